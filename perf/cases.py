@@ -3,7 +3,7 @@
 A case is a dict of plain values.  `listed()` are the fixed ones, `draw(rng)` makes another one of
 the same ranges, `prepare` builds what a program keeps (weights on the device, filled KV caches,
 recorded steps), `run` is one pass through the public entry points, `work` what that pass cannot do
-without, `tolerance` how far another correct implementation may be.
+without, `tolerance` how far another correct implementation may be, `exact` the results in 64 bits.
 
 Kinds:
   decode   tokens of a running conversation: Llama2.decode_greedy at batch 1, then the logits
@@ -23,6 +23,7 @@ from __future__ import annotations
 import math
 
 import numpy as np
+import torch
 
 import wgml_amd as W
 from wgml_amd import _lib
@@ -285,19 +286,27 @@ def _gpt2_weights(case, seed, p):
 
 # ---- prepare and run ----------------------------------------------------------------------------
 
+def _gpt2_params(case):
+    return Gpt2Params(case["vocab"], 1024, case["dim"], case["heads"], case["layers"], case["hidden"],
+                      3 * case["dim"])
+
+
+def _llama_config(case):
+    positions = case["pos"] + case["tokens"] + case["steps"] + 1
+    return Llama2Config(case["dim"], case["hidden"], case["layers"], case["heads"], case["kv_heads"],
+                        case["vocab"], max(512, (positions + 255) // 256 * 256), case["rope_base"], 1.0e-5)
+
+
 def prepare(case, seed):
     gpu = W.GpuInstance(0)
     tokens = W.rng_tokens(seed + 17, max(1, case["tokens"]), min(SUCCESSORS, case["vocab"]) - 1)
     state = {"case": case, "gpu": gpu, "tokens": tokens, "seed": seed}
     if case["kind"] == "gpt2":
-        p = Gpt2Params(case["vocab"], 1024, case["dim"], case["heads"], case["layers"], case["hidden"],
-                       3 * case["dim"])
+        p = _gpt2_params(case)
         state["model"] = Gpt2(gpu, p).load(_gpt2_weights(case, seed, p))
         state["model"].record_steps(case["tokens"] + case["steps"])
         return state
-    positions = case["pos"] + case["tokens"] + case["steps"] + 1
-    cfg = Llama2Config(case["dim"], case["hidden"], case["layers"], case["heads"], case["kv_heads"],
-                       case["vocab"], max(512, (positions + 255) // 256 * 256), case["rope_base"], 1.0e-5)
+    cfg = _llama_config(case)
     host, w = _llama_weights(case, seed, cfg)
     if case["kind"] == "ops":
         return _prepare_ops(state, cfg, host, w)
@@ -445,3 +454,162 @@ def tolerance(case):
         return {"rel": 4e-5, "max": 1.6e-4, "differ": 0.02}
     # every product takes its input as 16-bit block fixed point
     return {"rel": 1.5e-4, "max": 6e-4, "differ": 0.02}
+
+# ---- the same results in 64 bits -----------------------------------------------------------------
+
+def _device():
+    return torch.device("cuda" if torch.cuda.is_available() else "cpu")
+
+
+def _f64(a):
+    return torch.tensor(np.asarray(a), device=_device()).double()
+
+
+def _half(b, at):
+    return b[:, at:at + 2].contiguous().view(torch.float16).double()
+
+
+def _scales_k(b):  # the 6-bit scales and minima of Q4_K and Q5_K
+    lo, mid, hi = b[:, 4:8], b[:, 8:12], b[:, 12:16]
+    sc = torch.cat([lo & 63, (hi & 15) | ((lo >> 6) << 4)], 1)
+    mn = torch.cat([mid & 63, (hi >> 4) | ((mid >> 6) << 4)], 1)
+    return (_half(b, 0) * sc)[:, :, None], (_half(b, 2) * mn)[:, :, None]
+
+
+def _dequantize(m):
+    """The matrix that the blocks of a GGUF tensor stand for."""
+    b = torch.tensor(m.data, device=_device()).reshape(-1, _file_bytes(m.qtype, 256) if m.qtype not in (
+        _lib.Q8_0, _lib.Q4_0) else _file_bytes(m.qtype, 32))
+    n = len(b)
+    if m.qtype == _lib.F16:
+        v = b.view(torch.float16).double()
+    elif m.qtype == _lib.Q8_0:
+        v = _half(b, 0) * b[:, 2:].contiguous().view(torch.int8)
+    elif m.qtype == _lib.Q4_0:
+        v = _half(b, 0) * (torch.cat([b[:, 2:] & 15, b[:, 2:] >> 4], 1).double() - 8)
+    elif m.qtype in (_lib.Q4_K, _lib.Q5_K):
+        qs = b[:, -128:].reshape(n, 4, 1, 32)
+        q = torch.cat([qs & 15, qs >> 4], 2).reshape(n, 8, 32)
+        if m.qtype == _lib.Q5_K:
+            bit = torch.arange(8, dtype=torch.uint8, device=b.device).reshape(1, 8, 1)
+            q = q | (((b[:, None, 16:48] >> bit) & 1) << 4)
+        scale, low = _scales_k(b)
+        v = scale * q - low
+    else:
+        ql, qh = b[:, :128].reshape(n, 2, 2, 32), b[:, 128:192].reshape(n, 2, 1, 32)
+        shift = torch.arange(0, 8, 2, dtype=torch.uint8, device=b.device).reshape(1, 1, 4, 1)
+        q = torch.cat([ql & 15, ql >> 4], 2) | (((qh >> shift) & 3) << 4)
+        scale = _half(b, 208) * b[:, 192:208].contiguous().view(torch.int8)
+        v = (q.double() - 32).reshape(n, 16, 16) * scale[:, :, None]
+    return v.reshape(m.nrows, m.ncols)
+
+
+class _Exact:
+    """A decoder in plain torch and 64 bits: `forward` takes tokens at the next positions and gives
+    the last one's logits."""
+
+    def __init__(self, case, host, caches):
+        val = lambda v: _dequantize(v) if isinstance(v, HostMatrix) else _f64(v)  # noqa: E731
+        self.case, self.gpt2 = case, case["kind"] == "gpt2"
+        self.layers = [{k: val(v) for k, v in layer.items()} for layer in host.layers]
+        self.caches = caches
+        if self.gpt2:
+            self.embd, self.pos_embd, self.head = _f64(host.wte), _f64(host.wpe), _dequantize(host.lm_head)
+            self.last = (_f64(host.ln_f_g), _f64(host.ln_f_b))
+        else:
+            self.embd, self.head, self.last = _f64(host.token_embd), _dequantize(host.output), (_f64(host.output_norm),)
+
+    def _norm(self, x, gain, bias=None):
+        if bias is None:
+            return x / torch.sqrt((x * x).mean(1, keepdim=True) + 1.0e-5) * gain
+        x = x - x.mean(1, keepdim=True)
+        return x / torch.sqrt((x * x).mean(1, keepdim=True) + 1.0e-5) * gain + bias
+
+    def _rope(self, x, start):
+        size = self.case["dim"] // self.case["heads"]
+        angle = self.case["rope_base"] ** (-torch.arange(0, size, 2, device=x.device).double() / size)
+        angle = (start + torch.arange(len(x), device=x.device).double())[:, None, None] * angle
+        c, s = angle.cos(), angle.sin()
+        x = x.reshape(len(x), -1, size)
+        if self.case["qwen2"]:
+            a, b = x[..., :size // 2], x[..., size // 2:]
+            return torch.cat([c * a - s * b, s * a + c * b], 2).reshape(len(x), -1)
+        a, b = x[..., 0::2], x[..., 1::2]
+        return torch.stack([c * a - s * b, s * a + c * b], 3).reshape(len(x), -1)
+
+    def _attention(self, l, q, k, v):
+        n, heads = len(q), self.case["heads"]
+        size, groups = self.case["dim"] // heads, k.shape[1] // (self.case["dim"] // heads)
+        k, v = self.caches[l] = [torch.cat([old, new]) for old, new in zip(self.caches[l], (k, v))]
+        q = q.reshape(n, groups, heads // groups, size).permute(1, 2, 0, 3).reshape(groups, -1, size)
+        score = torch.matmul(q, k.reshape(-1, groups, size).permute(1, 2, 0).contiguous()) / math.sqrt(size)
+        seen = torch.arange(len(k), device=q.device) <= len(k) - n + torch.arange(n, device=q.device)[:, None]
+        score = score.reshape(groups, -1, n, len(k)).masked_fill(~seen, -math.inf).softmax(3)
+        out = torch.matmul(score.reshape(groups, -1, len(k)), v.reshape(-1, groups, size).permute(1, 0, 2).contiguous())
+        return out.reshape(heads, n, size).permute(1, 0, 2).reshape(n, -1)
+
+    def forward(self, tokens, pos):
+        x = self.embd[torch.tensor([int(t) for t in tokens], device=self.embd.device)]
+        if self.gpt2:
+            x = x + self.pos_embd[pos:pos + len(x)]
+        for l, w in enumerate(self.layers):
+            if self.gpt2:
+                qkv = self._norm(x, w["ln_1_g"], w["ln_1_b"]) @ w["attn_w"].T + w["attn_b"]
+                x = x + self._attention(l, *qkv.chunk(3, 1)) @ w["attn_proj_w"].T + w["attn_proj_b"]
+                h = self._norm(x, w["ln_2_g"], w["ln_2_b"]) @ w["mlp_fc_w"].T + w["mlp_fc_b"]
+                h = 0.5 * h * (1 + torch.tanh(math.sqrt(2 / math.pi) * (h + 0.044715 * h ** 3)))
+                x = x + h @ w["mlp_proj_w"].T + w["mlp_proj_b"]
+                continue
+            y = self._norm(x, w["attn_norm"])
+            q, k, v = (y @ w["attn_" + n].T + w.get("attn_%s_bias" % n, 0.0) for n in "qkv")
+            y = self._attention(l, self._rope(q, pos), self._rope(k, pos), v)
+            x = x + y @ w["attn_output"].T
+            y = self._norm(x, w["ffn_norm"])
+            x = x + (torch.nn.functional.silu(y @ w["ffn_gate"].T) * (y @ w["ffn_up"].T)) @ w["ffn_down"].T
+        return (self._norm(x[-1:], *self.last) @ self.head.T)[0].cpu().numpy()
+
+
+def _sample64(logits, temperature, topp, coin):
+    p = np.exp((logits - logits.max()) / temperature)
+    p /= p.sum()
+    order = np.argsort(-p, kind="stable")
+    total = np.cumsum(p[order])
+    last = int(np.searchsorted(total, topp, side="right"))  # the first that exceeds topp
+    return order[min(last, int(np.searchsorted(total, coin * total[last], side="right")))]
+
+
+def exact(case, seed):
+    """What `run` returns, from the same blocks and vectors."""
+    kind, pos, steps = case["kind"], case["pos"], case["steps"]
+    tokens = W.rng_tokens(seed + 17, max(1, case["tokens"]), min(SUCCESSORS, case["vocab"]) - 1)
+    if kind == "gpt2":
+        host, kv, caches = _gpt2_weights(case, seed, _gpt2_params(case)), case["dim"], None
+    else:
+        cfg = _llama_config(case)
+        host, w = _llama_weights(case, seed, cfg)
+        kv, caches = cfg.kv_dim, None
+        if pos:  # an operator program's caches are filled to their ends
+            n = (cfg.seq_len if kind == "ops" else pos) * kv
+            caches = [[_f64(w.normal(n)[:pos * kv].reshape(pos, kv)) for _ in range(2)] for _ in host.layers]
+    model = _Exact(case, host, caches or [[_f64(np.empty((0, kv)))] * 2 for _ in host.layers])
+    if kind == "ops":
+        logits = model.forward(tokens, pos)
+        return {"token": int(logits.argmax()), "logits": logits}
+    if kind == "prompt":
+        return {"logits": model.forward(tokens, pos)}
+    out, result = [], {}
+    if kind == "turn":
+        result["first"] = logits = model.forward(tokens, pos)
+        pos, token = pos + len(tokens), int(logits.argmax())
+    elif kind == "decode":
+        token = int(tokens[0])
+    else:  # the loops that step through their prompt
+        steps, token = len(tokens) + steps, int(tokens[0])
+        coins = W.rng_uniform(seed + 5, steps)
+    for i in range(steps):
+        logits = model.forward([token], pos + i)
+        best = int(logits.argmax()) if kind != "sampled" else int(_sample64(logits, 0.8, 0.9, coins[i]))
+        token = int(tokens[i + 1]) if kind in ("sampled", "gpt2") and i + 1 < len(tokens) else best
+        out.append(best)
+    result.update(tokens=np.array(out, np.uint32), logits=logits)
+    return result
