@@ -432,6 +432,51 @@ struct FmtQ5K {
     }
 };
 
+// ------------------------------------------------------------- dense f32 ----
+// Rows of a multiple of 16 floats (F32 tensors, and F16 ones, which are expanded when the matrix
+// is created).  A tile is 16 elements, 64 bytes: a wave's step covers 1024 columns and asks for
+// 4 KB, as the quantized formats do.  No sums of x are needed.  HBM-bound where tall (GPT-2's
+// 50257x768 output projection), launch-bound elsewhere: what it brings is the folded norms,
+// epilogues and Q/K/V launch, and with them the recorded step -- GPT-2 124M from an F16 file
+// 331 us per token, 625 with a launch per operation and gemv_f32_kernel.
+struct FmtF32 {
+    static constexpr int TILE = 16;
+    static constexpr int CHUNKS = 4;
+    static constexpr int NSUM = 0;
+    struct Row {
+        float4 a[4];
+    };
+    struct RowBase {
+        const float4 *row;
+    };
+    __device__ static RowBase row_base(const GemvParams &p, uint32_t row) {
+        return {reinterpret_cast<const float4 *>(p.p0) + (size_t)row * (p.ncols / 4)};
+    }
+    __device__ static void map(uint32_t g, uint32_t &tile, uint32_t &chunk) {
+        tile = g >> 2;
+        chunk = g & 3;
+    }
+    __device__ static void load(Row &w, const RowBase &rb, uint32_t tile) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) w.a[c] = rb.row[(size_t)tile * 4 + c];
+    }
+    template <int R>
+    __device__ static void accumulate(const Row (&w)[R], const float4 *xl, const float *, uint32_t,
+                                      float (&acc)[R]) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const float4 xv = xl[c * 64];
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                acc[r] = fmaf(w[r].a[c].x, xv.x, acc[r]);
+                acc[r] = fmaf(w[r].a[c].y, xv.y, acc[r]);
+                acc[r] = fmaf(w[r].a[c].z, xv.z, acc[r]);
+                acc[r] = fmaf(w[r].a[c].w, xv.w, acc[r]);
+            }
+        }
+    }
+};
+
 // LDS layout: x as float4 xs[step][chunk][lane]; then sums[sum][tile_padded].
 template <class F>
 __device__ __forceinline__ uint32_t lds_slot(uint32_t tile, uint32_t chunk) {
@@ -832,7 +877,8 @@ struct FFmt {
     using W = WFmt;
     static constexpr bool F32X = true;
     static constexpr int TILE = WFmt::TILE, CHUNKS = WFmt::CHUNKS, NSUM = WFmt::NSUM;
-    static constexpr int XB = WFmt::TILE / WFmt::NSUM, NXB = 0;  // elements per sum of x
+    // elements per sum of x
+    static constexpr int XB = WFmt::NSUM ? WFmt::TILE / (WFmt::NSUM ? WFmt::NSUM : 1) : WFmt::TILE, NXB = 0;
     struct X {};
 };
 
@@ -1462,6 +1508,9 @@ template <> struct FusedFmt<WGML_Q8_0, false> { using T = IFmtQ8_0; };
 template <> struct FusedFmt<WGML_Q4_K, true> { using T = FFmt<FmtQ4K>; };
 template <> struct FusedFmt<WGML_Q6_K, true> { using T = FFmt<FmtQ6K>; };
 template <> struct FusedFmt<WGML_Q8_0, true> { using T = FFmt<FmtQ8_0>; };
+// (WGML_F32 is 0, which as FMT stands for mixed formats)
+constexpr int kFusedDenseF32 = 1000;
+template <> struct FusedFmt<kFusedDenseF32, true> { using T = FFmt<FmtF32>; };
 template <> struct FusedFmt<WGML_Q5_K, false> { using T = IFmtQ5K; };
 template <> struct FusedFmt<WGML_Q8_K, false> { using T = IFmtQ8K; };
 template <> struct FusedFmt<WGML_Q4_0, false> { using T = IFmtQ4_0; };
@@ -1501,7 +1550,9 @@ __global__ __launch_bounds__(MAXT, MINW) void gemv_fused_kernel(const FusedParam
 }
 
 // ------------------------------------------------------------- dense f32 ----
-// out = A v, A row-major f32 (p.p0).  One wave per row, float4 loads, x from LDS.
+// out = A v, A row-major f32 (p.p0).  One wave per row, float4 loads, x from LDS.  For what the
+// shared body does not take: f32 tensors as operator arguments (any width and alignment) and
+// matrices whose rows are not a multiple of 16 floats.
 __global__ __launch_bounds__(256) void gemv_f32_kernel(const GemvParams p, int vec4) {
     extern __shared__ float4 smem[];
     __shared__ float red[16];
@@ -1707,12 +1758,17 @@ int launch_fmt_f32(wgml_ctx *ctx, const GemvParams &p) {
         return set_error(WGML_E_UNSUPPORTED,
                          "gemv_quant: %u columns need %zu bytes of LDS (limit %zu)", p.ncols, lds,
                          kMaxLds);
-    if (p.part_n) return launch_variant_i8<F, 1, 1, 1024, 4, true>(ctx, p, lds);
-    const int waves = ctx->tuning[WGML_TUNE_GEMV_WAVES_PER_WG];
+    if constexpr (!std::is_same_v<WF, FmtF32>) {
+        if (p.part_n) return launch_variant_i8<F, 1, 1, 1024, 4, true>(ctx, p, lds);
+    }
+    // (the workgroup size is selectable for the quantized formats only)
+    const int waves = std::is_same_v<WF, FmtF32> ? 16 : ctx->tuning[WGML_TUNE_GEMV_WAVES_PER_WG];
     if (p.ln_g && (p.ncols >> 2) > 3u * (waves == 8 ? 512u : 1024u))  // XP float4 per thread
         return set_error(WGML_E_UNSUPPORTED, "gemv_quant: %u columns are too many for the folded "
                                              "LayerNorm", p.ncols);
-    if (waves == 8) return launch_variant_i8<F, 1, 2, 512, 2>(ctx, p, lds);
+    if constexpr (!std::is_same_v<WF, FmtF32>) {
+        if (waves == 8) return launch_variant_i8<F, 1, 2, 512, 2>(ctx, p, lds);
+    }
     return launch_variant_i8<F, 1, 1, 1024, 4>(ctx, p, lds);
 }
 
@@ -1743,6 +1799,11 @@ int launch_gemv_f32(wgml_ctx *ctx, float *out, const float *a, uint32_t nrows, u
     WGML_CHECK_LAUNCH();
     ctx->launches++;
     return WGML_OK;
+}
+
+// Dense f32 matrices that run in the shared body: whole tiles, and x within the LDS limit.
+static bool dense_f32_in_shared_body(const wgml_qmat *m) {
+    return m->type == WGML_F32 && m->ncols % FmtF32::TILE == 0 && (size_t)m->ncols * 4 <= kMaxLds;
 }
 
 bool gemv_partials_supported(const wgml_ctx *, const wgml_qmat *m) {
@@ -1788,9 +1849,10 @@ int launch_gemv_quant(wgml_ctx *ctx, float *out, const wgml_qmat *m, const float
         return set_error(WGML_E_INVALID, "gemv_quant: the input vector must be 16-byte aligned");
     }
     (void)main_fmt;
+    if (m->type == WGML_F32 && dense_f32_in_shared_body(m)) return launch_fmt_f32<FmtF32>(ctx, p);
     if ((p.ln_g || p.act) && m->type == WGML_F32)
-        return set_error(WGML_E_UNSUPPORTED,
-                         "gemv_quant: LayerNorm / activation folding needs a quantized matrix");
+        return set_error(WGML_E_UNSUPPORTED, "gemv_quant: LayerNorm / activation folding needs rows of a "
+                                             "multiple of 16 elements");
     if (m->type == WGML_F32) {
         const size_t lds = (size_t)m->ncols * 4;
         if (lds > kMaxLds)
@@ -1839,6 +1901,7 @@ static size_t lds_bytes_of(uint32_t ncols) {
 }
 static size_t lds_bytes_fused(int type, uint32_t ncols, bool f32) {
     switch (type) {
+    case WGML_F32: return lds_bytes_of<FFmt<FmtF32>>(ncols);
     case WGML_Q4_K: return f32 ? lds_bytes_of<FFmt<FmtQ4K>>(ncols) : lds_bytes_of<IFmtQ4K>(ncols);
     case WGML_Q6_K: return f32 ? lds_bytes_of<FFmt<FmtQ6K>>(ncols) : lds_bytes_of<IFmtQ6K>(ncols);
     case WGML_Q8_0: return f32 ? lds_bytes_of<FFmt<FmtQ8_0>>(ncols) : lds_bytes_of<IFmtQ8_0>(ncols);
@@ -1853,14 +1916,15 @@ static bool main_format(int type) { return type == WGML_Q4_K || type == WGML_Q6_
 bool gemv_fused_supported(const wgml_qmat *m) {
     if (!m) return false;
     switch (m->type) {
+    case WGML_F32: return dense_f32_in_shared_body(m);
     case WGML_Q4_K: case WGML_Q6_K: case WGML_Q8_0: case WGML_Q5_K: case WGML_Q8_K: case WGML_Q4_0:
     case WGML_Q4_1: case WGML_Q5_0: case WGML_Q5_1: return true;
     default: return false;
     }
 }
 
-// One launch takes matrices of one format (any of the nine), or a mix of Q4_K / Q6_K / Q8_0; with
-// fp32 activations only those three.
+// One launch takes matrices of one format (any of the nine, or dense f32), or a mix of Q4_K / Q6_K
+// / Q8_0; with fp32 activations only those three, or dense f32.
 bool gemv_fused_set_supported(const wgml_ctx *ctx, const wgml_qmat *const *mats, int n) {
     bool same = true, all_main = true;
     for (int i = 0; i < n; ++i) {
@@ -1868,7 +1932,7 @@ bool gemv_fused_set_supported(const wgml_ctx *ctx, const wgml_qmat *const *mats,
         same = same && mats[i]->type == mats[0]->type;
         all_main = all_main && main_format(mats[i]->type);
     }
-    if (ctx->tuning[WGML_TUNE_GEMV_F32_ACTIVATIONS]) return all_main;
+    if (ctx->tuning[WGML_TUNE_GEMV_F32_ACTIVATIONS]) return all_main || (same && mats[0]->type == WGML_F32);
     return same || all_main;
 }
 
@@ -1900,7 +1964,7 @@ static int launch_gemv_fused_variant(wgml_ctx *ctx, const FusedGemv &f, uint32_t
         const FusedGemvJob &s = f.jobs[i];
         if (!gemv_fused_supported(s.a) || s.a->ncols != ncols)
             return set_error(WGML_E_INVALID, "gemv_fused: job %d has an unsupported matrix", i);
-        if (f32 && !main_format(s.a->type))
+        if (f32 && !main_format(s.a->type) && s.a->type != WGML_F32)
             return set_error(WGML_E_UNSUPPORTED, "gemv_fused: fp32 activations exist for Q4_K, Q6_K "
                                                  "and Q8_0 only");
         GemvJob &j = P.jobs[i];
@@ -1914,6 +1978,7 @@ static int launch_gemv_fused_variant(wgml_ctx *ctx, const FusedGemv &f, uint32_t
                 return set_error(WGML_E_INVALID, "gemv_fused: job %d: bad row slice", i);
             const uint64_t r = s.row0, nb = r * (ncols / 256), nb32 = r * (ncols / 32);
             switch (s.a->type) {
+            case WGML_F32: j.a0 += r * ncols * 4; break;
             case WGML_Q4_K: j.a0 += nb * 144; break;
             case WGML_Q5_K: j.a0 += nb * 176; break;
             case WGML_Q8_K: j.a0 += nb * 292; break;
@@ -1952,9 +2017,9 @@ static int launch_gemv_fused_variant(wgml_ctx *ctx, const FusedGemv &f, uint32_t
         return set_error(WGML_E_UNSUPPORTED,
                          "gemv_fused: %u columns are too many for the folded LayerNorm", ncols);
     // one kernel per format when all matrices share it, else the mixed one
-    int fmt = P.jobs[0].type, slot = 0;
+    int fmt = P.jobs[0].type == WGML_F32 ? kFusedDenseF32 : P.jobs[0].type;
     for (int i = 1; i < f.njobs; ++i)
-        if (P.jobs[i].type != fmt) fmt = 0;
+        if (P.jobs[i].type != P.jobs[0].type) fmt = 0;
     if (fmt == 0)
         for (int i = 0; i < f.njobs; ++i)
             if (!main_format(P.jobs[i].type))
@@ -1963,8 +2028,9 @@ static int launch_gemv_fused_variant(wgml_ctx *ctx, const FusedGemv &f, uint32_t
     // the mixed-format kernel is held to 96 registers (5 waves per SIMD): it fits without
     // spilling, and the waves of a workgroup start sooner the fewer registers they take
     void (*kern)(const FusedParams) = gemv_fused_kernel<D, MAXT, (MAXT == 1024 ? 5 : MINW), 0>;
-    (void)slot;
-    if (f32) {
+    if (fmt == kFusedDenseF32) {
+        kern = gemv_fused_kernel<D, MAXT, MINW, kFusedDenseF32, true>;
+    } else if (f32) {
         kern = gemv_fused_kernel<D, MAXT, MINW, 0, true>;
         switch (fmt) {
         case WGML_Q4_K: kern = gemv_fused_kernel<D, MAXT, MINW, WGML_Q4_K, true>; break;

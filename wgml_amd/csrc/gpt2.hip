@@ -230,8 +230,10 @@ namespace {
 // v are row slices of the one attn_w matrix, k and v written straight into their
 // cache columns (:329-353 copies them).  fusion 0 keeps layernorm, GELU and the
 // cache copies as launches of their own.
-// The folded launches exist for the quantized formats only.
+// The folded launches exist for the quantized formats and for dense f32 rows of whole tiles, and
+// the folded LayerNorm holds its row in registers (12 elements per thread).
 bool can_fold(const wgml_gpt2 *m) {
+    if (m->p.n_embd > 12u * 1024u) return false;
     if (!gemv_fused_supported(m->lm_head)) return false;
     for (const Gpt2Layer &w : m->layers)
         if (!gemv_fused_supported(w.attn_w) || !gemv_fused_supported(w.proj_w) ||

@@ -479,7 +479,7 @@ int run_recorded(wgml_llama2 *m, uint32_t first_token, uint32_t start_pos, uint3
 
 // The batched products take these formats, and weights that fit their f16 operands.
 bool gemm_supported(const wgml_qmat *q) {
-    return gemv_fused_supported(q) && q->max_abs <= kGemmMaxWeight;  // the nine quantized formats
+    return q->type != WGML_F32 && gemv_fused_supported(q) && q->max_abs <= kGemmMaxWeight;  // the nine quantized formats
 }
 
 // One run of T <= kPrefillMaxTokens prompt tokens at positions pos0 .. pos0 + T - 1: the
