@@ -364,7 +364,7 @@ WGML_API int wgml_llama2_decode_greedy_sync(wgml_llama2 *m, uint32_t first_token
  * start_pos + n_tokens - 1 of every layer and the logits of the last token (read
  * them with wgml_llama2_read_logits) -- with every matrix-vector product of the
  * step replaced by one product with up to 128 token vectors on the matrix cores
- * (wgml_gemm_quant; longer prompts go through in runs of 128).  The layer matrices
+ * (as wgml_gemm_quant; longer prompts go through in runs of up to 1024).  The layer matrices
  * are multiplied at the precision set with wgml_ctx_set_gemm_precision (default:
  * to fp32 rounding); norms, RoPE, attention and the output matrix are fp32 as in
  * the step, so with the default the logits agree with the step-by-step pass as two

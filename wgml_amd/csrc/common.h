@@ -300,8 +300,9 @@ int launch_argmax_next(wgml_ctx *ctx, const float *v, uint32_t n, DynState *dyn,
 int launch_dequantize(wgml_ctx *ctx, float *out, const wgml_qmat *m);
 
 // ---- batched products for prompt processing (prefill.hip) ---------------------
-constexpr uint32_t kPrefillMaxTokens = 128;
-uint32_t prefill_tpad(uint32_t T);  // tokens rounded up to 16, 32, 64 or 128
+constexpr uint32_t kPrefillMaxTokens = 128;  // of one product through the public entry point
+constexpr uint32_t kPrefillMaxRun = 1024;    // of one run of a prompt pass (more than 128: wider tiles)
+uint32_t prefill_tpad(uint32_t T);  // tokens rounded up to 16, 32, 64, 128 or a multiple of 256
 uint32_t prefill_kpad(uint32_t K);  // columns rounded up to a multiple of 128
 int ensure_prefill_scratch(wgml_ctx *ctx, size_t xh_bytes);
 // xh[tpad][kpad] (f16) <- x[T][K] (f32, rows x_stride apart): RMS-normalised with

@@ -56,6 +56,7 @@ struct wgml_llama2 {
     // state of the batched prompt pass, allocated at its first use: one row per token
     // of a run (up to kPrefillMaxTokens)
     float *pf_x = nullptr, *pf_xb = nullptr, *pf_q = nullptr, *pf_hb = nullptr, *pf_hb2 = nullptr;
+    uint32_t pf_rows = 0;  // tokens the pf_ buffers hold
     uint32_t *pf_tokens = nullptr;
     std::vector<void *> allocs;
     uint64_t launches_last = 0;   // launches of the last step that ran
@@ -482,7 +483,17 @@ bool gemm_supported(const wgml_qmat *q) {
     return q->type != WGML_F32 && gemv_fused_supported(q) && q->max_abs <= kGemmMaxWeight;  // the nine quantized formats
 }
 
-// One run of T <= kPrefillMaxTokens prompt tokens at positions pos0 .. pos0 + T - 1: the
+// Tokens of the next run of a prompt pass with `left` tokens to go.  Runs of more than 128 tokens
+// multiply in tiles of 256: the rest of a prompt beyond whole tiles goes into the same run if it
+// fills more than half a tile, and into a run of its own otherwise.
+uint32_t prefill_run_length(uint32_t left, uint32_t max_run) {
+    if (left >= max_run) return max_run;
+    if (left <= kPrefillMaxTokens) return left;
+    const uint32_t rest = left % 256;
+    return rest > kPrefillMaxTokens ? left : left - rest;
+}
+
+// One run of T <= kPrefillMaxRun prompt tokens at positions pos0 .. pos0 + T - 1: the
 // launches of enqueue_step with every matrix-vector product replaced by a product
 // with the T vectors at once.  Leaves the last token's residual stream in m->x.
 int enqueue_prefill_run(wgml_llama2 *m, const uint32_t *tokens, uint32_t T, uint32_t pos0) {
@@ -765,27 +776,43 @@ int wgml_llama2_prefill(wgml_llama2 *m, const uint32_t *tokens, uint32_t n_token
         m->launches_last = ctx->launches - launches0;
         return WGML_OK;
     }
-    if (!m->pf_x) {
-        int rc = WGML_OK;
-        auto A = [&](float **p, uint64_t n) {
-            if (rc == WGML_OK) rc = dev_alloc(m, p, n, false);
-        };
-        A(&m->pf_xb, (uint64_t)kPrefillMaxTokens * c.dim);
-        A(&m->pf_q, (uint64_t)kPrefillMaxTokens * c.dim);
-        A(&m->pf_hb, (uint64_t)kPrefillMaxTokens * c.hidden_dim);
-        A(&m->pf_hb2, (uint64_t)kPrefillMaxTokens * c.hidden_dim);
-        if (rc == WGML_OK) rc = dev_alloc_bytes(m, (void **)&m->pf_tokens, kPrefillMaxTokens * 4, false);
-        A(&m->pf_x, (uint64_t)kPrefillMaxTokens * c.dim);  // last: marks the set as complete
-        WGML_TRY(rc);
-    }
     const uint32_t kmax = c.dim > c.hidden_dim ? c.dim : c.hidden_dim;
-    WGML_TRY(ensure_prefill_scratch(ctx, (size_t)kPrefillMaxTokens * prefill_kpad(kmax) * 2));
+    // Workspaces for runs of up to `rows` tokens; a smaller set that queued work may still read
+    // stays with the model (there are two sizes).
+    auto reserve = [&](uint32_t rows) -> int {
+        if (m->pf_rows < rows) {
+            int rc = WGML_OK;
+            auto A = [&](float **p, uint64_t n) {
+                if (rc == WGML_OK) rc = dev_alloc(m, p, n, false);
+            };
+            m->pf_rows = 0;
+            A(&m->pf_xb, (uint64_t)rows * c.dim);
+            A(&m->pf_q, (uint64_t)rows * c.dim);
+            A(&m->pf_hb, (uint64_t)rows * c.hidden_dim);
+            A(&m->pf_hb2, (uint64_t)rows * c.hidden_dim);
+            if (rc == WGML_OK) rc = dev_alloc_bytes(m, (void **)&m->pf_tokens, rows * 4, false);
+            A(&m->pf_x, (uint64_t)rows * c.dim);
+            WGML_TRY(rc);
+            m->pf_rows = rows;
+        }
+        return ensure_prefill_scratch(ctx, (size_t)prefill_tpad(rows) * prefill_kpad(kmax) * 2);
+    };
     const uint64_t launches0 = ctx->launches;
-    ctx->gemm_pending_ks = 0;  // nothing is owed from an earlier call that failed half way
-    ctx->gemm_pending_pair = 0;
-    for (uint32_t done = 0; done < n_tokens; done += kPrefillMaxTokens) {
-        const uint32_t T = n_tokens - done < kPrefillMaxTokens ? n_tokens - done : kPrefillMaxTokens;
-        WGML_TRY(enqueue_prefill_run(m, tokens + done, T, start_pos + done));
+    uint32_t max_run = kPrefillMaxRun;
+    for (uint32_t done = 0; done < n_tokens;) {
+        const uint32_t T = prefill_run_length(n_tokens - done, max_run);
+        ctx->gemm_pending_ks = 0;  // nothing is owed from an earlier run that failed half way
+        ctx->gemm_pending_pair = 0;
+        int rc = reserve(T > kPrefillMaxTokens ? kPrefillMaxRun : kPrefillMaxTokens);
+        if (rc == WGML_OK) rc = enqueue_prefill_run(m, tokens + done, T, start_pos + done);
+        if (rc != WGML_OK && T > kPrefillMaxTokens) {
+            // no memory for the workspaces of a long run: short runs leave the same state
+            (void)hipGetLastError();
+            max_run = kPrefillMaxTokens;
+            continue;
+        }
+        WGML_TRY(rc);
+        done += T;
     }
     // logits of the last token, as a decode step ends (final norm folded into the product)
     GemvEpilogue eo;
