@@ -275,6 +275,8 @@ int launch_silu(wgml_ctx *ctx, float *h1, const float *h2, uint32_t n);
 int launch_unary(wgml_ctx *ctx, int op, float *x, uint32_t n, const float *args4);
 int launch_op_assign(wgml_ctx *ctx, int op, float *a, const float *b, uint32_t n);
 int launch_argmax(wgml_ctx *ctx, const float *v, uint32_t n, uint32_t *d_out);
+// d_out[t] = first index of the maximum of v[t * n .. t * n + n - 1]
+int launch_argmax_rows(wgml_ctx *ctx, const float *v, uint32_t n, uint32_t rows, uint32_t *d_out);
 // Token-loop state on the device: {pos, token, n_generated, n_prompt}.
 struct DynState {
     uint32_t pos, token, count, n_prompt;
@@ -308,10 +310,11 @@ int ensure_prefill_scratch(wgml_ctx *ctx, size_t xh_bytes);
 // xh[tpad][kpad] (f16) <- x[T][K] (f32, rows x_stride apart): RMS-normalised with
 // norm_w first when that is non-null; replaced by up[t][k] * silu(x[t][k]) when `up`
 // is non-null.  xscale[tpad] receives what a token's products must be multiplied with.
+// With ln_beta the norm is LayerNorm (gamma = norm_w); with gelu the input is gelu(x).
 // If the product before left partial sums for x (defer_reduce), they are added to x first.
 int launch_prefill_prep(wgml_ctx *ctx, float *x, uint32_t x_stride, const float *up,
                         const float *norm_w, float eps, void *xh, float *xscale, uint32_t K,
-                        uint32_t T);
+                        uint32_t T, const float *ln_beta = nullptr, int gelu = 0);
 // Adds partial sums left for x by a product with defer_reduce (no-op if there are none).
 int launch_gemm_flush(wgml_ctx *ctx, float *x, uint32_t x_stride, const float *xscale, uint32_t K,
                       uint32_t T);
@@ -352,7 +355,11 @@ int launch_gemm_quant_multi(wgml_ctx *ctx, const GemmTarget *targets, int n, con
                             const float *xscale, uint32_t T, int accumulate,
                             bool defer_reduce = false, GemmRope *rope = nullptr);
 int launch_embed_rows(wgml_ctx *ctx, float *x, const float *table, const uint32_t *d_tokens,
-                      uint32_t dim, uint32_t T);
+                      uint32_t dim, uint32_t T, const float *pos_table = nullptr, uint32_t pos0 = 0);
+// k and v of T rows of (q, k, v), each n wide, to T cache rows (n a multiple of 4)
+int launch_cache_rows(wgml_ctx *ctx, const float *qkv, float *k, float *v, uint32_t n, uint32_t T);
+// The batched products take these formats, and weights that fit their f16 operands.
+bool gemm_supported(const wgml_qmat *q);
 // q (q_len wide) and k (kv_dim wide) of T tokens rotated in place; either may be null
 int launch_rope_rows(wgml_ctx *ctx, int variant, uint32_t head_size, uint32_t kv_dim, uint32_t pos0,
                      float base_freq, float *q, uint32_t q_len, uint32_t q_stride, float *k,

@@ -478,11 +478,6 @@ int run_recorded(wgml_llama2 *m, uint32_t first_token, uint32_t start_pos, uint3
     return WGML_OK;
 }
 
-// The batched products take these formats, and weights that fit their f16 operands.
-bool gemm_supported(const wgml_qmat *q) {
-    return q->type != WGML_F32 && gemv_fused_supported(q) && q->max_abs <= kGemmMaxWeight;  // the nine quantized formats
-}
-
 // Tokens of the next run of a prompt pass with `left` tokens to go.  Runs of more than 128 tokens
 // multiply in tiles of 256: the rest of a prompt beyond whole tiles goes into the same run if it
 // fills more than half a tile, and into a run of its own otherwise.

@@ -209,8 +209,8 @@ __device__ __forceinline__ uint32_t block_argmax(const float *__restrict__ v, ui
 
 __global__ __launch_bounds__(1024) void argmax_kernel(const float *__restrict__ v, uint32_t n,
                                                       uint32_t *__restrict__ out) {
-    const uint32_t idx = block_argmax(v, n);
-    if (threadIdx.x == 0) out[0] = idx;
+    const uint32_t idx = block_argmax(v + (size_t)blockIdx.x * n, n);
+    if (threadIdx.x == 0) out[blockIdx.x] = idx;
 }
 
 // Greedy sampling + the token loop's bookkeeping on the device
@@ -356,7 +356,11 @@ int launch_op_assign(wgml_ctx *ctx, int op, float *a, const float *b, uint32_t n
 }
 
 int launch_argmax(wgml_ctx *ctx, const float *v, uint32_t n, uint32_t *d_out) {
-    argmax_kernel<<<dim3(1), dim3(1024), 0, ctx->stream>>>(v, n, d_out);
+    return launch_argmax_rows(ctx, v, n, 1, d_out);
+}
+
+int launch_argmax_rows(wgml_ctx *ctx, const float *v, uint32_t n, uint32_t rows, uint32_t *d_out) {
+    argmax_kernel<<<dim3(rows), dim3(1024), 0, ctx->stream>>>(v, n, d_out);
     WGML_CHECK_LAUNCH();
     ctx->launches++;
     return WGML_OK;

@@ -1045,6 +1045,7 @@ __global__ __launch_bounds__(PREP_THREADS) void prep_x_kernel(float *__restrict_
                                                      uint32_t part_pair,
                                                      const float *__restrict__ up,
                                                      const float *__restrict__ norm_w, float eps,
+                                                     const float *__restrict__ ln_beta, int gelu,
                                                      uint4 *__restrict__ xh, uint4 *__restrict__ xl,
                                                      float *__restrict__ xscale, uint32_t K,
                                                      uint32_t kpad, uint32_t T) {
@@ -1091,6 +1092,7 @@ __global__ __launch_bounds__(PREP_THREADS) void prep_x_kernel(float *__restrict_
     auto raw = [&](uint32_t k) -> float {  // the value before normalisation
         if (k >= K) return 0.f;
         const float xv = xr[k];
+        if (gelu) return gelu_tanh(xv);
         return ur ? ur[k] * (xv / (1.0f + expf(-xv))) : xv;
     };
     if (cached) {
@@ -1132,13 +1134,30 @@ __global__ __launch_bounds__(PREP_THREADS) void prep_x_kernel(float *__restrict_
                     for (int e = 0; e < 8; ++e) v[i][e] = uv[e] * (xv[e] / (1.0f + expf(-xv[e])));
                 } else {
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) v[i][e] = xv[e];
+                    for (int e = 0; e < 8; ++e) v[i][e] = gelu ? gelu_tanh(xv[e]) : xv[e];
                 }
             }
         }
     }
-    float rs = 1.f;
-    if (norm_w) {
+    float rs = 1.f, mean = 0.f;
+    if (ln_beta) {  // LayerNorm, in registers only (the launcher sees to that)
+        float sum = 0.f;
+#pragma unroll
+        for (int i = 0; i < PREP_GROUPS; ++i) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) sum += v[i][e];
+        }
+        mean = block_sum(sum, red) / (float)K;
+        float ss = 0.f;
+#pragma unroll
+        for (int i = 0; i < PREP_GROUPS; ++i) {
+            if (8 * (tid + i * PREP_THREADS) < K) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) ss = fmaf(v[i][e] - mean, v[i][e] - mean, ss);
+            }
+        }
+        rs = 1.0f / sqrtf(block_sum(ss, red) / (float)K + eps);
+    } else if (norm_w) {
         float ss = 0.f;
         if (cached) {
 #pragma unroll
@@ -1151,7 +1170,10 @@ __global__ __launch_bounds__(PREP_THREADS) void prep_x_kernel(float *__restrict_
         }
         rs = 1.0f / sqrtf(block_sum(ss, red) / (float)K + eps);
     }
-    auto value = [&](uint32_t k, float r) { return norm_w && k < K ? (r * rs) * norm_w[k] : r; };
+    auto value = [&](uint32_t k, float r) {
+        if (ln_beta && k < K) return ((r - mean) * rs) * norm_w[k] + ln_beta[k];
+        return norm_w && k < K ? (r * rs) * norm_w[k] : r;
+    };
     float amax = 0.f;
     if (cached) {
 #pragma unroll
@@ -1211,10 +1233,24 @@ __global__ __launch_bounds__(PREP_THREADS) void prep_x_kernel(float *__restrict_
 }
 
 // X[t] = table[tokens[t]]  (embedding rows of the prompt tokens)
+// pos_table (GPT-2's learned positions): the row of position pos0 + t is added.
 __global__ void embed_rows_kernel(float *__restrict__ x, const float *__restrict__ table,
-                                  const uint32_t *__restrict__ tokens, uint32_t dim) {
+                                  const uint32_t *__restrict__ tokens, uint32_t dim,
+                                  const float *__restrict__ pos_table, uint32_t pos0) {
     const uint32_t t = blockIdx.y, i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < dim) x[(size_t)t * dim + i] = table[(size_t)tokens[t] * dim + i];
+    if (i >= dim) return;
+    float v = table[(size_t)tokens[t] * dim + i];
+    if (pos_table) v += pos_table[(size_t)(pos0 + t) * dim + i];
+    x[(size_t)t * dim + i] = v;
+}
+
+// Rows of q, k and v side by side (3 n wide, n a multiple of 4): k and v of token t to its cache rows.
+__global__ void cache_rows_kernel(const float *__restrict__ qkv, float *__restrict__ k, float *__restrict__ v,
+                                  uint32_t n) {
+    const uint32_t t = blockIdx.y, i = (blockIdx.x * blockDim.x + threadIdx.x) * 4;
+    if (i >= 2 * n) return;
+    const float4 w = *reinterpret_cast<const float4 *>(qkv + (size_t)t * 3 * n + n + i);
+    *reinterpret_cast<float4 *>((i < n ? k + i : v + (i - n)) + (size_t)t * n) = w;
 }
 
 // RoPE of q[t] and of the K-cache row of position pos0 + t, for every token t
@@ -1597,6 +1633,10 @@ uint32_t prefill_tpad(uint32_t T) {
 }
 uint32_t prefill_kpad(uint32_t K) { return (K + 2 * KC - 1) / (2 * KC) * (2 * KC); }
 
+bool gemm_supported(const wgml_qmat *q) {
+    return q->type != WGML_F32 && gemv_fused_supported(q) && q->max_abs <= kGemmMaxWeight;  // the nine quantized formats
+}
+
 int ensure_prefill_scratch(wgml_ctx *ctx, size_t xh_bytes) {
     if (!ctx->prefill_xscale)
         WGML_CHECK_HIP(hipMalloc((void **)&ctx->prefill_xscale, kPrefillMaxRun * sizeof(float)));
@@ -1615,7 +1655,11 @@ int ensure_prefill_scratch(wgml_ctx *ctx, size_t xh_bytes) {
 
 int launch_prefill_prep(wgml_ctx *ctx, float *x, uint32_t x_stride, const float *up,
                         const float *norm_w, float eps, void *xh, float *xscale, uint32_t K,
-                        uint32_t T) {
+                        uint32_t T, const float *ln_beta, int gelu) {
+    if (ln_beta && !(norm_w && !up && K % 8 == 0 && x_stride % 4 == 0 &&
+                     prefill_kpad(K) / 8 <= (uint32_t)(PREP_GROUPS * PREP_THREADS) &&
+                     (reinterpret_cast<uintptr_t>(x) & 15u) == 0))
+        return set_error(WGML_E_UNSUPPORTED, "prefill_prep: LayerNorm of rows of %u columns", K);
     // partial sums a product with defer_reduce left: for x (K wide; x is its output), or for a
     // gate / up pair (2 K wide; x and up are then not read)
     const uint32_t pending = ctx->gemm_pending_ks, pair = ctx->gemm_pending_pair;
@@ -1628,7 +1672,7 @@ int launch_prefill_prep(wgml_ctx *ctx, float *x, uint32_t x_stride, const float 
                                          "most %d columns", 8 * PREP_GROUPS * PREP_THREADS);
     prep_x_kernel<<<dim3(prefill_tpad(T)), dim3(PREP_THREADS), 0, ctx->stream>>>(
         x, x_stride, pending ? ctx->gemm_part : nullptr, pending, pair, up, norm_w, eps,
-        reinterpret_cast<uint4 *>(xh), ctx->gemm_precise ? reinterpret_cast<uint4 *>(ctx->prefill_xl) : nullptr,
+        ln_beta, gelu, reinterpret_cast<uint4 *>(xh), ctx->gemm_precise ? reinterpret_cast<uint4 *>(ctx->prefill_xl) : nullptr,
         xscale, K, prefill_kpad(K), T);
     WGML_CHECK_LAUNCH();
     ctx->launches++;
@@ -1784,9 +1828,16 @@ int launch_gemm_quant(wgml_ctx *ctx, float *out, uint32_t out_stride, const wgml
 }
 
 int launch_embed_rows(wgml_ctx *ctx, float *x, const float *table, const uint32_t *d_tokens,
-                      uint32_t dim, uint32_t T) {
-    embed_rows_kernel<<<dim3((dim + 255) / 256, T), dim3(256), 0, ctx->stream>>>(x, table, d_tokens,
-                                                                                 dim);
+                      uint32_t dim, uint32_t T, const float *pos_table, uint32_t pos0) {
+    embed_rows_kernel<<<dim3((dim + 255) / 256, T), dim3(256), 0, ctx->stream>>>(x, table, d_tokens, dim,
+                                                                                 pos_table, pos0);
+    WGML_CHECK_LAUNCH();
+    ctx->launches++;
+    return WGML_OK;
+}
+
+int launch_cache_rows(wgml_ctx *ctx, const float *qkv, float *k, float *v, uint32_t n, uint32_t T) {
+    cache_rows_kernel<<<dim3((n / 2 + 255) / 256, T), dim3(256), 0, ctx->stream>>>(qkv, k, v, n);
     WGML_CHECK_LAUNCH();
     ctx->launches++;
     return WGML_OK;
