@@ -56,6 +56,9 @@ struct wgml_llama2 {
     // state of the batched prompt pass, allocated at its first use: one row per token
     // of a run (up to kPrefillMaxTokens)
     float *pf_x = nullptr, *pf_xb = nullptr, *pf_q = nullptr, *pf_hb = nullptr, *pf_hb2 = nullptr;
+    float *h_logits = nullptr;  // pinned host memory for logits (generate_sampled)
+    size_t h_logits_n = 0;
+    float *pf_logits = nullptr;  // of every token of a run (generate_sampled)
     uint32_t pf_rows = 0;  // tokens the pf_ buffers hold
     uint32_t *pf_tokens = nullptr;
     std::vector<void *> allocs;
@@ -564,6 +567,97 @@ int enqueue_prefill_run(wgml_llama2 *m, const uint32_t *tokens, uint32_t T, uint
     return WGML_OK;
 }
 
+bool all_gemm_supported(const wgml_llama2 *m) {
+    for (const LlamaLayer &w : m->layers)
+        for (const wgml_qmat *q : {w.attn_q, w.attn_k, w.attn_v, w.attn_output, w.ffn_gate, w.ffn_up,
+                                   w.ffn_down})
+            if (!gemm_supported(q)) return false;
+    return true;
+}
+
+// Workspaces for runs of up to `rows` tokens; a smaller set that queued work may still read stays
+// with the model (there are two sizes).
+int reserve_prefill(wgml_llama2 *m, uint32_t rows) {
+    const wgml_llama2_config &c = m->cfg;
+    if (m->pf_rows < rows) {
+        int rc = WGML_OK;
+        auto A = [&](float **p, uint64_t n) {
+            if (rc == WGML_OK) rc = dev_alloc(m, p, n, false);
+        };
+        m->pf_rows = 0;
+        A(&m->pf_xb, (uint64_t)rows * c.dim);
+        A(&m->pf_q, (uint64_t)rows * c.dim);
+        A(&m->pf_hb, (uint64_t)rows * c.hidden_dim);
+        A(&m->pf_hb2, (uint64_t)rows * c.hidden_dim);
+        if (rc == WGML_OK) rc = dev_alloc_bytes(m, (void **)&m->pf_tokens, rows * 4, false);
+        A(&m->pf_x, (uint64_t)rows * c.dim);
+        WGML_TRY(rc);
+        m->pf_rows = rows;
+    }
+    const uint32_t kmax = c.dim > c.hidden_dim ? c.dim : c.hidden_dim;
+    return ensure_prefill_scratch(m->ctx, (size_t)prefill_tpad(rows) * prefill_kpad(kmax) * 2);
+}
+
+int enqueue_read_logits(wgml_llama2 *m, float *host_out) {
+    WGML_CHECK_HIP(hipMemcpyAsync(host_out, m->logits, (size_t)m->cfg.vocab_size * 4,
+                                  hipMemcpyDeviceToHost, m->ctx->stream));
+    return WGML_OK;
+}
+
+// Pinned host memory for n logits, kept with the model (at most a run's rows): a copy to it needs no
+// staging and runs beside the host's work.  Null where there is none.
+float *reserve_host_logits(wgml_llama2 *m, size_t n) {
+    if (m->h_logits_n >= n) return m->h_logits;
+    (void)hipStreamSynchronize(m->ctx->stream);
+    if (m->h_logits) (void)hipHostFree(m->h_logits);
+    m->h_logits = nullptr;
+    m->h_logits_n = 0;
+    if (hipHostMalloc((void **)&m->h_logits, n * 4, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        m->h_logits = nullptr;
+        return nullptr;
+    }
+    m->h_logits_n = n;
+    return m->h_logits;
+}
+
+// generate_sampled takes prompts of at least this many tokens (and at most one run) in one pass: the
+// pass is 12 launches of 5-20 us per layer, a step 5 or 6 of 5-7 us and a read-back.
+constexpr uint32_t kSampledPromptMin = 6;
+
+// Plain f16 products are further from 64 bits than the step's 16-bit fixed point, and fp32
+// activations closer than split f16: under those settings the prompt stays with the steps.
+bool can_batch_sampled_prompt(const wgml_llama2 *m) {
+    return m->ctx->gemm_precise && !m->ctx->tuning[WGML_TUNE_GEMV_F32_ACTIVATIONS] && all_gemm_supported(m) &&
+           gemm_supported(m->output) && m->head_size % 4 == 0 && m->head_size <= 256 && m->kv_dim % 4 == 0 &&
+           m->cfg.dim % 4 == 0;
+}
+
+// np <= kPrefillMaxTokens prompt tokens from position 0 in one run: cache rows, the logits after
+// every one of them on the host (row after row) and the last ones in m->logits, as np steps leave.
+int prompt_logits(wgml_llama2 *m, const uint32_t *prompt, uint32_t np, float *host) {
+    const wgml_llama2_config &c = m->cfg;
+    wgml_ctx *ctx = m->ctx;
+    const size_t row = (size_t)c.vocab_size * 4;
+    if (!m->pf_logits)
+        WGML_TRY(dev_alloc(m, &m->pf_logits, (uint64_t)kPrefillMaxTokens * c.vocab_size, false));
+    WGML_TRY(reserve_prefill(m, kPrefillMaxTokens));
+    const uint64_t launches0 = ctx->launches;
+    ctx->gemm_pending_ks = 0;  // nothing is owed from an earlier run that failed half way
+    ctx->gemm_pending_pair = 0;
+    WGML_TRY(enqueue_prefill_run(m, prompt, np, 0));
+    WGML_TRY(launch_prefill_prep(ctx, m->pf_x, c.dim, nullptr, m->output_norm, c.rms_norm_eps, ctx->prefill_xh,
+                                 ctx->prefill_xscale, c.dim, np));
+    WGML_TRY(launch_gemm_quant(ctx, m->pf_logits, c.vocab_size, m->output, ctx->prefill_xh, ctx->prefill_xscale,
+                               np, nullptr, 0));
+    WGML_CHECK_HIP(hipMemcpyAsync(m->logits, m->pf_logits + (size_t)(np - 1) * c.vocab_size, row,
+                                  hipMemcpyDeviceToDevice, ctx->stream));
+    WGML_CHECK_HIP(hipMemcpyAsync(host, m->pf_logits, row * np, hipMemcpyDeviceToHost, ctx->stream));
+    WGML_CHECK_HIP(hipStreamSynchronize(ctx->stream));
+    m->launches_last = (ctx->launches - launches0) / np;
+    return WGML_OK;
+}
+
 }  // namespace
 
 extern "C" {
@@ -630,6 +724,7 @@ int wgml_llama2_destroy(wgml_llama2 *m) {
     if (m->ctx && m->ctx->stream) (void)hipStreamSynchronize(m->ctx->stream);
     drop_graph(m);
     for (void *p : m->allocs) (void)hipFree(p);
+    if (m->h_logits) (void)hipHostFree(m->h_logits);
     ctx_release(m->ctx);
     delete m;
     return WGML_OK;
@@ -757,12 +852,7 @@ int wgml_llama2_prefill(wgml_llama2 *m, const uint32_t *tokens, uint32_t n_token
         WGML_REQUIRE(tokens[i] < c.vocab_size,
                      "wgml_llama2_prefill: token %u outside vocabulary %u", tokens[i], c.vocab_size);
     wgml_ctx *ctx = m->ctx;
-    bool batched = true;
-    for (const LlamaLayer &w : m->layers)
-        for (const wgml_qmat *q : {w.attn_q, w.attn_k, w.attn_v, w.attn_output, w.ffn_gate, w.ffn_up,
-                                   w.ffn_down})
-            if (!gemm_supported(q)) batched = false;
-    if (!batched) {
+    if (!all_gemm_supported(m)) {
         // The batched products exist for the quantized formats, with weights of at most
         // 255.875 in magnitude.  A model with any other matrix takes the prompt the way the reference does: one step per token
         // (chat_llama2.rs:155-228), which leaves the same state.
@@ -771,34 +861,13 @@ int wgml_llama2_prefill(wgml_llama2 *m, const uint32_t *tokens, uint32_t n_token
         m->launches_last = ctx->launches - launches0;
         return WGML_OK;
     }
-    const uint32_t kmax = c.dim > c.hidden_dim ? c.dim : c.hidden_dim;
-    // Workspaces for runs of up to `rows` tokens; a smaller set that queued work may still read
-    // stays with the model (there are two sizes).
-    auto reserve = [&](uint32_t rows) -> int {
-        if (m->pf_rows < rows) {
-            int rc = WGML_OK;
-            auto A = [&](float **p, uint64_t n) {
-                if (rc == WGML_OK) rc = dev_alloc(m, p, n, false);
-            };
-            m->pf_rows = 0;
-            A(&m->pf_xb, (uint64_t)rows * c.dim);
-            A(&m->pf_q, (uint64_t)rows * c.dim);
-            A(&m->pf_hb, (uint64_t)rows * c.hidden_dim);
-            A(&m->pf_hb2, (uint64_t)rows * c.hidden_dim);
-            if (rc == WGML_OK) rc = dev_alloc_bytes(m, (void **)&m->pf_tokens, rows * 4, false);
-            A(&m->pf_x, (uint64_t)rows * c.dim);
-            WGML_TRY(rc);
-            m->pf_rows = rows;
-        }
-        return ensure_prefill_scratch(ctx, (size_t)prefill_tpad(rows) * prefill_kpad(kmax) * 2);
-    };
     const uint64_t launches0 = ctx->launches;
     uint32_t max_run = kPrefillMaxRun;
     for (uint32_t done = 0; done < n_tokens;) {
         const uint32_t T = prefill_run_length(n_tokens - done, max_run);
         ctx->gemm_pending_ks = 0;  // nothing is owed from an earlier run that failed half way
         ctx->gemm_pending_pair = 0;
-        int rc = reserve(T > kPrefillMaxTokens ? kPrefillMaxRun : kPrefillMaxTokens);
+        int rc = reserve_prefill(m, T > kPrefillMaxTokens ? kPrefillMaxRun : kPrefillMaxTokens);
         if (rc == WGML_OK) rc = enqueue_prefill_run(m, tokens + done, T, start_pos + done);
         if (rc != WGML_OK && T > kPrefillMaxTokens) {
             // no memory for the workspaces of a long run: short runs leave the same state
@@ -837,8 +906,7 @@ int wgml_llama2_prefill_decode_greedy(wgml_llama2 *m, const uint32_t *prompt, ui
 
 int wgml_llama2_read_logits(wgml_llama2 *m, float *host_out) {
     WGML_REQUIRE(m && host_out, "wgml_llama2_read_logits: null argument");
-    WGML_CHECK_HIP(hipMemcpyAsync(host_out, m->logits, (size_t)m->cfg.vocab_size * 4,
-                                  hipMemcpyDeviceToHost, m->ctx->stream));
+    WGML_TRY(enqueue_read_logits(m, host_out));
     WGML_CHECK_HIP(hipStreamSynchronize(m->ctx->stream));
     return WGML_OK;
 }
@@ -922,17 +990,58 @@ int wgml_llama2_generate_sampled(wgml_llama2 *m, const uint32_t *prompt, uint32_
                  "wgml_llama2_generate_sampled: %u positions exceed seq_len %u", n_total,
                  m->cfg.seq_len);
     if (n_total == 0) return WGML_OK;
-    std::vector<float> logits(m->cfg.vocab_size), coins(n_total);
+    const uint32_t vocab = m->cfg.vocab_size, np = n_prompt < n_total ? n_prompt : n_total;
+    std::vector<float> coins(n_total);
     WGML_TRY(wgml_rng_uniform_f32(seed, coins.data(), n_total));
-    uint32_t token = prompt[0];
+    // The logits of the positions not yet sampled; [0, np) are the prompt's.  What is sampled inside
+    // the prompt is returned but not fed back (the prompt's next token wins), so those samples are
+    // drawn on the host while the GPU runs the steps that follow.
+    WGML_TRY(check_ready(m));
+    float *logits = nullptr;
+    std::vector<float> pageable;
+    uint32_t batched = 0;  // prompt positions whose logits one pass over the prompt has left
+    if (np >= kSampledPromptMin && np <= kPrefillMaxTokens && can_batch_sampled_prompt(m)) {
+        bool valid = true;
+        for (uint32_t i = 0; i < np; ++i) valid = valid && prompt[i] < vocab;
+        if (valid) logits = reserve_host_logits(m, (size_t)np * vocab);
+        if (logits && prompt_logits(m, prompt, np, logits) == WGML_OK)
+            batched = np;
+        else
+            (void)hipGetLastError();  // no memory for its workspaces: the steps need none of them
+    }
+    if (!batched && !(logits = reserve_host_logits(m, (size_t)2 * vocab))) {
+        pageable.resize((size_t)2 * vocab);
+        logits = pageable.data();
+    }
+    uint32_t open = 0;  // first prompt position still to be sampled
+    auto sample = [&](float *l, uint32_t pos) {
+        return wgml_sample(l, vocab, temperature, topp, coins[pos], out_tokens + pos);
+    };
+    if (batched) {
+        WGML_TRY(sample(logits + (size_t)(np - 1) * vocab, np - 1));
+        for (uint32_t pos = np; pos < n_total; ++pos) {
+            // row np - 1 is free from here on: the steps' logits go there
+            float *row = logits + (size_t)(np - 1) * vocab;
+            WGML_TRY(wgml_llama2_forward(m, out_tokens[pos - 1], pos));
+            WGML_TRY(enqueue_read_logits(m, row));
+            if (open + 1 < np) {
+                WGML_TRY(sample(logits + (size_t)open * vocab, open));
+                ++open;
+            }
+            WGML_CHECK_HIP(hipStreamSynchronize(m->ctx->stream));
+            WGML_TRY(sample(row, pos));
+        }
+        for (; open + 1 < np; ++open) WGML_TRY(sample(logits + (size_t)open * vocab, open));
+        return WGML_OK;
+    }
     for (uint32_t pos = 0; pos < n_total; ++pos) {
-        WGML_TRY(wgml_llama2_forward(m, token, pos));
-        WGML_TRY(wgml_llama2_read_logits(m, logits.data()));
-        uint32_t next = 0;
-        WGML_TRY(wgml_sample(logits.data(), m->cfg.vocab_size, temperature, topp, coins[pos],
-                             &next));
-        out_tokens[pos] = next;
-        token = (pos + 1 < n_prompt) ? prompt[pos + 1] : next;
+        const bool forced = pos > 0 && pos < np;
+        float *row = logits + (size_t)(pos & 1) * vocab;
+        WGML_TRY(wgml_llama2_forward(m, pos < np ? prompt[pos] : out_tokens[pos - 1], pos));
+        WGML_TRY(enqueue_read_logits(m, row));
+        if (forced) WGML_TRY(sample(logits + (size_t)((pos - 1) & 1) * vocab, pos - 1));
+        WGML_CHECK_HIP(hipStreamSynchronize(m->ctx->stream));
+        if (pos + 1 >= np) WGML_TRY(sample(row, pos));
     }
     return WGML_OK;
 }
