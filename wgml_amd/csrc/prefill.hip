@@ -386,6 +386,12 @@ struct GemmQ8K {
 // a lane's t = 8 g + 4 e + i, so lanes g < 2 take low nibbles and g >= 2 high nibbles of the
 // same eight bytes.  Blocks are 2-byte aligned: the loads below are unaligned, which gfx950
 // serves.  A block of the padded K range that does not exist reads the last one and expands to 0.
+// (A load per halfword instead, nine per chunk: 21 tokens through four layers of 3072 x 8192 in Q4_0
+// 901 us against 522, Q8_0 557.)
+template <class T>
+struct __attribute__((packed, aligned(2))) Half2Aligned {
+    T v;
+};
 template <int BYTES, bool HAS_M, bool HAS_QH>
 struct GemmLegacy {
     struct Raw {
@@ -410,18 +416,14 @@ struct GemmLegacy {
 #pragma unroll
         for (int s2 = 0; s2 < 2; ++s2) {
             const uint8_t *blk = m.p0 + (size_t)min(b0 + s2, nb - 1) * BYTES;
-            // 2-byte aligned: halfwords are loaded as such and put together
-            const uint32_t d = load_at<uint16_t>(blk, l.blk);
-            uint32_t mm = 0;
-            if (HAS_M) mm = load_at<uint16_t>(blk + 2, l.blk);
-            r.dm[s2] = d | (mm << 16);
+            if (HAS_M)
+                r.dm[s2] = load_at<Half2Aligned<uint32_t>>(blk, l.blk).v;
+            else
+                r.dm[s2] = load_at<uint16_t>(blk, l.blk);
             r.qh[s2] = 0;
-            if (HAS_QH)
-                r.qh[s2] = (uint32_t)load_at<uint16_t>(blk + (HAS_M ? 4 : 2), l.blk) |
-                           ((uint32_t)load_at<uint16_t>(blk + (HAS_M ? 6 : 4), l.blk) << 16);
-            const uint32_t q0 = (uint32_t)load_at<uint16_t>(blk, l.q) | ((uint32_t)load_at<uint16_t>(blk + 2, l.q) << 16);
-            const uint32_t q1 = (uint32_t)load_at<uint16_t>(blk + 4, l.q) | ((uint32_t)load_at<uint16_t>(blk + 6, l.q) << 16);
-            r.q[s2] = make_uint2(q0, q1);
+            if (HAS_QH) r.qh[s2] = load_at<Half2Aligned<uint32_t>>(blk + (HAS_M ? 4 : 2), l.blk).v;
+            const uint64_t q = load_at<Half2Aligned<uint64_t>>(blk, l.q).v;
+            r.q[s2] = make_uint2((uint32_t)q, (uint32_t)(q >> 32));
         }
     }
     __device__ static void pre(Pre &p, const Raw &r, uint32_t ncols, uint32_t chunk, uint32_t g) {
