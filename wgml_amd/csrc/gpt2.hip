@@ -535,14 +535,25 @@ int reserve_prompt(wgml_gpt2 *m) {
     const wgml_gpt2_params &p = m->p;
     if (!m->pf_x) {
         const uint64_t T = kPrefillMaxTokens;
-        float *tokens = nullptr;
-        WGML_TRY(dev_alloc(m, &tokens, T, false));
+        const size_t kept = m->allocs.size();
+        int rc = WGML_OK;
+        auto A = [&](uint64_t n) {
+            float *d = nullptr;
+            if (rc == WGML_OK) rc = dev_alloc(m, &d, n, false);
+            return d;
+        };
+        float *x = A(T * p.n_embd), *qkv = A(T * 3 * p.n_embd), *att = A(T * p.n_embd), *h = A(T * p.ff_len);
+        float *logits = A(T * p.n_vocab), *tokens = A(T);
+        if (rc != WGML_OK) {  // all of them or none: a later call must not find less memory
+            for (; m->allocs.size() > kept; m->allocs.pop_back()) (void)hipFree(m->allocs.back());
+            return rc;
+        }
+        m->pf_x = x;
+        m->pf_qkv = qkv;
+        m->pf_att = att;
+        m->pf_h = h;
+        m->pf_logits = logits;
         m->pf_tokens = reinterpret_cast<uint32_t *>(tokens);
-        WGML_TRY(dev_alloc(m, &m->pf_qkv, T * 3 * p.n_embd, false));
-        WGML_TRY(dev_alloc(m, &m->pf_att, T * p.n_embd, false));
-        WGML_TRY(dev_alloc(m, &m->pf_h, T * p.ff_len, false));
-        WGML_TRY(dev_alloc(m, &m->pf_logits, T * p.n_vocab, false));
-        WGML_TRY(dev_alloc(m, &m->pf_x, T * p.n_embd, false));  // last: marks the set as complete
     }
     const uint32_t kmax = p.n_embd > p.ff_len ? p.n_embd : p.ff_len;
     return ensure_prefill_scratch(m->ctx, (size_t)kPrefillMaxTokens * prefill_kpad(kmax) * 2);

@@ -83,6 +83,11 @@ int dev_alloc(wgml_llama2 *m, float **p, uint64_t n_floats, bool zero) {
     return dev_alloc_bytes(m, (void **)p, n_floats * 4, zero);
 }
 
+// Gives back what was allocated behind the first `kept` blocks and never used.
+void free_allocs_from(wgml_llama2 *m, size_t kept) {
+    for (; m->allocs.size() > kept; m->allocs.pop_back()) (void)hipFree(m->allocs.back());
+}
+
 int check_ready(const wgml_llama2 *m) {
     for (size_t l = 0; l < m->layers.size(); ++l) {
         const LlamaLayer &w = m->layers[l];
@@ -576,22 +581,31 @@ bool all_gemm_supported(const wgml_llama2 *m) {
 }
 
 // Workspaces for runs of up to `rows` tokens; a smaller set that queued work may still read stays
-// with the model (there are two sizes).
+// with the model (there are two sizes).  Where there is no memory for all of a set nothing of it is
+// kept, and the model goes on with the set it has.
 int reserve_prefill(wgml_llama2 *m, uint32_t rows) {
     const wgml_llama2_config &c = m->cfg;
     if (m->pf_rows < rows) {
+        const size_t kept = m->allocs.size();
         int rc = WGML_OK;
-        auto A = [&](float **p, uint64_t n) {
-            if (rc == WGML_OK) rc = dev_alloc(m, p, n, false);
+        auto A = [&](uint64_t n) {
+            float *p = nullptr;
+            if (rc == WGML_OK) rc = dev_alloc(m, &p, n, false);
+            return p;
         };
-        m->pf_rows = 0;
-        A(&m->pf_xb, (uint64_t)rows * c.dim);
-        A(&m->pf_q, (uint64_t)rows * c.dim);
-        A(&m->pf_hb, (uint64_t)rows * c.hidden_dim);
-        A(&m->pf_hb2, (uint64_t)rows * c.hidden_dim);
-        if (rc == WGML_OK) rc = dev_alloc_bytes(m, (void **)&m->pf_tokens, rows * 4, false);
-        A(&m->pf_x, (uint64_t)rows * c.dim);
-        WGML_TRY(rc);
+        float *x = A((uint64_t)rows * c.dim), *xb = A((uint64_t)rows * c.dim), *q = A((uint64_t)rows * c.dim);
+        float *hb = A((uint64_t)rows * c.hidden_dim), *hb2 = A((uint64_t)rows * c.hidden_dim);
+        float *tokens = A(rows);
+        if (rc != WGML_OK) {
+            free_allocs_from(m, kept);
+            return rc;
+        }
+        m->pf_x = x;
+        m->pf_xb = xb;
+        m->pf_q = q;
+        m->pf_hb = hb;
+        m->pf_hb2 = hb2;
+        m->pf_tokens = reinterpret_cast<uint32_t *>(tokens);
         m->pf_rows = rows;
     }
     const uint32_t kmax = c.dim > c.hidden_dim ? c.dim : c.hidden_dim;

@@ -1643,13 +1643,13 @@ int ensure_prefill_scratch(wgml_ctx *ctx, size_t xh_bytes) {
     if (!ctx->prefill_xscale)
         WGML_CHECK_HIP(hipMalloc((void **)&ctx->prefill_xscale, kPrefillMaxRun * sizeof(float)));
     if (xh_bytes <= ctx->prefill_xh_bytes) return WGML_OK;
-    // work already enqueued may still read the old buffer: retire it, free with the context
-    if (ctx->prefill_xh) ctx->retired.push_back(ctx->prefill_xh);
-    ctx->prefill_xh = nullptr;
-    ctx->prefill_xh_bytes = 0;
     xh_bytes = (xh_bytes + 255) & ~(size_t)255;
     // two arrays: the f16 activations and, behind them, their low parts (split precision)
-    WGML_CHECK_HIP(hipMalloc(&ctx->prefill_xh, 2 * xh_bytes));
+    void *xh = nullptr;
+    WGML_CHECK_HIP(hipMalloc(&xh, 2 * xh_bytes));  // without it the old buffer stays in use
+    // work already enqueued may still read the old buffer: retire it, free with the context
+    if (ctx->prefill_xh) ctx->retired.push_back(ctx->prefill_xh);
+    ctx->prefill_xh = xh;
     ctx->prefill_xl = (char *)ctx->prefill_xh + xh_bytes;
     ctx->prefill_xh_bytes = xh_bytes;
     return WGML_OK;
@@ -1707,11 +1707,11 @@ int launch_gemm_flush(wgml_ctx *ctx, float *x, uint32_t x_stride, const float *x
 
 int ensure_gemm_partials(wgml_ctx *ctx, size_t bytes) {
     if (bytes <= ctx->gemm_part_bytes) return WGML_OK;
-    if (ctx->gemm_part) ctx->retired.push_back(ctx->gemm_part);  // may still be read by queued work
-    ctx->gemm_part = nullptr;
-    ctx->gemm_part_bytes = 0;
     bytes = (bytes + (size_t(8) << 20)) & ~((size_t(1) << 20) - 1);  // grow in steps
-    WGML_CHECK_HIP(hipMalloc((void **)&ctx->gemm_part, bytes));
+    float *part = nullptr;
+    WGML_CHECK_HIP(hipMalloc((void **)&part, bytes));  // without it the old buffer stays in use
+    if (ctx->gemm_part) ctx->retired.push_back(ctx->gemm_part);  // may still be read by queued work
+    ctx->gemm_part = part;
     ctx->gemm_part_bytes = bytes;
     return WGML_OK;
 }
