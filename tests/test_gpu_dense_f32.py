@@ -1,5 +1,6 @@
-"""Dense f32 matrices (F32 tensors, F16 ones expanded at creation) in the shared GEMV body: rows of
-a multiple of 16 columns; other widths stay on the general kernel.  Against float64."""
+"""Dense f32 matrices (F32 tensors, F16 ones expanded at creation): rows of a multiple of 16 columns
+in the shared GEMV body, other widths and most narrow matrices on the general kernel
+(test_host_routes.py has the line).  Against float64."""
 import numpy as np
 import pytest
 
@@ -37,13 +38,15 @@ def test_gemv_f32_rows(gpu, nrows, ncols):
     assert (err <= _bound(a, x)).all(), err.max()
 
 
-def test_gemv_f32_tall(gpu):
-    # more rows than one result per lane and wave of the machine
+# rows below a step in the shared body; more rows than one result per lane and wave of the machine in
+# the shared body and in the general kernel
+@pytest.mark.parametrize("nrows,ncols", [(8193, 272), (8193, 1008), (32769, 144), (300001, 272), (300001, 32)])
+def test_gemv_f32_tall(gpu, nrows, ncols):
     rng = np.random.default_rng(5)
-    a = rng.standard_normal((300001, 32)).astype(np.float32)
-    x = rng.standard_normal(32).astype(np.float32)
+    a = rng.standard_normal((nrows, ncols), dtype=np.float32)
+    x = rng.standard_normal(ncols).astype(np.float32)
     out = W.GpuVector.uninit(gpu, len(a))
-    m = W.GpuQuantMatrix(gpu, W.F32, len(a), 32, a.view(np.uint8).reshape(-1))
+    m = W.GpuQuantMatrix(gpu, W.F32, len(a), ncols, a.view(np.uint8).reshape(-1))
     W.GemvQuant.from_device(gpu).dispatch(out, m, W.GpuVector.init(gpu, x))
     assert (np.abs(out.read() - a.astype(np.float64) @ x) <= _bound(a, x)).all()
 

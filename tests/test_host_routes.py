@@ -1,0 +1,28 @@
+"""Which kernels the library's calls launch, what they allocate and what they do when a call of the
+HIP runtime fails, on the CPU: the runtime is host_hip.c, which runs no kernel."""
+import pytest
+
+import host_hip
+
+
+@pytest.fixture(scope="module")
+def runtime(tmp_path_factory):
+    return host_hip.build(tmp_path_factory)
+
+
+def test_narrow_dense_matrices_take_the_general_kernel(runtime):
+    # on both sides of each part of the rule, and the matrices the shared body cannot take
+    host_hip.run(runtime, """
+    def general(nrows, ncols):
+        m = W.GpuQuantMatrix(gpu, W.F32, nrows, ncols, np.zeros(4 * nrows * ncols, np.uint8))
+        out, x = W.GpuVector.uninit(gpu, nrows), W.GpuVector.uninit(gpu, ncols)
+        names = launched(lambda: W.GemvQuant(gpu).dispatch(out, m, x))
+        assert len(names) == 1
+        return "gemv_f32_kernel" in names[0]
+
+    for shape in ((1, 16), (4096, 64), (50257, 128), (300001, 128), (515, 512), (8192, 1008), (32768, 256),
+                  (262145, 256), (17, 20), (50257, 772)):
+        assert general(*shape), shape
+    for shape in ((1, 1024), (17, 4096), (8193, 272), (8193, 1008), (32769, 256), (262144, 256), (262145, 272)):
+        assert not general(*shape), shape
+    """)

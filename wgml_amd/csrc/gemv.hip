@@ -1551,8 +1551,9 @@ __global__ __launch_bounds__(MAXT, MINW) void gemv_fused_kernel(const FusedParam
 
 // ------------------------------------------------------------- dense f32 ----
 // out = A v, A row-major f32 (p.p0).  One wave per row, float4 loads, x from LDS.  For what the
-// shared body does not take: f32 tensors as operator arguments (any width and alignment) and
-// matrices whose rows are not a multiple of 16 floats.
+// shared body does not take -- f32 tensors as operator arguments (any width and alignment) and
+// matrices whose rows are not a multiple of 16 floats -- and for what it takes longer for
+// (dense_f32_general_faster).
 __global__ __launch_bounds__(256) void gemv_f32_kernel(const GemvParams p, int vec4) {
     extern __shared__ float4 smem[];
     __shared__ float red[16];
@@ -1806,6 +1807,22 @@ static bool dense_f32_in_shared_body(const wgml_qmat *m) {
     return m->type == WGML_F32 && m->ncols % FmtF32::TILE == 0 && (size_t)m->ncols * 4 <= kMaxLds;
 }
 
+// Plain products (no folded norm or activation) of such matrices that gemv_f32_kernel does faster.
+// In the shared body a lane takes 16 columns of a row, there 4: rows of less than a step of 1024
+// columns leave most of a wave idle here, which costs more than the general kernel's single load in
+// flight while the matrix is small, and at any size for rows of up to 128 columns.  Beyond 64
+// results in each of the machine's waves of rows the body needs a second round of workgroups.
+// Measured, general / shared: 4096x64 2.0 / 3.0 us, 4096x256 2.4 / 3.3, 515x512 2.1 / 2.5, 8192x512
+// 4.6 / 4.8, 50257x128 9.1 / 9.8, 32768x256 7.7 / 8.3, 300001x256 69 / 100; on the other side of the
+// line 515x1024 2.5 / 2.5, 4096x2048 9.0 / 7.2, 12288x768 9.6 / 8.2, 50257x256 13.9 / 13.5, 300001x384
+// 114 / 109.
+static bool dense_f32_general_faster(const wgml_ctx *ctx, uint32_t nrows, uint32_t ncols) {
+    const uint32_t cu = ctx->n_cu > 0 ? (uint32_t)ctx->n_cu : 256u;
+    if (ncols <= 128) return true;
+    if (ncols < 1024 && nrows <= 8192) return true;
+    return ncols <= 256 && (nrows <= 32768 || nrows > cu * 16 * 64);
+}
+
 bool gemv_partials_supported(const wgml_ctx *, const wgml_qmat *m) {
     return m && (m->type == WGML_Q4_K || m->type == WGML_Q6_K || m->type == WGML_Q8_0);
 }
@@ -1849,7 +1866,9 @@ int launch_gemv_quant(wgml_ctx *ctx, float *out, const wgml_qmat *m, const float
         return set_error(WGML_E_INVALID, "gemv_quant: the input vector must be 16-byte aligned");
     }
     (void)main_fmt;
-    if (m->type == WGML_F32 && dense_f32_in_shared_body(m)) return launch_fmt_f32<FmtF32>(ctx, p);
+    if (dense_f32_in_shared_body(m) &&
+        (p.ln_g || p.act || p.norm_w || !dense_f32_general_faster(ctx, p.nrows, p.ncols)))
+        return launch_fmt_f32<FmtF32>(ctx, p);
     if ((p.ln_g || p.act) && m->type == WGML_F32)
         return set_error(WGML_E_UNSUPPORTED, "gemv_quant: LayerNorm / activation folding needs rows of a "
                                              "multiple of 16 elements");
