@@ -396,8 +396,9 @@ WGML_API int wgml_llama2_launches_per_token(const wgml_llama2 *m);
  * 1: bias and residual adds folded into the GEMV epilogues; 2: also every
  * RMSNorm folded into the GEMVs that consume it; 3 (default): also Q, K and V
  * (with bias, RoPE and the KV-cache write) in one launch and gate and up (with
- * the SiLU gating) in one launch.  All levels give the same results to fp32
- * rounding. */
+ * the SiLU gating) in one launch.  wgml_llama2_generate_sampled takes the prompt in
+ * one pass from level 1 on; wgml_llama2_prefill does at every level.  All levels give
+ * the same results to fp32 rounding. */
 WGML_API int wgml_llama2_set_fusion(wgml_llama2 *m, int level);
 
 /* ---- GPT-2: Gpt2 / Gpt2State / Gpt2Weights -------------------------------- */

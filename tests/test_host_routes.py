@@ -26,3 +26,17 @@ def test_narrow_dense_matrices_take_the_general_kernel(runtime):
     for shape in ((1, 1024), (17, 4096), (8193, 272), (8193, 1008), (32769, 256), (262144, 256), (262145, 272)):
         assert not general(*shape), shape
     """)
+
+
+def test_sampled_generation_follows_the_fusion_level(runtime):
+    # level 0 is one launch per operation of the reference, in the prompt too
+    host_hip.run(runtime, """
+    m = llama(gpu, Llama2Config(256, 512, 2, 4, 2, 331, 64))
+    prompt = np.zeros(20, np.uint32)
+    for level, batched in ((0, False), (1, True), (2, True), (3, True)):
+        m.set_fusion(level)
+        one = launched(lambda: m.forward(0, 0))
+        names = launched(lambda: m.generate_sampled(prompt, 23, 0.7, 0.9, 1))
+        assert (count(names, "gemm_lds_kernel") > 0) == batched, level
+        assert batched or names == one * 23
+    """)

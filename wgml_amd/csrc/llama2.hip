@@ -640,9 +640,10 @@ float *reserve_host_logits(wgml_llama2 *m, size_t n) {
 constexpr uint32_t kSampledPromptMin = 6;
 
 // Plain f16 products are further from 64 bits than the step's 16-bit fixed point, and fp32
-// activations closer than split f16: under those settings the prompt stays with the steps.
+// activations closer than split f16: under those settings the prompt stays with the steps.  So it
+// does at fusion level 0, which is one launch per operation of the reference.
 bool can_batch_sampled_prompt(const wgml_llama2 *m) {
-    return m->ctx->gemm_precise && !m->ctx->tuning[WGML_TUNE_GEMV_F32_ACTIVATIONS] && all_gemm_supported(m) &&
+    return m->fusion >= 1 && m->ctx->gemm_precise && !m->ctx->tuning[WGML_TUNE_GEMV_F32_ACTIVATIONS] && all_gemm_supported(m) &&
            gemm_supported(m->output) && m->head_size % 4 == 0 && m->head_size <= 256 && m->kv_dim % 4 == 0 &&
            m->cfg.dim % 4 == 0;
 }
