@@ -40,3 +40,21 @@ def test_sampled_generation_follows_the_fusion_level(runtime):
         assert (count(names, "gemm_lds_kernel") > 0) == batched, level
         assert batched or names == one * 23
     """)
+
+
+def test_sampled_generation_refuses_a_temperature_before_it_starts(runtime):
+    # (refused by the first sample, it left a copy of logits under way to memory that the call frees
+    # where there is no pinned memory)
+    host_hip.run(runtime, """
+    m = llama(gpu, Llama2Config(256, 512, 2, 4, 2, 331, 64))
+    for n_prompt, temperature in ((1, -1.0), (3, -1.0), (20, -0.5), (3, float("nan"))):
+        def call():
+            try:
+                m.generate_sampled(np.zeros(n_prompt, np.uint32), 23, temperature, 0.9, 1)
+            except W.WgmlError as e:
+                assert e.code == _lib.E_INVALID and "temperature" in str(e)
+            else:
+                assert False
+        assert launched(call) == []
+    m.generate_sampled(np.zeros(3, np.uint32), 0, -1.0, 0.9, 1)  # nothing to do: accepted as before
+    """)

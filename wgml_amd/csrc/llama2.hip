@@ -1005,6 +1005,8 @@ int wgml_llama2_generate_sampled(wgml_llama2 *m, const uint32_t *prompt, uint32_
                  "wgml_llama2_generate_sampled: %u positions exceed seq_len %u", n_total,
                  m->cfg.seq_len);
     if (n_total == 0) return WGML_OK;
+    // what the sampler refuses is refused here: below, copies to the host are under way
+    WGML_REQUIRE(temperature >= 0.0f, "wgml_llama2_generate_sampled: temperature %g", (double)temperature);
     const uint32_t vocab = m->cfg.vocab_size, np = n_prompt < n_total ? n_prompt : n_total;
     std::vector<float> coins(n_total);
     WGML_TRY(wgml_rng_uniform_f32(seed, coins.data(), n_total));
