@@ -58,3 +58,14 @@ def test_sampled_generation_refuses_a_temperature_before_it_starts(runtime):
         assert launched(call) == []
     m.generate_sampled(np.zeros(3, np.uint32), 0, -1.0, 0.9, 1)  # nothing to do: accepted as before
     """)
+
+
+def test_rows_whose_long_runs_the_products_cannot_address_go_in_short_ones(runtime):
+    # 2^20 columns: the low halves of 1024 packed tokens would lie 2^31 bytes behind the high ones
+    host_hip.run(runtime, """
+    m = llama(gpu, Llama2Config(256, 1 << 20, 1, 4, 4, 331, 400))
+    names = launched(lambda: m.prefill(np.zeros(300, np.uint32)))
+    assert count(names, "gemm_tile") == 0 and count(names, "gemm_lds") > 0
+    m = llama(gpu, Llama2Config(256, 1 << 19, 1, 4, 4, 331, 400))
+    assert count(launched(lambda: m.prefill(np.zeros(300, np.uint32))), "gemm_tile") > 0
+    """)

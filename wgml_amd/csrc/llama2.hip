@@ -580,6 +580,17 @@ bool all_gemm_supported(const wgml_llama2 *m) {
     return true;
 }
 
+// Bytes of the packed activations of `rows` tokens, as wide as the widest product of the model.
+size_t prefill_xh_bytes(const wgml_llama2_config &c, uint32_t rows) {
+    return (size_t)prefill_tpad(rows) * prefill_kpad(c.dim > c.hidden_dim ? c.dim : c.hidden_dim) * 2;
+}
+
+// The longest run of a prompt pass.  The products address the low halves of the packed activations
+// with 31 bits from the high ones, so models of 2^20 columns and more stay with short runs.
+uint32_t prefill_max_run(const wgml_llama2 *m) {
+    return prefill_xh_bytes(m->cfg, kPrefillMaxRun) < (size_t(1) << 31) ? kPrefillMaxRun : kPrefillMaxTokens;
+}
+
 // Workspaces for runs of up to `rows` tokens; a smaller set that queued work may still read stays
 // with the model (there are two sizes).  Where there is no memory for all of a set nothing of it is
 // kept, and the model goes on with the set it has.
@@ -608,8 +619,7 @@ int reserve_prefill(wgml_llama2 *m, uint32_t rows) {
         m->pf_tokens = reinterpret_cast<uint32_t *>(tokens);
         m->pf_rows = rows;
     }
-    const uint32_t kmax = c.dim > c.hidden_dim ? c.dim : c.hidden_dim;
-    return ensure_prefill_scratch(m->ctx, (size_t)prefill_tpad(rows) * prefill_kpad(kmax) * 2);
+    return ensure_prefill_scratch(m->ctx, prefill_xh_bytes(c, rows));
 }
 
 int enqueue_read_logits(wgml_llama2 *m, float *host_out) {
@@ -877,7 +887,7 @@ int wgml_llama2_prefill(wgml_llama2 *m, const uint32_t *tokens, uint32_t n_token
         return WGML_OK;
     }
     const uint64_t launches0 = ctx->launches;
-    uint32_t max_run = kPrefillMaxRun;
+    uint32_t max_run = prefill_max_run(m);
     for (uint32_t done = 0; done < n_tokens;) {
         const uint32_t T = prefill_run_length(n_tokens - done, max_run);
         ctx->gemm_pending_ks = 0;  // nothing is owed from an earlier run that failed half way
