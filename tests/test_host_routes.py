@@ -69,3 +69,52 @@ def test_rows_whose_long_runs_the_products_cannot_address_go_in_short_ones(runti
     m = llama(gpu, Llama2Config(256, 1 << 19, 1, 4, 4, 331, 400))
     assert count(launched(lambda: m.prefill(np.zeros(300, np.uint32))), "gemm_tile") > 0
     """)
+
+
+def test_only_missing_memory_sends_a_prompt_down_the_slower_path(runtime):
+    # runs of 1024 tokens, then of 128, then (where a loop has them) steps; any other failure of the
+    # faster path is the caller's to see
+    host_hip.run(runtime, """
+    def failure(call):
+        try:
+            call()
+        except W.WgmlError as e:
+            return e.code
+    prompt, long_prompt = np.zeros(20, np.uint32), np.zeros(300, np.uint32)
+    cfg = Llama2Config(256, 512, 2, 4, 2, 331, 400)
+    p = Gpt2Params(n_vocab=331, n_seq=64, n_embd=128, n_head=4, n_layer=2, ff_len=512, attn_b=384)
+    sampled = lambda m: m.generate_sampled(prompt, 23, 0.7, 0.9, 1)
+
+    # no memory for the larger workspaces, or for any
+    m = llama(gpu, cfg)
+    fake.host_hip_malloc_limit(1 << 20)
+    names = launched(lambda: m.prefill(long_prompt))
+    assert count(names, "gemm_tile") == 0 and count(names, "gemm_lds") > 0
+    fake.host_hip_malloc_limit(NO_LIMIT)
+    assert count(launched(lambda: m.prefill(long_prompt)), "gemm_tile") > 0
+    m, g = llama(gpu, cfg), gpt2(gpu, p)
+    one = launched(lambda: m.forward(0, 0))
+    g.record_steps(23)
+    fake.host_hip_malloc_limit(1 << 10)
+    assert launched(lambda: sampled(m)) == one * 23
+    assert count(launched(lambda: g.generate_greedy(prompt, 23)), "gemm_") == 0
+    fake.host_hip_malloc_limit(NO_LIMIT)
+    assert count(launched(lambda: sampled(m)), "gemm_lds") > 0
+    assert count(launched(lambda: g.generate_greedy(prompt, 23)), "gemm_lds") > 0
+
+    # no memory for the partial sums of a product, in the middle of a run
+    wide = llama(W.GpuInstance(0), Llama2Config(1024, 2816, 2, 8, 8, 331, 400))
+    one = launched(lambda: wide.forward(0, 0))
+    fake.host_hip_malloc_limit(6 << 20)
+    names = launched(lambda: sampled(wide))
+    assert count(names, "prep_x") == 1 and names[-23 * len(one):] == one * 23
+    assert failure(lambda: wide.prefill(long_prompt)) == _lib.E_OOM
+    fake.host_hip_malloc_limit(NO_LIMIT)
+
+    # a launch that fails
+    fake.host_hip_fail_kernel(b"gemm_tile_kernel")
+    assert failure(lambda: m.prefill(long_prompt)) == _lib.E_HIP
+    fake.host_hip_fail_kernel(b"gemm_lds_kernel")
+    assert failure(lambda: sampled(m)) == _lib.E_HIP
+    assert failure(lambda: g.generate_greedy(prompt, 23)) == _lib.E_HIP
+    """)

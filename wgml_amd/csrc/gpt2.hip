@@ -54,9 +54,11 @@ namespace {
 int dev_alloc(wgml_gpt2 *m, float **p, uint64_t n_floats, bool zero) {
     void *d = nullptr;
     hipError_t e = hipMalloc(&d, n_floats * 4);
-    if (e != hipSuccess)
+    if (e != hipSuccess) {
+        (void)hipGetLastError();  // not the next launch's error
         return set_error(WGML_E_OOM, "wgml_gpt2: hipMalloc(%llu) failed: %s",
                          (unsigned long long)(n_floats * 4), hipGetErrorString(e));
+    }
     m->allocs.push_back(d);
     if (zero) WGML_CHECK_HIP(hipMemsetAsync(d, 0, n_floats * 4, m->ctx->stream));
     *p = (float *)d;
@@ -522,13 +524,12 @@ constexpr uint32_t kBatchedPromptMin = 8;
 // of 4.
 bool can_batch_prompt(const wgml_gpt2 *m) {
     const uint32_t n = m->p.n_embd;
-    if (!m->ctx->gemm_precise || m->ctx->tuning[WGML_TUNE_GEMV_F32_ACTIVATIONS] || (n / m->p.n_head) % 4 != 0 || n % 8 != 0 || !gemm_supported(m->lm_head))
+    if (!m->ctx->gemm_precise || m->ctx->tuning[WGML_TUNE_GEMV_F32_ACTIVATIONS] || (n / m->p.n_head) % 4 != 0 || n % 8 != 0)
         return false;
+    auto fits = [](const wgml_qmat *q) { return gemm_supported(q) && gemm_addressable(q); };
     for (const Gpt2Layer &w : m->layers)
-        if (!gemm_supported(w.attn_w) || !gemm_supported(w.proj_w) || !gemm_supported(w.fc_w) ||
-            !gemm_supported(w.mlp_proj_w))
-            return false;
-    return true;
+        if (!fits(w.attn_w) || !fits(w.proj_w) || !fits(w.fc_w) || !fits(w.mlp_proj_w)) return false;
+    return fits(m->lm_head);
 }
 
 int reserve_prompt(wgml_gpt2 *m) {
@@ -705,11 +706,13 @@ int wgml_gpt2_generate_greedy(wgml_gpt2 *m, const uint32_t *prompt, uint32_t n_p
     uint32_t first = 0;  // the loop's first position: behind the prompt where that goes in batched
     if (np >= kBatchedPromptMin && can_batch_prompt(m)) {
         const uint64_t l0 = ctx->launches;
-        if (enqueue_prompt(m, np, at) == WGML_OK) {
+        const int rc = enqueue_prompt(m, np, at);
+        if (rc == WGML_OK) {
             first = np;
             m->launches_last = (ctx->launches - l0) / np;
-        } else {
-            (void)hipGetLastError();  // no memory for its workspaces: the steps need none of them
+        } else if (rc != WGML_E_OOM) {  // no memory for its workspaces: the steps need none of them
+            (void)hipStreamSynchronize(ctx->stream);  // a copy of `at` may be under way
+            return rc;
         }
     }
     if (first == 0) {

@@ -70,9 +70,11 @@ namespace {
 int dev_alloc_bytes(wgml_llama2 *m, void **p, uint64_t bytes, bool zero) {
     void *d = nullptr;
     hipError_t e = hipMalloc(&d, bytes);
-    if (e != hipSuccess)
+    if (e != hipSuccess) {
+        (void)hipGetLastError();  // not the next launch's error
         return set_error(WGML_E_OOM, "wgml_llama2: hipMalloc(%llu) failed: %s",
                          (unsigned long long)bytes, hipGetErrorString(e));
+    }
     m->allocs.push_back(d);
     if (zero) WGML_CHECK_HIP(hipMemsetAsync(d, 0, bytes, m->ctx->stream));
     *p = d;
@@ -653,6 +655,10 @@ constexpr uint32_t kSampledPromptMin = 6;
 // activations closer than split f16: under those settings the prompt stays with the steps.  So it
 // does at fusion level 0, which is one launch per operation of the reference.
 bool can_batch_sampled_prompt(const wgml_llama2 *m) {
+    for (const LlamaLayer &w : m->layers)
+        for (const wgml_qmat *q : {w.attn_q, w.attn_k, w.attn_v, w.attn_output, w.ffn_gate, w.ffn_up, w.ffn_down,
+                                   m->output})
+            if (!gemm_addressable(q)) return false;
     return m->fusion >= 1 && m->ctx->gemm_precise && !m->ctx->tuning[WGML_TUNE_GEMV_F32_ACTIVATIONS] && all_gemm_supported(m) &&
            gemm_supported(m->output) && m->head_size % 4 == 0 && m->head_size <= 256 && m->kv_dim % 4 == 0 &&
            m->cfg.dim % 4 == 0;
@@ -894,9 +900,8 @@ int wgml_llama2_prefill(wgml_llama2 *m, const uint32_t *tokens, uint32_t n_token
         ctx->gemm_pending_pair = 0;
         int rc = reserve_prefill(m, T > kPrefillMaxTokens ? kPrefillMaxRun : kPrefillMaxTokens);
         if (rc == WGML_OK) rc = enqueue_prefill_run(m, tokens + done, T, start_pos + done);
-        if (rc != WGML_OK && T > kPrefillMaxTokens) {
+        if (rc == WGML_E_OOM && T > kPrefillMaxTokens) {
             // no memory for the workspaces of a long run: short runs leave the same state
-            (void)hipGetLastError();
             max_run = kPrefillMaxTokens;
             continue;
         }
@@ -1031,10 +1036,13 @@ int wgml_llama2_generate_sampled(wgml_llama2 *m, const uint32_t *prompt, uint32_
         bool valid = true;
         for (uint32_t i = 0; i < np; ++i) valid = valid && prompt[i] < vocab;
         if (valid) logits = reserve_host_logits(m, (size_t)np * vocab);
-        if (logits && prompt_logits(m, prompt, np, logits) == WGML_OK)
-            batched = np;
-        else
-            (void)hipGetLastError();  // no memory for its workspaces: the steps need none of them
+        if (logits) {
+            const int rc = prompt_logits(m, prompt, np, logits);
+            if (rc == WGML_OK)
+                batched = np;
+            else if (rc != WGML_E_OOM)  // no memory for its workspaces: the steps need none of them
+                return rc;
+        }
     }
     if (!batched && !(logits = reserve_host_logits(m, (size_t)2 * vocab))) {
         pageable.resize((size_t)2 * vocab);

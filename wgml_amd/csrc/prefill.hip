@@ -1645,14 +1645,29 @@ bool gemm_supported(const wgml_qmat *q) {
     return q->type != WGML_F32 && gemv_fused_supported(q) && q->max_abs <= kGemmMaxWeight;  // the nine quantized formats
 }
 
+// The kernels address a matrix plane with 32-bit lane offsets (at most 1 byte per element).
+bool gemm_addressable(const wgml_qmat *q) {
+    return (uint64_t)q->nrows * q->ncols < (uint64_t(1) << 32) - 4096;
+}
+
+// hipMalloc for a workspace: callers with a path that needs none of it go on with that where the
+// memory is missing (WGML_E_OOM), and only there.
+static int workspace_alloc(void **p, size_t bytes) {
+    const hipError_t e = hipMalloc(p, bytes);
+    if (e == hipSuccess) return WGML_OK;
+    (void)hipGetLastError();  // not the next launch's error
+    *p = nullptr;
+    return set_error(WGML_E_OOM, "prompt workspace: hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
+}
+
 int ensure_prefill_scratch(wgml_ctx *ctx, size_t xh_bytes) {
     if (!ctx->prefill_xscale)
-        WGML_CHECK_HIP(hipMalloc((void **)&ctx->prefill_xscale, kPrefillMaxRun * sizeof(float)));
+        WGML_TRY(workspace_alloc((void **)&ctx->prefill_xscale, kPrefillMaxRun * sizeof(float)));
     if (xh_bytes <= ctx->prefill_xh_bytes) return WGML_OK;
     xh_bytes = (xh_bytes + 255) & ~(size_t)255;
     // two arrays: the f16 activations and, behind them, their low parts (split precision)
     void *xh = nullptr;
-    WGML_CHECK_HIP(hipMalloc(&xh, 2 * xh_bytes));  // without it the old buffer stays in use
+    WGML_TRY(workspace_alloc(&xh, 2 * xh_bytes));  // without it the old buffer stays in use
     // work already enqueued may still read the old buffer: retire it, free with the context
     if (ctx->prefill_xh) ctx->retired.push_back(ctx->prefill_xh);
     ctx->prefill_xh = xh;
@@ -1716,7 +1731,7 @@ int ensure_gemm_partials(wgml_ctx *ctx, size_t bytes) {
     if (bytes <= ctx->gemm_part_bytes) return WGML_OK;
     bytes = (bytes + (size_t(8) << 20)) & ~((size_t(1) << 20) - 1);  // grow in steps
     float *part = nullptr;
-    WGML_CHECK_HIP(hipMalloc((void **)&part, bytes));  // without it the old buffer stays in use
+    WGML_TRY(workspace_alloc((void **)&part, bytes));  // without it the old buffer stays in use
     if (ctx->gemm_part) ctx->retired.push_back(ctx->gemm_part);  // may still be read by queued work
     ctx->gemm_part = part;
     ctx->gemm_part_bytes = bytes;
@@ -1742,8 +1757,7 @@ int launch_gemm_quant_multi(wgml_ctx *ctx, const GemmTarget *targets, int n, con
                              "gemm_quant: a weight of magnitude up to %g does not fit the f16 operands of "
                              "the batched product (up to %g only); use the per-token product",
                              (double)q->max_abs, (double)kGemmMaxWeight);
-        // the kernel addresses a matrix plane with 32-bit lane offsets (at most 1 byte per element)
-        if ((uint64_t)q->nrows * q->ncols >= (uint64_t(1) << 32) - 4096)
+        if (!gemm_addressable(q))
             return set_error(WGML_E_UNSUPPORTED, "gemm_quant: a matrix of %u x %u elements (below 2^32 only)",
                              q->nrows, q->ncols);
         GemmMat &g = a.m[i];
