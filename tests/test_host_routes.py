@@ -118,3 +118,18 @@ def test_only_missing_memory_sends_a_prompt_down_the_slower_path(runtime):
     assert failure(lambda: sampled(m)) == _lib.E_HIP
     assert failure(lambda: g.generate_greedy(prompt, 23)) == _lib.E_HIP
     """)
+
+
+def test_partial_sums_of_growing_prompts_keep_little_memory(runtime):
+    # buffers that were outgrown stay with the context; a buffer holds at most 136 MiB here
+    host_hip.run(runtime, """
+    def kept(lengths):
+        m = llama(W.GpuInstance(0), Llama2Config(4096, 11008, 1, 32, 32, 331, 1100))
+        before = fake.host_hip_allocated()
+        for n in lengths:
+            m.prefill(np.zeros(n, np.uint32))
+        return fake.host_hip_allocated() - before
+
+    assert kept(range(1, 1025, 3)) - kept((1, 1024)) <= 2 * 136 << 20
+    assert kept(range(1, 129)) - kept((1,)) <= 2 * 136 << 20
+    """)

@@ -1729,12 +1729,20 @@ int launch_gemm_flush(wgml_ctx *ctx, float *x, uint32_t x_stride, const float *x
 
 int ensure_gemm_partials(wgml_ctx *ctx, size_t bytes) {
     if (bytes <= ctx->gemm_part_bytes) return WGML_OK;
-    bytes = (bytes + (size_t(8) << 20)) & ~((size_t(1) << 20) - 1);  // grow in steps
+    // Old buffers stay until the context goes (queued work, or a graph the caller recorded, may read
+    // them), so each is at least twice the one before, up to what a long run takes at most: together
+    // they are no larger than the last.
+    constexpr size_t kStep = size_t(8) << 20, kUsual = kTilePartBytes + kStep;
+    const size_t need = (bytes + kStep) & ~((size_t(1) << 20) - 1);
+    size_t size = need > 2 * ctx->gemm_part_bytes ? need : 2 * ctx->gemm_part_bytes;
+    if (size > kUsual) size = need > kUsual ? need : kUsual;
     float *part = nullptr;
-    WGML_TRY(workspace_alloc((void **)&part, bytes));  // without it the old buffer stays in use
-    if (ctx->gemm_part) ctx->retired.push_back(ctx->gemm_part);  // may still be read by queued work
+    int rc = workspace_alloc((void **)&part, size);
+    if (rc != WGML_OK && size > need) rc = workspace_alloc((void **)&part, size = need);
+    WGML_TRY(rc);  // without it the old buffer stays in use
+    if (ctx->gemm_part) ctx->retired.push_back(ctx->gemm_part);
     ctx->gemm_part = part;
-    ctx->gemm_part_bytes = bytes;
+    ctx->gemm_part_bytes = size;
     return WGML_OK;
 }
 
