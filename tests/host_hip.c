@@ -13,7 +13,7 @@ static int n_functions;
 static const char *launches[MAX_LAUNCHES];
 static int n_launches;
 static struct { void *p; size_t bytes; } blocks[MAX_BLOCKS];
-static int n_blocks;
+static int n_blocks, n_pinned;
 static size_t allocated, malloc_limit = (size_t)-1;
 static char failing[64];
 static hipError_t last_error;
@@ -26,6 +26,7 @@ void host_hip_clear(void) { n_launches = 0; }
 int host_hip_launches(void) { return n_launches; }
 const char *host_hip_launch(int i) { return launches[i]; }
 size_t host_hip_allocated(void) { return allocated; }
+int host_hip_pinned(void) { return n_pinned; } /* requests for pinned memory so far */
 
 static hipError_t done(hipError_t e) {
     if (e != hipSuccess) last_error = e;
@@ -102,7 +103,7 @@ hipError_t hipMalloc(void **p, size_t bytes) {
     return e;
 }
 hipError_t hipFree(void *p) { allocated -= take(p); return hipSuccess; }
-hipError_t hipHostMalloc(void **p, size_t bytes, unsigned flags) { (void)flags; return give(p, bytes); }
+hipError_t hipHostMalloc(void **p, size_t bytes, unsigned flags) { (void)flags; ++n_pinned; return give(p, bytes); }
 hipError_t hipHostFree(void *p) { take(p); return hipSuccess; }
 hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind k) {
     (void)k;

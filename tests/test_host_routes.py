@@ -133,3 +133,13 @@ def test_partial_sums_of_growing_prompts_keep_little_memory(runtime):
     assert kept(range(1, 1025, 3)) - kept((1, 1024)) <= 2 * 136 << 20
     assert kept(range(1, 129)) - kept((1,)) <= 2 * 136 << 20
     """)
+
+
+def test_longer_prompts_pin_no_new_memory(runtime):
+    host_hip.run(runtime, """
+    m = llama(gpu, Llama2Config(256, 512, 2, 4, 2, 331, 400))
+    before = fake.host_hip_pinned()
+    for n in (1, 6, 7, 12, 40, 128, 129, 5):
+        assert m.generate_sampled(np.zeros(n, np.uint32), n + 9, 0.7, 0.9, 1).size == n + 9
+    assert fake.host_hip_pinned() == before + 1
+    """)

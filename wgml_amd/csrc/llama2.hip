@@ -56,8 +56,7 @@ struct wgml_llama2 {
     // state of the batched prompt pass, allocated at its first use: one row per token
     // of a run (up to kPrefillMaxTokens)
     float *pf_x = nullptr, *pf_xb = nullptr, *pf_q = nullptr, *pf_hb = nullptr, *pf_hb2 = nullptr;
-    float *h_logits = nullptr;  // pinned host memory for logits (generate_sampled)
-    size_t h_logits_n = 0;
+    float *h_logits = nullptr;  // pinned host memory for kHostRows rows of logits (generate_sampled)
     float *pf_logits = nullptr;  // of every token of a run (generate_sampled)
     uint32_t pf_rows = 0;  // tokens the pf_ buffers hold
     uint32_t *pf_tokens = nullptr;
@@ -630,20 +629,21 @@ int enqueue_read_logits(wgml_llama2 *m, float *host_out) {
     return WGML_OK;
 }
 
-// Pinned host memory for n logits, kept with the model (at most a run's rows): a copy to it needs no
-// staging and runs beside the host's work.  Null where there is none.
-float *reserve_host_logits(wgml_llama2 *m, size_t n) {
-    if (m->h_logits_n >= n) return m->h_logits;
-    (void)hipStreamSynchronize(m->ctx->stream);
-    if (m->h_logits) (void)hipHostFree(m->h_logits);
-    m->h_logits = nullptr;
-    m->h_logits_n = 0;
-    if (hipHostMalloc((void **)&m->h_logits, n * 4, hipHostMallocDefault) != hipSuccess) {
+// Rows of logits that generate_sampled keeps on the host: that of the newest position, and two groups
+// of the prompt's rows, one being sampled while the other is on its way.  (With a row for every
+// prompt token, every longer prompt pinned new memory: 128 rows of 128256 logits 23 ms, more than
+// the pass over that prompt saves.)
+constexpr uint32_t kRowGroup = 4, kHostRows = 1 + 2 * kRowGroup;
+
+// Pinned host memory for them, kept with the model: a copy to it needs no staging and runs beside
+// the host's work.  Null where there is none.
+float *reserve_host_logits(wgml_llama2 *m) {
+    if (!m->h_logits &&
+        hipHostMalloc((void **)&m->h_logits, (size_t)kHostRows * m->cfg.vocab_size * 4, hipHostMallocDefault) !=
+            hipSuccess) {
         (void)hipGetLastError();
         m->h_logits = nullptr;
-        return nullptr;
     }
-    m->h_logits_n = n;
     return m->h_logits;
 }
 
@@ -665,8 +665,8 @@ bool can_batch_sampled_prompt(const wgml_llama2 *m) {
 }
 
 // np <= kPrefillMaxTokens prompt tokens from position 0 in one run: cache rows, the logits after
-// every one of them on the host (row after row) and the last ones in m->logits, as np steps leave.
-int prompt_logits(wgml_llama2 *m, const uint32_t *prompt, uint32_t np, float *host) {
+// every one of them in pf_logits (row after row) and the last ones in m->logits, as np steps leave.
+int enqueue_prompt_logits(wgml_llama2 *m, const uint32_t *prompt, uint32_t np) {
     const wgml_llama2_config &c = m->cfg;
     wgml_ctx *ctx = m->ctx;
     const size_t row = (size_t)c.vocab_size * 4;
@@ -683,11 +683,36 @@ int prompt_logits(wgml_llama2 *m, const uint32_t *prompt, uint32_t np, float *ho
                                np, nullptr, 0));
     WGML_CHECK_HIP(hipMemcpyAsync(m->logits, m->pf_logits + (size_t)(np - 1) * c.vocab_size, row,
                                   hipMemcpyDeviceToDevice, ctx->stream));
-    WGML_CHECK_HIP(hipMemcpyAsync(host, m->pf_logits, row * np, hipMemcpyDeviceToHost, ctx->stream));
-    WGML_CHECK_HIP(hipStreamSynchronize(ctx->stream));
     m->launches_last = (ctx->launches - launches0) / np;
     return WGML_OK;
 }
+
+// The samples of a prompt's positions before its last, drawn on the host in order from the rows that
+// enqueue_prompt_logits leaves: a group of rows is sampled while the next one is on its way.
+struct PromptSamples {
+    wgml_llama2 *m;
+    float *host;     // two groups of rows
+    uint32_t n;      // positions to sample
+    uint32_t next = 0;
+
+    float *row(uint32_t pos) const { return host + (size_t)(pos % (2 * kRowGroup)) * m->cfg.vocab_size; }
+    // Enqueues the copy of the group that starts at position `first`, to where the group before the
+    // one being sampled was.  It is there once the stream has been synchronised.
+    int fetch(uint32_t first) {
+        if (first >= n) return WGML_OK;
+        const uint32_t rows = n - first < kRowGroup ? n - first : kRowGroup;
+        WGML_CHECK_HIP(hipMemcpyAsync(row(first), m->pf_logits + (size_t)first * m->cfg.vocab_size,
+                                      (size_t)rows * m->cfg.vocab_size * 4, hipMemcpyDeviceToHost, m->ctx->stream));
+        return WGML_OK;
+    }
+    template <class Sample>
+    int draw(Sample &&sample) {
+        if (next % kRowGroup == 0) WGML_TRY(fetch(next + kRowGroup));
+        WGML_TRY(sample(row(next), next));
+        ++next;
+        return WGML_OK;
+    }
+};
 
 }  // namespace
 
@@ -1025,49 +1050,45 @@ int wgml_llama2_generate_sampled(wgml_llama2 *m, const uint32_t *prompt, uint32_
     const uint32_t vocab = m->cfg.vocab_size, np = n_prompt < n_total ? n_prompt : n_total;
     std::vector<float> coins(n_total);
     WGML_TRY(wgml_rng_uniform_f32(seed, coins.data(), n_total));
-    // The logits of the positions not yet sampled; [0, np) are the prompt's.  What is sampled inside
-    // the prompt is returned but not fed back (the prompt's next token wins), so those samples are
-    // drawn on the host while the GPU runs the steps that follow.
+    // What is sampled inside the prompt is returned but not fed back (the prompt's next token wins),
+    // so those samples are drawn on the host while the GPU runs the steps that follow.
     WGML_TRY(check_ready(m));
-    float *logits = nullptr;
-    std::vector<float> pageable;
-    uint32_t batched = 0;  // prompt positions whose logits one pass over the prompt has left
-    if (np >= kSampledPromptMin && np <= kPrefillMaxTokens && can_batch_sampled_prompt(m)) {
-        bool valid = true;
-        for (uint32_t i = 0; i < np; ++i) valid = valid && prompt[i] < vocab;
-        if (valid) logits = reserve_host_logits(m, (size_t)np * vocab);
-        if (logits) {
-            const int rc = prompt_logits(m, prompt, np, logits);
-            if (rc == WGML_OK)
-                batched = np;
-            else if (rc != WGML_E_OOM)  // no memory for its workspaces: the steps need none of them
-                return rc;
-        }
-    }
-    if (!batched && !(logits = reserve_host_logits(m, (size_t)2 * vocab))) {
-        pageable.resize((size_t)2 * vocab);
-        logits = pageable.data();
-    }
-    uint32_t open = 0;  // first prompt position still to be sampled
+    float *logits = reserve_host_logits(m);
     auto sample = [&](float *l, uint32_t pos) {
         return wgml_sample(l, vocab, temperature, topp, coins[pos], out_tokens + pos);
     };
+    bool batched = logits && np >= kSampledPromptMin && np <= kPrefillMaxTokens && can_batch_sampled_prompt(m);
+    for (uint32_t i = 0; i < np; ++i) batched = batched && prompt[i] < vocab;
     if (batched) {
-        WGML_TRY(sample(logits + (size_t)(np - 1) * vocab, np - 1));
+        const int rc = enqueue_prompt_logits(m, prompt, np);
+        if (rc == WGML_E_OOM)
+            batched = false;  // no memory for its workspaces: the steps need none of them
+        else
+            WGML_TRY(rc);
+    }
+    if (batched) {
+        PromptSamples inside{m, logits + vocab, np - 1};
+        WGML_TRY(enqueue_read_logits(m, logits));
+        WGML_TRY(inside.fetch(0));
+        WGML_CHECK_HIP(hipStreamSynchronize(m->ctx->stream));
+        WGML_TRY(sample(logits, np - 1));
         for (uint32_t pos = np; pos < n_total; ++pos) {
-            // row np - 1 is free from here on: the steps' logits go there
-            float *row = logits + (size_t)(np - 1) * vocab;
             WGML_TRY(wgml_llama2_forward(m, out_tokens[pos - 1], pos));
-            WGML_TRY(enqueue_read_logits(m, row));
-            if (open + 1 < np) {
-                WGML_TRY(sample(logits + (size_t)open * vocab, open));
-                ++open;
-            }
+            WGML_TRY(enqueue_read_logits(m, logits));
+            if (inside.next < inside.n) WGML_TRY(inside.draw(sample));
             WGML_CHECK_HIP(hipStreamSynchronize(m->ctx->stream));
-            WGML_TRY(sample(row, pos));
+            WGML_TRY(sample(logits, pos));
         }
-        for (; open + 1 < np; ++open) WGML_TRY(sample(logits + (size_t)open * vocab, open));
+        while (inside.next < inside.n) {
+            if (inside.next % kRowGroup == 0) WGML_CHECK_HIP(hipStreamSynchronize(m->ctx->stream));
+            WGML_TRY(inside.draw(sample));
+        }
         return WGML_OK;
+    }
+    std::vector<float> pageable;
+    if (!logits) {
+        pageable.resize((size_t)2 * vocab);
+        logits = pageable.data();
     }
     for (uint32_t pos = 0; pos < n_total; ++pos) {
         const bool forced = pos > 0 && pos < np;
