@@ -2,6 +2,10 @@
 algorithm fixes (closed forms on small distributions, an independent numpy construction of the
 nucleus, the empirical distribution over many coins); the library's sampler must then return
 the oracle's token for every coin.  No GPU needed."""
+import ctypes as C
+import subprocess
+from pathlib import Path
+
 import numpy as np
 import pytest
 
@@ -86,3 +90,54 @@ def test_argument_checks_and_coins():
     c = W.rng_uniform(9, 10000)
     assert c.min() >= 0.0 and c.max() < 1.0 and abs(c.mean() - 0.5) < 0.02
     assert np.array_equal(c[:100], W.rng_uniform(9, 100))
+
+
+def _exp_arguments():
+    """Every 1009th float of [-104, -0], those around -87 (where the sampler hands over to std::exp)
+    and around the smallest results, both zeros and -inf."""
+    bits = np.arange(0x80000000, np.float32(-104).view(np.uint32), 1009, dtype=np.uint64).astype(np.uint32)
+    near = [np.float32(v).view(np.uint32) + np.arange(-40, 41) for v in (-87.0, -87.33655, -103.27893, -0.6931472)]
+    return np.concatenate([bits.view(np.float32), np.concatenate(near).astype(np.uint32).view(np.float32),
+                           np.float32([0.0, -0.0, -np.inf, np.finfo(np.float32).min])])
+
+
+@pytest.fixture(scope="module")
+def exp_block(tmp_path_factory):
+    here = Path(__file__).parent
+    out = tmp_path_factory.mktemp("exp_block") / "exp_block.so"
+    subprocess.run(["g++", "-shared", "-fPIC", "-O2", "-std=c++17", "-ffp-contract=off", "-D__HIP_PLATFORM_AMD__",
+                    "-I/opt/rocm/include", "-o", str(out), str(here / "exp_block.cpp")], check=True,
+                   capture_output=True)
+    return C.CDLL(str(out))
+
+
+@pytest.mark.parametrize("avx2", [0, 1])
+def test_blocks_of_exp_are_std_exp_bit_for_bit(exp_block, avx2):
+    if avx2 and not exp_block.cpu_has_avx2():
+        pytest.skip("no AVX2 on this machine")
+    x = _exp_arguments()
+    p = lambda a: a.ctypes.data_as(C.c_void_p)
+    got, want, asked = np.empty_like(x), np.empty_like(x), C.c_uint32()
+    exp_block.std_exp(p(x), x.size, p(want))
+    exp_block.take_exp(p(x), x.size, avx2, p(got), C.byref(asked))
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+    ordinary = x >= -87  # std::exp answers for about 4 % of these and for all of the others
+    assert asked.value - (~ordinary).sum() < 0.06 * ordinary.sum()
+
+
+# one element, a block short of one, a whole one, one into the next, many
+@pytest.mark.parametrize("n", [1, 255, 256, 257, 4000])
+def test_probabilities_are_those_of_the_oracle_bit_for_bit(n):
+    x = _exp_arguments()
+    rng = np.random.default_rng(n)
+    for trial in range(60):
+        logits = rng.choice(x[x > -30] if trial % 3 else x, n)
+        logits[rng.integers(n)] = 0.0  # the maximum
+        if trial % 4 == 0:
+            logits = logits + np.float32(3.7)
+        got, want = logits.copy(), logits.copy()
+        coin, t = float(W.rng_uniform(trial, 1)[0]), (1.0, 0.7)[trial % 2]
+        a = W.Sampler(None, t, (0.9, 0.0)[trial % 2]).sample(got, coin)
+        b = orc.lib.orc_sample(want.ctypes.data_as(C.c_void_p), n, t, (0.9, 0.0)[trial % 2], coin)
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+        assert a == b
