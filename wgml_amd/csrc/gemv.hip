@@ -1808,18 +1808,21 @@ static bool dense_f32_in_shared_body(const wgml_qmat *m) {
 }
 
 // Plain products (no folded norm or activation) of such matrices that gemv_f32_kernel does faster.
-// In the shared body a lane takes 16 columns of a row, there 4: rows of less than a step of 1024
-// columns leave most of a wave idle here, which costs more than the general kernel's single load in
-// flight while the matrix is small, and at any size for rows of up to 128 columns.  Beyond 64
-// results in each of the machine's waves of rows the body needs a second round of workgroups.
-// Measured, general / shared: 4096x64 2.0 / 3.0 us, 4096x256 2.4 / 3.3, 515x512 2.1 / 2.5, 8192x512
-// 4.6 / 4.8, 50257x128 9.1 / 9.8, 32768x256 7.7 / 8.3, 300001x256 69 / 100; on the other side of the
-// line 515x1024 2.5 / 2.5, 4096x2048 9.0 / 7.2, 12288x768 9.6 / 8.2, 50257x256 13.9 / 13.5, 300001x384
-// 114 / 109.
+// In the shared body a lane takes 16 columns of a row, there 4, so rows of few columns leave most of
+// a wave idle here; but the body requests its weights ahead of x, which the general kernel does
+// behind it, a memory round trip that shows where x comes from the launch before.  Beyond 64
+// results in each of the machine's waves the body needs a second round of workgroups.  General /
+// shared, us, each with x at rest and as part of a chain of dependent products (with the product
+// that leads back to x):
+//     4096x64     2.0 /  3.0    5.9 /  6.7        8192x512    4.6 /  4.8    9.0 /  9.0
+//     4096x256    2.4 /  3.3    6.5 /  6.9        768x768     2.3 /  2.5    6.5 /  5.8
+//     768x512     2.1 /  2.5    5.8 /  5.7        4096x1024   4.7 /  4.8    9.8 /  9.2 (1008)
+//     32768x256   7.7 /  8.3   12.0 / 12.2        50257x256  13.9 / 13.5
+//     50000x128   9.1 /  9.8   13.8 / 14.9        262160x256  69 / 100 (300001)  47 / 82
 static bool dense_f32_general_faster(const wgml_ctx *ctx, uint32_t nrows, uint32_t ncols) {
     const uint32_t cu = ctx->n_cu > 0 ? (uint32_t)ctx->n_cu : 256u;
     if (ncols <= 128) return true;
-    if (ncols < 1024 && nrows <= 8192) return true;
+    if (ncols <= 512 && nrows <= 8192) return true;
     return ncols <= 256 && (nrows <= 32768 || nrows > cu * 16 * 64);
 }
 
