@@ -25,6 +25,12 @@ def test_narrow_dense_matrices_take_the_general_kernel(runtime):
         assert general(*shape), shape
     for shape in ((1, 528), (768, 768), (17, 4096), (8193, 272), (8193, 512), (32769, 256), (262144, 256), (262145, 272)):
         assert not general(*shape), shape
+
+    # folded norms (fusion level 2: Q, K, V, gate, up, output): the general kernel up to 128 columns
+    for dim, hidden, n_general in ((128, 352, 8), (288, 768, 1)):
+        m = llama(gpu, Llama2Config(dim, hidden, 1, 4, 4, 331, 64), W.F32)
+        m.set_fusion(2)
+        assert count(launched(lambda: m.forward(0, 0)), "gemv_f32_kernel") == n_general, dim
     """)
 
 

@@ -1807,7 +1807,7 @@ static bool dense_f32_in_shared_body(const wgml_qmat *m) {
     return m->type == WGML_F32 && m->ncols % FmtF32::TILE == 0 && (size_t)m->ncols * 4 <= kMaxLds;
 }
 
-// Plain products (no folded norm or activation) of such matrices that gemv_f32_kernel does faster.
+// Products of such matrices (without LayerNorm or activation) that gemv_f32_kernel does faster.
 // In the shared body a lane takes 16 columns of a row, there 4, so rows of few columns leave most of
 // a wave idle here; but the body requests its weights ahead of x, which the general kernel does
 // behind it, a memory round trip that shows where x comes from the launch before.  Beyond 64
@@ -1819,9 +1819,12 @@ static bool dense_f32_in_shared_body(const wgml_qmat *m) {
 //     768x512     2.1 /  2.5    5.8 /  5.7        4096x1024   4.7 /  4.8    9.8 /  9.2 (1008)
 //     32768x256   7.7 /  8.3   12.0 / 12.2        50257x256  13.9 / 13.5
 //     50000x128   9.1 /  9.8   13.8 / 14.9        262160x256  69 / 100 (300001)  47 / 82
-static bool dense_f32_general_faster(const wgml_ctx *ctx, uint32_t nrows, uint32_t ncols) {
+// A folded RMSNorm makes the general kernel pass over x twice: up to 128 columns it is the faster one
+// still (a Llama of dimension 128 at fusion level 2, 40 tokens: 4.29 / 4.40 ms; of 288: 8.0 / 7.0).
+static bool dense_f32_general_faster(const wgml_ctx *ctx, uint32_t nrows, uint32_t ncols, bool norm) {
     const uint32_t cu = ctx->n_cu > 0 ? (uint32_t)ctx->n_cu : 256u;
     if (ncols <= 128) return true;
+    if (norm) return false;
     if (ncols <= 512 && nrows <= 8192) return true;
     return ncols <= 256 && (nrows <= 32768 || nrows > cu * 16 * 64);
 }
@@ -1870,7 +1873,7 @@ int launch_gemv_quant(wgml_ctx *ctx, float *out, const wgml_qmat *m, const float
     }
     (void)main_fmt;
     if (dense_f32_in_shared_body(m) &&
-        (p.ln_g || p.act || p.norm_w || !dense_f32_general_faster(ctx, p.nrows, p.ncols)))
+        (p.ln_g || p.act || !dense_f32_general_faster(ctx, p.nrows, p.ncols, p.norm_w != nullptr)))
         return launch_fmt_f32<FmtF32>(ctx, p);
     if ((p.ln_g || p.act) && m->type == WGML_F32)
         return set_error(WGML_E_UNSUPPORTED, "gemv_quant: LayerNorm / activation folding needs rows of a "
