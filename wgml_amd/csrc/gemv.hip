@@ -1802,6 +1802,12 @@ int launch_gemv_f32(wgml_ctx *ctx, float *out, const float *a, uint32_t nrows, u
     return WGML_OK;
 }
 
+// Dense f32 in the shared body.  Defined behind everything else in this file, so that its kernels
+// come last in the code object: between the others they moved those by 10 to 30 KB, and decoding the
+// 7B shape took 22.82 ms for 16 tokens instead of 22.69, with the same instructions.
+static int launch_dense_f32(wgml_ctx *ctx, const GemvParams &p);
+static void (*dense_f32_fused_kernel(int threads))(const FusedParams);
+
 // Dense f32 matrices that run in the shared body: whole tiles, and x within the LDS limit.
 static bool dense_f32_in_shared_body(const wgml_qmat *m) {
     return m->type == WGML_F32 && m->ncols % FmtF32::TILE == 0 && (size_t)m->ncols * 4 <= kMaxLds;
@@ -1874,7 +1880,7 @@ int launch_gemv_quant(wgml_ctx *ctx, float *out, const wgml_qmat *m, const float
     (void)main_fmt;
     if (dense_f32_in_shared_body(m) &&
         (p.ln_g || p.act || !dense_f32_general_faster(ctx, p.nrows, p.ncols, p.norm_w != nullptr)))
-        return launch_fmt_f32<FmtF32>(ctx, p);
+        return launch_dense_f32(ctx, p);
     if ((p.ln_g || p.act) && m->type == WGML_F32)
         return set_error(WGML_E_UNSUPPORTED, "gemv_quant: LayerNorm / activation folding needs rows of a "
                                              "multiple of 16 elements");
@@ -2054,7 +2060,7 @@ static int launch_gemv_fused_variant(wgml_ctx *ctx, const FusedGemv &f, uint32_t
     // spilling, and the waves of a workgroup start sooner the fewer registers they take
     void (*kern)(const FusedParams) = gemv_fused_kernel<D, MAXT, (MAXT == 1024 ? 5 : MINW), 0>;
     if (fmt == kFusedDenseF32) {
-        kern = gemv_fused_kernel<D, MAXT, MINW, kFusedDenseF32, true>;
+        kern = dense_f32_fused_kernel(MAXT);
     } else if (f32) {
         kern = gemv_fused_kernel<D, MAXT, MINW, 0, true>;
         switch (fmt) {
@@ -2172,3 +2178,14 @@ int wgml_gemv_f32(wgml_ctx *ctx, wgml_view out, wgml_view a, uint32_t nrows, uin
 }
 
 }  // extern "C"
+
+namespace wgml {
+
+static int launch_dense_f32(wgml_ctx *ctx, const GemvParams &p) { return launch_fmt_f32<FmtF32>(ctx, p); }
+
+static void (*dense_f32_fused_kernel(int threads))(const FusedParams) {
+    return threads == 768 ? gemv_fused_kernel<1, 768, 1, kFusedDenseF32, true>
+                          : gemv_fused_kernel<1, 1024, 1, kFusedDenseF32, true>;
+}
+
+}  // namespace wgml
