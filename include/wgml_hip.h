@@ -94,7 +94,9 @@ enum {
                                                 (single-matrix launches then use 16) */
     WGML_TUNE_GEMV_WG_PER_CU,                /* cap on resident workgroups per compute unit, 1..8 */
     WGML_TUNE_GEMV_DEPTH,                    /* weight tiles in flight per wave, 1..4 */
-    WGML_TUNE_GEMV_F32_ACTIVATIONS,          /* 1: fp32 activations instead of 16-bit block fixed point */
+    WGML_TUNE_GEMV_F32_ACTIVATIONS,          /* 1: fp32 activations instead of 16-bit block fixed point
+                                                (wgml_llama2_generate_sampled and wgml_gpt2_generate_greedy
+                                                then step through their prompts) */
     WGML_TUNE_GEMM_K_SPLIT,                  /* 1..8 workgroups share the K range of a batched product */
     WGML_TUNE_PREFILL_ATTENTION_PER_TOKEN,   /* 1: one workgroup per (head, token) in the prompt pass */
     WGML_TUNE_ATTN_WIDE_POSITIONS,           /* decode attention planned for up to this many positions
@@ -183,7 +185,10 @@ WGML_API int wgml_gemv_quant(wgml_ctx *ctx, wgml_view out, const wgml_qmat *m, w
  * and 65504 is the largest finite f16): a bound on the largest weight is computed when the
  * matrix is created, and a matrix whose bound is larger is refused with WGML_E_UNSUPPORTED
  * (wgml_gemv_quant takes any value;
- * wgml_llama2_prefill steps through the prompt token by token for such a model). */
+ * wgml_llama2_prefill steps through the prompt token by token for such a model).
+ * Level 0 also makes wgml_llama2_generate_sampled and wgml_gpt2_generate_greedy step
+ * through their prompts, which is slower: they take them in one pass only where that is
+ * at least as precise as the steps. */
 WGML_API int wgml_ctx_set_gemm_precision(wgml_ctx *ctx, int level);
 WGML_API int wgml_gemm_quant(wgml_ctx *ctx, wgml_view out, const wgml_qmat *m, wgml_view x,
                              uint32_t n_tokens);
@@ -363,9 +368,10 @@ WGML_API int wgml_llama2_decode_greedy_sync(wgml_llama2 *m, uint32_t first_token
  * state those n_tokens steps leave behind -- KV-cache rows start_pos ..
  * start_pos + n_tokens - 1 of every layer and the logits of the last token (read
  * them with wgml_llama2_read_logits) -- with every matrix-vector product of the
- * step replaced by one product with up to 128 token vectors on the matrix cores
- * (as wgml_gemm_quant; longer prompts go through in runs of up to 1024).  The layer matrices
- * are multiplied at the precision set with wgml_ctx_set_gemm_precision (default:
+ * step replaced by one product with the vectors of a run of up to 1024 tokens on the
+ * matrix cores (the arithmetic of wgml_gemm_quant; longer prompts go through in several
+ * runs, and in runs of 128 where there is no memory for the workspaces of longer ones or a
+ * matrix has 2^20 columns or more).  The layer matrices are multiplied at the precision set with wgml_ctx_set_gemm_precision (default:
  * to fp32 rounding); norms, RoPE, attention and the output matrix are fp32 as in
  * the step, so with the default the logits agree with the step-by-step pass as two
  * fp32 implementations do (2e-4 of their range is the bound the tests use); with
@@ -430,7 +436,9 @@ WGML_API int wgml_gpt2_set_embeddings(wgml_gpt2 *m, const float *wte, const floa
 /* Gpt2::dispatch (models/gpt2/transformer.rs:265-477). */
 WGML_API int wgml_gpt2_forward(wgml_gpt2 *m, uint32_t token, uint32_t pos);
 WGML_API int wgml_gpt2_read_logits(wgml_gpt2 *m, float *host_out);
-/* ChatGpt2::forward's loop with greedy sampling (wgml-chat/src/chat_gpt2.rs:43-151). */
+/* ChatGpt2::forward's loop with greedy sampling (wgml-chat/src/chat_gpt2.rs:43-151).  A
+ * prompt of 8 tokens and more goes through the layers in runs of up to 128, on the same
+ * conditions as in wgml_llama2_generate_sampled (fusion level 1). */
 WGML_API int wgml_gpt2_generate_greedy(wgml_gpt2 *m, const uint32_t *prompt, uint32_t n_prompt,
                                        uint32_t n_total, uint32_t *out_tokens);
 /* As wgml_llama2_record_steps, for positions 0 .. n_total - 1. */
@@ -548,7 +556,11 @@ WGML_API int wgml_sample(float *logits, uint32_t n, float temperature, float top
 /* The token loop of ChatLlama2::forward with that sampler (chat_llama2.rs:51-153;
  * the reference uses temperature 0.7, top-p 0.95 there, wgml-chat/src/sampler.rs:109):
  * logits are read back after every step and sampled on the host; the coin of position
- * p is the p-th output of the library's counter-based generator for `seed`. */
+ * p is the p-th output of the library's counter-based generator for `seed`.
+ * A prompt of 6 to 128 tokens goes through the layers and the output matrix in one pass
+ * (as wgml_llama2_prefill) where every matrix has a batched product, the gemm precision is
+ * the default, activations are not fp32 and the fusion level is at least 1; its samples are
+ * drawn while later steps run.  Other prompts take a step per token. */
 WGML_API int wgml_llama2_generate_sampled(wgml_llama2 *m, const uint32_t *prompt,
                                           uint32_t n_prompt, uint32_t n_total, float temperature,
                                           float topp, uint64_t seed, uint32_t *out_tokens);

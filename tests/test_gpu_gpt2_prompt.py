@@ -4,8 +4,8 @@ A context with plain-f16 products leaves the prompt to the steps, so the same mo
 The step's products take their input as 16-bit block fixed point (up to 1e-3 of the largest logit
 over a whole model, the bound of test_gpu_models.py), the batched ones are exact to fp32 rounding:
 about 1e-6 of a row's magnitude each, so that the logits after a prompt are within PROMPT of the
-oracle's (three layers of four products and the output matrix; 1.2e-6 measured).  LayerNorm or GELU rows without their
-low halves would put them off by 7e-5 to 4e-4 here.
+oracle's (three layers of four products and the output matrix; 1.2e-6 measured).  LayerNorm or GELU
+rows without their low halves would put them off by 7e-5 to 4e-4 here.
 """
 import numpy as np
 import pytest

@@ -46,7 +46,6 @@ struct wgml_gpt2 {
     uint64_t launches_last = 0;   // launches of the last step that ran
     // workspaces of the batched prompt pass, for kPrefillMaxTokens tokens (allocated on first use)
     float *pf_x = nullptr, *pf_qkv = nullptr, *pf_att = nullptr, *pf_h = nullptr, *pf_logits = nullptr;
-    uint32_t *pf_tokens = nullptr;
 };
 
 namespace {
@@ -513,15 +512,17 @@ int record_steps(wgml_gpt2 *m, uint32_t n_total) {
     return WGML_OK;
 }
 
-// Prompts of at least this many tokens go through the layers together.  A run is 14 launches of
-// 5-10 us per layer whatever its length, a step 5 launches of 4 us: eight steps cost more.
-// GPT-2 124M in Q8_0, 32 prompt tokens and 96 generated: 27.1 ms against 34.5 in steps.
+// Prompts of at least this many tokens go through the layers together.  A run is 11 launches of
+// 3-12 us per layer whatever its length, a step 5 or 6 of 3-6 us.  Measured, 8 tokens and nothing
+// behind them: 124M in Q8_0 0.95 ms against 2.11 in steps, 12 layers of 1024 in Q4_K 0.97 / 2.29, 2
+// layers of 256 0.18 / 0.39, so the lines cross near 4 tokens (shorter runs were not timed).
+// 32 prompt tokens and 96 generated, 124M: 27.0 ms against 34.3.
 constexpr uint32_t kBatchedPromptMin = 8;
 
 // The batched products take quantized matrices; the split-f16 form of them is closer to 64 bits than
 // the step's 16-bit fixed point (plain f16 is not, and fp32 activations are closer still: those
 // settings leave the prompt to the steps); attention over a run takes head sizes that are multiples
-// of 4.
+// of 4 up to 256 (the model has none above), LayerNorm rows of up to 16384 (can_fold: 12288).
 bool can_batch_prompt(const wgml_gpt2 *m) {
     const uint32_t n = m->p.n_embd;
     if (!m->ctx->gemm_precise || m->ctx->tuning[WGML_TUNE_GEMV_F32_ACTIVATIONS] || (n / m->p.n_head) % 4 != 0 || n % 8 != 0)
@@ -544,7 +545,7 @@ int reserve_prompt(wgml_gpt2 *m) {
             return d;
         };
         float *x = A(T * p.n_embd), *qkv = A(T * 3 * p.n_embd), *att = A(T * p.n_embd), *h = A(T * p.ff_len);
-        float *logits = A(T * p.n_vocab), *tokens = A(T);
+        float *logits = A(T * p.n_vocab);
         if (rc != WGML_OK) {  // all of them or none: a later call must not find less memory
             for (; m->allocs.size() > kept; m->allocs.pop_back()) (void)hipFree(m->allocs.back());
             return rc;
@@ -554,7 +555,6 @@ int reserve_prompt(wgml_gpt2 *m) {
         m->pf_att = att;
         m->pf_h = h;
         m->pf_logits = logits;
-        m->pf_tokens = reinterpret_cast<uint32_t *>(tokens);
     }
     const uint32_t kmax = p.n_embd > p.ff_len ? p.n_embd : p.ff_len;
     return ensure_prefill_scratch(m->ctx, (size_t)kPrefillMaxTokens * prefill_kpad(kmax) * 2);

@@ -63,7 +63,9 @@ class GpuInstance:
 
     def set_gemm_precision(self, level: int) -> None:
         """Batched products (GemmQuant, Llama2.prefill): 1 = split-f16 operands, results to fp32
-        rounding (default); 0 = plain f16 operands, faster, about 3e-4 of a row's magnitude."""
+        rounding (default); 0 = plain f16 operands, faster, about 3e-4 of a row's magnitude.  At 0
+        Llama2.generate_sampled and Gpt2.generate_greedy step through their prompts (slower): they
+        take them in one pass only where that is at least as precise."""
         call("wgml_ctx_set_gemm_precision", self._h, level)
 
     def info(self):
