@@ -71,6 +71,7 @@ struct wgml_ctx {
     // grown on demand
     void *prefill_xh = nullptr;
     void *prefill_xl = nullptr;  // low parts of the same activations (inside the same allocation)
+    void *prefill_xsum = nullptr;  // sums of 32 activations, behind the low parts
     size_t prefill_xh_bytes = 0;
     int gemm_precise = 1;  // batched products: 1 = split-f16 operands (fp32-grade), 0 = f16
     float *prefill_xscale = nullptr;
@@ -120,8 +121,8 @@ struct wgml_qmat {
     float max_abs = 0.f;
 };
 
-// The batched products (prefill.hip) expand weights into f16 times 2^8: a dequantized weight
-// beyond 65504 / 2^8 (the largest finite f16) would round to infinity there, so a matrix whose
+// The batched products (gemm_kernel.h) may round a weight to f16, times 2^8: a dequantized weight
+// beyond 65504 / 2^8 (the largest finite f16) would be infinite there, so a matrix whose
 // bound exceeds this goes through the per-token kernels, which take any f32 value.
 constexpr float kGemmMaxWeight = 65504.f / 256.f;  // 255.875
 
@@ -304,8 +305,8 @@ int launch_dequantize(wgml_ctx *ctx, float *out, const wgml_qmat *m);
 // ---- batched products for prompt processing (prefill.hip) ---------------------
 constexpr uint32_t kPrefillMaxTokens = 128;  // of one product through the public entry point
 constexpr uint32_t kPrefillMaxRun = 1024;    // of one run of a prompt pass (more than 128: wider tiles)
-uint32_t prefill_tpad(uint32_t T);  // tokens rounded up to 16, 32, 64, 128 or a multiple of 256
-uint32_t prefill_kpad(uint32_t K);  // columns rounded up to a multiple of 128
+uint32_t prefill_tpad(uint32_t T);  // tokens rounded up to 16, 32, 48, 64, 96, 128 or a multiple of 256
+uint32_t prefill_kpad(uint32_t K);  // columns rounded up to a multiple of 256
 int ensure_prefill_scratch(wgml_ctx *ctx, size_t xh_bytes);
 // xh[tpad][kpad] (f16) <- x[T][K] (f32, rows x_stride apart): RMS-normalised with
 // norm_w first when that is non-null; replaced by up[t][k] * silu(x[t][k]) when `up`

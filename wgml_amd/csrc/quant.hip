@@ -416,6 +416,11 @@ int wgml_quant_matrix_create(wgml_ctx *ctx, int type, uint32_t nrows, uint32_t n
                          hipGetErrorString(err));
     };
 
+    // The batched products read whole units of 256 columns: behind a last row that ends inside one
+    // they multiply what follows the last block by zeros, so there are no NaN scales there.
+    const uint64_t end = type == WGML_Q8_0 ? o1 + nblocks * 2 : type == WGML_Q6_K ? o3 + nblocks * 2 : m->gguf_bytes;
+    e = hipMemsetAsync(m->base + end, 0, total - end, ctx->stream);
+    if (e != hipSuccess) return fail(e, "spare bytes");
     if (kept_raw(type)) {
         e = hipMemcpyAsync(m->base, gguf_bytes, gguf, hipMemcpyHostToDevice, ctx->stream);
         if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
