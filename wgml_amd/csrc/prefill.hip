@@ -105,6 +105,9 @@ __global__ __launch_bounds__(256) void gemm_reduce_rope_kernel(const GemmArgs a)
     }
 }
 
+// Bound by its chain of one memory trip (row, partial sums and norm weights together), a reduction and
+// a store: 8.4 us for 128 rows of 4096 that add four partial sums, 5.8 us for 21 rows of 3072 (9.5 and 6.4 with
+// the weights requested after the first of two reductions).
 // One workgroup per token: X[t] (fp32, optionally RMS-normalised with weights w as
 // the reference does: (x * rsqrt(mean(x^2) + eps)) * w, ops/rms_norm.rs:55-63) -> f16
 // in the packed order described at the top, times the power of two that brings the row's
@@ -142,14 +145,28 @@ __device__ __forceinline__ void add_part_batch(float (&acc)[N][8], const float *
         }
     }
 }
-// all ks parts, four, two or one at a time
+// all ks parts, eight (of one row), four, two or one at a time
 template <int N>
 __device__ __forceinline__ void add_parts(float (&acc)[N][8], const float *__restrict__ part, size_t ystride,
                                           const size_t (&off)[N], uint32_t ks) {
     uint32_t y = 0;
+    if (N == 1)
+        for (; y + 8 <= ks; y += 8) add_part_batch<8, N>(acc, part, ystride, off, y);
     for (; y + 4 <= ks; y += 4) add_part_batch<4, N>(acc, part, ystride, off, y);
     for (; y + 2 <= ks; y += 2) add_part_batch<2, N>(acc, part, ystride, off, y);
     for (; y < ks; ++y) add_part_batch<1, N>(acc, part, ystride, off, y);
+}
+
+__device__ __forceinline__ void load8(float (&o)[8], const float *p) {  // 16-byte aligned
+    const float4 a = reinterpret_cast<const float4 *>(p)[0], b = reinterpret_cast<const float4 *>(p)[1];
+    o[0] = a.x;
+    o[1] = a.y;
+    o[2] = a.z;
+    o[3] = a.w;
+    o[4] = b.x;
+    o[5] = b.y;
+    o[6] = b.z;
+    o[7] = b.w;
 }
 
 constexpr int PREP_THREADS = 1024;
@@ -167,7 +184,7 @@ __global__ __launch_bounds__(PREP_THREADS) void prep_x_kernel(float *__restrict_
                                                      _Float16 *__restrict__ xsum,
                                                      float *__restrict__ xscale, uint32_t K,
                                                      uint32_t kpad, uint32_t T, uint32_t nt) {
-    __shared__ float red[16];
+    __shared__ float red[32];
     const uint32_t t = blockIdx.x, tid = threadIdx.x;
     // 16-byte word of (token t, columns 8 k8 .. 8 k8 + 7)
     auto word_index = [&](uint32_t k8) {
@@ -184,8 +201,9 @@ __global__ __launch_bounds__(PREP_THREADS) void prep_x_kernel(float *__restrict_
     // columns per thread and group, and kept in registers (v); longer rows are re-read from
     // memory by the later passes.  (K is a multiple of 32 for every quantized format.)
     const bool cached = ngroups <= PREP_GROUPS * PREP_THREADS && K % 8 == 0 && x_stride % 4 == 0 &&
-                        ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(up) |
-                          reinterpret_cast<uintptr_t>(part)) & 15u) == 0;  // 16-byte loads below
+                        ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(up_or_beta) |
+                          reinterpret_cast<uintptr_t>(norm_w) | reinterpret_cast<uintptr_t>(part)) & 15u) == 0;
+    // (16-byte loads below)
     // the product before this kernel may have left  x[t] += xscale[t] * (part[0][t] + part[1][t]
     // + ...)  to be done here (part: [part_ks][T][K], xscale[t] still that product's factor)
     // With part_pair the partial sums are 2 K wide and hold a gate product in [0, K) and an up
@@ -202,6 +220,21 @@ __global__ __launch_bounds__(PREP_THREADS) void prep_x_kernel(float *__restrict_
         __syncthreads();  // every thread reads what others wrote (same workgroup only)
     }
     float v[PREP_GROUPS][8];
+    // the norm's weights, requested together with the row: after the reductions they would be one more
+    // trip to memory
+    const bool normed = MODE != PREP_GELU && norm_w;
+    float nw[PREP_GROUPS][8], nb[PREP_GROUPS][8];
+    if (cached && normed) {
+#pragma unroll
+        for (int i = 0; i < PREP_GROUPS; ++i) {
+            const uint32_t k0 = 8 * (tid + i * PREP_THREADS);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) nw[i][e] = nb[i][e] = 0.f;
+            if (k0 >= K) continue;
+            load8(nw[i], norm_w + k0);
+            if (MODE == PREP_LN) load8(nb[i], up_or_beta + k0);
+        }
+    }
     auto raw = [&](uint32_t k) -> float {  // the value before normalisation
         if (k >= K) return 0.f;
         const float xv = xr[k];
@@ -253,6 +286,7 @@ __global__ __launch_bounds__(PREP_THREADS) void prep_x_kernel(float *__restrict_
         }
     }
     float rs = 1.f, mean = 0.f;
+    auto value = [&](uint32_t k, float r) { return normed && k < K ? (r * rs) * norm_w[k] : r; };  // not cached
     if (MODE == PREP_LN) {  // in registers only (the launcher sees to that)
         float sum = 0.f;
 #pragma unroll
@@ -270,47 +304,66 @@ __global__ __launch_bounds__(PREP_THREADS) void prep_x_kernel(float *__restrict_
             }
         }
         rs = 1.0f / sqrtf(block_sum(ss, red) / (float)K + eps);
-    } else if (MODE == PREP_RMS && norm_w) {
-        float ss = 0.f;
-        if (cached) {
-#pragma unroll
-            for (int i = 0; i < PREP_GROUPS; ++i) {
-#pragma unroll
-                for (int e = 0; e < 8; ++e) ss = fmaf(v[i][e], v[i][e], ss);
-            }
-        } else {
-            for (uint32_t k = tid; k < K; k += PREP_THREADS) ss = fmaf(xr[k], xr[k], ss);
-        }
-        rs = 1.0f / sqrtf(block_sum(ss, red) / (float)K + eps);
     }
-    auto value = [&](uint32_t k, float r) {
-        if constexpr (MODE == PREP_LN) return k < K ? ((r - mean) * rs) * norm_w[k] + up_or_beta[k] : r;
-        return MODE == PREP_RMS && norm_w && k < K ? (r * rs) * norm_w[k] : r;
-    };
     float amax = 0.f;
-    if (cached) {
+    if (MODE == PREP_RMS && normed && cached) {
+        // The sum of squares and the largest |x w| in one reduction: the factor between them is
+        // positive and the same for the whole row, and only a power of two is taken from the largest value.
+        float ss = 0.f;
 #pragma unroll
         for (int i = 0; i < PREP_GROUPS; ++i) {
-            const uint32_t k0 = 8 * (tid + i * PREP_THREADS);
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-                v[i][e] = value(k0 + e, v[i][e]);
+                ss = fmaf(v[i][e], v[i][e], ss);
+                amax = fmaxf(amax, fabsf(v[i][e] * nw[i][e]));
+            }
+        }
+        ss = wave_sum(ss);
+        amax = wave_max(amax);
+        if ((tid & 63) == 0) {
+            red[tid >> 6] = ss;
+            red[16 + (tid >> 6)] = amax;
+        }
+        __syncthreads();
+        ss = 0.f;
+#pragma unroll
+        for (int w = 0; w < PREP_THREADS / 64; ++w) {
+            ss += red[w];
+            amax = fmaxf(amax, red[16 + w]);
+        }
+        rs = 1.0f / sqrtf(ss / (float)K + eps);
+        amax *= rs;
+#pragma unroll
+        for (int i = 0; i < PREP_GROUPS; ++i) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[i][e] = (v[i][e] * rs) * nw[i][e];
+        }
+    } else if (cached) {
+#pragma unroll
+        for (int i = 0; i < PREP_GROUPS; ++i) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                if (MODE == PREP_LN) v[i][e] = ((v[i][e] - mean) * rs) * nw[i][e] + nb[i][e];
                 amax = fmaxf(amax, fabsf(v[i][e]));
             }
         }
+        amax = block_max(amax, red);
     } else {
+        if (normed) {
+            float ss = 0.f;
+            for (uint32_t k = tid; k < K; k += PREP_THREADS) ss = fmaf(xr[k], xr[k], ss);
+            rs = 1.0f / sqrtf(block_sum(ss, red) / (float)K + eps);
+        }
         for (uint32_t k = tid; k < K; k += PREP_THREADS) amax = fmaxf(amax, fabsf(value(k, raw(k))));
+        amax = block_max(amax, red);
     }
-    amax = block_max(amax, red);
-    float down = 1.f, undo = 1.f;
-    for (int it = 0; it < 120 && amax * down > 1024.f; ++it) {  // uniform over the workgroup
-        down *= 0.5f;
-        undo *= 2.f;
+    // the power of two that brings the largest value into (512, 1024], as far as 2^-120 .. 2^100 go
+    int shift = 0;
+    if (amax > 0.f) {
+        const float f = frexpf(amax, &shift);  // f in [0.5, 1), shift 0 for infinities
+        shift = amax <= 3.4028235e38f ? max(-120, min(100, 10 - shift + (f == 0.5f ? 1 : 0))) : -120;
     }
-    for (int it = 0; it < 100 && amax > 0.f && amax * down <= 512.f; ++it) {
-        down *= 2.f;
-        undo *= 0.5f;
-    }
+    const float down = ldexpf(1.f, shift), undo = ldexpf(1.f, -shift);
     // high parts f16(v); low parts f16(v - high) when the split-precision product is on
     auto store = [&](uint32_t k8, const float(&f)[8]) {
         _Float16 h[8], lo[8];
@@ -538,8 +591,12 @@ __global__ __launch_bounds__(256) void attn_rows_kernel(const AttnRowsArgs a) {
 //   online softmax per token: maximum and sum over the lane's 4 rows and the 4 lane groups;
 //   O^T[dim][token] += V^T · P^T : A = V^T (lane n = dimension 16 b + n, k-slot g = row 4 g + i
 //                     in step i), B = the lane's own P values -- no transposition anywhere.
-template <int HS16>
-__global__ __launch_bounds__(256) void attn_block_kernel(const AttnRowsArgs a, uint32_t T) {
+// WAVES 4: several workgroups fit a compute unit and cover each other's waits.  WAVES 8, where there are fewer
+// workgroups than compute units (a short run behind a long context): twice the waves share the cache rows,
+// and a wave requests its next block of them before it multiplies one (21 tokens behind 600, 24 heads of 128:
+// 39 -> 25 us; 45 behind 300, 32 heads: 24.5 -> 18; with 256 workgroups 9.8 us with four waves, 11.3 with eight).
+template <int HS16, int WAVES>
+__global__ __launch_bounds__(WAVES * 64) void attn_block_kernel(const AttnRowsArgs a, uint32_t T) {
     constexpr int HS = HS16 * 16;
     __shared__ float sm_m[4][16], sm_l[4][16];
     __shared__ float sm_o[4][HS][17];
@@ -561,19 +618,27 @@ __global__ __launch_bounds__(256) void attn_block_kernel(const AttnRowsArgs a, u
 #pragma unroll
     for (int b = 0; b < HS16; ++b) acc[b] = floatx4{0.f, 0.f, 0.f, 0.f};
     float m = -INFINITY, l = 0.f;
-    for (uint32_t blk = wave; blk < nblk; blk += 4) {  // uniform over the wave
+    struct Rows {
+        float4 k[HS16];
+        float v[HS16][4];
+    };
+    auto load = [&](Rows &r, uint32_t blk) {  // rows past the end repeat the last one and do not count
         const uint32_t pbase = blk * 16;
         const float *krow = a.kc + (size_t)min(pbase + n, last_pos) * a.kv_dim + head_off + 4 * g;
-        float4 k[HS16];
 #pragma unroll
-        for (int c = 0; c < HS16; ++c) k[c] = *reinterpret_cast<const float4 *>(krow + 16 * c);
-        float v[HS16][4];
+        for (int c = 0; c < HS16; ++c) r.k[c] = *reinterpret_cast<const float4 *>(krow + 16 * c);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const float *vrow = a.vc + (size_t)min(pbase + 4 * g + i, last_pos) * a.kv_dim + head_off + n;
 #pragma unroll
-            for (int b = 0; b < HS16; ++b) v[b][i] = vrow[16 * b];
+            for (int b = 0; b < HS16; ++b) r.v[b][i] = vrow[16 * b];
         }
+    };
+    constexpr bool AHEAD = WAVES == 8;
+    auto step = [&](const Rows &r, uint32_t blk) {
+        const uint32_t pbase = blk * 16;
+        const float4(&k)[HS16] = r.k;
+        const float(&v)[HS16][4] = r.v;
         floatx4 s = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int c = 0; c < HS16; ++c) {
@@ -609,19 +674,58 @@ __global__ __launch_bounds__(256) void attn_block_kernel(const AttnRowsArgs a, u
 #pragma unroll
             for (int i = 0; i < 4; ++i) acc[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[b][i], p[i], acc[b], 0, 0, 0);
         }
+    };
+    if (AHEAD) {
+        Rows r0, r1;
+        if (wave < nblk) load(r0, wave);
+        for (uint32_t blk = wave; blk < nblk; blk += 2 * WAVES) {  // uniform over the wave
+            load(r1, blk + WAVES);
+            __builtin_amdgcn_sched_barrier(0);  // requested before the products, not between them
+            step(r0, blk);
+            if (blk + WAVES >= nblk) break;
+            load(r0, blk + 2 * WAVES);
+            __builtin_amdgcn_sched_barrier(0);
+            step(r1, blk + WAVES);
+        }
+    } else {
+        for (uint32_t blk = wave; blk < nblk; blk += WAVES) {
+            Rows r;
+            load(r, blk);
+            step(r, blk);
+        }
     }
-    // acc[b][i] = O^T[dimension 16 b + 4 g + i][token n] of this wave's rows; merge the four waves
-    if (g == 0) {
-        sm_m[wave][n] = m;
-        sm_l[wave][n] = l;
-    }
+    // acc[b][i] = O^T[dimension 16 b + 4 g + i][token n] of this wave's rows; merge the waves, eight of
+    // them in two steps (wave w takes up wave w + 4 first)
+    auto leave = [&](uint32_t w) {
+        if (g == 0) {
+            sm_m[w][n] = m;
+            sm_l[w][n] = l;
+        }
 #pragma unroll
-    for (int b = 0; b < HS16; ++b) {
+        for (int b = 0; b < HS16; ++b) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) sm_o[wave][16 * b + 4 * g + i][n] = acc[b][i];
+            for (int i = 0; i < 4; ++i) sm_o[w][16 * b + 4 * g + i][n] = acc[b][i];
+        }
+    };
+    if (WAVES == 8) {
+        if (wave >= 4) leave(wave - 4);
+        __syncthreads();
+        if (wave < 4) {
+            const float m2 = sm_m[wave][n], l2 = sm_l[wave][n], mn = fmaxf(m, m2);
+            const float s1 = m == -INFINITY ? 0.f : __expf(m - mn), s2 = m2 == -INFINITY ? 0.f : __expf(m2 - mn);
+#pragma unroll
+            for (int b = 0; b < HS16; ++b) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    acc[b][i] = fmaf(acc[b][i], s1, sm_o[wave][16 * b + 4 * g + i][n] * s2);
+            }
+            l = fmaf(l, s1, l2 * s2);
+            m = mn;
+        }
     }
+    if (wave < 4) leave(wave);
     __syncthreads();
-    for (uint32_t idx = threadIdx.x; idx < 16 * HS; idx += 256) {
+    for (uint32_t idx = threadIdx.x; idx < 16 * HS; idx += WAVES * 64) {
         const uint32_t tok = idx / HS, d = idx % HS;
         if (t0 + tok >= T) continue;
         const float M = fmaxf(fmaxf(sm_m[0][tok], sm_m[1][tok]), fmaxf(sm_m[2][tok], sm_m[3][tok]));
@@ -644,6 +748,15 @@ void token_blocks(uint32_t T, uint32_t *tiles, uint32_t *nt) {
     const uint32_t n = (T + 15) / 16;
     *tiles = T <= kPrefillMaxTokens ? 1 : (T + TILE_TOKENS - 1) / TILE_TOKENS;
     *nt = T > kPrefillMaxTokens ? TILE_TOKENS / 16 : n == 5 ? 6 : n == 7 ? 8 : n;
+}
+
+template <int HS16>
+void launch_attn_block(wgml_ctx *ctx, const AttnRowsArgs &a, uint32_t n_heads, uint32_t T, bool few) {
+    const dim3 grid(n_heads, (T + 15) / 16);
+    if (few)
+        attn_block_kernel<HS16, 8><<<grid, dim3(512), 0, ctx->stream>>>(a, T);
+    else
+        attn_block_kernel<HS16, 4><<<grid, dim3(256), 0, ctx->stream>>>(a, T);
 }
 
 // How many workgroups share the K range of a row tile.
@@ -953,16 +1066,16 @@ int launch_attention_rows(wgml_ctx *ctx, const wgml_attn_params &p, uint32_t pos
     AttnRowsArgs a{q, kc, vc, xb, q_stride, xb_stride, p.kv_dim, p.kv_mul, p.head_size, pos0};
     if (p.head_size % 16 == 0 && p.head_size <= 128 && !ctx->tuning[WGML_TUNE_PREFILL_ATTENTION_PER_TOKEN]) {
         // 16 tokens per workgroup on the fp32 matrix cores
-        const dim3 bgrid(p.n_heads, (T + 15) / 16), bblock(256);
+        const bool few = (uint64_t)p.n_heads * ((T + 15) / 16) < (uint64_t)(ctx->n_cu > 0 ? ctx->n_cu : 256);
         switch (p.head_size / 16) {
-        case 1: attn_block_kernel<1><<<bgrid, bblock, 0, ctx->stream>>>(a, T); break;
-        case 2: attn_block_kernel<2><<<bgrid, bblock, 0, ctx->stream>>>(a, T); break;
-        case 3: attn_block_kernel<3><<<bgrid, bblock, 0, ctx->stream>>>(a, T); break;
-        case 4: attn_block_kernel<4><<<bgrid, bblock, 0, ctx->stream>>>(a, T); break;
-        case 5: attn_block_kernel<5><<<bgrid, bblock, 0, ctx->stream>>>(a, T); break;
-        case 6: attn_block_kernel<6><<<bgrid, bblock, 0, ctx->stream>>>(a, T); break;
-        case 7: attn_block_kernel<7><<<bgrid, bblock, 0, ctx->stream>>>(a, T); break;
-        default: attn_block_kernel<8><<<bgrid, bblock, 0, ctx->stream>>>(a, T); break;
+        case 1: launch_attn_block<1>(ctx, a, p.n_heads, T, few); break;
+        case 2: launch_attn_block<2>(ctx, a, p.n_heads, T, few); break;
+        case 3: launch_attn_block<3>(ctx, a, p.n_heads, T, few); break;
+        case 4: launch_attn_block<4>(ctx, a, p.n_heads, T, few); break;
+        case 5: launch_attn_block<5>(ctx, a, p.n_heads, T, few); break;
+        case 6: launch_attn_block<6>(ctx, a, p.n_heads, T, few); break;
+        case 7: launch_attn_block<7>(ctx, a, p.n_heads, T, few); break;
+        default: launch_attn_block<8>(ctx, a, p.n_heads, T, few); break;
         }
         WGML_CHECK_LAUNCH();
         ctx->launches++;
