@@ -221,7 +221,10 @@ struct FusedGemv {
     // optional table of (cos, sin) pairs for the current position, one per rotated
     // pair of a head (head_size / 2 entries); computed in-kernel when null
     const float *rope_cs = nullptr;
+    // Neox pairs for the jobs in ROPE mode (rows a multiple of head_size, at most kFusedNeoxRows)
+    bool rope_neox = false;
 };
+constexpr uint32_t kFusedNeoxRows = 1u << 24;  // rows / 2 * head_size / 2 stays below 2^32 (heads of up to 256)
 bool gemv_fused_supported(const wgml_qmat *m);
 // the matrices can share one launch_gemv_fused (with the context's settings): one format, or a
 // mix of Q4_K / Q6_K / Q8_0
@@ -229,6 +232,8 @@ bool gemv_fused_set_supported(const wgml_ctx *ctx, const wgml_qmat *const *mats,
 // launch_gemv_quant takes GemvEpilogue::partials for this matrix (with the context's settings)
 bool gemv_partials_supported(const wgml_ctx *ctx, const wgml_qmat *m);
 int launch_gemv_fused(wgml_ctx *ctx, const FusedGemv &f);
+// the kernel of a launch with Neox pairs (gemv_neox.hip): matrices of format fmt (0: a mix of the main ones)
+const void *gemv_neox_kernel(int fmt, int threads);
 
 int launch_gemv_quant(wgml_ctx *ctx, float *out, const wgml_qmat *m, const float *v,
                       const GemvEpilogue &ep);

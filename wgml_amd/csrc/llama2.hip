@@ -150,7 +150,10 @@ int enqueue_step(wgml_llama2 *m, bool dynamic, uint32_t token, uint32_t pos,
             gemv_fused_set_supported(ctx, gate_up, 2) && w.ffn_gate->type == w.ffn_up->type) {
             // 5 launches per layer: [norm + Q,K,V + bias + RoPE + KV-cache write],
             // attention (+ merge), [Wo + residual], [norm + gate,up + SiLU], [down + residual]
-            const bool rope_fused = variant == WGML_ROPE_ORIGINAL;
+            // (fp32 activations and f32 matrices keep the Neox rope launch of their own)
+            const bool rope_fused = variant == WGML_ROPE_ORIGINAL ||
+                                    (dim <= kFusedNeoxRows && w.attn_q->type != WGML_F32 &&
+                                     !ctx->tuning[WGML_TUNE_GEMV_F32_ACTIVATIONS]);
             FusedGemv f;
             f.njobs = 3;
             f.x = m->x;
@@ -160,6 +163,7 @@ int enqueue_step(wgml_llama2 *m, bool dynamic, uint32_t token, uint32_t pos,
             f.head_size = m->head_size;
             f.rope_base = c.rope_base_freq;
             f.rope_cs = m->rope_cs;
+            f.rope_neox = rope_fused && variant == WGML_ROPE_NEOX;
             f.jobs[0].a = w.attn_q;
             f.jobs[0].out = m->q;
             f.jobs[0].bias = w.bq;
