@@ -579,7 +579,7 @@ constexpr uint32_t gemm_lds_words(int nt) {  // 16-byte words
 }
 
 template <class F, int NT, bool SPLIT>
-__global__ __launch_bounds__(256, NT >= 8 ? 2 : NT >= 6 ? 3 : 4) void gemm_rows_kernel(const GemmArgs a) {
+__global__ __launch_bounds__(256, NT >= 8 ? 2 : NT >= 6 ? 3 : 4) void gemm_lds_kernel(const GemmArgs a) {
     extern __shared__ u32x4 xs[];  // [2][chunks][high: NT * 128 words (, low: the same)], [2][sums: NT * 32]
     constexpr int PARTS = SPLIT ? 2 : 1, CPS = gemm_stage_chunks(NT), NS = 4 / CPS;
     constexpr uint32_t CW = NT * 128, CWX = CW * PARTS, STAGE = CPS * CWX, SUMS = F::OFFSET ? NT * 32 : 0;
@@ -963,7 +963,7 @@ int launch_with_lds(wgml_ctx *ctx, K kernel, const GemmArgs &a, uint32_t grid, u
 
 template <class F, int NT, bool SPLIT>
 int launch_rows(wgml_ctx *ctx, const GemmArgs &a, uint32_t tiles) {
-    return launch_with_lds(ctx, gemm_rows_kernel<F, NT, SPLIT>, a, tiles * a.ks, 256,
+    return launch_with_lds(ctx, gemm_lds_kernel<F, NT, SPLIT>, a, tiles * a.ks, 256,
                            gemm_lds_words<F, SPLIT>(NT) * sizeof(u32x4));
 }
 

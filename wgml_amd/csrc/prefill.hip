@@ -891,7 +891,8 @@ int ensure_gemm_partials(wgml_ctx *ctx, size_t bytes) {
     // them), so each is at least twice the one before, up to what a long run takes at most: together
     // they are no larger than the last.
     constexpr size_t kStep = size_t(8) << 20, kUsual = kTilePartBytes + kStep;
-    const size_t need = (bytes + kStep) & ~((size_t(1) << 20) - 1);
+    // (half a MiB for the products of small models: K is split there too)
+    const size_t need = bytes <= kStep / 16 ? kStep / 16 : (bytes + kStep) & ~((size_t(1) << 20) - 1);
     size_t size = need > 2 * ctx->gemm_part_bytes ? need : 2 * ctx->gemm_part_bytes;
     if (size > kUsual) size = need > kUsual ? need : kUsual;
     float *part = nullptr;
