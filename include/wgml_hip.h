@@ -172,10 +172,10 @@ WGML_API int wgml_gemv_quant(wgml_ctx *ctx, wgml_view out, const wgml_qmat *m, w
  * out[t] = m * x[t], with x n_tokens x ncols and out n_tokens x nrows, both row-major.
  * No counterpart in the reference, which multiplies one vector at a time
  * (GemvQuant::dispatch above); it is the building block of wgml_llama2_prefill.
- * The weights are expanded with the reference's dequantization arithmetic (fp32).
- * Precision (wgml_ctx_set_gemm_precision): level 1, the default, feeds the matrix
- * cores pairs of f16 numbers per operand (high part + low part), three MFMAs per
- * product term group, fp32 sums: results agree with n_tokens calls of
+ * The matrix cores multiply the weights' integers, which f16 holds exactly; scales and
+ * minima are applied to the sums of a sub-block in fp32.
+ * Precision (wgml_ctx_set_gemm_precision): level 1, the default, takes the vectors as
+ * pairs of f16 numbers (high part + low part), two MFMAs per 32 terms, fp32 sums: results agree with n_tokens calls of
  * wgml_gemv_quant to fp32 rounding (about 1e-6 of a row's magnitude).  Level 0 rounds
  * weights and vectors to f16 once: 1.4x faster, about 3e-4 of a row's magnitude
  * (up to 1.4e-3 for single elements).  m: any of the nine quantized block formats

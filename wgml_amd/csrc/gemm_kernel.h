@@ -972,7 +972,7 @@ int launch_gemm_prec(wgml_ctx *ctx, const GemmArgs &a, uint32_t tiles) {
     if (a.tall)
         return launch_with_lds(ctx, gemm_tile_kernel<F, SPLIT>, a, tiles * a.ttiles * a.ks, 512,
                                TileLds<F, SPLIT>::WORDS * sizeof(u32x4));
-    switch (a.nt) {  // gemm_token_blocks
+    switch (a.nt) {  // token_blocks
     case 1: return launch_rows<F, 1, SPLIT>(ctx, a, tiles);
     case 2: return launch_rows<F, 2, SPLIT>(ctx, a, tiles);
     case 3: return launch_rows<F, 3, SPLIT>(ctx, a, tiles);

@@ -1098,8 +1098,8 @@ int launch_attention_rows(wgml_ctx *ctx, const wgml_attn_params &p, uint32_t pos
 
 extern "C" {
 
-// 1 (default): products of the batched path take both operands as pairs of f16 numbers (error
-// about 2^-22 per term, three MFMAs per sub-block); 0: plain f16 operands (2^-11, one MFMA).
+// 1 (default): products of the batched path take the activations as pairs of f16 numbers (error
+// about 2^-22 per term, two MFMAs per 32 terms); 0: plain f16 activations (2^-11, one MFMA).
 int wgml_ctx_set_gemm_precision(wgml_ctx *ctx, int level) {
     WGML_REQUIRE(ctx != nullptr, "wgml_ctx_set_gemm_precision: null context");
     WGML_REQUIRE(level == 0 || level == 1, "wgml_ctx_set_gemm_precision: level %d not in {0, 1}", level);
