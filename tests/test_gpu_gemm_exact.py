@@ -6,11 +6,16 @@ activation keeps 22 bits, so a result is off by at most 2^-22 of sum |w x| (half
 as rows scale to at most 1024), plus fp32 sums: K / 32 + 4 roundings of 2^-24 of sums no larger than
 sum |q scale x| + sum |min x|, the two parts of a weight apart.  Twice that is allowed.
 """
+import ctypes
+
 import numpy as np
 import pytest
 
+import npref
 import oracle as orc
 import wgml_amd as W
+from wgml_amd import _lib
+from wgml_amd.models import HostMatrix, Llama2, Llama2Config
 
 pytestmark = pytest.mark.gpu
 SIZES = {W.Q4_0: 18, W.Q4_1: 20, W.Q5_0: 22, W.Q5_1: 24, W.Q8_0: 34, W.Q4_K: 144, W.Q5_K: 176, W.Q6_K: 210, W.Q8_K: 292}
@@ -60,3 +65,57 @@ def test_nothing_behind_the_last_row_is_multiplied(gpu, qtype):
         W.GemmQuant.from_device(gpu).dispatch(out, m, W.GpuVector.init(gpu, x.reshape(-1)), 5)
         whole.append(out.read().reshape(5, rows)[:, 0])
     assert np.array_equal(whole[0], whole[1]) and np.isfinite(whole[0]).all()
+
+
+def v_rows(gpu, qtype, raw, nrows, ncols, x, precision=1):
+    """The product of a matrix with the rows of x, RMS-normalised, as a run of len(x) prompt tokens multiplies it: V of
+    the first layer, between matrices of the same format for Q and K (one launch), and what it multiplied."""
+    heads = ncols // 32
+    cfg = Llama2Config(dim=ncols, hidden_dim=256, n_layers=1, n_q_heads=heads, n_kv_heads=nrows // 32, vocab_size=len(x),
+                       seq_len=len(x), rope_base_freq=10000.0, rms_norm_eps=1e-5)
+    m = Llama2(gpu, cfg)
+    other = {"attn_q": (ncols, ncols), "attn_k": (nrows, ncols), "attn_output": (ncols, ncols), "ffn_gate": (256, ncols),
+             "ffn_up": (256, ncols), "ffn_down": (ncols, 256)}
+    for i, (name, (r, c)) in enumerate(other.items()):
+        m.set_matrix(name, 0, HostMatrix(qtype, r, c, random_blocks(qtype, r * c, 50 + i)))
+    m.set_matrix("attn_v", 0, HostMatrix(qtype, nrows, ncols, raw))
+    m.set_matrix("output", 0, HostMatrix(W.F32, len(x), ncols, np.zeros(4 * len(x) * ncols, np.uint8)))
+    for name in ("attn_norm", "ffn_norm", "output_norm"):
+        m.set_vector(name, 0, np.ones(ncols))
+    te = np.ascontiguousarray(x, np.float32)
+    _lib.call("wgml_llama2_set_token_embd", m._h, te.ctypes.data_as(ctypes.c_void_p))
+    gpu.set_gemm_precision(precision)
+    try:
+        m.prefill(np.arange(len(x), dtype=np.uint32))
+    finally:
+        gpu.set_gemm_precision(1)
+    xd = te.astype(np.float64)
+    return np.asarray(m.kv_download(0, 1, 0, len(x))), xd / np.sqrt((xd ** 2).mean(1, keepdims=True) + 1e-5)
+
+
+@pytest.mark.parametrize("long_run", [False, True], ids=["product", "long_run"])
+@pytest.mark.parametrize("qtype", list(SIZES))
+def test_parts_of_a_weight_do_not_cancel(gpu, qtype, long_run):
+    """Activations of one sign, weights around zero: d q and the minimum of a Q4_1 weight are each a hundred times the
+    sum of their products, so fp32 sums of the one and of the other would be off by 1.7e-6 (Q4_1, Q5_1) to 4e-6 (Q4_K,
+    Q5_K) of its rms.  Sums no larger than the result: N = 3 K / 32 + K / 256 roundings of 2^-24 / sqrt(3) at most, with
+    random signs: sqrt(N) 3.4e-8 = 3.5e-7 of it at K = 1024, and 1.2e-7 for the second parts of activations and
+    of sums of 32 (23 bits).  A factor common to a row of V is that row's norm, in fp32 on the device."""
+    K, R, T = 1024, 256, 200 if long_run else 48
+    values = W.rng_normal(1, R * K, 0.0, 0.02)
+    raw = npref.encode_simple(qtype, values) if qtype in (W.Q4_0, W.Q4_1, W.Q5_0, W.Q5_1, W.Q5_K, W.Q8_K) \
+        else np.asarray(W.quantize(qtype, values))
+    w = orc.dequantize(qtype, raw, R * K).reshape(R, K).astype(np.float64)
+    z = W.rng_normal(2, T * K).reshape(T, K)
+    for x in (np.abs(z), z + np.float32(3), np.maximum(z, np.float32(-0.2))):
+        if long_run:
+            got, xd = v_rows(gpu, qtype, raw, R, K, x)
+        else:
+            out, xd = W.GpuVector.uninit(gpu, T * R), x.astype(np.float64)
+            m = W.GpuQuantMatrix(gpu, qtype, R, K, raw)
+            W.GemmQuant.from_device(gpu).dispatch(out, m, W.GpuVector.init(gpu, x.reshape(-1)), T)
+            got = out.read().reshape(T, R)
+        want = xd @ w.T
+        factor = (got * want).sum(1, keepdims=True) / (want ** 2).sum(1, keepdims=True)
+        assert np.abs(factor - 1).max() <= 1e-6
+        assert np.sqrt(((got - factor * want) ** 2).mean()) <= 5e-7 * np.sqrt((want ** 2).mean())

@@ -22,6 +22,7 @@ struct GemmMat {
     uint32_t tile0;                    // first row tile of this matrix in the launch (64 or TILE_ROWS rows)
     uint32_t roff;                     // rows of the matrices before this one in the launch
     uint32_t rope;                     // the reduction rotates this matrix' rows (GemmArgs::rope_*)
+    float offset_up, offset_down;      // power of two that brings offsets of weights into f16 range, and its inverse
 };
 
 struct GemmArgs {

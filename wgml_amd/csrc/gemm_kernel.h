@@ -30,12 +30,19 @@ struct __attribute__((packed, aligned(2))) Half2Aligned {
 // A weight of every format is an exact small integer times the scale of its block (plus, in some,
 // an offset shared by 32 elements).  The matrix cores multiply the integers, which f16 holds
 // exactly, and the scale multiplies the fp32 sums of a block:
-//   blocks of 32 (Q8_0, Q4_0, Q4_1, Q5_0, Q5_1)   q in [-128, 127], d per 32 elements
-//   Q8_K                                          q in [-128, 127], d per 256
-//   Q4_K, Q5_K    q * scale <= 31 * 63 = 1953, d per 256; the minima meet the sums of 32
-//                 activations in one more MFMA per 256 elements
+//   Q8_0, Q8_K    q in [-128, 127], d per 32 (Q8_K: 256) elements
+//   Q4_0, Q5_0    q - 8, q - 16, d per 32
+//   Q4_1, Q5_1    q - 7.5, q - 15.5, d per 32
+//   Q4_K, Q5_K    (q - 7.5) * scale, (q - 15.5) * scale: up to 977, d per 256
 //   Q6_K          (q - 32) * scale up to 4096: f16 holds 11 bits, so a pair hi + lo (exact), d per 256
-// Nothing is rounded on the weights' side, and an element takes about one vector instruction (a
+// What these integers leave of a weight d q + m (Q4_1, Q5_1) or d scale q - dmin min (Q4_K, Q5_K) is an offset shared by
+// 32 elements, 7.5 d + m and the like, which meets the sums of 32 activations in one more MFMA per 256 elements, as a pair
+// of f16 numbers of which the second holds what rounding the first left.
+// The integers are taken from the middle of q's range because d q and m alone are each about a hundred times the result
+// where activations have one sign, and cancel only in the fp32 sums: error of Q4_K, |N(0,1)| activations, K = 4096, 3.6e-6 of
+// the result's rms with q from 0, 3.9e-7 around 8, 2.8e-7 around 7.5 (zero-mean activations 4.1e-7, 1.8e-7, 1.9e-7;
+// shorter chains of MFMAs take it further, CHAIN below).
+// Nothing else is rounded on the weights' side, and an element takes about one vector instruction (a
 // byte permutation makes f16 numbers 1024 + q out of two bytes of q at a time; one packed multiply-add
 // takes the 1024 off again and applies the block's integer scale).
 //
@@ -46,6 +53,7 @@ struct __attribute__((packed, aligned(2))) Half2Aligned {
 //   Dec       what is decoded once per unit
 //   operand   the 8 halves of half chunk Q, and the low parts where the format has them
 //   scale     of half chunk Q (blocks of 32) or of the unit
+//   offsets   of sub-blocks 2 g and 2 g + 1 times `up`, as f16 pairs hi and lo
 // Elements beyond the row's end (32-element blocks, last unit) are whatever follows in the matrix or
 // in the zeroed bytes behind it: finite, and multiplied by activations that are zero.
 __device__ __forceinline__ half2v as_half2(uint32_t v) {
@@ -80,13 +88,28 @@ __device__ __forceinline__ void bytes_plus(uint32_t (&o)[4], uint32_t lo4, uint3
     o[2] = as_u32(bytes_1024<0>(hi4) + k);
     o[3] = as_u32(bytes_1024<1>(hi4) + k);
 }
-// eight bytes q (two words) to q * s; s and -1024 s are integers that f16 holds (s <= 63)
+// eight bytes b (two words) to b / 2 + off (0x6000 is 512, its last place is 1/2)
+__device__ __forceinline__ void bytes_halved(uint32_t (&o)[4], uint32_t lo4, uint32_t hi4, float off) {
+    const half2v k = splat(off - 512.f);
+    o[0] = as_u32(as_half2(__builtin_amdgcn_perm(0x60606060u, lo4, 0x04010400u)) + k);
+    o[1] = as_u32(as_half2(__builtin_amdgcn_perm(0x60606060u, lo4, 0x04030402u)) + k);
+    o[2] = as_u32(as_half2(__builtin_amdgcn_perm(0x60606060u, hi4, 0x04010400u)) + k);
+    o[3] = as_u32(as_half2(__builtin_amdgcn_perm(0x60606060u, hi4, 0x04030402u)) + k);
+}
+// eight bytes n q + n / 2 (two words) to (q - c) * n s, c = 128 / n - 1/2 (the middle of q's range), where n s is a scale of
+// up to 63: s, 1152 s and the result (multiples of 1/2 up to 977) are numbers that f16 holds
 __device__ __forceinline__ void bytes_times(uint32_t (&o)[4], uint32_t lo4, uint32_t hi4, half2v s) {
-    const half2v k = s * splat(-1024.f);
+    const half2v k = s * splat(-(1024.f + 128.f));
     o[0] = as_u32(__builtin_elementwise_fma(bytes_1024<0>(lo4), s, k));
     o[1] = as_u32(__builtin_elementwise_fma(bytes_1024<1>(lo4), s, k));
     o[2] = as_u32(__builtin_elementwise_fma(bytes_1024<0>(hi4), s, k));
     o[3] = as_u32(__builtin_elementwise_fma(bytes_1024<1>(hi4), s, k));
+}
+// two offsets, and what rounding them to f16 left
+__device__ __forceinline__ void offset_pair(uint32_t &hi, uint32_t &lo, float a, float b) {
+    const half2v h{(_Float16)a, (_Float16)b};
+    hi = as_u32(h);
+    lo = as_u32(half2v{(_Float16)(a - (float)h[0]), (_Float16)(b - (float)h[1])});
 }
 
 // Plain f16 in runs of more than 128 tokens: the weight itself, rounded to f16 once, times 2^8 (undone at
@@ -113,14 +136,21 @@ struct ScalesK {
         s[1] = (h.w & 0x0f0f0f0fu) | ((h.y >> 2) & 0x30303030u);
         m[1] = ((h.w >> 4) & 0x0f0f0f0fu) | ((h.z >> 2) & 0x30303030u);
     }
-    template <int Q>
+    // of sub-block Q over N (16 or 8)
+    template <int Q, int N>
     __device__ half2v scale() const {
-        return byte_1024<Q & 3>(s[Q >> 2]) - splat(1024.f);
+        return __builtin_elementwise_fma(byte_1024<Q & 3>(s[Q >> 2]), splat(1.f / N), splat(-1024.f / N));
     }
-    __device__ void mins(uint32_t (&o)[4]) const { bytes_plus(o, m[0], m[1], 0.f); }
-    template <int Q>
+    template <int N>
+    __device__ void offsets(uint32_t &hi, uint32_t &lo, uint32_t g, float up) const {
+        const uint32_t sc = (g & 2 ? s[1] : s[0]) >> (16 * (g & 1)), mn = (g & 2 ? m[1] : m[0]) >> (16 * (g & 1));
+        const float centre = d * up * (128.f / N - 0.5f), least = dmin * up;
+        offset_pair(hi, lo, fmaf(centre, (float)(sc & 0xffu), -(least * (float)(mn & 0xffu))),
+                    fmaf(centre, (float)((sc >> 8) & 0xffu), -(least * (float)((mn >> 8) & 0xffu))));
+    }
+    template <int Q, int N>
     __device__ void direct(uint32_t (&o)[4], uint32_t lo4, uint32_t hi4) const {
-        bytes_direct(o, lo4, hi4, d * kDirectScale * (float)((s[Q >> 2] >> (8 * (Q & 3))) & 0xffu),
+        bytes_direct(o, lo4, hi4, d * (kDirectScale / N) * (float)((s[Q >> 2] >> (8 * (Q & 3))) & 0xffu),
                      -(dmin * kDirectScale * (float)((m[Q >> 2] >> (8 * (Q & 3))) & 0xffu)));
     }
 };
@@ -148,20 +178,23 @@ struct GemmQ4K {
     }
     __device__ static void decode(Dec &d, const Unit &r, uint32_t) { d.decode(r.hdr); }
     template <int Q>
-    __device__ static u32x2 bytes(const Unit &r) { return (r.qs[Q / 2] >> (4 * (Q & 1))) & 0x0f0f0f0fu; }
+    __device__ static u32x2 bytes(const Unit &r) {  // 16 q
+        return (Q & 1 ? r.qs[Q / 2] : r.qs[Q / 2] << 4) & 0xf0f0f0f0u;
+    }
     template <int Q>
     __device__ static void operand(uint32_t (&hi)[4], uint32_t (&)[4], const Dec &d, const Unit &r, uint32_t) {
-        const u32x2 q = bytes<Q>(r);
-        bytes_times(hi, q.x, q.y, d.scale<Q>());
+        const u32x2 q = bytes<Q>(r) | 0x08080808u;
+        bytes_times(hi, q.x, q.y, d.scale<Q, 16>());
     }
     template <int Q>
     __device__ static void direct(uint32_t (&o)[4], const Dec &d, const Unit &r, uint32_t) {
         const u32x2 q = bytes<Q>(r);
-        d.direct<Q>(o, q.x, q.y);
+        d.direct<Q, 16>(o, q.x, q.y);
     }
     __device__ static float unit_scale(const Dec &d) { return d.d; }
-    __device__ static void mins(uint32_t (&o)[4], const Dec &d) { d.mins(o); }
-    __device__ static float min_scale(const Dec &d) { return -d.dmin; }
+    __device__ static void offsets(uint32_t &hi, uint32_t &lo, const Dec &d, uint32_t g, float up) {
+        d.offsets<16>(hi, lo, g, up);
+    }
 };
 
 // Q5_K (176 B: d, dmin, scales[12] as Q4_K, 32 bytes of fifth bits, 128 bytes of nibbles;
@@ -199,22 +232,23 @@ struct GemmQ5K {
         d.qh = r.qh;
     }
     template <int Q>
-    __device__ static u32x2 bytes(const Dec &d, const Unit &r) {
-        return ((r.qs[Q / 2] >> (4 * (Q & 1))) & 0x0f0f0f0fu) | (((d.qh >> Q) & 0x01010101u) << 4);
+    __device__ static u32x2 bytes(const Dec &d, const Unit &r) {  // 8 q
+        return ((Q & 1 ? r.qs[Q / 2] >> 1 : r.qs[Q / 2] << 3) & 0x78787878u) | (((d.qh >> Q) & 0x01010101u) << 7);
     }
     template <int Q>
     __device__ static void operand(uint32_t (&hi)[4], uint32_t (&)[4], const Dec &d, const Unit &r, uint32_t) {
-        const u32x2 q = bytes<Q>(d, r);
-        bytes_times(hi, q.x, q.y, d.k.scale<Q>());
+        const u32x2 q = bytes<Q>(d, r) | 0x04040404u;
+        bytes_times(hi, q.x, q.y, d.k.scale<Q, 8>());
     }
     template <int Q>
     __device__ static void direct(uint32_t (&o)[4], const Dec &d, const Unit &r, uint32_t) {
         const u32x2 q = bytes<Q>(d, r);
-        d.k.direct<Q>(o, q.x, q.y);
+        d.k.direct<Q, 8>(o, q.x, q.y);
     }
     __device__ static float unit_scale(const Dec &d) { return d.k.d; }
-    __device__ static void mins(uint32_t (&o)[4], const Dec &d) { d.k.mins(o); }
-    __device__ static float min_scale(const Dec &d) { return -d.k.dmin; }
+    __device__ static void offsets(uint32_t &hi, uint32_t &lo, const Dec &d, uint32_t g, float up) {
+        d.k.offsets<8>(hi, lo, g, up);
+    }
 };
 
 // Element 32 Q + 8 g + i of a super-block: nibble (Q >> 1) & 1 of ql[64 (Q >> 2) + 32 (Q & 1) + 8 g + i],
@@ -400,7 +434,7 @@ struct GemmLegacy {
         uint32_t dm[2];  // of blocks 2 g and 2 g + 1: d (low half) and m (high half) as stored
     };
     struct Dec {
-        uint32_t dm[8];
+        uint32_t dm[8], own[HAS_M ? 2 : 1];  // of all blocks; of blocks 2 g and 2 g + 1
     };
     struct Lane {
         uint32_t blk, dm, q;
@@ -435,39 +469,52 @@ struct GemmLegacy {
         const int j4 = (int)(threadIdx.x & 15) * 4;
 #pragma unroll
         for (int b = 0; b < 8; ++b) d.dm[b] = (uint32_t)__builtin_amdgcn_ds_bpermute((b / 2) * 64 + j4, (int)r.dm[b & 1]);
+        if (HAS_M) {
+            d.own[0] = r.dm[0];
+            d.own[HAS_M ? 1 : 0] = r.dm[1];
+        }
     }
-    template <int Q>
+    // q << SHIFT in eight bytes
+    template <int Q, int SHIFT>
     __device__ static u32x2 bytes(const Unit &r, uint32_t g) {
-        uint32_t a = (r.q[Q].x >> (4 * (g >> 1))) & 0x0f0f0f0fu, b = (r.q[Q].y >> (4 * (g >> 1))) & 0x0f0f0f0fu;
+        const uint32_t right = (4 * (g >> 1) - SHIFT) & 31u, mask = 0x0f0f0f0fu << SHIFT;  // (a rotation)
+        uint32_t a = __builtin_amdgcn_alignbit(r.q[Q].x, r.q[Q].x, right) & mask;
+        uint32_t b = __builtin_amdgcn_alignbit(r.q[Q].y, r.q[Q].y, right) & mask;
         if (HAS_QH) {
             // bits 8 g .. 8 g + 7 of qh moved to bit 4 of the eight bytes
             const uint32_t bits = r.qh[Q] >> (8 * g);
-            a |= (((bits & 15u) * 0x00204081u) & 0x01010101u) << 4;
-            b |= ((((bits >> 4) & 15u) * 0x00204081u) & 0x01010101u) << 4;
+            a |= (((bits & 15u) * 0x00204081u) & 0x01010101u) << (4 + SHIFT);
+            b |= ((((bits >> 4) & 15u) * 0x00204081u) & 0x01010101u) << (4 + SHIFT);
         }
         return u32x2{a, b};
     }
-    static constexpr float ZERO = HAS_M ? 0.f : HAS_QH ? -16.f : -8.f;
+    static constexpr float CENTRE = HAS_QH ? 16.f : 8.f;
     template <int Q>
     __device__ static void operand(uint32_t (&hi)[4], uint32_t (&)[4], const Dec &, const Unit &r, uint32_t g) {
-        const u32x2 q = bytes<Q>(r, g);
-        bytes_plus(hi, q.x, q.y, ZERO);
+        const u32x2 q = HAS_M ? bytes<Q, 1>(r, g) | 0x01010101u : bytes<Q, 0>(r, g);
+        if constexpr (HAS_M)
+            bytes_halved(hi, q.x, q.y, -CENTRE);  // q - 7.5, q - 15.5 out of bytes 2 q + 1
+        else
+            bytes_plus(hi, q.x, q.y, -CENTRE);
     }
     template <int Q>
     __device__ static void direct(uint32_t (&o)[4], const Dec &d, const Unit &r, uint32_t g) {
-        const u32x2 q = bytes<Q>(r, g);
+        const u32x2 q = bytes<Q, 0>(r, g);
         const float s = scale<Q>(d) * kDirectScale;
-        bytes_direct(o, q.x, q.y, s, HAS_M ? f16_bits_to_f32((uint16_t)(d.dm[Q] >> 16)) * kDirectScale : ZERO * s);
+        bytes_direct(o, q.x, q.y, s, HAS_M ? f16_bits_to_f32((uint16_t)(d.dm[Q] >> 16)) * kDirectScale : -CENTRE * s);
     }
     template <int Q>
     __device__ static float scale(const Dec &d) {
         return f16_bits_to_f32((uint16_t)(d.dm[Q] & 0xffffu));
     }
-    __device__ static void mins(uint32_t (&o)[4], const Dec &d) {
+    __device__ static void offsets(uint32_t &hi, uint32_t &lo, const Dec &d, uint32_t, float up) {
+        float c[2];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) o[k] = (d.dm[2 * k] >> 16) | (d.dm[2 * k + 1] & 0xffff0000u);
+        for (int b = 0; b < 2; ++b)
+            c[b] = fmaf(CENTRE - 0.5f, f16_bits_to_f32((uint16_t)(d.own[HAS_M ? b : 0] & 0xffffu)),
+                        f16_bits_to_f32((uint16_t)(d.own[HAS_M ? b : 0] >> 16))) * up;
+        offset_pair(hi, lo, c[0], c[1]);
     }
-    __device__ static float min_scale(const Dec &) { return 1.f; }
 };
 using GemmQ4_0 = GemmLegacy<18, false, false>;
 using GemmQ4_1 = GemmLegacy<20, true, false>;
@@ -552,6 +599,22 @@ __device__ __forceinline__ void add_scaled(floatx4 &acc, const floatx4 &t, float
     for (int k = 0; k < 4; ++k) acc[k] = fmaf(t[k], s, acc[k]);
 }
 
+// Offsets as an MFMA operand: lane (g, j) comes with hi and lo of its two sub-blocks and leaves with the eight hi of row j
+// for g < 2, the eight lo otherwise.  The sums opposite are their first part for even g and their second for odd,
+// so that the four products of parts are summed.
+__device__ __forceinline__ void gather_offsets(uint32_t (&o)[4], uint32_t hi, uint32_t lo) {
+    // rows of 16 lanes: [h0 h1 h2 h3] twice -> [h0 h0 h2 h2], [h1 h1 h3 h3]; then the upper halves of those against the
+    // lower halves of lo's
+    const u32x2 h = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane16_swap(hi, hi, false, false));
+    const u32x2 l = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane16_swap(lo, lo, false, false));
+    const u32x2 even = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(h.x, l.x, false, false));
+    const u32x2 odd = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(h.y, l.y, false, false));
+    o[0] = even.x;
+    o[1] = odd.x;
+    o[2] = even.y;
+    o[3] = odd.y;
+}
+
 // What computes `v` stays in front of this: instruction selection would move sums that nothing in the
 // loop reads to its end, and keep what they are made of in registers until there.
 __device__ __forceinline__ void keep_here(floatx4 &v) { asm volatile("" : "+v"(v)); }
@@ -585,6 +648,11 @@ __global__ __launch_bounds__(256, NT >= 8 ? 2 : NT >= 6 ? 3 : 4) void gemm_lds_k
     constexpr uint32_t CW = NT * 128, CWX = CW * PARTS, STAGE = CPS * CWX, SUMS = F::OFFSET ? NT * 32 : 0;
     constexpr int SW = STAGE / 256;  // staged words per thread
     constexpr bool WLO = F::PAIR && SPLIT, G32 = F::GROUP == 32;
+    // half chunks whose products pile up before the scale multiplies them.  An MFMA's own additions round more than a
+    // multiply-add does: eight of them, as in the other formats with a scale per unit, give 2.7e-7 of the result's rms
+    // (Q4_K, |N(0,1)| activations, K = 512 .. 4096), four 2.2e-7, two 1.9e-7 to 2.0e-7; weights expanded to fp32 first gave
+    // 2.1e-7.  Two against eight cost 1 % of a pass of 5 .. 64 tokens, 4 % of 128 (7B widths).
+    constexpr int CHAIN = F::OFFSET && SPLIT ? 2 : 8;
     const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
     const uint32_t tid = threadIdx.x, lane = tid & 63;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
@@ -639,12 +707,8 @@ __global__ __launch_bounds__(256, NT >= 8 ? 2 : NT >= 6 ? 3 : 4) void gemm_lds_k
         const uint32_t next = unit_at(u + 1);
         typename F::Dec ndec;
         floatx4 tmp[G32 ? 1 : NT];
-        uint32_t mins[4];
-        if constexpr (F::OFFSET) {
-            F::mins(mins, dec);
-#pragma unroll
-            for (int k = 0; k < 4; ++k) mins[k] = g < 2 ? mins[k] : 0u;
-        }
+        uint32_t off_hi = 0, off_lo = 0;
+        if constexpr (F::OFFSET) F::offsets(off_hi, off_lo, dec, g, m.offset_up);
         static_for<0, NS>([&](auto s_c) {
             constexpr int s = decltype(s_c)::value;
             u32x4 *buf = xs + (NS > 1 ? (uint32_t)(s & 1) : (u & 1)) * STAGE;
@@ -677,7 +741,7 @@ __global__ __launch_bounds__(256, NT >= 8 ? 2 : NT >= 6 ? 3 : 4) void gemm_lds_k
                 Op &o = op[q & 1];
                 if constexpr (i + AHEAD < NSTEP) fetch(std::integral_constant<int, i + AHEAD>{});
                 const half8 x8 = as_half8(bh[slot]);
-                floatx4 t = mfma(x8, as_half8(o.hi), G32 || q == 0 ? zero : tmp[G32 ? 0 : n]);
+                floatx4 t = mfma(x8, as_half8(o.hi), G32 || q % CHAIN == 0 ? zero : tmp[G32 ? 0 : n]);
                 if constexpr (SPLIT) t = mfma(as_half8(bl[slot]), as_half8(o.hi), t);
                 if constexpr (WLO) t = mfma(x8, as_half8(o.lo), t);
                 if constexpr (n == 0) {
@@ -696,6 +760,9 @@ __global__ __launch_bounds__(256, NT >= 8 ? 2 : NT >= 6 ? 3 : 4) void gemm_lds_k
                     late = t;
                     late_scale = o.scale;
                 } else {
+                    if constexpr (q % CHAIN == CHAIN - 1 && n > 0) add_scaled(acc[n - 1], tmp[n - 1], F::unit_scale(dec));
+                    if constexpr (q % CHAIN == 0 && q > 0 && n == 0)
+                        add_scaled(acc[NT - 1], tmp[NT - 1], F::unit_scale(dec));
                     tmp[n] = t;
                 }
                 __builtin_amdgcn_sched_barrier(0);
@@ -703,11 +770,13 @@ __global__ __launch_bounds__(256, NT >= 8 ? 2 : NT >= 6 ? 3 : 4) void gemm_lds_k
         });
         if constexpr (!G32 || F::OFFSET) {
             const u32x4 *sums = xs + 2 * STAGE + (u & 1) * SUMS + (lane & 31);
+            uint32_t offs[4];
+            if constexpr (F::OFFSET) gather_offsets(offs, off_hi, off_lo);
+            if constexpr (!G32) add_scaled(acc[NT - 1], tmp[NT - 1], F::unit_scale(dec));
+            if constexpr (F::OFFSET) {
 #pragma unroll
-            for (int n = 0; n < NT; ++n) {
-                if constexpr (!G32) add_scaled(acc[n], tmp[n], F::unit_scale(dec));
-                if constexpr (F::OFFSET)
-                    add_scaled(acc[n], mfma(as_half8(sums[n * 32]), as_half8(mins), zero), F::min_scale(dec));
+                for (int n = 0; n < NT; ++n)
+                    add_scaled(acc[n], mfma(as_half8(sums[n * 32]), as_half8(offs), zero), m.offset_down);
             }
         }
         dec = ndec;
@@ -735,8 +804,8 @@ template <class F, bool SPLIT>
 struct TileLds {  // 16-byte words
     static constexpr uint32_t WPARTS = F::PAIR && SPLIT ? 2 : 1, XPARTS = SPLIT ? 2 : 1;
     static constexpr uint32_t W = 8 * WPARTS * 64, X = XPARTS * 16 * 64, SLOT = W + X + 32;  // + 128 scales
-    // per unit, twice: 128 scales, 128 scales of the minima, the minima, the sums
-    static constexpr uint32_t UNIT = !SPLIT ? 0 : F::OFFSET ? 64 + 8 * 32 + 16 * 32 : F::GROUP == 256 ? 32 : 0;
+    // per unit, twice: 128 scales, the offsets (per row block 16 words of their first parts, 16 of the second), the sums
+    static constexpr uint32_t UNIT = !SPLIT ? 0 : F::OFFSET ? 32 + 8 * 32 + 16 * 32 : F::GROUP == 256 ? 32 : 0;
     static constexpr uint32_t WORDS = 2 * (SLOT + UNIT);
 };
 
@@ -747,6 +816,7 @@ __global__ __launch_bounds__(512) void gemm_tile_kernel(const GemmArgs a) {
     // plain f16: the sums need no scaling per block (direct), split f16: per 32 columns or per unit (tmp)
     constexpr bool DIRECT = !SPLIT, OFFSET = F::OFFSET && SPLIT, WLO = L::WPARTS == 2;
     constexpr bool G32 = F::GROUP == 32 && SPLIT, TMP = F::GROUP == 256 && SPLIT;
+    constexpr int CHAIN = F::OFFSET ? 4 : 8;  // as in gemm_lds_kernel: 2.1e-7 to 2.4e-7 (expanded weights 2.7e-7 to 3.7e-7)
     constexpr int SW = 2 * L::XPARTS;  // staged words of activations per thread and half chunk
     const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
     const uint32_t tid = threadIdx.x, lane = tid & 63;
@@ -815,7 +885,7 @@ __global__ __launch_bounds__(512) void gemm_tile_kernel(const GemmArgs a) {
             if (g == 0) reinterpret_cast<float *>(xs + slot * L::SLOT + L::W + L::X)[wave * 16 + j] = op.scale;
         }
     };
-    // what is shared per unit: scales (and those of the minima), minima, sums
+    // what is shared per unit: scales, offsets, sums
     auto unit_words = [&](uint32_t parity) { return xs + 2 * L::SLOT + parity * L::UNIT; };
     auto unit_store = [&](uint32_t parity, const typename F::Dec &d) {
         u32x4 *w = unit_words(parity);
@@ -823,13 +893,12 @@ __global__ __launch_bounds__(512) void gemm_tile_kernel(const GemmArgs a) {
             if (g == 0) reinterpret_cast<float *>(w)[wave * 16 + j] = F::unit_scale(d);
         }
         if constexpr (OFFSET) {
-            if (g == 0) reinterpret_cast<float *>(w + 32)[wave * 16 + j] = F::min_scale(d);
-            uint32_t mins[4];
-            F::mins(mins, d);
-            u32x4 mw;
-            __builtin_memcpy(&mw, mins, 16);
-            if (g < 2) w[64 + wave * 32 + lane] = mw;
-            w[64 + 8 * 32 + tid] = ss;
+            uint32_t hi, lo;
+            F::offsets(hi, lo, d, g, m.offset_up);
+            uint32_t *o = reinterpret_cast<uint32_t *>(w + 32 + wave * 32 + j) + g;
+            o[0] = hi;
+            o[16 * 4] = lo;
+            w[32 + 8 * 32 + tid] = ss;
         }
     };
     typename F::Unit un;
@@ -863,6 +932,8 @@ __global__ __launch_bounds__(512) void gemm_tile_kernel(const GemmArgs a) {
                 if (WLO) al[b] = aw[b * L::WPARTS * 64 + 64];
                 if (G32)
                     sc[b] = reinterpret_cast<const float *>(xs + (q & 1) * L::SLOT + L::W + L::X)[(wr * 4 + b) * 16 + j];
+                if (TMP && q % CHAIN == CHAIN - 1)
+                    sc[b] = reinterpret_cast<const float *>(unit_words(u & 1))[(wr * 4 + b) * 16 + j];
             }
             __builtin_amdgcn_sched_barrier(0);
             stage_store(1 - (q & 1));
@@ -880,7 +951,7 @@ __global__ __launch_bounds__(512) void gemm_tile_kernel(const GemmArgs a) {
                 floatx4 t[4];
 #pragma unroll
                 for (int b = 0; b < 4; ++b)
-                    t[b] = mfma(x8, as_half8(ah[b]), DIRECT ? acc[b][n] : G32 || q == 0 ? zero : tmp[TMP ? b : 0][TMP ? n : 0]);
+                    t[b] = mfma(x8, as_half8(ah[b]), DIRECT ? acc[b][n] : G32 || q % CHAIN == 0 ? zero : tmp[TMP ? b : 0][TMP ? n : 0]);
                 if constexpr (SPLIT) {
                     const half8 l8 = as_half8(bl[cur]);
 #pragma unroll
@@ -902,6 +973,10 @@ __global__ __launch_bounds__(512) void gemm_tile_kernel(const GemmArgs a) {
                     } else if constexpr (DIRECT) {
                         acc[b][n] = t[b];
                     } else {
+                        if constexpr (q % CHAIN == CHAIN - 1 && n > 0) {
+                            add_scaled(acc[b][n - 1], tmp[b][n - 1], sc[b]);
+                            keep_here(acc[b][n - 1]);
+                        }
                         tmp[b][n] = t[b];
                     }
                 }
@@ -913,6 +988,13 @@ __global__ __launch_bounds__(512) void gemm_tile_kernel(const GemmArgs a) {
                 }
                 __builtin_amdgcn_sched_barrier(0);
             });
+            if constexpr (TMP && q % CHAIN == CHAIN - 1) {
+#pragma unroll
+                for (int b = 0; b < 4; ++b) {
+                    add_scaled(acc[b][3], tmp[b][3], sc[b]);
+                    keep_here(acc[b][3]);
+                }
+            }
             if constexpr (G32) {
 #pragma unroll
                 for (int b = 0; b < 4; ++b) {
@@ -922,20 +1004,22 @@ __global__ __launch_bounds__(512) void gemm_tile_kernel(const GemmArgs a) {
             }
             if constexpr (q == 7 && (TMP || OFFSET)) {
                 const u32x4 *w = unit_words(u & 1);
-                const float *scale = reinterpret_cast<const float *>(w) + wr * 64 + j;
+                u32x4 o[4];
 #pragma unroll
                 for (int b = 0; b < 4; ++b) {
-#pragma unroll
-                    for (int n = 0; n < 4; ++n) {
-                        if constexpr (TMP) add_scaled(acc[b][n], tmp[b][n], scale[b * 16]);
-                        if constexpr (OFFSET) {
-                            const half8 s8 = as_half8(w[64 + 8 * 32 + (wc * 4 + n) * 32 + (lane & 31)]);
-                            u32x4 mw = w[64 + (wr * 4 + b) * 32 + (lane & 31)];
-                            if (g >= 2) mw = u32x4{0, 0, 0, 0};
-                            add_scaled(acc[b][n], mfma(s8, as_half8(mw), zero), scale[128 + b * 16]);
-                        }
-                    }
+                    if (OFFSET) o[b] = w[32 + (wr * 4 + b) * 32 + 16 * (g >> 1) + j];
                 }
+                static_for<0, 4>([&](auto n_c) {
+                    constexpr int n = decltype(n_c)::value;
+                    u32x4 sums;
+                    if (OFFSET) sums = w[32 + 8 * 32 + (wc * 4 + n) * 32 + (lane & 31)];
+#pragma unroll
+                    for (int b = 0; b < 4; ++b) {
+                        if constexpr (OFFSET)
+                            add_scaled(acc[b][n], mfma(as_half8(sums), as_half8(o[b]), zero), m.offset_down);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                });
                 unit_store((u + 1) & 1, dec);
             }
             __syncthreads();

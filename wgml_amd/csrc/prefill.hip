@@ -937,6 +937,12 @@ int launch_gemm_quant_multi(wgml_ctx *ctx, const GemmTarget *targets, int n, con
         g.bias = targets[i].bias;
         g.nrows = q->nrows;
         g.rope = targets[i].rope ? 1u : 0u;
+        // offsets (no larger than a weight can be) up to 2^15: their second parts stay clear of the bottom of the f16 range
+        int e = 0;
+        if (q->max_abs > 0.f) frexpf(q->max_abs, &e);
+        e = 15 - e < 100 ? 15 - e : 100;
+        g.offset_up = ldexpf(1.f, e);
+        g.offset_down = ldexpf(1.f, -e);
         g.out_stride = targets[i].out_stride;
         g.tile0 = tiles;
         g.roff = a.total_rows;
