@@ -633,16 +633,26 @@ __device__ __forceinline__ void keep_here(floatx4 &v) { asm volatile("" : "+v"(v
 // a time per unit); 8 waves that share rows and tokens out; activations requested two stages ahead
 // (spills below 128 registers, no faster where it fits).
 //
-// Chunks of 64 columns staged per barrier: 16 KB of activations, twice, for up to 64 tokens (32 KB
-// beyond), so that four (two) workgroups fit a compute unit.
+// Chunks of 64 columns staged per barrier: 16 KB of activations in split precision for up to 16, 32 and 64 tokens, 24 KB
+// for 48 and 96, 32 KB for 128, half of that in plain f16; twice, with 512 bytes of sums per 16 tokens.
 constexpr int gemm_stage_chunks(int nt) { return nt == 1 ? 4 : nt <= 3 ? 2 : 1; }
 template <class F, bool SPLIT>
 constexpr uint32_t gemm_lds_words(int nt) {  // 16-byte words
     return 2 * (gemm_stage_chunks(nt) * nt * 128 * (SPLIT ? 2 : 1) + (F::OFFSET ? nt * 32 : 0));
 }
+// Workgroups per compute unit that registers are kept for (128 each at four, 168 at three): no more than fit its 160 KB of LDS
+// in split precision (three for 48 tokens, two or three for 96, two for 128), and three for 64 tokens, where four fit: at
+// 128 registers the formats with most to decode spill (four layers, 2080 x 5600 in Q5_1, us: 45 tokens 507 with four ->
+// 410, 64 tokens 482 -> 438; 4096 x 11008 in Q5_K 651 -> 604, 703 -> 663) and the others gain nothing (+-0.6 %).
+template <class F, bool SPLIT>
+constexpr int gemm_workgroups(int nt) {
+    const int fit = (int)(160 * 1024 / (16 * gemm_lds_words<F, SPLIT>(nt)));
+    const int most = nt >= 8 ? 2 : nt >= (SPLIT ? 3 : 6) ? 3 : 4;
+    return fit < most ? fit : most;
+}
 
 template <class F, int NT, bool SPLIT>
-__global__ __launch_bounds__(256, NT >= 8 ? 2 : NT >= 6 ? 3 : 4) void gemm_lds_kernel(const GemmArgs a) {
+__global__ __launch_bounds__(256, (gemm_workgroups<F, SPLIT>(NT))) void gemm_lds_kernel(const GemmArgs a) {
     extern __shared__ u32x4 xs[];  // [2][chunks][high: NT * 128 words (, low: the same)], [2][sums: NT * 32]
     constexpr int PARTS = SPLIT ? 2 : 1, CPS = gemm_stage_chunks(NT), NS = 4 / CPS;
     constexpr uint32_t CW = NT * 128, CWX = CW * PARTS, STAGE = CPS * CWX, SUMS = F::OFFSET ? NT * 32 : 0;
