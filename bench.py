@@ -36,6 +36,7 @@ from __future__ import annotations
 
 import argparse
 import ctypes as C
+import hashlib
 import json
 import os
 import sys
@@ -54,6 +55,15 @@ def log(*a):
 def gemv_bytes(qtype_bytes_per_matrix: int, nrows: int, ncols: int) -> int:
     """Algorithmic bytes of one GEMV: GGUF bytes of W + x (f32) + y (f32)."""
     return qtype_bytes_per_matrix + 4 * ncols + 4 * nrows
+
+
+def gemv_sources_sha256(csrc: str = os.path.join(ROOT, "wgml_amd", "csrc")) -> str:
+    """What the GEMV kernels and their launches are made of (file times say nothing after a checkout)."""
+    digest = hashlib.sha256()
+    for name in ("gemv.hip", "gemv_kernels.h", "device_utils.h"):
+        with open(os.path.join(csrc, name), "rb") as f:
+            digest.update(f.read())
+    return digest.hexdigest()
 
 
 DTYPE = ("quantized weights (q4_k/q6_k/q8_0 ints) x 16-bit block-fixed-point activations on "
@@ -682,9 +692,8 @@ def main():
             traffic = tj.get("gemv_fused_gate_up_bytes_per_launch")
             traffic_src = tj.get("source")
             # the counters were read for the kernel as it was then: say so when it has changed
-            ksrc = os.path.join(ROOT, "wgml_amd", "csrc", "gemv.hip")
-            if os.path.exists(ksrc) and os.path.getmtime(ksrc) > os.path.getmtime(tpath) + 1:
-                log("WARNING: wgml_amd/csrc/gemv.hip is newer than profiles/traffic.json: "
+            if tj.get("kernel_sources_sha256") != gemv_sources_sha256():
+                log("WARNING: the sources of the GEMV kernels are not those of profiles/traffic.json: "
                     "roofline.traffic was measured for an earlier build of the kernel")
                 traffic_src = (traffic_src or "") + " (measured before the kernel source last changed)"
         gate = [W.GpuQuantMatrix(gpu, W.Q4_K, cfg.hidden_dim, cfg.dim, l["ffn_gate"].data)
