@@ -67,6 +67,27 @@ def test_nothing_behind_the_last_row_is_multiplied(gpu, qtype):
     assert np.array_equal(whole[0], whole[1]) and np.isfinite(whole[0]).all()
 
 
+def test_rows_beyond_four_gigabytes(gpu):
+    """Q8_K takes 292 bytes for 256 weights: a matrix of fewer than 2^32 weights whose last rows start behind 2^32 bytes."""
+    nrows, ncols = 58000, 1 << 16
+    row = ncols // 256 * 292
+    raw, rows = np.zeros(nrows * row, np.uint8), [0, 1, 542, 543, (1 << 32) // row, (1 << 32) // row + 1, nrows - 1]
+    some = random_blocks(W.Q8_K, len(rows) * ncols, 9)
+    for i, r in enumerate(rows):
+        raw[r * row:(r + 1) * row] = some[i * row:(i + 1) * row]
+    x = W.rng_normal(4, 2 * ncols).reshape(2, ncols)
+    out, few = W.GpuVector.uninit(gpu, 2 * nrows), W.GpuVector.uninit(gpu, 2 * len(rows))
+    m = W.GpuQuantMatrix(gpu, W.Q8_K, nrows, ncols, raw)
+    W.GemmQuant.from_device(gpu).dispatch(out, m, W.GpuVector.init(gpu, x.reshape(-1)), 2)
+    got = out.read().reshape(2, nrows)
+    m = W.GpuQuantMatrix(gpu, W.Q8_K, len(rows), ncols, some)
+    W.GemmQuant.from_device(gpu).dispatch(few, m, W.GpuVector.init(gpu, x.reshape(-1)), 2)
+    # (the few rows are a product of their own with another split of K: 2048 fp32 sums in another order, sqrt(2048) 2^-24)
+    want = few.read().reshape(2, len(rows))
+    assert np.abs(got[:, rows] - want).max() <= 4e-6 * np.abs(want).max()
+    assert not np.delete(got, rows, axis=1).any()
+
+
 def v_rows(gpu, qtype, raw, nrows, ncols, x, precision=1):
     """The product of a matrix with the rows of x, RMS-normalised, as a run of len(x) prompt tokens multiplies it: V of
     the first layer, between matrices of the same format for Q and K (one launch), and what it multiplied."""

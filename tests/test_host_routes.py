@@ -77,6 +77,27 @@ def test_rows_whose_long_runs_the_products_cannot_address_go_in_short_ones(runti
     """)
 
 
+def test_matrices_that_the_products_address(runtime):
+    # rows of a tile at 32-bit offsets from its first one: below 2^32 weights as before, also where they take more bytes
+    # (Q8_K, 292 per 256), unless one tile alone does
+    host_hip.run(runtime, """
+    def product(nrows, ncols):
+        m = W.GpuQuantMatrix(gpu, W.Q8_K, nrows, ncols, np.zeros(W.quant_bytes(W.Q8_K, nrows * ncols), np.uint8))
+        out, x = W.GpuVector.uninit(gpu, nrows), W.GpuVector.uninit(gpu, ncols)
+        try:
+            return count(launched(lambda: W.GemmQuant.from_device(gpu).dispatch(out, m, x, 1)), "gemm_lds_kernel")
+        except W.WgmlError as e:
+            assert e.code == _lib.E_UNSUPPORTED
+            return 0
+
+    assert product(58000, 1 << 16) == 1
+    assert product(112, 1 << 22) == 1 and product(1000, 1 << 21) == 1
+    assert product(1 << 16, 1 << 16) == 0
+    gpu.set_gemm_precision(0)
+    assert product(112, 1 << 25) == 1 and product(114, 1 << 25) == 0
+    """)
+
+
 def test_only_missing_memory_sends_a_prompt_down_the_slower_path(runtime):
     # runs of 1024 tokens, then of 128, then (where a loop has them) steps; any other failure of the
     # faster path is the caller's to see

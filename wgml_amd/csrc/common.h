@@ -366,7 +366,7 @@ int launch_embed_rows(wgml_ctx *ctx, float *x, const float *table, const uint32_
 int launch_cache_rows(wgml_ctx *ctx, const float *qkv, float *k, float *v, uint32_t n, uint32_t T);
 // The batched products take these formats, and weights that fit their f16 operands.
 bool gemm_supported(const wgml_qmat *q);
-// ... and matrices of fewer than 2^32 elements.
+// ... and matrices of fewer than 2^32 elements, 128 rows of fewer than 2^32 bytes.
 bool gemm_addressable(const wgml_qmat *q);
 // q (q_len wide) and k (kv_dim wide) of T tokens rotated in place; either may be null
 int launch_rope_rows(wgml_ctx *ctx, int variant, uint32_t head_size, uint32_t kv_dim, uint32_t pos0,

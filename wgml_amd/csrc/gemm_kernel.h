@@ -49,7 +49,8 @@ struct __attribute__((packed, aligned(2))) Half2Aligned {
 // Lane (g, j) of a wave holds, for half chunk Q of row j of its row block, the elements
 // 256 u + 32 Q + 8 g .. + 7 (u: unit of 256 columns, Q in 0..7).  A format provides
 //   Unit      the bytes of one unit, in four pieces (piece c: what half chunks 2 c and 2 c + 1 need
-//             and the pieces before it have not fetched; rows are addressed with 32-bit offsets)
+//             and the pieces before it have not fetched)
+//   to_row    moves a matrix to the first row of a tile; its lanes' rows are 32-bit offsets from there
 //   Dec       what is decoded once per unit
 //   operand   the 8 halves of half chunk Q, and the low parts where the format has them
 //   scale     of half chunk Q (blocks of 32) or of the unit
@@ -166,6 +167,7 @@ struct GemmQ4K {
     struct Lane {
         uint32_t hdr, qs;
     };
+    __device__ static void to_row(GemmMat &m, uint32_t ncols, uint32_t row) { m.p0 += (size_t)row * (ncols / 256) * 144; }
     __device__ static void lane_init(Lane &l, uint32_t ncols, uint32_t row, uint32_t g) {
         l.hdr = row * (ncols / 256) * 144;
         l.qs = l.hdr + 16 + 8 * g;
@@ -213,6 +215,7 @@ struct GemmQ5K {
     struct Lane {
         uint32_t hdr, qh, qs;
     };
+    __device__ static void to_row(GemmMat &m, uint32_t ncols, uint32_t row) { m.p0 += (size_t)row * (ncols / 256) * 176; }
     __device__ static void lane_init(Lane &l, uint32_t ncols, uint32_t row, uint32_t g) {
         l.hdr = row * (ncols / 256) * 176;
         l.qh = l.hdr + 16 + 8 * g;
@@ -268,6 +271,13 @@ struct GemmQ6K {
     struct Lane {
         uint32_t ql, qh, sc, d;
     };
+    __device__ static void to_row(GemmMat &m, uint32_t ncols, uint32_t row) {
+        const size_t blk = (size_t)row * (ncols / 256);
+        m.p0 += blk * 128;
+        m.p1 += blk * 64;
+        m.p2 += blk * 16;
+        m.p3 += blk * 2;
+    }
     __device__ static void lane_init(Lane &l, uint32_t ncols, uint32_t row, uint32_t g) {
         const uint32_t blk = row * (ncols / 256);
         l.ql = blk * 128 + 8 * g;
@@ -347,6 +357,10 @@ struct GemmQ8_0 {
     struct Lane {
         uint32_t q, d;
     };
+    __device__ static void to_row(GemmMat &m, uint32_t ncols, uint32_t row) {
+        m.p0 += (size_t)row * ncols;
+        m.p1 += (size_t)row * (ncols / 32) * 2;
+    }
     __device__ static void lane_init(Lane &l, uint32_t ncols, uint32_t row, uint32_t g) {
         l.q = row * ncols + 8 * g;
         l.d = row * (ncols / 32) * 2;
@@ -393,6 +407,7 @@ struct GemmQ8K {
     struct Lane {
         uint32_t d, q;
     };
+    __device__ static void to_row(GemmMat &m, uint32_t ncols, uint32_t row) { m.p0 += (size_t)row * (ncols / 256) * 292; }
     __device__ static void lane_init(Lane &l, uint32_t ncols, uint32_t row, uint32_t g) {
         l.d = row * (ncols / 256) * 292;
         l.q = l.d + 4 + 8 * g;
@@ -440,6 +455,7 @@ struct GemmLegacy {
         uint32_t blk, dm, q;
     };
     static constexpr uint32_t QS = 2 + (HAS_M ? 2 : 0) + (HAS_QH ? 4 : 0);
+    __device__ static void to_row(GemmMat &m, uint32_t ncols, uint32_t row) { m.p0 += (size_t)row * (ncols / 32) * BYTES; }
     __device__ static void lane_init(Lane &l, uint32_t ncols, uint32_t row, uint32_t g) {
         l.blk = row * (ncols / 32) * BYTES;
         l.dm = l.blk + 2 * g * BYTES;
@@ -668,10 +684,11 @@ __global__ __launch_bounds__(256, (gemm_workgroups<F, SPLIT>(NT))) void gemm_lds
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
     const uint32_t j = lane & 15, g = lane >> 4;
     const uint32_t ky = blockIdx.x % a.ks, tile = blockIdx.x / a.ks;
-    const GemmMat m = matrix_of_tile(a, tile);
-    const uint32_t row0 = (tile - m.tile0) * 64 + wave * 16;
+    GemmMat m = matrix_of_tile(a, tile);
+    const uint32_t tile_row = (tile - m.tile0) * 64, row0 = tile_row + wave * 16;
+    F::to_row(m, a.ncols, tile_row);
     typename F::Lane wl;
-    F::lane_init(wl, a.ncols, min(row0 + j, m.nrows - 1), g);
+    F::lane_init(wl, a.ncols, min(wave * 16 + j, m.nrows - 1 - tile_row), g);
     const uint32_t nunits = a.kpad / KU, u0 = nunits * ky / a.ks, u1 = nunits * (ky + 1) / a.ks;
 
     floatx4 acc[NT];
@@ -840,10 +857,11 @@ __global__ __launch_bounds__(512) void gemm_tile_kernel(const GemmArgs a) {
     const uint32_t v = xcd * q8 + min(xcd, r8) + (blockIdx.x >> 3);
     const uint32_t tt = v % a.ttiles, rtiles = n_wg / (a.ttiles * a.ks);
     const uint32_t tile = (v / a.ttiles) % rtiles, ky = v / a.ttiles / rtiles;
-    const GemmMat m = matrix_of_tile(a, tile);
+    GemmMat m = matrix_of_tile(a, tile);
     const uint32_t row0 = (tile - m.tile0) * TILE_ROWS;
+    F::to_row(m, a.ncols, row0);
     typename F::Lane wl;
-    F::lane_init(wl, a.ncols, min(row0 + 16 * wave + j, m.nrows - 1), g);
+    F::lane_init(wl, a.ncols, min(16 * wave + j, m.nrows - 1 - row0), g);
     const uint32_t nunits = a.kpad / KU, u0 = nunits * ky / a.ks, u1 = nunits * (ky + 1) / a.ks;
 
     floatx4 acc[4][4];

@@ -802,9 +802,12 @@ bool gemm_supported(const wgml_qmat *q) {
     return q->type != WGML_F32 && gemv_fused_supported(q) && q->max_abs <= kGemmMaxWeight;  // the nine quantized formats
 }
 
-// The kernels address a matrix plane with 32-bit lane offsets (at most 1 byte per element).
+// The kernels address the rows of a tile in a plane with 32-bit offsets: at most 1 byte per element, but 292 per 256 in Q8_K,
+// which matters to tiles of 2^32 bytes only.
 bool gemm_addressable(const wgml_qmat *q) {
-    return (uint64_t)q->nrows * q->ncols < (uint64_t(1) << 32) - 4096;
+    constexpr uint64_t limit = (uint64_t(1) << 32) - 4096;
+    const uint64_t rows = q->nrows < TILE_ROWS ? q->nrows : TILE_ROWS;
+    return (uint64_t)q->nrows * q->ncols < limit && (q->type != WGML_Q8_K || rows * (q->ncols / 256) * 292 < limit);
 }
 
 // hipMalloc for a workspace: callers with a path that needs none of it go on with that where the
@@ -926,8 +929,8 @@ int launch_gemm_quant_multi(wgml_ctx *ctx, const GemmTarget *targets, int n, con
                              "the batched product (up to %g only); use the per-token product",
                              (double)q->max_abs, (double)kGemmMaxWeight);
         if (!gemm_addressable(q))
-            return set_error(WGML_E_UNSUPPORTED, "gemm_quant: a matrix of %u x %u elements (below 2^32 only)",
-                             q->nrows, q->ncols);
+            return set_error(WGML_E_UNSUPPORTED, "gemm_quant: a matrix of %u x %u elements (below 2^32 only, 128 rows below "
+                             "2^32 bytes)", q->nrows, q->ncols);
         GemmMat &g = a.m[i];
         g.p0 = q->p0;
         g.p1 = q->p1;
