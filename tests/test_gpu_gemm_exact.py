@@ -1,4 +1,4 @@
-"""GPU parity: the batched product where its tiles, units and operand forms end, on random block bits.
+"""GPU parity: the batched products, short and long runs, where tiles, units and operand forms end, on random block bits.
 
 Random bytes reach the largest integers of a format (Q6_K: (q - 32) * scale of 4064 and more, which one f16
 number does not hold; Q5_K: 31 * 63) and every sign.  With split operands the weights are exact and an
@@ -46,10 +46,35 @@ def test_products_to_fp32_rounding(gpu, qtype, T, nrows, units):
     W.GemmQuant.from_device(gpu).dispatch(out, m, W.GpuVector.init(gpu, x.reshape(-1)), T)
     got = out.read().reshape(T, nrows)
     xa = np.abs(x).astype(np.float64)
+    assert (np.abs(got - x.astype(np.float64) @ w.T) <= 2 * split_bound(qtype, xa, w)).all()
+
+
+def split_bound(qtype, xa, w):
     parts = xa @ np.abs(w).T + (xa.sum(1)[:, None] * 2 * np.abs(w).max() if qtype in (W.Q4_1, W.Q5_1, W.Q4_K, W.Q5_K) else 0)
-    low = np.abs(x).max(1)[:, None] * 2.0 ** -34 * np.abs(w).sum(1)[None, :]  # low parts at the bottom of f16
-    bound = 2 * (2.0 ** -22 * (xa @ np.abs(w).T) + (ncols / 32 + 4) * 2.0 ** -24 * parts + low)
-    assert (np.abs(got - x.astype(np.float64) @ w.T) <= bound).all()
+    low = xa.max(1)[:, None] * 2.0 ** -34 * np.abs(w).sum(1)[None, :]  # low parts at the bottom of f16
+    return 2.0 ** -22 * (xa @ np.abs(w).T) + (xa.shape[1] / 32 + 4) * 2.0 ** -24 * parts + low
+
+
+@pytest.mark.parametrize("qtype", list(SIZES))
+@pytest.mark.parametrize("T,nrows,units", [(1, 17, 2), (16, 64, 1), (17, 65, 3), (33, 130, 2), (49, 63, 5), (65, 64, 2),
+                                           (96, 130, 3), (97, 16, 1), (128, 65, 9)])
+def test_products_in_plain_f16(gpu, qtype, T, nrows, units):
+    """An activation keeps 11 bits (half a last place: 2^-11 of |w x|, low parts as above), integers of a weight
+    are exact but for Q6_K's products, which keep 11 bits too; fp32 sums as in split precision."""
+    ncols = 256 * units - (0 if SIZES[qtype] > 40 else 32 * (units + T) % 224)
+    raw = random_blocks(qtype, nrows * ncols, T)
+    w = orc.dequantize(qtype, raw, nrows * ncols).reshape(nrows, ncols).astype(np.float64)
+    x = W.rng_normal(T, T * ncols).reshape(T, ncols)
+    out = W.GpuVector.init(gpu, np.full(T * nrows, np.nan, dtype=np.float32))
+    m = W.GpuQuantMatrix(gpu, qtype, nrows, ncols, raw)
+    gpu.set_gemm_precision(0)
+    try:
+        W.GemmQuant.from_device(gpu).dispatch(out, m, W.GpuVector.init(gpu, x.reshape(-1)), T)
+    finally:
+        gpu.set_gemm_precision(1)
+    xa = np.abs(x).astype(np.float64)
+    bound = 2.0 ** -11 * (2 if qtype == W.Q6_K else 1) * (xa @ np.abs(w).T) + 2 * split_bound(qtype, xa, w)
+    assert (np.abs(out.read().reshape(T, nrows) - x.astype(np.float64) @ w.T) <= bound).all()
 
 
 @pytest.mark.parametrize("qtype", list(SIZES))
@@ -112,6 +137,25 @@ def v_rows(gpu, qtype, raw, nrows, ncols, x, precision=1):
         gpu.set_gemm_precision(1)
     xd = te.astype(np.float64)
     return np.asarray(m.kv_download(0, 1, 0, len(x))), xd / np.sqrt((xd ** 2).mean(1, keepdims=True) + 1e-5)
+
+
+@pytest.mark.parametrize("precision", [1, 0], ids=["split_f16", "plain_f16"])
+@pytest.mark.parametrize("qtype", list(SIZES))
+@pytest.mark.parametrize("T,nrows,ncols", [(129, 32, 512), (200, 96, 288), (256, 160, 320), (257, 320, 1280), (300, 64, 256),
+                                           (513, 256, 512)])
+def test_long_runs(gpu, qtype, T, nrows, ncols, precision):
+    """As above, in tiles of 128 rows x 256 tokens (K and V beside the Q matrix, which is ncols rows): two more roundings of
+    2^-22 in the norm; plain f16 rounds the weights themselves as well, times 2^8, of which the smallest keep 2^-25."""
+    if ncols % 256 and SIZES[qtype] > 40:
+        nrows, ncols = 96, 768
+    raw = random_blocks(qtype, nrows * ncols, T)
+    w = orc.dequantize(qtype, raw, nrows * ncols).reshape(nrows, ncols).astype(np.float64)
+    got, x = v_rows(gpu, qtype, raw, nrows, ncols, W.rng_normal(T, T * ncols).reshape(T, ncols), precision)
+    xa = np.abs(x)
+    bound = 2 * split_bound(qtype, xa, w) + 2.0 ** -21 * (xa @ np.abs(w).T)
+    if precision == 0:
+        bound += 2.0 ** -10 * (xa @ np.abs(w).T) + 2.0 ** -33 * xa.sum(1)[:, None]
+    assert (np.abs(got - x @ w.T) <= bound).all()
 
 
 @pytest.mark.parametrize("long_run", [False, True], ids=["product", "long_run"])

@@ -88,3 +88,26 @@ def test_rows_and_columns_beyond_whole_tiles(gpu, k_split, dim, heads, kv_heads,
         compare(gpu, cfg, weights(cfg, "q8_0", True), LlamaModelType.Qwen2, 210)
     finally:
         gpu.set_tuning(gpu.TUNE_GEMM_K_SPLIT, 0)
+
+
+@pytest.mark.parametrize("n,start", [(300, 0), (100, 37), (272, 41)])
+@pytest.mark.parametrize("head_size", [16, 32, 48, 64, 80, 96, 112, 128])
+def test_attention_in_four_and_in_eight_waves(gpu, head_size, n, start):
+    """16 tokens per workgroup, of four waves where heads x blocks of tokens are at least as many as the 256 compute units
+    (16 heads, 300 and 272 tokens: 304 and 272) and of eight below (100 tokens: 112), against a workgroup per token."""
+    cfg = config(16 * head_size, 256, 16, 4, 400)
+    w = weights(cfg, "q8_0", False)
+    toks = W.prompt_tokens(9, start + n, cfg.vocab_size)
+    got = []
+    for per_token in (0, 1):
+        m = Llama2(gpu, cfg, LlamaModelType.Llama).load(w)
+        gpu.set_tuning(gpu.TUNE_PREFILL_ATTENTION_PER_TOKEN, per_token)
+        try:
+            if start:
+                m.prefill(toks[:start])
+            m.prefill(toks[start:], start_pos=start)
+        finally:
+            gpu.set_tuning(gpu.TUNE_PREFILL_ATTENTION_PER_TOKEN, 0)
+        got.append(state(m, cfg, start + n))
+    for a, b in zip(*got):
+        assert np.isfinite(a).all() and np.abs(a - b).max() <= 2e-4 * np.abs(b).max()
