@@ -77,6 +77,24 @@ def test_rows_whose_long_runs_the_products_cannot_address_go_in_short_ones(runti
     """)
 
 
+def test_partial_sums_take_a_launch_only_where_it_pays(runtime):
+    # nothing adds a product's partial sums on its way: two parts of 512 columns were slower than one for a few vectors
+    host_hip.run(runtime, """
+    def reductions(nrows, ncols, n, qtype=W.Q8_0):
+        m = W.GpuQuantMatrix(gpu, qtype, nrows, ncols, np.zeros(W.quant_bytes(qtype, nrows * ncols), np.uint8))
+        out, x = W.GpuVector.uninit(gpu, n * nrows), W.GpuVector.uninit(gpu, n * ncols)
+        names = launched(lambda: W.GemmQuant.from_device(gpu).dispatch(out, m, x, n))
+        assert count(names, "gemm_lds_kernel") == 1 and len(names) == 2 + count(names, "gemm_reduce_kernel")
+        return count(names, "gemm_reduce_kernel")
+
+    for shape in ((64, 256, 128), (64, 288, 1), (64, 512, 16), (4096, 512, 16), (1024, 768, 1), (32000, 1024, 48)):
+        assert reductions(*shape) == 0, shape
+    for shape in ((64, 512, 128), (64, 1024, 128), (64, 4096, 1), (4096, 4096, 1), (256, 16384, 16)):
+        assert reductions(*shape) == 1, shape
+    assert reductions(1024, 768, 1, W.Q4_0) == 1  # a unit takes longer there
+    """)
+
+
 def test_matrices_that_the_products_address(runtime):
     # rows of a tile at 32-bit offsets from its first one: below 2^32 weights as before, also where they take more bytes
     # (Q8_K, 292 per 256), unless one tile alone does

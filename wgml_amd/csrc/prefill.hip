@@ -41,6 +41,21 @@ using namespace wgml;
 
 namespace {
 
+// p[0] + p[stride] + ..., n of them in this order, eight loads at a time (one by one they are a chain of trips to memory)
+__device__ __forceinline__ float sum_of_parts(const float *p, size_t stride, uint32_t n) {
+    float v = 0.f;
+    uint32_t y = 0;
+    for (; y + 8 <= n; y += 8) {
+        float q[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) q[k] = p[(y + k) * stride];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v += q[k];
+    }
+    for (; y < n; ++y) v += p[y * stride];
+    return v;
+}
+
 // out[t][r] (= or +=) xscale[t] * (part[0][t][r] + part[1][t][r] + ...) + bias[r]
 __global__ __launch_bounds__(256) void gemm_reduce_kernel(const GemmArgs a) {
     const uint32_t rg = blockIdx.x * 256 + threadIdx.x, t = blockIdx.y;  // row among all matrices
@@ -50,9 +65,7 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(const GemmArgs a) {
     if (a.nmat > 2 && rg >= a.m[2].roff) mi = 2;
     const GemmMat &m = a.m[mi];
     const uint32_t r = rg - m.roff;
-    const float *p = a.part + (size_t)t * a.total_rows + rg;
-    float v = p[0];
-    for (uint32_t y = 1; y < a.ks; ++y) v += p[(size_t)y * a.T * a.total_rows];
+    float v = sum_of_parts(a.part + (size_t)t * a.total_rows + rg, (size_t)a.T * a.total_rows, a.ks);
     v *= a.xscale ? a.xscale[t] : 1.f;
     if (m.bias) v += m.bias[r];
     float *o = m.out + (size_t)t * m.out_stride + r;
@@ -764,19 +777,40 @@ void launch_attn_block(wgml_ctx *ctx, const AttnRowsArgs &a, uint32_t n_heads, u
 //   first bytes of each, so K is split into about 448 workgroups of the same number of units (256, 320,
 //   384, 512, 600 instead: 0-6 % slower over a pass of 4 .. 128 tokens through the 7B shape, 3072 x 8192 and
 //   768 x 2048; workgroups of one unit each up to 40 %).
+//   Where the partial sums take a launch of their own (nothing behind the product adds or rotates its rows), no more than
+//   pays: with T = 16 nt tokens a unit takes about 0.2 + 0.5 nt us (Q4_0 .. Q5_1, whose blocks come in pieces, 1.4 + 0.5 nt), the
+//   launch 3.1 - 0.25 nt, a part 0.09 and 1.5 (1 + nt) ns per tile, and workgroups that share a compute unit slow each other by a
+//   third (fitted to 1, 16, 45 and 128 tokens, 16 .. 4096 rows, 512 .. 65536 columns, Q8_0 and Q4_K, ks from 1 to 256: 1.1 % above
+//   the best ks on average, 20 % at most).  Against 448 workgroups here too, one vector: 256 x 512 in Q8_0 11.9 us -> 9.2,
+//   256 x 16384 26.7 -> 17.4; 128 vectors 40.1 -> 28.8.
 //   longer runs: one workgroup per compute unit; the ks with the least time in units of K, one unit per
 //   round of the grid for its start, end and results.
 constexpr size_t kTilePartBytes = size_t(128) << 20;
-uint32_t gemm_k_split(const wgml_ctx *ctx, uint32_t tiles, uint32_t units, bool tall, size_t part_bytes) {
+uint32_t gemm_k_split(const wgml_ctx *ctx, int type, uint32_t tiles, uint32_t units, uint32_t nt, bool tall,
+                      bool own_launch, size_t part_bytes) {
     const int forced = ctx->tuning[WGML_TUNE_GEMM_K_SPLIT];
     if (forced) return min((uint32_t)forced, units);
-    if (!tall) {
-        const uint32_t want = 448, per = max(1u, (units * tiles + want / 2) / want);
-        return per >= units ? 1 : (units + per - 1) / per;
-    }
     const uint32_t cu = ctx->n_cu > 0 ? (uint32_t)ctx->n_cu : 256u;
     uint32_t best = 1;
     float best_cost = 1e30f;
+    if (!tall) {
+        const uint32_t want = 448, per = max(1u, (units * tiles + want / 2) / want);
+        const uint32_t most = per >= units ? 1 : (units + per - 1) / per;
+        if (!own_launch) return most;
+        const bool pieces = type == WGML_Q4_0 || type == WGML_Q4_1 || type == WGML_Q5_0 || type == WGML_Q5_1;
+        const float unit = (pieces ? 1.4f : 0.2f) + 0.5f * (float)nt;
+        const float part = 0.09f + 1.5e-3f * (float)(tiles * (1 + nt));
+        for (uint32_t ks = 1; ks <= most; ++ks) {
+            const float shared = tiles * ks > cu ? (float)(tiles * ks - cu) / (float)cu : 0.f;
+            const float cost = (float)((units + ks - 1) / ks) * unit * (1.f + 0.35f * shared) +
+                               (ks > 1 ? 3.1f - 0.25f * (float)nt + (float)ks * part : 0.f);
+            if (cost < best_cost) {
+                best_cost = cost;
+                best = ks;
+            }
+        }
+        return best;
+    }
     for (uint32_t ks = 1; ks <= 8 && ks <= units && (ks == 1 || ks * part_bytes <= kTilePartBytes); ++ks) {
         const float cost = (float)((tiles * ks + cu - 1) / cu) * ((float)((units + ks - 1) / ks) + 1.f);
         if (cost < best_cost) {
@@ -973,31 +1007,31 @@ int launch_gemm_quant_multi(wgml_ctx *ctx, const GemmTarget *targets, int n, con
     if (ctx->gemm_pending_ks)
         return set_error(WGML_E_INVALID, "gemm_quant: the partial sums a previous product left for its "
                                          "output were not added yet (launch_prefill_prep / launch_gemm_flush)");
-    a.ks = gemm_k_split(ctx, tiles * a.ttiles, a.kpad / KU, a.tall, (size_t)T * a.total_rows * sizeof(float));
+    // the caller's next kernel adds the partial sums up itself: one matrix, plain += only, ...
+    const bool residual = n == 1 && accumulate && !targets[0].bias;
+    // ... or a gate / up pair whose next kernel is the gated launch_prefill_prep on (gate out, up out)
+    const bool pair = n == 2 && !accumulate && !targets[0].bias && !targets[1].bias &&
+                      targets[0].m->nrows == targets[1].m->nrows && targets[0].m->nrows % 8 == 0 &&
+                      targets[0].m->nrows <= 8u * 2 * 1024;
+    const bool defer = defer_reduce && (residual || pair);
+    // the kernel that adds them rotates the marked targets, if rows come in pairs
+    bool rotate = rope && !defer && !accumulate && rope->head_size >= 2 && rope->head_size % 2 == 0;
+    for (int i = 0; rotate && i < n; ++i)
+        rotate = targets[i].m->nrows % 2 == 0 && (!targets[i].rope || targets[i].m->nrows % rope->head_size == 0);
+    a.ks = gemm_k_split(ctx, first->type, tiles * a.ttiles, a.kpad / KU, a.nt, a.tall, !defer && !rotate,
+                        (size_t)T * a.total_rows * sizeof(float));
     if (a.ks > 1) {
         WGML_TRY(ensure_gemm_partials(ctx, (size_t)a.ks * T * a.total_rows * sizeof(float)));
         a.part = ctx->gemm_part;
-        // the caller's next kernel adds the partial sums up itself (one matrix, plain += only)
-        const bool residual = n == 1 && accumulate && !targets[0].bias;
-        // a gate / up pair whose next kernel is the gated launch_prefill_prep on (gate out, up out)
-        const bool pair = n == 2 && !accumulate && !targets[0].bias && !targets[1].bias &&
-                          targets[0].m->nrows == targets[1].m->nrows && targets[0].m->nrows % 8 == 0 &&
-                          targets[0].m->nrows <= 8u * 2 * 1024;
-        a.defer = defer_reduce && (residual || pair);
-        if (a.defer) {
+        a.defer = defer;
+        if (defer) {
             ctx->gemm_pending_ks = a.ks;
             ctx->gemm_pending_pair = pair ? 1 : 0;
         }
     }
     if (rope) {
-        // the kernel that adds the partial sums rotates the marked targets, if there is one and
-        // rows come in pairs
-        bool pairs = a.ks > 1 && !a.defer && !accumulate && rope->head_size >= 2 && rope->head_size % 2 == 0;
-        for (int i = 0; i < n; ++i)
-            pairs = pairs && targets[i].m->nrows % 2 == 0 &&
-                    (!targets[i].rope || targets[i].m->nrows % rope->head_size == 0);
-        rope->applied = pairs;
-        if (pairs) {
+        rope->applied = rotate && a.ks > 1;
+        if (rope->applied) {
             a.rope_head_size = rope->head_size;
             a.rope_pos0 = rope->pos0;
             a.rope_base = rope->base_freq;
