@@ -674,11 +674,13 @@ __global__ __launch_bounds__(256, (gemm_workgroups<F, SPLIT>(NT))) void gemm_lds
     constexpr uint32_t CW = NT * 128, CWX = CW * PARTS, STAGE = CPS * CWX, SUMS = F::OFFSET ? NT * 32 : 0;
     constexpr int SW = STAGE / 256;  // staged words per thread
     constexpr bool WLO = F::PAIR && SPLIT, G32 = F::GROUP == 32;
-    // half chunks whose products pile up before the scale multiplies them.  An MFMA's own additions round more than a
-    // multiply-add does: eight of them, as in the other formats with a scale per unit, give 2.7e-7 of the result's rms
-    // (Q4_K, |N(0,1)| activations, K = 512 .. 4096), four 2.2e-7, two 1.9e-7 to 2.0e-7; weights expanded to fp32 first gave
-    // 2.1e-7.  Two against eight cost 1 % of a pass of 5 .. 64 tokens, 4 % of 128 (7B widths).
-    constexpr int CHAIN = F::OFFSET && SPLIT ? 2 : 8;
+    // Half chunks whose products pile up before the scale multiplies them.  An MFMA's own additions round more than a
+    // multiply-add does: eight half chunks of high and low parts in one sum, as in the other formats with a scale per unit, give
+    // 2.7e-7 of the result's rms (Q4_K, |N(0,1)| activations, K = 512 .. 4096); weights expanded to fp32 first gave 2.1e-7.
+    // Where weights have an offset the low parts, a thousandth as large, have a sum of their own, and the high parts one of four
+    // half chunks: 1.9e-7 (in one sum of two half chunks 2.0e-7, and 4 % slower at 128 tokens of the 7B widths).
+    constexpr int CHAIN = F::OFFSET && SPLIT && !G32 ? 4 : 8;
+    constexpr bool APART = F::OFFSET && SPLIT && !G32;
     const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
     const uint32_t tid = threadIdx.x, lane = tid & 63;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
@@ -733,7 +735,7 @@ __global__ __launch_bounds__(256, (gemm_workgroups<F, SPLIT>(NT))) void gemm_lds
     for (uint32_t u = u0; u < u1; ++u) {
         const uint32_t next = unit_at(u + 1);
         typename F::Dec ndec;
-        floatx4 tmp[G32 ? 1 : NT];
+        floatx4 tmp[G32 ? 1 : NT], low[APART ? NT : 1];
         uint32_t off_hi = 0, off_lo = 0;
         if constexpr (F::OFFSET) F::offsets(off_hi, off_lo, dec, g, m.offset_up);
         static_for<0, NS>([&](auto s_c) {
@@ -769,7 +771,10 @@ __global__ __launch_bounds__(256, (gemm_workgroups<F, SPLIT>(NT))) void gemm_lds
                 if constexpr (i + AHEAD < NSTEP) fetch(std::integral_constant<int, i + AHEAD>{});
                 const half8 x8 = as_half8(bh[slot]);
                 floatx4 t = mfma(x8, as_half8(o.hi), G32 || q % CHAIN == 0 ? zero : tmp[G32 ? 0 : n]);
-                if constexpr (SPLIT) t = mfma(as_half8(bl[slot]), as_half8(o.hi), t);
+                if constexpr (APART)
+                    low[n] = mfma(as_half8(bl[slot]), as_half8(o.hi), q == 0 ? zero : low[n]);
+                else if constexpr (SPLIT)
+                    t = mfma(as_half8(bl[slot]), as_half8(o.hi), t);
                 if constexpr (WLO) t = mfma(x8, as_half8(o.lo), t);
                 if constexpr (n == 0) {
                     if constexpr (q < 7) {
@@ -802,8 +807,10 @@ __global__ __launch_bounds__(256, (gemm_workgroups<F, SPLIT>(NT))) void gemm_lds
             if constexpr (!G32) add_scaled(acc[NT - 1], tmp[NT - 1], F::unit_scale(dec));
             if constexpr (F::OFFSET) {
 #pragma unroll
-                for (int n = 0; n < NT; ++n)
+                for (int n = 0; n < NT; ++n) {
+                    if constexpr (APART) add_scaled(acc[n], low[n], F::unit_scale(dec));
                     add_scaled(acc[n], mfma(as_half8(sums[n * 32]), as_half8(offs), zero), m.offset_down);
+                }
             }
         }
         dec = ndec;
@@ -843,7 +850,7 @@ __global__ __launch_bounds__(512) void gemm_tile_kernel(const GemmArgs a) {
     // plain f16: the sums need no scaling per block (direct), split f16: per 32 columns or per unit (tmp)
     constexpr bool DIRECT = !SPLIT, OFFSET = F::OFFSET && SPLIT, WLO = L::WPARTS == 2;
     constexpr bool G32 = F::GROUP == 32 && SPLIT, TMP = F::GROUP == 256 && SPLIT;
-    constexpr int CHAIN = F::OFFSET ? 4 : 8;  // as in gemm_lds_kernel: 2.1e-7 to 2.4e-7 (expanded weights 2.7e-7 to 3.7e-7)
+    constexpr int CHAIN = F::OFFSET ? 4 : 8;  // see gemm_lds_kernel: 2.2e-7 (expanded weights 2.7e-7 to 3.7e-7)
     constexpr int SW = 2 * L::XPARTS;  // staged words of activations per thread and half chunk
     const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
     const uint32_t tid = threadIdx.x, lane = tid & 63;
