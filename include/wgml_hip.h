@@ -172,17 +172,20 @@ WGML_API int wgml_gemv_quant(wgml_ctx *ctx, wgml_view out, const wgml_qmat *m, w
  * out[t] = m * x[t], with x n_tokens x ncols and out n_tokens x nrows, both row-major.
  * No counterpart in the reference, which multiplies one vector at a time
  * (GemvQuant::dispatch above); it is the building block of wgml_llama2_prefill.
- * The matrix cores multiply the weights' integers, which f16 holds exactly; scales and
- * minima are applied to the sums of a sub-block in fp32.
+ * The matrix cores multiply the weights' integers, which f16 holds exactly; scales are
+ * applied to fp32 sums, and what a weight has beside its integer (the minima of Q4_K, Q5_K,
+ * Q4_1, Q5_1) is multiplied with the sums of 32 vector elements, both as pairs of f16 numbers.
  * Precision (wgml_ctx_set_gemm_precision): level 1, the default, takes the vectors as
- * pairs of f16 numbers (high part + low part), two MFMAs per 32 terms, fp32 sums: results agree with n_tokens calls of
- * wgml_gemv_quant to fp32 rounding (about 1e-6 of a row's magnitude).  Level 0 rounds
- * weights and vectors to f16 once: 1.4x faster, about 3e-4 of a row's magnitude
- * (up to 1.4e-3 for single elements).  m: any of the nine quantized block formats
+ * pairs of f16 numbers (high part + low part), two MFMAs per 32 terms (three for Q6_K, whose
+ * products of quant and scale take a pair too), fp32 sums: 0.9e-7 to 2.4e-7 of the results' RMS from
+ * the exact product of the dequantized weights (512 to 11008 columns, elements of both signs or of one).
+ * Level 0 rounds the vectors to f16 once, and Q6_K's products of quant and scale: one MFMA, up to
+ * 1.1x faster for one vector and 1.4x for 128, about 2e-4 of the results' RMS (runs of more than
+ * 128 tokens in wgml_llama2_prefill round every weight once as well: 3e-4).  m: any of the nine quantized block formats
  * (Q8_0, Q4_K, Q6_K, Q4_0, Q4_1, Q5_0, Q5_1, Q5_K, Q8_K); not F32 / F16.
  * Vectors of any magnitude are taken (scaled per vector by a power of two); the
- * dequantized weights must not exceed 255.875 in magnitude (they pass through f16 times 2^8,
- * and 65504 is the largest finite f16): a bound on the largest weight is computed when the
+ * dequantized weights must not exceed 255.875 in magnitude (long runs at level 0 pass them
+ * through f16 times 2^8, and 65504 is the largest finite f16; one rule serves all): a bound on the largest weight is computed when the
  * matrix is created, and a matrix whose bound is larger is refused with WGML_E_UNSUPPORTED
  * (wgml_gemv_quant takes any value;
  * wgml_llama2_prefill steps through the prompt token by token for such a model).

@@ -4,7 +4,7 @@ Random bytes reach the largest integers of a format (Q6_K: (q - 32) * scale of 4
 number does not hold; Q5_K: 31 * 63) and every sign.  With split operands the weights are exact and an
 activation keeps 22 bits, so a result is off by at most 2^-22 of sum |w x| (half a last place of the low part,
 as rows scale to at most 1024), plus fp32 sums: K / 32 + 4 roundings of 2^-24 of sums no larger than
-sum |q scale x| + sum |min x|, the two parts of a weight apart.  Twice that is allowed.
+sum |w x| or, where a weight is an integer's part and an offset, sum |x| times twice the largest weight.  Twice that is allowed.
 """
 import ctypes
 

@@ -5,13 +5,13 @@ The reference has neither: it runs the prompt through its batch-1 step token by 
 sequence -- the oracle's N single-token steps on the same quantized bytes.
 
 Two precisions (wgml_ctx_set_gemm_precision), both tested:
-  1 (default)  operands as pairs of f16 numbers (high + low part), fp32 sums: products agree with
+  1 (default)  activations as pairs of f16 numbers (high + low part), fp32 sums: products agree with
                the exact product of the dequantized weights to fp32 rounding.  Bounds:
                |gpu - ref| <= 1e-4 * |ref| + 2e-5 * rms(ref) for products, 2e-4 * max|ref| for
                logits and cache rows after a whole model pass (the tolerance of the step itself is
                1e-3; observed ~1e-6 and ~2e-5).
-  0            operands rounded to f16 once: a product's error is about 2^-11 / sqrt(3) per term,
-               random in sign, ~3e-4 of rms(ref) observed.  Bounds: 1e-3 * |ref| + 2e-3 * rms(ref)
+  0            activations rounded to f16 once (in runs of more than 128 tokens weights too): a product's
+               error is about 2^-12 / sqrt(3) per term and operand, random in sign, 2e-4 to 3e-4 of rms(ref) observed.  Bounds: 1e-3 * |ref| + 2e-3 * rms(ref)
                for products, 3e-3 * max|ref| after a whole pass of the 2-layer models.
 """
 import numpy as np
@@ -175,9 +175,8 @@ def test_gemm_large_activations_stay_finite(gpu, k_split, qtype):
 @pytest.mark.parametrize("qtype", QT)
 @pytest.mark.parametrize("x_scale,w_std", [(1e-3, 0.02), (300.0, 0.02), (1.0, 1.0), (1.0, 1e-3), (1.0, 20.0)])
 def test_gemm_operand_magnitudes(gpu, qtype, x_scale, w_std):
-    # The low parts of the split operands are small numbers: activations are scaled per token into
-    # (512, 1024] (up as well as down) and weights expanded times 2^8 so that they stay f16
-    # numbers.  Small and large activations, small and large weights (|w| <= 255.875 is the limit),
+    # The low parts of the activations are small numbers: activations are scaled per token into
+    # (512, 1024] (up as well as down) so that they stay f16 numbers; weights are integers times fp32 scales.  Small and large activations, small and large weights (|w| <= 255.875 is the limit),
     # one outlier in a row: the bounds hold unchanged (observed 2e-7 rms, 2e-6 worst, split f16).
     nrows, ncols, T = 96, 2048, 40
     raw = W.quantize(qtype, W.rng_normal(31, nrows * ncols, 0, w_std))
@@ -188,7 +187,7 @@ def test_gemm_operand_magnitudes(gpu, qtype, x_scale, w_std):
 
 @pytest.mark.parametrize("qtype", QT)
 def test_gemm_weight_magnitude_limit(gpu, qtype):
-    # Weights pass through f16 times 2^8, so a matrix is taken only while a bound on its largest
+    # Long runs of plain f16 round weights to f16 times 2^8, and one rule serves all: a matrix is taken only while a bound on its largest
     # dequantized weight stays within 65504 / 256 = 255.875 (computed when the matrix is created: exact for Q8_0,
     # the ends of each sub-block's quant range for Q4_K, |d| |scale| 32 for Q6_K).  Just inside the limit the product
     # is as accurate as anywhere else; at or beyond it the call is refused and the per-token

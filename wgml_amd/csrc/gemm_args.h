@@ -28,17 +28,17 @@ struct GemmMat {
 struct GemmArgs {
     GemmMat m[3];
     uint32_t nmat;
-    const u32x4 *xh;                   // packed f16 activations (see above)
+    const u32x4 *xh;                   // packed f16 activations (order: top of prefill.hip)
     const u32x4 *xl;                   // their low parts in the same order (split precision only)
     uint32_t xl_offset;                // bytes from xh to xl
-    const u32x4 *xsum;                 // sums of 32 activations (see above)
+    const u32x4 *xsum;                 // sums of 32 activations (order: top of prefill.hip)
     uint32_t ttiles;                   // tiles of tokens
     uint32_t tall;                     // gemm_tile_kernel
     const float *xscale;               // [tpad] factor to multiply a token's results with
     uint32_t ncols, kpad, T, nt;       // nt: blocks of 16 tokens per tile
     int accumulate;                    // out += result
     float *part;                       // [ks][T][total_rows] partial sums (ks > 1)
-    uint32_t ks;                       // ways K is split between workgroups (grid.y)
+    uint32_t ks;                       // ways K is split between workgroups (its part varies fastest in the grid up to 128 tokens, slowest beyond)
     uint32_t total_rows;               // rows of all matrices of the launch
     int defer;                         // ks > 1: leave the partial sums to the next kernel
     // rotary encoding applied by gemm_reduce_rope_kernel to the matrices marked `rope`

@@ -641,10 +641,11 @@ __device__ __forceinline__ void keep_here(floatx4 &v) { asm volatile("" : "+v"(v
 // its operands in registers, each weight once, while the matrix cores multiply the half chunk
 // before, and refills the bytes of a unit piece by piece as they are used up.
 // What bounds it: with few tokens the first bytes of each workgroup and about 2.6 vector instructions per
-// weight, with many the activations, which every 64 rows read again (leave-one-out at 128 tokens: LDS reads
-// 11 %, staging 12 %, weight loads 7 %, no single one dominates).  Four layers, one pass, us, with operands
-// expanded to fp32 and three MFMAs per term -> now: 7B shape Q4_K_M 4 tokens 582 -> 487, 45: 790 -> 636, 128: 1188 ->
-// 1026 (plain f16 872 -> 751); 768 x 2048 Q8_0 4: 272 -> 232, 128: 439 -> 311.
+// weight, with many the activations, which every 64 rows read again (leave-one-out at 128 tokens, with one sum per result
+// and unit: LDS reads 11 %, staging 12 %, weight loads 7 %, no single one dominates; now MFMAs for 29 % of the cycles, 2.8 other vector
+// instructions each).  Four layers, one pass, us, with operands
+// expanded to fp32 and three MFMAs per term -> now: 7B shape Q4_K_M 4 tokens 594 -> 471, 45: 801 -> 618, 128: 1199 ->
+// 1015 (plain f16 886 -> 745); 768 x 2048 Q8_0 4: 297 -> 206, 128: 458 -> 299.
 // Measured and dropped: two row blocks per wave (128 tokens 1048 -> 1272: fewer workgroups, and no shorter
 // a time per unit); 8 waves that share rows and tokens out; activations requested two stages ahead
 // (spills below 128 registers, no faster where it fits).
@@ -826,12 +827,12 @@ __global__ __launch_bounds__(256, (gemm_workgroups<F, SPLIT>(NT))) void gemm_lds
 // blocks it multiplies.  K is walked in half chunks of 32 columns, two LDS slots in turn, one barrier
 // each: during half chunk Q slot Q & 1 is multiplied, the other one takes the activations (requested
 // during Q - 1) and weights (made during Q - 1) of Q + 1, and the operands of Q + 2 are made.
-// What bounds it: a half chunk takes about 2500 cycles for 1100 of MFMAs (18 each), 1100 of LDS and 400-800 of
-// vector instructions, which hide beside each other only in part (two waves per SIMD: 8 MFMAs and 32
-// multiply-adds take 403 cycles, apart 292 and 203).  So sums are scaled per unit where the format
+// What bounds it (Q8_0): a half chunk takes 2350 cycles for 1090 of MFMAs (17 each), 1100 of LDS and, per MFMA, 2.7
+// vector instructions, which hide beside each other only in part (two waves per SIMD: 8 MFMAs, then 32
+// multiply-adds take 452 cycles, apart 271 and 289).  So sums are scaled per unit where the format
 // allows it (tmp), not per 32 columns, and not at all in plain f16, where the weight itself is rounded.
-// Four layers, one pass of 1000 tokens, us, with three MFMAs per term -> now: 3072 x 8192 Q8_0 3543 -> 2949, plain
-// f16 2422 -> 2228; 7B shape Q4_K_M 5561 -> 5196, 3390 -> 3303.  Measured and dropped: activations requested two
+// Four layers, one pass of 1000 tokens, us, with three MFMAs per term -> now: 3072 x 8192 Q8_0 3508 -> 2830, plain
+// f16 2441 -> 2144; 7B shape Q4_K_M 5503 -> 4733, 3306 -> 3164.  Measured and dropped: activations requested two
 // half chunks ahead (5262 against 5042), tiles of 128 tokens in workgroups of 4 waves (5750), Q8_0 as pairs of
 // f16 products with a third MFMA (3535 against 3137).
 template <class F, bool SPLIT>

@@ -13,7 +13,7 @@
 //                        512 < max |x| <= 1024 so that the low parts stay clear of the bottom of the f16
 //                        range (the matrix cores take subnormal f16 inputs as they are); the weights'
 //                        integers are exact, so the product is W X_hi + W X_lo: two MFMAs per term group
-//                        (three for Q6_K), results to fp32 rounding (about 2e-7 of a row's magnitude);
+//                        (three for Q6_K), results to fp32 rounding (0.9e-7 to 2.4e-7 of their RMS, K = 512 .. 11008);
 //   plain f16            the activations rounded to f16 once, one MFMA: about 2e-4 of a row's RMS (in runs
 //                        of more than 128 tokens the weights are rounded once too: 3e-4).
 //
@@ -118,15 +118,6 @@ __global__ __launch_bounds__(256) void gemm_reduce_rope_kernel(const GemmArgs a)
     }
 }
 
-// Bound by its chain of one memory trip (row, partial sums and norm weights together), a reduction and
-// a store: 8.4 us for 128 rows of 4096 that add four partial sums, 5.8 us for 21 rows of 3072 (9.5 and 6.4 with
-// the weights requested after the first of two reductions).
-// One workgroup per token: X[t] (fp32, optionally RMS-normalised with weights w as
-// the reference does: (x * rsqrt(mean(x^2) + eps)) * w, ops/rms_norm.rs:55-63) -> f16
-// in the packed order described at the top, times the power of two that brings the row's
-// largest |x| into (512, 1024]; the factor to undo it goes to xscale[t].  Columns from K on are zero (tokens
-// from T on hold anything: a token's results are its own).  With `up` non-null the input is the gated activation
-// up[k] * silu(x[k]) (ops/silu.wgsl:13-27) instead of x itself (no normalisation then).
 // acc[n][0..7] += part[y .. y + B - 1][off[n] .. off[n] + 7], part by part in the order of y; the
 // loads of all B parts are requested before the first sum (a chain of memory round trips
 // otherwise).  ystride: floats from one part to the next.
@@ -187,6 +178,15 @@ constexpr int PREP_GROUPS = 2;  // groups of 8 columns a thread keeps in registe
 // A form of its own for LayerNorm and for GELU: tested per element at run time they cost the other
 // rows 3 % of a short prompt (8 layers of the 7B shape, 45 tokens in plain f16: 1620 us against 1574).
 enum PrepMode { PREP_RMS, PREP_LN, PREP_GELU };
+// Bound by its chain of one memory trip (row, partial sums and norm weights together), a reduction and
+// a store: 8.4 us for 128 rows of 4096 that add four partial sums, 5.8 us for 21 rows of 3072 (9.5 and 6.4 with
+// the weights requested after the first of two reductions).
+// One workgroup per token: X[t] (fp32, optionally RMS-normalised with weights w as
+// the reference does: (x * rsqrt(mean(x^2) + eps)) * w, ops/rms_norm.rs:55-63) -> f16
+// in the packed order described at the top, times the power of two that brings the row's
+// largest |x| into (512, 1024]; the factor to undo it goes to xscale[t].  Columns from K on are zero (tokens
+// from T on hold anything: a token's results are its own).  With `up` non-null the input is the gated activation
+// up[k] * silu(x[k]) (ops/silu.wgsl:13-27) instead of x itself (no normalisation then).
 template <int MODE>
 __global__ __launch_bounds__(PREP_THREADS) void prep_x_kernel(float *__restrict__ x, uint32_t x_stride,
                                                      const float *__restrict__ part, uint32_t part_ks,

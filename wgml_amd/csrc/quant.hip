@@ -53,7 +53,7 @@ __global__ void repack_q6_k(const uint16_t *__restrict__ raw, uint16_t *__restri
 // An upper bound on |w| over the dequantized matrix: Q8_0 and Q8_K |d| max|q| (exact); Q4_K and
 // Q5_K max(|dmin m|, |d sc 15 (31) - dmin m|) per sub-block (the two ends of the quant range);
 // Q6_K |d| |scale| 32 per sub-block; the 32-element blocks the ends of their ranges likewise.  The batched
-// products expand weights into f16 times 2^8 and need it within 255.875.  NaN / inf scales give
+// products round weights to f16 times 2^8 in long runs of plain f16 and need it within 255.875 there; one rule serves all.  NaN / inf scales give
 // inf.  Non-negative floats order like their bit patterns, so the maximum is an atomicMax on
 // the bits.
 __device__ __forceinline__ float nan_to_inf(float v) { return v == v ? v : INFINITY; }
