@@ -106,6 +106,9 @@ struct wgml_buf {
 //         (nrows*ncols/32 f16), so that quants load as aligned 128-bit words.
 //   Q6_K: four planes: ql (128 B/block), qh (64 B/block), scales (16 B/block),
 //         d (2 B/block), each row-major in block order.
+//   Q4_0, Q4_1, Q5_0, Q5_1: planes p0 nibbles (16 B/block), p2 fifth bits (4 B/block, Q5 only) and
+//         p1 d (2 B/block; {d, m}, 4 B/block, in the _1 formats), each row-major in block order.
+//   Q5_K, Q8_K: the GGUF bytes unchanged.
 // Plane offsets are multiples of 256 bytes; the byte total equals the GGUF size
 // up to that padding.
 struct wgml_qmat {
@@ -234,6 +237,11 @@ bool gemv_partials_supported(const wgml_ctx *ctx, const wgml_qmat *m);
 int launch_gemv_fused(wgml_ctx *ctx, const FusedGemv &f);
 // the kernel of a launch with Neox pairs (gemv_neox.hip): matrices of format fmt (0: a mix of the main ones)
 const void *gemv_neox_kernel(int fmt, int threads);
+// the kernels of a format with a source file of its own
+struct GemvKernels {
+    const void *plain, *fused1024, *fused768;
+};
+GemvKernels gemv_legacy_kernels(int fmt);  // gemv_legacy.hip: a 32-element format, or kLegacyWide + one
 
 int launch_gemv_quant(wgml_ctx *ctx, float *out, const wgml_qmat *m, const float *v,
                       const GemvEpilogue &ep);

@@ -432,62 +432,64 @@ struct GemmQ8K {
     __device__ static float unit_scale(const Dec &d) { return d.d; }
 };
 
-// The 32-element blocks Q4_0 (18 B: d, 16 B of nibbles), Q4_1 (20 B: d, m, nibbles), Q5_0 (22 B:
-// d, 32 fifth bits, nibbles), Q5_1 (24 B: d, m, fifth bits, nibbles); quantization.rs:47-162.
-// Element t of a block is the low nibble of qs[t] for t < 16 and the high nibble of qs[t - 16]
+// The 32-element blocks Q4_0, Q4_1, Q5_0, Q5_1 (quantization.rs:47-162), as planes of nibbles (p0), d or {d, m} (p1) and
+// fifth bits (p2).  Element t of a block is the low nibble of qs[t] for t < 16 and the high nibble of qs[t - 16]
 // otherwise, with bit t of qh as its fifth bit.  Half chunk Q is block 8 u + Q; a lane's t = 8 g + i, so
-// lanes g < 2 take low nibbles and g >= 2 high nibbles of the same eight bytes.  Blocks are 2-byte
-// aligned: the loads are unaligned, which gfx950 serves (a load per halfword instead, 21 tokens
-// through four layers of 3072 x 8192 in Q4_0: 901 us against 522).
-template <int BYTES, bool HAS_M, bool HAS_QH>
+// lanes g < 2 take low nibbles and g >= 2 high nibbles of the same eight bytes.
+template <bool HAS_M, bool HAS_QH>
 struct GemmLegacy {
     static constexpr int GROUP = 32;
     static constexpr bool OFFSET = HAS_M, PAIR = false;
     struct Unit {
         u32x2 q[8];
-        uint32_t qh[8];
-        uint32_t dm[2];  // of blocks 2 g and 2 g + 1: d (low half) and m (high half) as stored
+        u32x2 qh[4];
+        u32x2 dm;   // d (low half) and m (high half) of blocks 2 g and 2 g + 1 where there is an m
+        u32x4 d;    // the unit's eight scales where there is none
     };
     struct Dec {
-        uint32_t dm[8], own[HAS_M ? 2 : 1];  // of all blocks; of blocks 2 g and 2 g + 1
+        uint32_t dm[HAS_M ? 8 : 4], own[HAS_M ? 2 : 1];  // of all blocks (two to a word without m); of blocks 2 g and 2 g + 1
     };
     struct Lane {
-        uint32_t blk, dm, q;
+        uint32_t q, dm, qh;
     };
-    static constexpr uint32_t QS = 2 + (HAS_M ? 2 : 0) + (HAS_QH ? 4 : 0);
-    __device__ static void to_row(GemmMat &m, uint32_t ncols, uint32_t row) { m.p0 += (size_t)row * (ncols / 32) * BYTES; }
+    __device__ static void to_row(GemmMat &m, uint32_t ncols, uint32_t row) {
+        const size_t blk = (size_t)row * (ncols / 32);
+        m.p0 += blk * 16;
+        m.p1 += blk * (HAS_M ? 4 : 2);
+        m.p2 += blk * 4;
+    }
     __device__ static void lane_init(Lane &l, uint32_t ncols, uint32_t row, uint32_t g) {
-        l.blk = row * (ncols / 32) * BYTES;
-        l.dm = l.blk + 2 * g * BYTES;
-        l.q = l.blk + QS + 8 * (g & 1);
+        const uint32_t blk = row * (ncols / 32);
+        l.q = blk * 16 + 8 * (g & 1);
+        l.dm = HAS_M ? blk * 4 + 8 * g : blk * 2;
+        l.qh = blk * 4;
     }
     template <int C>
     __device__ static void load(Unit &r, const GemmMat &m, const Lane &l, uint32_t u) {
-        const uint8_t *unit = m.p0 + (size_t)u * (8 * BYTES);
         if (C == 0) {
-#pragma unroll
-            for (int b = 0; b < 2; ++b) {
-                if (HAS_M)
-                    r.dm[b] = load_at<Half2Aligned<uint32_t>>(unit + b * BYTES, l.dm).v;
-                else
-                    r.dm[b] = load_at<uint16_t>(unit + b * BYTES, l.dm);
-            }
+            if constexpr (HAS_M)
+                r.dm = load_at<Half2Aligned<u32x2>>(m.p1 + (size_t)u * 32, l.dm).v;
+            else
+                r.d = load_at<Half2Aligned<u32x4>>(m.p1 + (size_t)u * 16, l.dm).v;
         }
-#pragma unroll
-        for (int b = 2 * C; b < 2 * C + 2; ++b) {
-            if (HAS_QH) r.qh[b] = load_at<Half2Aligned<uint32_t>>(unit + b * BYTES + (HAS_M ? 4 : 2), l.blk).v;
-            r.q[b] = load_at<Half2Aligned<u32x2>>(unit + b * BYTES, l.q).v;
-        }
+        if constexpr (HAS_QH) r.qh[C] = load_at<Half2Aligned<u32x2>>(m.p2 + (size_t)u * 32 + 8 * C, l.qh).v;
+        r.q[2 * C] = load_at<u32x2>(m.p0 + (size_t)u * 128 + 32 * C, l.q);
+        r.q[2 * C + 1] = load_at<u32x2>(m.p0 + (size_t)u * 128 + 32 * C + 16, l.q);
     }
-    // the eight scales of a row come from its four lanes (a load of each by every lane, 16 instead of 10
-    // loads per unit: 21 tokens through eight layers of 3072 x 8192 in Q4_0 140 us more)
+    // With minima the eight pairs of a row come from its four lanes (all eight of them in every lane take six registers more
+    // through the whole unit).
     __device__ static void decode(Dec &d, const Unit &r, uint32_t) {
-        const int j4 = (int)(threadIdx.x & 15) * 4;
+        if constexpr (HAS_M) {
+            const int j4 = (int)(threadIdx.x & 15) * 4;
 #pragma unroll
-        for (int b = 0; b < 8; ++b) d.dm[b] = (uint32_t)__builtin_amdgcn_ds_bpermute((b / 2) * 64 + j4, (int)r.dm[b & 1]);
-        if (HAS_M) {
-            d.own[0] = r.dm[0];
-            d.own[HAS_M ? 1 : 0] = r.dm[1];
+            for (int b = 0; b < 8; ++b) d.dm[b] = (uint32_t)__builtin_amdgcn_ds_bpermute((b / 2) * 64 + j4, (int)(b & 1 ? r.dm.y : r.dm.x));
+            d.own[0] = r.dm.x;
+            d.own[1] = r.dm.y;
+        } else {
+            d.dm[0] = r.d.x;
+            d.dm[1] = r.d.y;
+            d.dm[2] = r.d.z;
+            d.dm[3] = r.d.w;
         }
     }
     // q << SHIFT in eight bytes
@@ -498,7 +500,7 @@ struct GemmLegacy {
         uint32_t b = __builtin_amdgcn_alignbit(r.q[Q].y, r.q[Q].y, right) & mask;
         if (HAS_QH) {
             // bits 8 g .. 8 g + 7 of qh moved to bit 4 of the eight bytes
-            const uint32_t bits = r.qh[Q] >> (8 * g);
+            const uint32_t bits = (Q & 1 ? r.qh[Q / 2].y : r.qh[Q / 2].x) >> (8 * g);
             a |= (((bits & 15u) * 0x00204081u) & 0x01010101u) << (4 + SHIFT);
             b |= ((((bits >> 4) & 15u) * 0x00204081u) & 0x01010101u) << (4 + SHIFT);
         }
@@ -517,11 +519,11 @@ struct GemmLegacy {
     __device__ static void direct(uint32_t (&o)[4], const Dec &d, const Unit &r, uint32_t g) {
         const u32x2 q = bytes<Q, 0>(r, g);
         const float s = scale<Q>(d) * kDirectScale;
-        bytes_direct(o, q.x, q.y, s, HAS_M ? f16_bits_to_f32((uint16_t)(d.dm[Q] >> 16)) * kDirectScale : -CENTRE * s);
+        bytes_direct(o, q.x, q.y, s, HAS_M ? f16_bits_to_f32((uint16_t)(d.dm[HAS_M ? Q : 0] >> 16)) * kDirectScale : -CENTRE * s);
     }
     template <int Q>
     __device__ static float scale(const Dec &d) {
-        return f16_bits_to_f32((uint16_t)(d.dm[Q] & 0xffffu));
+        return f16_bits_to_f32((uint16_t)(HAS_M ? d.dm[HAS_M ? Q : 0] & 0xffffu : d.dm[Q / 2] >> (16 * (Q & 1))));
     }
     __device__ static void offsets(uint32_t &hi, uint32_t &lo, const Dec &d, uint32_t, float up) {
         float c[2];
@@ -532,10 +534,10 @@ struct GemmLegacy {
         offset_pair(hi, lo, c[0], c[1]);
     }
 };
-using GemmQ4_0 = GemmLegacy<18, false, false>;
-using GemmQ4_1 = GemmLegacy<20, true, false>;
-using GemmQ5_0 = GemmLegacy<22, false, true>;
-using GemmQ5_1 = GemmLegacy<24, true, true>;
+using GemmQ4_0 = GemmLegacy<false, false>;
+using GemmQ4_1 = GemmLegacy<true, false>;
+using GemmQ5_0 = GemmLegacy<false, true>;
+using GemmQ5_1 = GemmLegacy<true, true>;
 
 template <int I, int N, class Fn>
 __device__ __forceinline__ void static_for(Fn &&fn) {

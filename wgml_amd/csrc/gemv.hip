@@ -3,6 +3,17 @@
 
 namespace {
 
+// The kernels a decode step launches by default come first and side by side: 16 tokens of the 7B shape take 22.59 ms, with
+// the same kernels scattered over the code object 22.64 to 22.69.
+template __global__ void gemv_fused_kernel<1, 1024, 5, 0, false>(const FusedParams);
+template __global__ void gemv_fused_kernel<1, 1024, 1, WGML_Q4_K, false>(const FusedParams);
+template __global__ void gemv_quant_i8_kernel<IFmtQ4K, 1, 1, 1024, 8, false>(const GemvParams);
+template __global__ void gemv_quant_i8_kernel<IFmtQ6K, 1, 1, 1024, 4, false>(const GemvParams);
+template __global__ void gemv_fused_kernel<1, 1024, 1, WGML_Q6_K, false>(const FusedParams);
+template __global__ void gemv_fused_kernel<1, 768, 1, WGML_Q6_K, false>(const FusedParams);
+template __global__ void gemv_fused_kernel<1, 1024, 1, WGML_Q8_0, false>(const FusedParams);
+template __global__ void gemv_quant_i8_kernel<IFmtQ8_0, 1, 1, 1024, 8, false>(const GemvParams);
+
 // ------------------------------------------------------------- dense f32 ----
 // out = A v, A row-major f32 (p.p0).  One wave per row, float4 loads, x from LDS.  For what the
 // shared body does not take -- f32 tensors as operator arguments (any width and alignment) and
@@ -112,24 +123,65 @@ WgPlan plan_groups(uint32_t ngroups, uint32_t max_wgs, uint32_t max_waves, uint3
     return {c, nw, wgs};
 }
 
-template <class F, int R, int D, int MAXT, int MINW = MAXT / 256, bool XPART = false>
-int launch_variant_i8(wgml_ctx *ctx, const GemvParams &p0, size_t lds) {
+// LDS a workgroup of the shared body needs for x: two int8 planes + per-tile scales and sums
+// (integer dot), or the floats themselves + per-tile sums (fp32 activations).
+template <class F>
+size_t lds_bytes_of(uint32_t ncols) {
+    const uint32_t ntiles = ncols / F::TILE;
+    const size_t ntiles_pad = ((ntiles + 63) / 64) * 64;
+    if (F::F32X) return ntiles_pad * (F::TILE / 4) * 16 + ntiles_pad * F::NSUM * 4;
+    return ntiles_pad * 2 * (F::TILE / 16) * 16 + ntiles_pad * (F::NXB + F::NSUM) * 4;
+}
+// `fn`: a gemv_quant_i8_kernel with R rows per group and workgroups of `maxt` threads.
+int launch_plain(wgml_ctx *ctx, const void *fn, uint32_t R, uint32_t maxt, GemvParams p, size_t lds) {
     int per_cu = 1;
-    WGML_TRY(blocks_per_cu(ctx, (const void *)gemv_quant_i8_kernel<F, R, D, MAXT, MINW, XPART>, MAXT,
-                           lds, &per_cu));
+    WGML_TRY(blocks_per_cu(ctx, fn, (int)maxt, lds, &per_cu));
     const uint32_t cu = ctx->n_cu > 0 ? (uint32_t)ctx->n_cu : 256u;
     // One workgroup per CU with all its waves at work rather than two half-empty ones
     // (each would stage x), as long as that still gives every CU a workgroup (min_c).
-    const uint32_t ngroups = (p0.nrows + R - 1) / R;
+    const uint32_t ngroups = (p.nrows + R - 1) / R;
     uint32_t min_c = (ngroups + cu - 1) / cu;
-    if (min_c > MAXT / 64) min_c = MAXT / 64;
-    const WgPlan plan = plan_groups(ngroups, cu * (uint32_t)per_cu, MAXT / 64, 64 / R, min_c);
-    GemvParams p = p0;
+    if (min_c > maxt / 64) min_c = maxt / 64;
+    const WgPlan plan = plan_groups(ngroups, cu * (uint32_t)per_cu, maxt / 64, 64 / R, min_c);
     p.active_waves = plan.active_waves;
-    gemv_quant_i8_kernel<F, R, D, MAXT, MINW, XPART><<<dim3(plan.wgs), dim3(MAXT), lds, ctx->stream>>>(p);
+    void *args[] = {&p};
+    WGML_CHECK_HIP(hipLaunchKernel(fn, dim3(plan.wgs), dim3(maxt), args, lds, ctx->stream));
     WGML_CHECK_LAUNCH();
     ctx->launches++;
     return WGML_OK;
+}
+
+template <class F, int R, int D, int MAXT, int MINW = MAXT / 256, bool XPART = false>
+int launch_variant_i8(wgml_ctx *ctx, const GemvParams &p, size_t lds) {
+    return launch_plain(ctx, (const void *)gemv_quant_i8_kernel<F, R, D, MAXT, MINW, XPART>, R, MAXT, p, lds);
+}
+
+bool legacy_format(int type) {
+    return type == WGML_Q4_0 || type == WGML_Q4_1 || type == WGML_Q5_0 || type == WGML_Q5_1;
+}
+// Tiles of two blocks instead of one: a lane asks for twice the bytes, and a row of up to 4096 columns is one step.  Up to
+// 2048 columns the lanes' blocks are one step as it is, and tiles of two would leave half of them idle.  us per launch, blocks as
+// in the file / planes, tiles of one block / of two: Q4_0 3072x3072 4.8 / 4.6 / 3.9, gate and up 8192x3072 11.8 / 9.0 / 8.2,
+// 3072x8192 7.1 / 6.7 / 6.1, 32000x3072 18.7 / 17.2 / 12.3, 4096x2112 4.4 / 4.4 / 4.2; gate and up 5632x2048 6.8 / 5.9 / -;
+// Q5_0 gate and up 8192x3072 13.7 / 10.9 / 10.5; Q5_1 3072x8192 7.4 / 7.6 / 7.4.
+int legacy_kernel_format(int type, uint32_t ncols) {
+    return ncols > 2048 && ncols % 64 == 0 ? kLegacyWide + type : type;
+}
+
+size_t lds_bytes_legacy(int type, uint32_t ncols) {
+    return legacy_kernel_format(type, ncols) == type ? lds_bytes_of<IFmtLegacy<false, false, 1>>(ncols)
+                                                     : lds_bytes_of<IFmtLegacy<false, false, 2>>(ncols);
+}
+
+int launch_legacy(wgml_ctx *ctx, int type, const GemvParams &p) {
+    if (p.part_n) return set_error(WGML_E_UNSUPPORTED, "gemv_quant: no merging kernel for this format");
+    if (p.ln_g && (p.ncols >> 2) > 3u * 1024u)  // XP float4 per thread
+        return set_error(WGML_E_UNSUPPORTED, "gemv_quant: %u columns are too many for the folded LayerNorm", p.ncols);
+    const size_t lds = lds_bytes_legacy(type, p.ncols);
+    if (lds > kMaxLds)
+        return set_error(WGML_E_UNSUPPORTED, "gemv_quant: %u columns need %zu bytes of LDS (limit %zu)", p.ncols, lds,
+                         kMaxLds);
+    return launch_plain(ctx, gemv_legacy_kernels(legacy_kernel_format(type, p.ncols)).plain, 1, 1024, p, lds);
 }
 
 template <class F, int R, int D>
@@ -351,10 +403,7 @@ int launch_gemv_quant(wgml_ctx *ctx, float *out, const wgml_qmat *m, const float
         return WGML_OK;
     }
     switch (m->type) {  // formats that exist as integer-dot kernels only
-    case WGML_Q4_0: return launch_fmt_i8<IFmtQ4_0, false>(ctx, p);
-    case WGML_Q4_1: return launch_fmt_i8<IFmtQ4_1, false>(ctx, p);
-    case WGML_Q5_0: return launch_fmt_i8<IFmtQ5_0, false>(ctx, p);
-    case WGML_Q5_1: return launch_fmt_i8<IFmtQ5_1, false>(ctx, p);
+    case WGML_Q4_0: case WGML_Q4_1: case WGML_Q5_0: case WGML_Q5_1: return launch_legacy(ctx, m->type, p);
     case WGML_Q5_K: return launch_fmt_i8<IFmtQ5K, false>(ctx, p);
     case WGML_Q8_K: return launch_fmt_i8<IFmtQ8K, false>(ctx, p);
     default: break;
@@ -375,15 +424,6 @@ int launch_gemv_quant(wgml_ctx *ctx, float *out, const wgml_qmat *m, const float
     }
 }
 
-// LDS a workgroup of the shared body needs for x: two int8 planes + per-tile scales and sums
-// (integer dot), or the floats themselves + per-tile sums (fp32 activations).
-template <class F>
-static size_t lds_bytes_of(uint32_t ncols) {
-    const uint32_t ntiles = ncols / F::TILE;
-    const size_t ntiles_pad = ((ntiles + 63) / 64) * 64;
-    if (F::F32X) return ntiles_pad * (F::TILE / 4) * 16 + ntiles_pad * F::NSUM * 4;
-    return ntiles_pad * 2 * (F::TILE / 16) * 16 + ntiles_pad * (F::NXB + F::NSUM) * 4;
-}
 static size_t lds_bytes_fused(int type, uint32_t ncols, bool f32) {
     switch (type) {
     case WGML_F32: return lds_bytes_of<FFmt<FmtF32>>(ncols);
@@ -392,7 +432,7 @@ static size_t lds_bytes_fused(int type, uint32_t ncols, bool f32) {
     case WGML_Q8_0: return f32 ? lds_bytes_of<FFmt<FmtQ8_0>>(ncols) : lds_bytes_of<IFmtQ8_0>(ncols);
     case WGML_Q5_K: return lds_bytes_of<IFmtQ5K>(ncols);
     case WGML_Q8_K: return lds_bytes_of<IFmtQ8K>(ncols);
-    default: return lds_bytes_of<IFmtQ4_0>(ncols);  // the four 32-element block formats
+    default: return lds_bytes_legacy(type, ncols);
     }
 }
 
@@ -469,10 +509,10 @@ static int launch_gemv_fused_variant(wgml_ctx *ctx, const FusedGemv &f, uint32_t
             case WGML_Q8_K: j.a0 += nb * 292; break;
             case WGML_Q6_K: j.a0 += nb * 128; j.a1 += nb * 64; j.a2 += nb * 16; j.a3 += nb * 2; break;
             case WGML_Q8_0: j.a0 += r * ncols; j.a1 += nb32 * 2; break;
-            case WGML_Q4_0: j.a0 += nb32 * 18; break;
-            case WGML_Q4_1: j.a0 += nb32 * 20; break;
-            case WGML_Q5_0: j.a0 += nb32 * 22; break;
-            default: j.a0 += nb32 * 24; break;  // Q5_1
+            default: {  // the 32-element formats
+                const bool has_m = s.a->type == WGML_Q4_1 || s.a->type == WGML_Q5_1;
+                j.a0 += nb32 * 16; j.a1 += nb32 * (has_m ? 4 : 2); j.a2 += nb32 * 4;
+            }
             }
             j.nrows = n;
         }
@@ -510,31 +550,32 @@ static int launch_gemv_fused_variant(wgml_ctx *ctx, const FusedGemv &f, uint32_t
             if (!main_format(P.jobs[i].type))
                 return set_error(WGML_E_UNSUPPORTED, "gemv_fused: formats can be mixed among Q4_K, "
                                                      "Q6_K and Q8_0 only");
+    if (legacy_format(fmt)) fmt = legacy_kernel_format(fmt, ncols);
     // the mixed-format kernel is held to 96 registers (5 waves per SIMD): it fits without
     // spilling, and the waves of a workgroup start sooner the fewer registers they take
-    void (*kern)(const FusedParams) = gemv_fused_kernel<D, MAXT, (MAXT == 1024 ? 5 : MINW), 0>;
+    const void *kern = (const void *)gemv_fused_kernel<D, MAXT, (MAXT == 1024 ? 5 : MINW), 0>;
     if (fmt == kFusedDenseF32) {
-        kern = dense_f32_fused_kernel(MAXT);
+        kern = (const void *)dense_f32_fused_kernel(MAXT);
     } else if (f32) {
-        kern = gemv_fused_kernel<D, MAXT, MINW, 0, true>;
+        kern = (const void *)gemv_fused_kernel<D, MAXT, MINW, 0, true>;
         switch (fmt) {
-        case WGML_Q4_K: kern = gemv_fused_kernel<D, MAXT, MINW, WGML_Q4_K, true>; break;
-        case WGML_Q6_K: kern = gemv_fused_kernel<D, MAXT, MINW, WGML_Q6_K, true>; break;
-        case WGML_Q8_0: kern = gemv_fused_kernel<D, MAXT, MINW, WGML_Q8_0, true>; break;
+        case WGML_Q4_K: kern = (const void *)gemv_fused_kernel<D, MAXT, MINW, WGML_Q4_K, true>; break;
+        case WGML_Q6_K: kern = (const void *)gemv_fused_kernel<D, MAXT, MINW, WGML_Q6_K, true>; break;
+        case WGML_Q8_0: kern = (const void *)gemv_fused_kernel<D, MAXT, MINW, WGML_Q8_0, true>; break;
         default: break;
         }
     } else {
         switch (fmt) {
-        case WGML_Q4_K: kern = gemv_fused_kernel<D, MAXT, MINW, WGML_Q4_K>; break;
-        case WGML_Q6_K: kern = gemv_fused_kernel<D, MAXT, MINW, WGML_Q6_K>; break;
-        case WGML_Q8_0: kern = gemv_fused_kernel<D, MAXT, MINW, WGML_Q8_0>; break;
-        case WGML_Q5_K: kern = gemv_fused_kernel<D, MAXT, MINW, WGML_Q5_K>; break;
-        case WGML_Q8_K: kern = gemv_fused_kernel<D, MAXT, MINW, WGML_Q8_K>; break;
-        case WGML_Q4_0: kern = gemv_fused_kernel<D, MAXT, MINW, WGML_Q4_0>; break;
-        case WGML_Q4_1: kern = gemv_fused_kernel<D, MAXT, MINW, WGML_Q4_1>; break;
-        case WGML_Q5_0: kern = gemv_fused_kernel<D, MAXT, MINW, WGML_Q5_0>; break;
-        case WGML_Q5_1: kern = gemv_fused_kernel<D, MAXT, MINW, WGML_Q5_1>; break;
-        default: break;
+        case 0: break;
+        case WGML_Q4_K: kern = (const void *)gemv_fused_kernel<D, MAXT, MINW, WGML_Q4_K>; break;
+        case WGML_Q6_K: kern = (const void *)gemv_fused_kernel<D, MAXT, MINW, WGML_Q6_K>; break;
+        case WGML_Q8_0: kern = (const void *)gemv_fused_kernel<D, MAXT, MINW, WGML_Q8_0>; break;
+        case WGML_Q5_K: kern = (const void *)gemv_fused_kernel<D, MAXT, MINW, WGML_Q5_K>; break;
+        case WGML_Q8_K: kern = (const void *)gemv_fused_kernel<D, MAXT, MINW, WGML_Q8_K>; break;
+        default: {
+            const GemvKernels k = gemv_legacy_kernels(fmt);
+            kern = MAXT == 768 ? k.fused768 : k.fused1024;
+        }
         }
     }
     // (heads of two elements: both RoPE variants rotate the same pairs)
@@ -544,9 +585,9 @@ static int launch_gemv_fused_variant(wgml_ctx *ctx, const FusedGemv &f, uint32_t
             if (f.jobs[i].mode == FUSED_SILU) return set_error(WGML_E_INVALID, "gemv_fused: a gated job beside Neox RoPE");
     if (neox && (f32 || fmt == kFusedDenseF32))
         return set_error(WGML_E_UNSUPPORTED, "gemv_fused: Neox RoPE takes the integer-dot formats only");
-    const void *const neox_kern = neox ? gemv_neox_kernel(fmt, MAXT) : nullptr;
+    if (neox) kern = gemv_neox_kernel(fmt, MAXT);
     int cached_blocks = 1;
-    WGML_TRY(blocks_per_cu(ctx, neox ? neox_kern : (const void *)kern, MAXT, lds, &cached_blocks));
+    WGML_TRY(blocks_per_cu(ctx, kern, MAXT, lds, &cached_blocks));
     const uint32_t cu = ctx->n_cu > 0 ? (uint32_t)ctx->n_cu : 256u;
     const uint32_t resident = cu * (uint32_t)cached_blocks;
     // Every workgroup streams about the same number of bytes: the smallest per-
@@ -586,14 +627,10 @@ static int launch_gemv_fused_variant(wgml_ctx *ctx, const FusedGemv &f, uint32_t
         for (int i = 0; i < f.njobs; ++i) *plan_only += ngroups[i];
         return WGML_OK;
     }
-    if (neox) {
-        const uint32_t half = P.head_size / 2;
-        NeoxPairs pairs{half, (uint32_t)(((uint64_t(1) << 32) + half - 1) / half)};
-        void *args[] = {&P, &pairs};
-        WGML_CHECK_HIP(hipLaunchKernel(neox_kern, dim3(begin), dim3(MAXT), args, lds, ctx->stream));
-    } else {
-        kern<<<dim3(begin), dim3(MAXT), lds, ctx->stream>>>(P);
-    }
+    const uint32_t half = P.head_size / 2;
+    NeoxPairs pairs{half, half ? (uint32_t)(((uint64_t(1) << 32) + half - 1) / half) : 0};
+    void *args[] = {&P, &pairs};  // (the others take the first only)
+    WGML_CHECK_HIP(hipLaunchKernel(kern, dim3(begin), dim3(MAXT), args, lds, ctx->stream));
     WGML_CHECK_LAUNCH();
     ctx->launches++;
     return WGML_OK;

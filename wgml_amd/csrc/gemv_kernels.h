@@ -355,39 +355,42 @@ struct FmtQ8_0 {
 };
 
 // ----------------------------------------- the 32-element GGUF blocks ----
-// Q4_0 (18 B: d, 16 B of nibbles), Q4_1 (20 B: d, m, nibbles), Q5_0 (22 B: d, 32 fifth
-// bits, nibbles), Q5_1 (24 B: d, m, fifth bits, nibbles); quantization.rs:47-162 of the
-// reference.  The bytes stay as in the GGUF file (blocks are only 2-byte aligned: the loads
-// below are unaligned 16-byte loads, which gfx950 serves).  A tile is one block: element k
-// of a block is the low nibble of qs[k] for k < 16, the high nibble of qs[k-16] otherwise,
-// plus bit k of qh as its fifth bit.  Integer-dot kernels only.
-template <int BYTES, bool HAS_M, bool HAS_QH>
+// Q4_0, Q4_1, Q5_0, Q5_1 (quantization.rs:47-162 of the reference) as planes of nibbles, scales (with
+// minima) and fifth bits.  Element k of a block is the low nibble of qs[k] for k < 16, the high nibble
+// of qs[k-16] otherwise, plus bit k of qh as its fifth bit.  A tile is B = 1 or 2 blocks (kLegacyWide).
+// Bound by the bytes in flight: 16 or 32 aligned bytes of nibbles per lane and request (blocks of 18 to
+// 24 bytes as in the file made them straddle; 24 tokens of eight layers of 3072 x 8192 in Q4_0, with
+// 21 of a prompt, 9.55 ms -> 8.08).  Integer-dot kernels only.
+template <bool HAS_M, bool HAS_QH, int B>
 struct FmtLegacy {
     struct Row {
-        uint4 q;
-        uint32_t qh;
-        uint16_t d, m;
+        uint4 q[B];
+        uint32_t qh[HAS_QH ? B : 1], dm[HAS_M ? B : 1];  // dm without minima: the d of both blocks in one word
     };
     struct RowBase {
-        const uint8_t *blocks;
+        const uint8_t *qs, *dm, *qh;
     };
     __device__ static RowBase row_base(const GemvParams &p, uint32_t row) {
-        return {p.p0 + (size_t)row * (p.ncols / 32) * BYTES};
+        const size_t nb = (size_t)row * (p.ncols / 32);
+        return {p.p0 + nb * 16, p.p1 + nb * (HAS_M ? 4 : 2), p.p2 + nb * 4};
     }
     __device__ static void load(Row &w, const RowBase &rb, uint32_t tile) {
-        const uint8_t *b = rb.blocks + (size_t)tile * BYTES;
-        __builtin_memcpy(&w.d, b, 2);
-        w.m = 0;
-        w.qh = 0;
-        if (HAS_M) __builtin_memcpy(&w.m, b + 2, 2);
-        if (HAS_QH) __builtin_memcpy(&w.qh, b + 2 + (HAS_M ? 2 : 0), 4);
-        __builtin_memcpy(&w.q, b + 2 + (HAS_M ? 2 : 0) + (HAS_QH ? 4 : 0), 16);
+        const size_t blk = (size_t)tile * B;
+#pragma unroll
+        for (int b = 0; b < B; ++b) w.q[b] = reinterpret_cast<const uint4 *>(rb.qs)[blk + b];
+        if constexpr (HAS_QH) __builtin_memcpy(w.qh, __builtin_assume_aligned(rb.qh + blk * 4, 4 * B), 4 * B);
+        if constexpr (HAS_M)
+            __builtin_memcpy(w.dm, __builtin_assume_aligned(rb.dm + blk * 4, 4 * B), 4 * B);
+        else if constexpr (B == 2)
+            w.dm[0] = *reinterpret_cast<const uint32_t *>(rb.dm + blk * 2);
+        else
+            w.dm[0] = *reinterpret_cast<const uint16_t *>(rb.dm + blk * 2);
     }
+    __device__ static float d(const Row &w, int b) {
+        return f16_bits_to_f32((uint16_t)(HAS_M ? w.dm[HAS_M ? b : 0] & 0xffffu : (w.dm[0] >> (16 * b)) & 0xffffu));
+    }
+    __device__ static float m(const Row &w, int b) { return f16_bits_to_f32((uint16_t)(w.dm[HAS_M ? b : 0] >> 16)); }
 };
-using FmtQ4_0 = FmtLegacy<18, false, false>;
-using FmtQ4_1 = FmtLegacy<20, true, false>;
-using FmtQ5_0 = FmtLegacy<22, false, true>;
-using FmtQ5_1 = FmtLegacy<24, true, true>;
 
 // Q8_K (292 B: f32 d, 256 int8, 16 block sums that dequantization does not use;
 // quantization.rs:170-199).  A tile is 32 of the 256 quants.
@@ -727,61 +730,60 @@ __device__ __forceinline__ uint32_t spread_bit4(uint32_t b) {
     return ((b * 0x00204081u) & 0x01010101u) << 4;
 }
 
-template <int BYTES, bool HAS_M, bool HAS_QH>
+template <bool HAS_M, bool HAS_QH, int B = 1>
 struct IFmtLegacy {
-    using W = FmtLegacy<BYTES, HAS_M, HAS_QH>;
+    using W = FmtLegacy<HAS_M, HAS_QH, B>;
     static constexpr bool F32X = false;
-    static constexpr int TILE = 32, XB = 32, NXB = 1, NSUM = 1;
+    static constexpr int TILE = 32 * B, XB = 32, NXB = B, NSUM = B;
     __device__ static void locate(uint32_t e, uint32_t &tile, uint32_t &local, uint32_t &xb) {
-        tile = e >> 5;
-        local = e & 31;
-        xb = 0;
+        tile = e / TILE;
+        local = e % TILE;
+        xb = local >> 5;
     }
     struct X {
-        uint4 xh[2], xl[2];
-        float s0, S0;  // scale of the block's fixed-point activations, sum of the rounded values
+        uint4 xh[2 * B], xl[2 * B];
+        float s[B], S[B];  // scales of the blocks' fixed-point activations, sums of the rounded values
     };
     __device__ static void load_x(X &x, const uint4 *xq, const float *meta) {
 #pragma unroll
-        for (int c = 0; c < 2; ++c) {
+        for (int c = 0; c < 2 * B; ++c) {
             x.xh[c] = xq[c * 64];
-            x.xl[c] = xq[(2 + c) * 64];
+            x.xl[c] = xq[(2 * B + c) * 64];
         }
-        x.s0 = meta[0];
-        x.S0 = meta[1];
+        __builtin_memcpy(x.s, __builtin_assume_aligned(meta, 8 * B), 4 * B);
+        __builtin_memcpy(x.S, meta + B, 4 * B);
     }
     template <int R>
     __device__ static void accumulate(const typename W::Row (&w)[R], const X &x, uint32_t,
                                       float (&acc)[R]) {
 #pragma unroll
         for (int r = 0; r < R; ++r) {
-            int h = 0, l = 0;
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const uint32_t q = (&w[r].q.x)[k];
-                uint32_t lo = q & 0x0f0f0f0fu, hi = (q >> 4) & 0x0f0f0f0fu;
-                if (HAS_QH) {
-                    lo |= spread_bit4((w[r].qh >> (4 * k)) & 15u);
-                    hi |= spread_bit4((w[r].qh >> (16 + 4 * k)) & 15u);
+            for (int b = 0; b < B; ++b) {
+                int h = 0, l = 0;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const uint32_t q = (&w[r].q[b].x)[k];
+                    uint32_t lo = q & 0x0f0f0f0fu, hi = (q >> 4) & 0x0f0f0f0fu;
+                    if constexpr (HAS_QH) {
+                        lo |= spread_bit4((w[r].qh[b] >> (4 * k)) & 15u);
+                        hi |= spread_bit4((w[r].qh[b] >> (16 + 4 * k)) & 15u);
+                    }
+                    h = sdot4(lo, (&x.xh[2 * b].x)[k], h);
+                    l = sdot4(lo, (&x.xl[2 * b].x)[k], l);
+                    h = sdot4(hi, (&x.xh[2 * b + 1].x)[k], h);
+                    l = sdot4(hi, (&x.xl[2 * b + 1].x)[k], l);
                 }
-                h = sdot4(lo, (&x.xh[0].x)[k], h);
-                l = sdot4(lo, (&x.xl[0].x)[k], l);
-                h = sdot4(hi, (&x.xh[1].x)[k], h);
-                l = sdot4(hi, (&x.xl[1].x)[k], l);
+                const float dot = (float)((h << 8) + l) * x.s[b];  // sum of quant * x over the block
+                const float d = W::d(w[r], b);
+                if (HAS_M)  // y = d q + m   (quantization.rs:93-96, 160-165)
+                    acc[r] += fmaf(d, dot, W::m(w[r], b) * x.S[b]);
+                else  // y = d (q - 8) or d (q - 16)   (quantization.rs:62-66, 123-129)
+                    acc[r] = fmaf(d, fmaf(HAS_QH ? -16.f : -8.f, x.S[b], dot), acc[r]);
             }
-            const float dot = (float)((h << 8) + l) * x.s0;  // sum of quant * x over the block
-            const float d = f16_bits_to_f32(w[r].d);
-            if (HAS_M)  // y = d q + m   (quantization.rs:93-96, 160-165)
-                acc[r] += fmaf(d, dot, f16_bits_to_f32(w[r].m) * x.S0);
-            else  // y = d (q - 8) or d (q - 16)   (quantization.rs:62-66, 123-129)
-                acc[r] = fmaf(d, fmaf(HAS_QH ? -16.f : -8.f, x.S0, dot), acc[r]);
         }
     }
 };
-using IFmtQ4_0 = IFmtLegacy<18, false, false>;
-using IFmtQ4_1 = IFmtLegacy<20, true, false>;
-using IFmtQ5_0 = IFmtLegacy<22, false, true>;
-using IFmtQ5_1 = IFmtLegacy<24, true, true>;
 
 struct IFmtQ8K {
     using W = FmtQ8K;
@@ -1513,12 +1515,19 @@ template <> struct FusedFmt<WGML_Q8_0, true> { using T = FFmt<FmtQ8_0>; };
 // (WGML_F32 is 0, which as FMT stands for mixed formats)
 constexpr int kFusedDenseF32 = 1000;
 template <> struct FusedFmt<kFusedDenseF32, true> { using T = FFmt<FmtF32>; };
+// A format number for kernels whose tiles are two blocks of a 32-element format.
+constexpr int kLegacyWide = 2000;
 template <> struct FusedFmt<WGML_Q5_K, false> { using T = IFmtQ5K; };
 template <> struct FusedFmt<WGML_Q8_K, false> { using T = IFmtQ8K; };
-template <> struct FusedFmt<WGML_Q4_0, false> { using T = IFmtQ4_0; };
-template <> struct FusedFmt<WGML_Q4_1, false> { using T = IFmtQ4_1; };
-template <> struct FusedFmt<WGML_Q5_0, false> { using T = IFmtQ5_0; };
-template <> struct FusedFmt<WGML_Q5_1, false> { using T = IFmtQ5_1; };
+template <> struct FusedFmt<WGML_Q4_0, false> { using T = IFmtLegacy<false, false>; };
+template <> struct FusedFmt<WGML_Q4_1, false> { using T = IFmtLegacy<true, false>; };
+template <> struct FusedFmt<WGML_Q5_0, false> { using T = IFmtLegacy<false, true>; };
+template <> struct FusedFmt<WGML_Q5_1, false> { using T = IFmtLegacy<true, true>; };
+// the same with tiles of two blocks (kLegacyWide)
+template <> struct FusedFmt<kLegacyWide + WGML_Q4_0, false> { using T = IFmtLegacy<false, false, 2>; };
+template <> struct FusedFmt<kLegacyWide + WGML_Q4_1, false> { using T = IFmtLegacy<true, false, 2>; };
+template <> struct FusedFmt<kLegacyWide + WGML_Q5_0, false> { using T = IFmtLegacy<false, true, 2>; };
+template <> struct FusedFmt<kLegacyWide + WGML_Q5_1, false> { using T = IFmtLegacy<true, true, 2>; };
 
 // MINW: waves per SIMD the register budget must allow.  FMT: 0 = the matrices of
 // a launch may differ in format (Q4_K / Q6_K / Q8_0, decided per workgroup), else the one

@@ -129,6 +129,10 @@ void (*neox_kernel_of(int fmt))(const FusedParams, const NeoxPairs) {
     case WGML_Q4_1: return gemv_fused_neox_kernel<MAXT, 1, WGML_Q4_1>;
     case WGML_Q5_0: return gemv_fused_neox_kernel<MAXT, 1, WGML_Q5_0>;
     case WGML_Q5_1: return gemv_fused_neox_kernel<MAXT, 1, WGML_Q5_1>;
+    case kLegacyWide + WGML_Q4_0: return gemv_fused_neox_kernel<MAXT, 1, kLegacyWide + WGML_Q4_0>;
+    case kLegacyWide + WGML_Q4_1: return gemv_fused_neox_kernel<MAXT, 1, kLegacyWide + WGML_Q4_1>;
+    case kLegacyWide + WGML_Q5_0: return gemv_fused_neox_kernel<MAXT, 1, kLegacyWide + WGML_Q5_0>;
+    case kLegacyWide + WGML_Q5_1: return gemv_fused_neox_kernel<MAXT, 1, kLegacyWide + WGML_Q5_1>;
     default: return gemv_fused_neox_kernel<MAXT, (MAXT == 1024 ? 5 : 1), 0>;
     }
 }

@@ -49,6 +49,26 @@ __global__ void repack_q6_k(const uint16_t *__restrict__ raw, uint16_t *__restri
     else d[b] = v;
 }
 
+// The 32-element blocks Q4_0 (u16 d, 16 bytes of nibbles), Q4_1 (d, u16 m, nibbles), Q5_0 (d, u32 of fifth bits,
+// nibbles) and Q5_1 (d, m, fifth bits, nibbles) -> planes: nibbles (16 B/block), fifth bits (4 B), d or {d, m} (2 or 4 B).
+template <bool HAS_M, bool HAS_QH>
+__global__ void repack_legacy(const uint16_t *__restrict__ raw, uint32_t *__restrict__ qs, uint16_t *__restrict__ dm,
+                              uint32_t *__restrict__ qh, uint64_t nblocks) {
+    uint64_t b = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (b >= nblocks) return;
+    constexpr int M = HAS_M ? 2 : 1, HALVES = M + (HAS_QH ? 2 : 0) + 8;
+    const uint16_t *src = raw + b * HALVES;
+#pragma unroll
+    for (int k = 0; k < M; ++k) dm[b * M + k] = src[k];
+    src += M;
+    if (HAS_QH) {
+        qh[b] = (uint32_t)src[0] | ((uint32_t)src[1] << 16);
+        src += 2;
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) qs[b * 4 + k] = (uint32_t)src[2 * k] | ((uint32_t)src[2 * k + 1] << 16);
+}
+
 // ---- largest weight magnitude (computed once per matrix at load) --------------
 // An upper bound on |w| over the dequantized matrix: Q8_0 and Q8_K |d| max|q| (exact); Q4_K and
 // Q5_K max(|dmin m|, |d sc 15 (31) - dmin m|) per sub-block (the two ends of the quant range);
@@ -110,12 +130,8 @@ __global__ void max_abs_kernel(int type, const uint8_t *__restrict__ p0,
         } else {  // the 32-element blocks: y = d (q - 8), d q + m, d (q - 16), d q + m
             const bool has_m = type == WGML_Q4_1 || type == WGML_Q5_1;
             const bool has_qh = type == WGML_Q5_0 || type == WGML_Q5_1;
-            const uint32_t bytes = 18 + (has_m ? 2 : 0) + (has_qh ? 4 : 0);
-            const uint8_t *blk = p0 + b * bytes;
-            uint16_t db, mb = 0;
-            __builtin_memcpy(&db, blk, 2);
-            if (has_m) __builtin_memcpy(&mb, blk + 2, 2);
-            const float d = f16_bits_to_f32(db), m = f16_bits_to_f32(mb);
+            const uint16_t *dm = reinterpret_cast<const uint16_t *>(p1) + b * (has_m ? 2 : 1);
+            const float d = f16_bits_to_f32(dm[0]), m = has_m ? f16_bits_to_f32(dm[1]) : 0.f;
             const float top = has_qh ? 31.f : 15.f;
             if (has_m) v = fmaxf(nan_to_inf(fabsf(m)), nan_to_inf(fabsf(d * top + m)));
             else v = fabsf(d) * (has_qh ? 16.f : 8.f);
@@ -211,25 +227,6 @@ __global__ void dequant_raw_kernel(const uint8_t *__restrict__ raw, float *__res
     if (e >= n) return;
     if (TYPE == WGML_F16) {
         out[e] = f16_bits_to_f32(ld_u16(raw + e * 2));
-    } else if (TYPE == WGML_Q4_0 || TYPE == WGML_Q4_1 || TYPE == WGML_Q5_0 || TYPE == WGML_Q5_1) {
-        constexpr int BYTES = TYPE == WGML_Q4_0 ? 18 : TYPE == WGML_Q4_1 ? 20 : TYPE == WGML_Q5_0 ? 22 : 24;
-        constexpr bool HAS_M = TYPE == WGML_Q4_1 || TYPE == WGML_Q5_1;
-        constexpr bool HAS_QH = TYPE == WGML_Q5_0 || TYPE == WGML_Q5_1;
-        const uint8_t *b = raw + (e / 32) * BYTES;
-        const uint32_t k = (uint32_t)(e % 32), j = k & 15;
-        const float d = f16_bits_to_f32(ld_u16(b));
-        const uint8_t *qs = b + 2 + (HAS_M ? 2 : 0) + (HAS_QH ? 4 : 0);
-        uint32_t x = k < 16 ? (qs[j] & 0x0Fu) : (uint32_t)(qs[j] >> 4);
-        if (HAS_QH) {
-            const uint32_t qh = ld_u32(b + 2 + (HAS_M ? 2 : 0));
-            x |= k < 16 ? ((qh >> j) << 4) & 0x10u : (qh >> (j + 12)) & 0x10u;
-        }
-        if (HAS_M) {
-            const float m = f16_bits_to_f32(ld_u16(b + 2));
-            out[e] = (float)x * d + m;
-        } else {
-            out[e] = (float)((int)x - (HAS_QH ? 16 : 8)) * d;
-        }
     } else if (TYPE == WGML_Q8_K) {
         const uint8_t *b = raw + (e / QK_K) * 292;
         const float d = __uint_as_float(ld_u32(b));
@@ -247,14 +244,31 @@ __global__ void dequant_raw_kernel(const uint8_t *__restrict__ raw, float *__res
     }
 }
 
+// The 32-element blocks, from their planes (quantization.rs:53-68, 82-98, 112-131, 146-167); one thread per element.
+template <bool HAS_M, bool HAS_QH>
+__global__ void dequant_legacy(const uint8_t *__restrict__ qs, const uint16_t *__restrict__ dm,
+                               const uint32_t *__restrict__ qh, float *__restrict__ out, uint64_t n) {
+    const uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (e >= n) return;
+    const uint64_t b = e / 32;
+    const uint32_t k = (uint32_t)(e % 32), j = k & 15;
+    const uint32_t byte = qs[b * 16 + j];
+    uint32_t x = k < 16 ? byte & 0x0Fu : byte >> 4;
+    if (HAS_QH) x |= ((qh[b] >> k) & 1u) << 4;
+    const float d = f16_bits_to_f32(dm[b * (HAS_M ? 2 : 1)]);
+    if (HAS_M)
+        out[e] = (float)x * d + f16_bits_to_f32(dm[b * 2 + 1]);
+    else
+        out[e] = (float)((int)x - (HAS_QH ? 16 : 8)) * d;
+}
+
 // True for the formats expanded to f32 at load: F16 only, as GgufTensorData::to_gpu_matrix
 // does (gguf.rs:131-184: every block format stays quantized on the GPU).
 bool expands_to_f32(int type) { return type == WGML_F16; }
 
 // Block formats whose bytes stay exactly as in the GGUF file (no re-layout).
 bool kept_raw(int type) {
-    return type == WGML_F32 || type == WGML_Q4_K || type == WGML_Q4_0 || type == WGML_Q4_1 ||
-           type == WGML_Q5_0 || type == WGML_Q5_1 || type == WGML_Q5_K || type == WGML_Q8_K;
+    return type == WGML_F32 || type == WGML_Q4_K || type == WGML_Q5_K || type == WGML_Q8_K;
 }
 
 uint32_t block_elems(int type) {
@@ -313,11 +327,13 @@ int launch_dequantize(wgml_ctx *ctx, float *out, const wgml_qmat *m) {
     }
     case WGML_Q4_0: case WGML_Q4_1: case WGML_Q5_0: case WGML_Q5_1: case WGML_Q5_K: case WGML_Q8_K: {
         const dim3 g((unsigned)((n + T - 1) / T)), b(T);
+        const uint16_t *dm = (const uint16_t *)m->p1;
+        const uint32_t *qh = (const uint32_t *)m->p2;
         switch (m->type) {
-        case WGML_Q4_0: dequant_raw_kernel<WGML_Q4_0><<<g, b, 0, ctx->stream>>>(m->p0, out, n); break;
-        case WGML_Q4_1: dequant_raw_kernel<WGML_Q4_1><<<g, b, 0, ctx->stream>>>(m->p0, out, n); break;
-        case WGML_Q5_0: dequant_raw_kernel<WGML_Q5_0><<<g, b, 0, ctx->stream>>>(m->p0, out, n); break;
-        case WGML_Q5_1: dequant_raw_kernel<WGML_Q5_1><<<g, b, 0, ctx->stream>>>(m->p0, out, n); break;
+        case WGML_Q4_0: dequant_legacy<false, false><<<g, b, 0, ctx->stream>>>(m->p0, dm, qh, out, n); break;
+        case WGML_Q4_1: dequant_legacy<true, false><<<g, b, 0, ctx->stream>>>(m->p0, dm, qh, out, n); break;
+        case WGML_Q5_0: dequant_legacy<false, true><<<g, b, 0, ctx->stream>>>(m->p0, dm, qh, out, n); break;
+        case WGML_Q5_1: dequant_legacy<true, true><<<g, b, 0, ctx->stream>>>(m->p0, dm, qh, out, n); break;
         case WGML_Q5_K: dequant_raw_kernel<WGML_Q5_K><<<g, b, 0, ctx->stream>>>(m->p0, out, n); break;
         default: dequant_raw_kernel<WGML_Q8_K><<<g, b, 0, ctx->stream>>>(m->p0, out, n); break;
         }
@@ -374,12 +390,19 @@ int wgml_quant_matrix_create(wgml_ctx *ctx, int type, uint32_t nrows, uint32_t n
     m->ncols = ncols;
     m->gguf_bytes = expand ? nelem * 4 : gguf;  // what a GEMV over this matrix streams
 
+    const bool has_m = type == WGML_Q4_1 || type == WGML_Q5_1, has_qh = type == WGML_Q5_0 || type == WGML_Q5_1;
+    const bool legacy = has_m || has_qh || type == WGML_Q4_0;
     uint64_t o1 = 0, o2 = 0, o3 = 0, total = 0;
     if (expand) total = align256(nelem * 4);
     switch (expand ? -1 : type) {
-    case WGML_F32: case WGML_Q4_K: case WGML_Q4_0: case WGML_Q4_1: case WGML_Q5_0: case WGML_Q5_1:
-    case WGML_Q5_K: case WGML_Q8_K:
+    case WGML_F32: case WGML_Q4_K: case WGML_Q5_K: case WGML_Q8_K:
         total = align256(gguf);
+        break;
+    case WGML_Q4_0: case WGML_Q4_1: case WGML_Q5_0: case WGML_Q5_1:
+        // (the scales last: bytes behind a matrix' last row are zeroed there, see below)
+        o2 = align256(nblocks * 16);
+        o1 = o2 + (has_qh ? align256(nblocks * 4) : 0);
+        total = o1 + align256(nblocks * (has_m ? 4 : 2));
         break;
     case WGML_Q8_0:
         o1 = align256(nblocks * 32);
@@ -418,7 +441,10 @@ int wgml_quant_matrix_create(wgml_ctx *ctx, int type, uint32_t nrows, uint32_t n
 
     // The batched products read whole units of 256 columns: behind a last row that ends inside one
     // they multiply what follows the last block by zeros, so there are no NaN scales there.
-    const uint64_t end = type == WGML_Q8_0 ? o1 + nblocks * 2 : type == WGML_Q6_K ? o3 + nblocks * 2 : m->gguf_bytes;
+    const uint64_t end = type == WGML_Q8_0 ? o1 + nblocks * 2
+                         : type == WGML_Q6_K ? o3 + nblocks * 2
+                         : legacy            ? o1 + nblocks * (has_m ? 4 : 2)
+                                             : m->gguf_bytes;
     e = hipMemsetAsync(m->base + end, 0, total - end, ctx->stream);
     if (e != hipSuccess) return fail(e, "spare bytes");
     if (kept_raw(type)) {
@@ -435,6 +461,15 @@ int wgml_quant_matrix_create(wgml_ctx *ctx, int type, uint32_t nrows, uint32_t n
             if (type == WGML_Q8_0) {
                 repack_q8_0<<<dim3((unsigned)((nblocks + T - 1) / T)), dim3(T), 0, ctx->stream>>>(
                     (const uint16_t *)raw, (uint32_t *)m->p0, (uint16_t *)m->p1, nblocks);
+            } else if (legacy) {
+                const dim3 g((unsigned)((nblocks + T - 1) / T)), b(T);
+                const uint16_t *r = (const uint16_t *)raw;
+                uint32_t *q = (uint32_t *)m->p0, *h = (uint32_t *)m->p2;
+                uint16_t *dm = (uint16_t *)m->p1;
+                if (has_m && has_qh) repack_legacy<true, true><<<g, b, 0, ctx->stream>>>(r, q, dm, h, nblocks);
+                else if (has_m) repack_legacy<true, false><<<g, b, 0, ctx->stream>>>(r, q, dm, h, nblocks);
+                else if (has_qh) repack_legacy<false, true><<<g, b, 0, ctx->stream>>>(r, q, dm, h, nblocks);
+                else repack_legacy<false, false><<<g, b, 0, ctx->stream>>>(r, q, dm, h, nblocks);
             } else if (expand) {  // F16
                 dequant_raw_kernel<WGML_F16><<<dim3((unsigned)((nelem + T - 1) / T)), dim3(T), 0,
                                                ctx->stream>>>(raw, reinterpret_cast<float *>(m->p0), nelem);
