@@ -237,11 +237,14 @@ bool gemv_partials_supported(const wgml_ctx *ctx, const wgml_qmat *m);
 int launch_gemv_fused(wgml_ctx *ctx, const FusedGemv &f);
 // the kernel of a launch with Neox pairs (gemv_neox.hip): matrices of format fmt (0: a mix of the main ones)
 const void *gemv_neox_kernel(int fmt, int threads);
-// the kernels of a format with a source file of its own
+// the kernels of a format
 struct GemvKernels {
-    const void *plain, *fused1024, *fused768;
+    const void *plain, *fused1024, *fused768, *gated1024, *gated768;
 };
 GemvKernels gemv_legacy_kernels(int fmt);  // gemv_legacy.hip: a 32-element format, or kLegacyWide + one
+// gemv_full.hip: with LayerNorm and activation (a format, kLegacyWide + one or kFusedDenseF32; no gated ones);
+// `rows` of a group of the plain kernel: 1, or 2 in Q8_0
+GemvKernels gemv_full_kernels(int fmt, bool f32, int rows);
 
 int launch_gemv_quant(wgml_ctx *ctx, float *out, const wgml_qmat *m, const float *v,
                       const GemvEpilogue &ep);

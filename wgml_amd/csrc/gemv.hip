@@ -8,11 +8,14 @@ namespace {
 template __global__ void gemv_fused_kernel<1, 1024, 5, 0, false>(const FusedParams);
 template __global__ void gemv_fused_kernel<1, 1024, 1, WGML_Q4_K, false>(const FusedParams);
 template __global__ void gemv_quant_i8_kernel<IFmtQ4K, 1, 1, 1024, 8, false>(const GemvParams);
+template __global__ void gemv_gated_kernel<1024, WGML_Q4_K>(const GatedParams);
 template __global__ void gemv_quant_i8_kernel<IFmtQ6K, 1, 1, 1024, 4, false>(const GemvParams);
 template __global__ void gemv_fused_kernel<1, 1024, 1, WGML_Q6_K, false>(const FusedParams);
 template __global__ void gemv_fused_kernel<1, 768, 1, WGML_Q6_K, false>(const FusedParams);
+template __global__ void gemv_gated_kernel<1024, WGML_Q6_K>(const GatedParams);
 template __global__ void gemv_fused_kernel<1, 1024, 1, WGML_Q8_0, false>(const FusedParams);
 template __global__ void gemv_quant_i8_kernel<IFmtQ8_0, 1, 1, 1024, 8, false>(const GemvParams);
+template __global__ void gemv_gated_kernel<1024, WGML_Q8_0>(const GatedParams);
 
 // ------------------------------------------------------------- dense f32 ----
 // out = A v, A row-major f32 (p.p0).  One wave per row, float4 loads, x from LDS.  For what the
@@ -175,8 +178,6 @@ size_t lds_bytes_legacy(int type, uint32_t ncols) {
 
 int launch_legacy(wgml_ctx *ctx, int type, const GemvParams &p) {
     if (p.part_n) return set_error(WGML_E_UNSUPPORTED, "gemv_quant: no merging kernel for this format");
-    if (p.ln_g && (p.ncols >> 2) > 3u * 1024u)  // XP float4 per thread
-        return set_error(WGML_E_UNSUPPORTED, "gemv_quant: %u columns are too many for the folded LayerNorm", p.ncols);
     const size_t lds = lds_bytes_legacy(type, p.ncols);
     if (lds > kMaxLds)
         return set_error(WGML_E_UNSUPPORTED, "gemv_quant: %u columns need %zu bytes of LDS (limit %zu)", p.ncols, lds,
@@ -192,6 +193,11 @@ int launch_rd_i8(wgml_ctx *ctx, const GemvParams &p, size_t lds, int waves) {
     default: return launch_variant_i8<F, R, D, 256>(ctx, p, lds);
     }
 }
+
+// GPT-2 124M's shapes, Q8_0 rows of 768 columns: 16-wave workgroups are as fast as 8-wave
+// ones or faster -- 3072x768 3.3 against 3.6 us, 50257x768 11.1 against 13.4 -- and the
+// tall output projection gains again from two rows per wave, 10.7 us.
+int rows_per_wave_q8(const GemvParams &p) { return p.ncols <= 1024 && p.nrows >= 16384 ? 2 : 1; }
 
 // SWEEP: the variants the tuning keys select (rows per wave, waves per workgroup, depth) exist
 // for this format; otherwise only the default one.
@@ -213,18 +219,12 @@ int launch_fmt_i8(wgml_ctx *ctx, const GemvParams &p) {
     int R = ctx->tuning[WGML_TUNE_GEMV_ROWS_PER_WAVE], waves = ctx->tuning[WGML_TUNE_GEMV_WAVES_PER_WG],
         depth = ctx->tuning[WGML_TUNE_GEMV_DEPTH];
     const bool q8 = F::TILE == 32;
-    // (GPT-2 124M's shapes, Q8_0 rows of 768 columns: 16-wave workgroups are as fast as 8-wave
-    // ones or faster -- 3072x768 3.3 against 3.6 us, 50257x768 11.1 against 13.4 -- and the
-    // tall output projection gains again from two rows per wave, 10.7 us)
-    if (!R) R = (q8 && SWEEP && p.ncols <= 1024 && p.nrows >= 16384) ? 2 : 1;
+    if (!R) R = q8 && SWEEP ? rows_per_wave_q8(p) : 1;
     if (!waves) waves = 16;
     if (waves == 12) waves = 16;  // 12-wave workgroups exist for the fused launches only
     // Q8_0 rows of five and more steps (over 8192 columns): four tiles in flight per wave
     // (4096x11008: 11.0 us against 13.4); everywhere else one tile is as fast or faster
     if (!depth) depth = (q8 && ntiles > 256 && SWEEP) ? 4 : 1;
-    if (p.ln_g && (p.ncols >> 2) > 3u * (uint32_t)waves * 64u)  // XP float4 per thread
-        return set_error(WGML_E_UNSUPPORTED, "gemv_quant: %u columns are too many for the folded "
-                                             "LayerNorm", p.ncols);
     if (p.part_n) {
         // the input is merged from attention partial results: one configuration (16-wave
         // workgroups with room for the partial results in registers)
@@ -245,9 +245,6 @@ int launch_fmt_i8(wgml_ctx *ctx, const GemvParams &p) {
         }
         return launch_rd_i8<F, 1, 1>(ctx, p, lds, waves);
     } else {
-        if (p.ln_g && (p.ncols >> 2) > 3u * 1024u)
-            return set_error(WGML_E_UNSUPPORTED, "gemv_quant: %u columns are too many for the "
-                                                 "folded LayerNorm", p.ncols);
         return launch_variant_i8<F, 1, 1, 1024>(ctx, p, lds);
     }
 }
@@ -270,9 +267,6 @@ int launch_fmt_f32(wgml_ctx *ctx, const GemvParams &p) {
     }
     // (the workgroup size is selectable for the quantized formats only)
     const int waves = std::is_same_v<WF, FmtF32> ? 16 : ctx->tuning[WGML_TUNE_GEMV_WAVES_PER_WG];
-    if (p.ln_g && (p.ncols >> 2) > 3u * (waves == 8 ? 512u : 1024u))  // XP float4 per thread
-        return set_error(WGML_E_UNSUPPORTED, "gemv_quant: %u columns are too many for the folded "
-                                             "LayerNorm", p.ncols);
     if constexpr (!std::is_same_v<WF, FmtF32>) {
         if (waves == 8) return launch_variant_i8<F, 1, 2, 512, 2>(ctx, p, lds);
     }
@@ -312,7 +306,7 @@ int launch_gemv_f32(wgml_ctx *ctx, float *out, const float *a, uint32_t nrows, u
 // come last in the code object: between the others they moved those by 10 to 30 KB, and decoding the
 // 7B shape took 22.82 ms for 16 tokens instead of 22.69, with the same instructions.
 static int launch_dense_f32(wgml_ctx *ctx, const GemvParams &p);
-static void (*dense_f32_fused_kernel(int threads))(const FusedParams);
+static GemvKernels dense_f32_kernels();
 
 // Dense f32 matrices that run in the shared body: whole tiles, and x within the LDS limit.
 static bool dense_f32_in_shared_body(const wgml_qmat *m) {
@@ -345,6 +339,42 @@ bool gemv_partials_supported(const wgml_ctx *, const wgml_qmat *m) {
     return m && (m->type == WGML_Q4_K || m->type == WGML_Q6_K || m->type == WGML_Q8_0);
 }
 
+static size_t lds_bytes_fused(int type, uint32_t ncols, bool f32) {
+    switch (type) {
+    case WGML_F32: return lds_bytes_of<FFmt<FmtF32>>(ncols);
+    case WGML_Q4_K: return f32 ? lds_bytes_of<FFmt<FmtQ4K>>(ncols) : lds_bytes_of<IFmtQ4K>(ncols);
+    case WGML_Q6_K: return f32 ? lds_bytes_of<FFmt<FmtQ6K>>(ncols) : lds_bytes_of<IFmtQ6K>(ncols);
+    case WGML_Q8_0: return f32 ? lds_bytes_of<FFmt<FmtQ8_0>>(ncols) : lds_bytes_of<IFmtQ8_0>(ncols);
+    case WGML_Q5_K: return lds_bytes_of<IFmtQ5K>(ncols);
+    case WGML_Q8_K: return lds_bytes_of<IFmtQ8K>(ncols);
+    default: return lds_bytes_legacy(type, ncols);
+    }
+}
+
+static bool main_format(int type) { return type == WGML_Q4_K || type == WGML_Q6_K || type == WGML_Q8_0; }
+
+// With LayerNorm or activation (gemv_full.hip): one variant per format, Q8_0 in one or two rows per wave.
+static int launch_full(wgml_ctx *ctx, const wgml_qmat *m, const GemvParams &p) {
+    if (m->type == WGML_F32 && !dense_f32_in_shared_body(m))
+        return set_error(WGML_E_UNSUPPORTED, "gemv_quant: LayerNorm / activation folding needs rows of a "
+                                             "multiple of 16 elements");
+    if (p.part_n) return set_error(WGML_E_UNSUPPORTED, "gemv_quant: no merging kernel with an activation");
+    const bool f32 = m->type == WGML_F32 || (main_format(m->type) && ctx->tuning[WGML_TUNE_GEMV_F32_ACTIVATIONS]);
+    const int waves = main_format(m->type) ? ctx->tuning[WGML_TUNE_GEMV_WAVES_PER_WG] : 0;
+    const uint32_t threads = waves == 8 ? 512u : waves && waves < 8 && !f32 ? 256u : 1024u;
+    if (p.ln_g && (p.ncols >> 2) > 3u * threads)  // XP float4 per thread
+        return set_error(WGML_E_UNSUPPORTED, "gemv_quant: %u columns are too many for the folded LayerNorm", p.ncols);
+    const size_t lds = lds_bytes_fused(m->type, p.ncols, f32);
+    if (lds > kMaxLds)
+        return set_error(WGML_E_UNSUPPORTED, "gemv_quant: %u columns need %zu bytes of LDS (limit %zu)", p.ncols, lds,
+                         kMaxLds);
+    const int fmt = m->type == WGML_F32 ? kFusedDenseF32
+                    : legacy_format(m->type) ? legacy_kernel_format(m->type, p.ncols)
+                                             : m->type;
+    const int rows = m->type == WGML_Q8_0 && !f32 ? rows_per_wave_q8(p) : 1;
+    return launch_plain(ctx, gemv_full_kernels(fmt, f32, rows).plain, (uint32_t)rows, 1024, p, lds);
+}
+
 int launch_gemv_quant(wgml_ctx *ctx, float *out, const wgml_qmat *m, const float *v,
                       const GemvEpilogue &ep) {
     GemvParams p{};
@@ -365,7 +395,6 @@ int launch_gemv_quant(wgml_ctx *ctx, float *out, const wgml_qmat *m, const float
     p.ln_g = ep.ln_gamma;
     p.ln_b = ep.ln_beta;
     p.act = ep.act;
-    const bool main_fmt = m->type == WGML_Q4_K || m->type == WGML_Q6_K || m->type == WGML_Q8_0;
     if (ep.partials.n) {
         const AttnPartials &a = ep.partials;
         if (!gemv_partials_supported(ctx, m) || a.n > 16 || !a.o || !a.ml || a.head_size == 0 ||
@@ -383,13 +412,9 @@ int launch_gemv_quant(wgml_ctx *ctx, float *out, const wgml_qmat *m, const float
     } else if ((uintptr_t)v % 16 != 0) {
         return set_error(WGML_E_INVALID, "gemv_quant: the input vector must be 16-byte aligned");
     }
-    (void)main_fmt;
-    if (dense_f32_in_shared_body(m) &&
-        (p.ln_g || p.act || !dense_f32_general_faster(ctx, p.nrows, p.ncols, p.norm_w != nullptr)))
+    if (p.ln_g || p.act) return launch_full(ctx, m, p);
+    if (dense_f32_in_shared_body(m) && !dense_f32_general_faster(ctx, p.nrows, p.ncols, p.norm_w != nullptr))
         return launch_dense_f32(ctx, p);
-    if ((p.ln_g || p.act) && m->type == WGML_F32)
-        return set_error(WGML_E_UNSUPPORTED, "gemv_quant: LayerNorm / activation folding needs rows of a "
-                                             "multiple of 16 elements");
     if (m->type == WGML_F32) {
         const size_t lds = (size_t)m->ncols * 4;
         if (lds > kMaxLds)
@@ -424,20 +449,6 @@ int launch_gemv_quant(wgml_ctx *ctx, float *out, const wgml_qmat *m, const float
     }
 }
 
-static size_t lds_bytes_fused(int type, uint32_t ncols, bool f32) {
-    switch (type) {
-    case WGML_F32: return lds_bytes_of<FFmt<FmtF32>>(ncols);
-    case WGML_Q4_K: return f32 ? lds_bytes_of<FFmt<FmtQ4K>>(ncols) : lds_bytes_of<IFmtQ4K>(ncols);
-    case WGML_Q6_K: return f32 ? lds_bytes_of<FFmt<FmtQ6K>>(ncols) : lds_bytes_of<IFmtQ6K>(ncols);
-    case WGML_Q8_0: return f32 ? lds_bytes_of<FFmt<FmtQ8_0>>(ncols) : lds_bytes_of<IFmtQ8_0>(ncols);
-    case WGML_Q5_K: return lds_bytes_of<IFmtQ5K>(ncols);
-    case WGML_Q8_K: return lds_bytes_of<IFmtQ8K>(ncols);
-    default: return lds_bytes_legacy(type, ncols);
-    }
-}
-
-static bool main_format(int type) { return type == WGML_Q4_K || type == WGML_Q6_K || type == WGML_Q8_0; }
-
 bool gemv_fused_supported(const wgml_qmat *m) {
     if (!m) return false;
     switch (m->type) {
@@ -461,13 +472,81 @@ bool gemv_fused_set_supported(const wgml_ctx *ctx, const wgml_qmat *const *mats,
     return same || all_main;
 }
 
-template <int D, int MAXT, int MINW>
-static int launch_gemv_fused_variant(wgml_ctx *ctx, const FusedGemv &f, uint32_t *plan_only = nullptr) {
-    constexpr uint32_t nwaves = MAXT / 64;
-    if (f.njobs < 1 || f.njobs > 3)
-        return set_error(WGML_E_INVALID, "gemv_fused: %d jobs", f.njobs);
-    if ((uintptr_t)f.x % 16 != 0)
-        return set_error(WGML_E_INVALID, "gemv_fused: the input vector must be 16-byte aligned");
+// The format number of a fused launch's kernel: that of its matrices, or 0 for a mix of the main ones.
+static int fused_format(const FusedGemv &f, uint32_t ncols) {
+    const int type = f.jobs[0].a->type;
+    for (int i = 1; i < f.njobs; ++i)
+        if (f.jobs[i].a->type != type) return 0;
+    return type == WGML_F32 ? kFusedDenseF32 : legacy_format(type) ? legacy_kernel_format(type, ncols) : type;
+}
+static GemvKernels fused_kernels(int fmt, bool f32) {
+    if (fmt == kFusedDenseF32) return dense_f32_kernels();
+    if (f32) {
+        switch (fmt) {
+        case WGML_Q4_K: return gemv_kernels_of<WGML_Q4_K, true, false>();
+        case WGML_Q6_K: return gemv_kernels_of<WGML_Q6_K, true, false>();
+        case WGML_Q8_0: return gemv_kernels_of<WGML_Q8_0, true, false>();
+        default:
+            return {nullptr, (const void *)gemv_fused_kernel<1, 1024, 1, 0, true>,
+                    (const void *)gemv_fused_kernel<1, 768, 1, 0, true>, nullptr, nullptr};
+        }
+    }
+    switch (fmt) {
+    // the mixed-format kernel is held to 96 registers (5 waves per SIMD): it fits without
+    // spilling, and the waves of a workgroup start sooner the fewer registers they take
+    case 0:
+        return {nullptr, (const void *)gemv_fused_kernel<1, 1024, 5, 0>, (const void *)gemv_fused_kernel<1, 768, 1, 0>,
+                nullptr, nullptr};
+    case WGML_Q4_K: return gemv_kernels_of<WGML_Q4_K, false, false>();
+    case WGML_Q6_K: return gemv_kernels_of<WGML_Q6_K, false, false>();
+    case WGML_Q8_0: return gemv_kernels_of<WGML_Q8_0, false, false>();
+    case WGML_Q5_K: return gemv_kernels_of<WGML_Q5_K, false, false>();
+    case WGML_Q8_K: return gemv_kernels_of<WGML_Q8_K, false, false>();
+    default: return gemv_legacy_kernels(fmt);
+    }
+}
+
+// Workgroups a fused launch is shared out over: one per compute unit, or as many as the machine holds at once where it streams
+// more than 64 MB.  A second workgroup on a compute unit stages x again, and the waves' row pairs are fewer and less even.  us
+// per launch, as many as fit (two of 64 registers) / one per compute unit: gate and up 8192x3072 in Q4_0 9.2 / 7.8, Q4_1 9.7 / 8.2,
+// Q8_0 (53 MB) 11.8 / 11.6, 9216x3072 rows in pairs in Q8_0 9.2 / 8.8, 2304x768 3.8 / 3.4; gate and up 11008x4096 in Q8_0 (96 MB)
+// 19.0 / 19.5.
+static uint32_t fused_workgroups(const wgml_ctx *ctx, int per_cu, uint64_t bytes) {
+    const uint32_t cu = ctx->n_cu > 0 ? (uint32_t)ctx->n_cu : 256u;
+    return bytes <= (uint64_t(64) << 20) ? cu : cu * (uint32_t)per_cu;
+}
+
+static int launch_gated(wgml_ctx *ctx, const FusedGemv &f, const FusedGemvJob &s, uint32_t threads) {
+    const uint32_t ncols = s.a->ncols;
+    const bool f32 = ctx->tuning[WGML_TUNE_GEMV_F32_ACTIVATIONS] != 0;
+    if (!s.b || s.b->type != s.a->type || s.b->nrows != s.a->nrows || s.b->ncols != ncols || s.row0 || s.nrows)
+        return set_error(WGML_E_INVALID, "gemv_fused: gate/up matrices differ");
+    if (f.ln_gamma) return set_error(WGML_E_UNSUPPORTED, "gemv_fused: a gated job behind a LayerNorm");
+    FusedGemv one = f;
+    one.jobs[0] = s;
+    one.njobs = 1;
+    const GemvKernels k = fused_kernels(fused_format(one, ncols), f32);
+    const void *kern = threads == 768 ? k.gated768 : k.gated1024;
+    const size_t lds = lds_bytes_fused(s.a->type, ncols, f32);
+    if (lds > kMaxLds)
+        return set_error(WGML_E_UNSUPPORTED, "gemv_fused: %u columns need %zu bytes of LDS", ncols, lds);
+    GatedParams P{s.a->p0, s.a->p1, s.a->p2, s.a->p3, s.b->p0, s.b->p1, s.b->p2, s.b->p3, f.x, f.norm_w, s.out,
+                  f.norm_eps, s.a->nrows, ncols, 0};
+    int per_cu = 1;
+    WGML_TRY(blocks_per_cu(ctx, kern, (int)threads, lds, &per_cu));
+    const uint32_t nwaves = threads / 64;
+    const WgPlan plan = plan_groups(P.nrows, fused_workgroups(ctx, per_cu, s.a->gguf_bytes * 2), nwaves, 32);
+    P.active_waves = plan.active_waves;
+    void *args[] = {&P};
+    WGML_CHECK_HIP(hipLaunchKernel(kern, dim3(plan.wgs), dim3(threads), args, lds, ctx->stream));
+    WGML_CHECK_LAUNCH();
+    ctx->launches++;
+    return WGML_OK;
+}
+
+// The jobs in PLAIN and ROPE mode.
+static int launch_jobs(wgml_ctx *ctx, const FusedGemv &f, uint32_t threads) {
+    const uint32_t nwaves = threads / 64, ncols = f.jobs[0].a->ncols;
     FusedParams P{};
     P.njobs = f.njobs;
     P.x = f.x;
@@ -479,7 +558,6 @@ static int launch_gemv_fused_variant(wgml_ctx *ctx, const FusedGemv &f, uint32_t
     P.head_size = f.head_size ? f.head_size : 2;
     P.rope_base = f.rope_base;
     P.rope_cs = reinterpret_cast<const float2 *>(f.rope_cs);
-    const uint32_t ncols = f.jobs[0].a->ncols;
     P.ncols = ncols;
     const bool f32 = ctx->tuning[WGML_TUNE_GEMV_F32_ACTIVATIONS] != 0;
     size_t lds = 0;
@@ -487,11 +565,6 @@ static int launch_gemv_fused_variant(wgml_ctx *ctx, const FusedGemv &f, uint32_t
     uint32_t ngroups[3];
     for (int i = 0; i < f.njobs; ++i) {
         const FusedGemvJob &s = f.jobs[i];
-        if (!gemv_fused_supported(s.a) || s.a->ncols != ncols)
-            return set_error(WGML_E_INVALID, "gemv_fused: job %d has an unsupported matrix", i);
-        if (f32 && !main_format(s.a->type) && s.a->type != WGML_F32)
-            return set_error(WGML_E_UNSUPPORTED, "gemv_fused: fp32 activations exist for Q4_K, Q6_K "
-                                                 "and Q8_0 only");
         GemvJob &j = P.jobs[i];
         j.a0 = s.a->p0; j.a1 = s.a->p1; j.a2 = s.a->p2; j.a3 = s.a->p3;
         j.out = s.out;
@@ -499,7 +572,7 @@ static int launch_gemv_fused_variant(wgml_ctx *ctx, const FusedGemv &f, uint32_t
         j.nrows = s.a->nrows;
         if (s.row0 || s.nrows) {  // a slice of the rows: move the plane pointers to its first row
             const uint32_t n = s.nrows ? s.nrows : s.a->nrows - s.row0;
-            if (s.mode == JOB_SILU || (uint64_t)s.row0 + n > s.a->nrows)
+            if ((uint64_t)s.row0 + n > s.a->nrows)
                 return set_error(WGML_E_INVALID, "gemv_fused: job %d: bad row slice", i);
             const uint64_t r = s.row0, nb = r * (ncols / 256), nb32 = r * (ncols / 32);
             switch (s.a->type) {
@@ -516,80 +589,33 @@ static int launch_gemv_fused_variant(wgml_ctx *ctx, const FusedGemv &f, uint32_t
             }
             j.nrows = n;
         }
-        j.type = s.a->type;
-        j.mode = s.mode;
-        j.accumulate = s.accumulate;
+        j.kind = gemv_kind(s.a->type, s.mode, s.accumulate);
         j.out_pos_stride = s.out_pos_stride;
         bytes[i] = s.a->gguf_bytes / s.a->nrows * j.nrows;
-        if (s.mode == JOB_SILU) {
-            if (!s.b || s.b->type != s.a->type || s.b->nrows != s.a->nrows || s.b->ncols != ncols)
-                return set_error(WGML_E_INVALID, "gemv_fused: job %d: gate/up matrices differ", i);
-            j.b0 = s.b->p0; j.b1 = s.b->p1; j.b2 = s.b->p2; j.b3 = s.b->p3;
-            bytes[i] += s.b->gguf_bytes;
-            ngroups[i] = j.nrows;
-        } else {
-            if (s.mode == JOB_ROPE && (j.nrows % 2 != 0 || P.head_size % 2 != 0))
-                return set_error(WGML_E_INVALID, "gemv_fused: RoPE needs even row counts");
-            ngroups[i] = (j.nrows + 1) / 2;
-        }
-        const size_t l = lds_bytes_fused(j.type, ncols, f32);
+        if (s.mode == JOB_ROPE && (j.nrows % 2 != 0 || P.head_size % 2 != 0))
+            return set_error(WGML_E_INVALID, "gemv_fused: RoPE needs even row counts");
+        ngroups[i] = (j.nrows + 1) / 2;
+        const size_t l = lds_bytes_fused(s.a->type, ncols, f32);
         if (l > lds) lds = l;
     }
     if (lds > kMaxLds)
         return set_error(WGML_E_UNSUPPORTED, "gemv_fused: %u columns need %zu bytes of LDS", ncols,
                          lds);
-    if (P.ln_g && (ncols >> 2) > 3u * (uint32_t)MAXT)  // XP float4 per thread
+    if (P.ln_g && (ncols >> 2) > 3u * threads)  // XP float4 per thread
         return set_error(WGML_E_UNSUPPORTED,
                          "gemv_fused: %u columns are too many for the folded LayerNorm", ncols);
-    // one kernel per format when all matrices share it, else the mixed one
-    int fmt = P.jobs[0].type == WGML_F32 ? kFusedDenseF32 : P.jobs[0].type;
-    for (int i = 1; i < f.njobs; ++i)
-        if (P.jobs[i].type != P.jobs[0].type) fmt = 0;
-    if (fmt == 0)
-        for (int i = 0; i < f.njobs; ++i)
-            if (!main_format(P.jobs[i].type))
-                return set_error(WGML_E_UNSUPPORTED, "gemv_fused: formats can be mixed among Q4_K, "
-                                                     "Q6_K and Q8_0 only");
-    if (legacy_format(fmt)) fmt = legacy_kernel_format(fmt, ncols);
-    // the mixed-format kernel is held to 96 registers (5 waves per SIMD): it fits without
-    // spilling, and the waves of a workgroup start sooner the fewer registers they take
-    const void *kern = (const void *)gemv_fused_kernel<D, MAXT, (MAXT == 1024 ? 5 : MINW), 0>;
-    if (fmt == kFusedDenseF32) {
-        kern = (const void *)dense_f32_fused_kernel(MAXT);
-    } else if (f32) {
-        kern = (const void *)gemv_fused_kernel<D, MAXT, MINW, 0, true>;
-        switch (fmt) {
-        case WGML_Q4_K: kern = (const void *)gemv_fused_kernel<D, MAXT, MINW, WGML_Q4_K, true>; break;
-        case WGML_Q6_K: kern = (const void *)gemv_fused_kernel<D, MAXT, MINW, WGML_Q6_K, true>; break;
-        case WGML_Q8_0: kern = (const void *)gemv_fused_kernel<D, MAXT, MINW, WGML_Q8_0, true>; break;
-        default: break;
-        }
-    } else {
-        switch (fmt) {
-        case 0: break;
-        case WGML_Q4_K: kern = (const void *)gemv_fused_kernel<D, MAXT, MINW, WGML_Q4_K>; break;
-        case WGML_Q6_K: kern = (const void *)gemv_fused_kernel<D, MAXT, MINW, WGML_Q6_K>; break;
-        case WGML_Q8_0: kern = (const void *)gemv_fused_kernel<D, MAXT, MINW, WGML_Q8_0>; break;
-        case WGML_Q5_K: kern = (const void *)gemv_fused_kernel<D, MAXT, MINW, WGML_Q5_K>; break;
-        case WGML_Q8_K: kern = (const void *)gemv_fused_kernel<D, MAXT, MINW, WGML_Q8_K>; break;
-        default: {
-            const GemvKernels k = gemv_legacy_kernels(fmt);
-            kern = MAXT == 768 ? k.fused768 : k.fused1024;
-        }
-        }
-    }
+    const int fmt = fused_format(f, ncols);
     // (heads of two elements: both RoPE variants rotate the same pairs)
     const bool neox = f.rope_neox && P.head_size > 2;
-    if (neox)
-        for (int i = 0; i < f.njobs; ++i)
-            if (f.jobs[i].mode == FUSED_SILU) return set_error(WGML_E_INVALID, "gemv_fused: a gated job beside Neox RoPE");
     if (neox && (f32 || fmt == kFusedDenseF32))
         return set_error(WGML_E_UNSUPPORTED, "gemv_fused: Neox RoPE takes the integer-dot formats only");
-    if (neox) kern = gemv_neox_kernel(fmt, MAXT);
-    int cached_blocks = 1;
-    WGML_TRY(blocks_per_cu(ctx, kern, MAXT, lds, &cached_blocks));
-    const uint32_t cu = ctx->n_cu > 0 ? (uint32_t)ctx->n_cu : 256u;
-    const uint32_t resident = cu * (uint32_t)cached_blocks;
+    if (P.ln_g && (neox || fmt == 0))
+        return set_error(WGML_E_UNSUPPORTED, "gemv_fused: LayerNorm before Neox RoPE or mixed formats");
+    const GemvKernels k = P.ln_g ? gemv_full_kernels(fmt, f32 || fmt == kFusedDenseF32, 1) : fused_kernels(fmt, f32);
+    const void *const kern = neox ? gemv_neox_kernel(fmt, (int)threads) : threads == 768 ? k.fused768 : k.fused1024;
+    int per_cu = 1;
+    WGML_TRY(blocks_per_cu(ctx, kern, (int)threads, lds, &per_cu));
+    const uint32_t resident = fused_workgroups(ctx, per_cu, bytes[0] + bytes[1] + bytes[2]);
     // Every workgroup streams about the same number of bytes: the smallest per-
     // workgroup budget T is searched for which the matrices together need no more
     // workgroups than the machine holds at once.
@@ -611,7 +637,7 @@ static int launch_gemv_fused_variant(wgml_ctx *ctx, const FusedGemv &f, uint32_t
         const double mid = 0.5 * (lo + hi);
         if (wgs_needed(mid) <= resident) hi = mid; else lo = mid;
     }
-    uint32_t begin = 0, max_nw = 1;
+    uint32_t begin = 0;
     for (int i = 0; i < f.njobs; ++i) {
         uint32_t c = (uint32_t)(hi / bpg[i]);
         if (c < 1) c = 1;
@@ -619,36 +645,59 @@ static int launch_gemv_fused_variant(wgml_ctx *ctx, const FusedGemv &f, uint32_t
         P.jobs[i].wg_begin = begin;
         P.jobs[i].wg_count = plan.wgs;
         P.jobs[i].active_waves = plan.active_waves;
-        if (plan.active_waves > max_nw) max_nw = plan.active_waves;
         begin += plan.wgs;
     }
-    if (plan_only) {  // the caller only asks how many row pairs the launch has
-        *plan_only = 0;
-        for (int i = 0; i < f.njobs; ++i) *plan_only += ngroups[i];
-        return WGML_OK;
-    }
     const uint32_t half = P.head_size / 2;
-    NeoxPairs pairs{half, half ? (uint32_t)(((uint64_t(1) << 32) + half - 1) / half) : 0};
-    void *args[] = {&P, &pairs};  // (the others take the first only)
-    WGML_CHECK_HIP(hipLaunchKernel(kern, dim3(begin), dim3(MAXT), args, lds, ctx->stream));
+    NeoxPairs neox_pairs{half, half ? (uint32_t)(((uint64_t(1) << 32) + half - 1) / half) : 0};
+    void *args[] = {&P, &neox_pairs};  // (the others take the first only)
+    WGML_CHECK_HIP(hipLaunchKernel(kern, dim3(begin), dim3(threads), args, lds, ctx->stream));
     WGML_CHECK_LAUNCH();
     ctx->launches++;
     return WGML_OK;
 }
 
 int launch_gemv_fused(wgml_ctx *ctx, const FusedGemv &f) {
-    const int depth = ctx->tuning[WGML_TUNE_GEMV_DEPTH], waves = ctx->tuning[WGML_TUNE_GEMV_WAVES_PER_WG];
-    (void)depth;  // deeper register rings spill in the fused kernels
-    if (waves == 12) return launch_gemv_fused_variant<1, 768, 1>(ctx, f);
-    if (waves == 16) return launch_gemv_fused_variant<1, 1024, 1>(ctx, f);
+    if (f.njobs < 1 || f.njobs > 3)
+        return set_error(WGML_E_INVALID, "gemv_fused: %d jobs", f.njobs);
+    if ((uintptr_t)f.x % 16 != 0)
+        return set_error(WGML_E_INVALID, "gemv_fused: the input vector must be 16-byte aligned");
+    const bool f32 = ctx->tuning[WGML_TUNE_GEMV_F32_ACTIVATIONS] != 0;
+    bool gated = false, mixed = false, all_main = true;
+    uint32_t pairs = 0;
+    for (int i = 0; i < f.njobs; ++i) {
+        const FusedGemvJob &s = f.jobs[i];
+        if (!gemv_fused_supported(s.a) || s.a->ncols != f.jobs[0].a->ncols)
+            return set_error(WGML_E_INVALID, "gemv_fused: job %d has an unsupported matrix", i);
+        if (f32 && !main_format(s.a->type) && s.a->type != WGML_F32)
+            return set_error(WGML_E_UNSUPPORTED, "gemv_fused: fp32 activations exist for Q4_K, Q6_K "
+                                                 "and Q8_0 only");
+        gated = gated || s.mode == FUSED_SILU;
+        mixed = mixed || s.a->type != f.jobs[0].a->type;
+        all_main = all_main && main_format(s.a->type);
+        const uint32_t rows = s.nrows ? s.nrows : s.a->nrows - s.row0;
+        pairs += s.mode == FUSED_SILU ? rows : (rows + 1) / 2;
+    }
+    if (mixed && !all_main)
+        return set_error(WGML_E_UNSUPPORTED, "gemv_fused: formats can be mixed among Q4_K, Q6_K and Q8_0 only");
+    if (gated && f.rope_neox && f.head_size > 2)
+        return set_error(WGML_E_INVALID, "gemv_fused: a gated job beside Neox RoPE");
     // 12-wave workgroups for launches with a little less than one row pair per wave of a
     // machine full of 16-wave workgroups (Q/K/V of 4096/1024/1024 rows: 8.6 us against 9.6;
     // small launches are better off with the 16-wave kernel: GPT-2's Q/K/V 5.1 us against 7.1)
-    uint32_t pairs = 0;
-    WGML_TRY((launch_gemv_fused_variant<1, 1024, 1>(ctx, f, &pairs)));
+    const int waves = ctx->tuning[WGML_TUNE_GEMV_WAVES_PER_WG];
     const uint32_t cu = ctx->n_cu > 0 ? (uint32_t)ctx->n_cu : 256u;
-    if (pairs > cu * 8 && pairs <= cu * 16) return launch_gemv_fused_variant<1, 768, 1>(ctx, f);
-    return launch_gemv_fused_variant<1, 1024, 1>(ctx, f);
+    const uint32_t threads = waves == 12 || (waves != 16 && pairs > cu * 8 && pairs <= cu * 16) ? 768 : 1024;
+    if (!gated) return launch_jobs(ctx, f, threads);
+    // gated jobs are a launch each
+    FusedGemv rest = f;
+    rest.njobs = 0;
+    for (int i = 0; i < f.njobs; ++i) {
+        if (f.jobs[i].mode == FUSED_SILU)
+            WGML_TRY(launch_gated(ctx, f, f.jobs[i], threads));
+        else
+            rest.jobs[rest.njobs++] = f.jobs[i];
+    }
+    return rest.njobs ? launch_jobs(ctx, rest, threads) : WGML_OK;
 }
 
 }  // namespace wgml
@@ -689,9 +738,6 @@ namespace wgml {
 
 static int launch_dense_f32(wgml_ctx *ctx, const GemvParams &p) { return launch_fmt_f32<FmtF32>(ctx, p); }
 
-static void (*dense_f32_fused_kernel(int threads))(const FusedParams) {
-    return threads == 768 ? gemv_fused_kernel<1, 768, 1, kFusedDenseF32, true>
-                          : gemv_fused_kernel<1, 1024, 1, kFusedDenseF32, true>;
-}
+static GemvKernels dense_f32_kernels() { return gemv_kernels_of<kFusedDenseF32, true, false>(); }
 
 }  // namespace wgml

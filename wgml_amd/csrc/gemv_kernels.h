@@ -887,6 +887,7 @@ struct FFmt {
 };
 
 // Row source / sink of a plain single-matrix GEMV: group g = rows g*R .. g*R+R-1.
+template <bool FULL>
 struct PlainPolicy {
     static constexpr int S = 1;  // passes per group
     const GemvParams &p;
@@ -927,7 +928,9 @@ struct PlainPolicy {
         const uint32_t row = (g0 + (lane / R) * GW) * R + lane % R;
         if (lane < n && row < p.nrows) {
             float v = mine + pre_bias;
-            if (p.act == 1) v = gelu_tanh(v);
+            if constexpr (FULL) {
+                if (p.act == 1) v = gelu_tanh(v);
+            }
             out[row] = v + pre_out;
         }
     }
@@ -945,7 +948,9 @@ struct PlainPolicy {
 // XREG: rows fit one step (ncols <= 64 tiles), so a lane's tile of x is the same
 // for every row and is read from LDS once instead of once per row.
 // XPART: x is not read from p.x but merged from attention partial results (merged_partials).
-template <class F, int R, int D, bool XREG, class Policy, bool XPART = false>
+// FULL: x may go through a LayerNorm (p.ln_g) on its way, and results through an activation.  Kernels of
+// their own (gemv_full.hip): the code that the others jump over costs every launch 0.05 to 0.1 us.
+template <class F, int R, int D, bool XREG, class Policy, bool XPART = false, bool FULL = false>
 __device__ __forceinline__ void gemv_i8_body(const GemvParams &p, Policy &pol, uint32_t wg,
                                              uint32_t nwg, uint32_t nw, uint32_t ngroups) {
     using WF = typename F::W;
@@ -1003,15 +1008,31 @@ __device__ __forceinline__ void gemv_i8_body(const GemvParams &p, Policy &pol, u
     // barrier.  (The folded LayerNorm has barriers of its own, so there every wave stages.)
     // (Merging partial results is several loads per float4: every wave takes a share.)
     uint32_t ns = ((n4 + 64 * XP - 1) / (64 * XP) + 3) & ~3u;
-    if (ns > nwaves || p.ln_g || XPART) ns = nwaves;
+    const float *const ln_g = FULL ? p.ln_g : nullptr;
+    if (ns > nwaves || ln_g || XPART) ns = nwaves;
+    // LayerNorm of up to LN_ROW float4: as many waves as hold them at one per lane stage, and each of these reads the
+    // whole vector and finds its mean and variance by itself.  Shared out over all waves that is two more barriers
+    // (with kernels without arguments of a second mode: GPT-2 124M in Q8_0 205 us per token -> 190, from an F16 file 331 -> 290).
+    constexpr int LN_REGS = 4;
+    constexpr uint32_t LN_ROW = 64 * LN_REGS;
+    const bool ln_row = ln_g && n4 <= LN_ROW;
+    if (ln_row) ns = (n4 + 63) / 64;
     const bool stager = wave < ns;
     // a wave with neither rows nor a share of x is done: the barrier below counts only the
     // waves that are still running, and it would be the last to reach it
     if (n_it == 0 && !stager) return;
     const uint32_t sthreads = ns * 64;
     float4 xv[XP], nv[XP], bv[XP];
-    const float4 *gsrc = p.ln_g ? reinterpret_cast<const float4 *>(p.ln_g) : nw4;
-    const float4 *bsrc = reinterpret_cast<const float4 *>(p.ln_b);
+    const float4 *gsrc = ln_g ? reinterpret_cast<const float4 *>(ln_g) : nw4;
+    const float4 *bsrc = FULL ? reinterpret_cast<const float4 *>(p.ln_b) : nullptr;
+    float4 xrow[FULL ? LN_REGS : 1];
+    if constexpr (FULL) {
+#pragma unroll
+        for (int i = 0; i < LN_REGS; ++i) {
+            xrow[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (ln_row && stager && lane + 64 * i < n4) xrow[i] = x4[lane + 64 * i];
+        }
+    }
 #pragma unroll
     for (int i = 0; i < XP; ++i) {
         const uint32_t g4 = stager ? tid + i * sthreads : n4;
@@ -1021,7 +1042,7 @@ __device__ __forceinline__ void gemv_i8_body(const GemvParams &p, Policy &pol, u
         if (g4 < n4) {
             if constexpr (!XPART) xv[i] = x4[g4];
             if (gsrc) nv[i] = gsrc[g4];
-            if (p.ln_g && bsrc) bv[i] = bsrc[g4];
+            if (ln_g && bsrc) bv[i] = bsrc[g4];
         }
     }
     // XPART: the first eight partial results of each thread's first float4 are requested here,
@@ -1051,7 +1072,28 @@ __device__ __forceinline__ void gemv_i8_body(const GemvParams &p, Policy &pol, u
             for (int i = 1; i < XP; ++i)
                 if (tid + i * sthreads < n4) xv[i] = merged_partials(p, tid + i * sthreads);
         }
-        if (p.ln_g) {
+        if constexpr (FULL) if (ln_row) {
+            float s1 = 0.f;
+#pragma unroll
+            for (int i = 0; i < LN_REGS; ++i) s1 += (xrow[i].x + xrow[i].y) + (xrow[i].z + xrow[i].w);
+            const float mean = wave_sum(s1) / (float)p.ncols;
+            float s2 = 0.f;
+#pragma unroll
+            for (int i = 0; i < LN_REGS; ++i) {
+                const bool there = lane + 64 * i < n4;
+                const float a = there ? xrow[i].x - mean : 0.f, b = there ? xrow[i].y - mean : 0.f,
+                            c = there ? xrow[i].z - mean : 0.f, d = there ? xrow[i].w - mean : 0.f;
+                s2 = fmaf(a, a, s2);
+                s2 = fmaf(b, b, s2);
+                s2 = fmaf(c, c, s2);
+                s2 = fmaf(d, d, s2);
+            }
+            const float rstd = 1.0f / sqrtf(wave_sum(s2) / (float)p.ncols + 1.0e-5f);
+            xv[0].x = ((xv[0].x - mean) * rstd) * nv[0].x + bv[0].x;
+            xv[0].y = ((xv[0].y - mean) * rstd) * nv[0].y + bv[0].y;
+            xv[0].z = ((xv[0].z - mean) * rstd) * nv[0].z + bv[0].z;
+            xv[0].w = ((xv[0].w - mean) * rstd) * nv[0].w + bv[0].w;
+        } else if (ln_g) {
             // LayerNorm folded in (host guarantees that the XP float4 per thread cover
             // x): mean, then variance about the mean (two exact passes over registers,
             // ops/layernorm.rs:46-53), then x <- (x - mean) * rstd * gamma + beta.
@@ -1330,55 +1372,63 @@ __device__ __forceinline__ void gemv_i8_body(const GemvParams &p, Policy &pol, u
 // MINW: waves per SIMD the register allocation must leave room for (MAXT / 256 = one
 // workgroup per CU; twice that caps the kernel at 64 vector registers, so that two
 // 1024-thread workgroups share a CU).
-template <class F, int R, int D, int MAXT, int MINW = MAXT / 256, bool XPART = false>
+template <class F, int R, int D, int MAXT, int MINW = MAXT / 256, bool XPART = false, bool FULL = false>
 __global__ __launch_bounds__(MAXT, MINW) void gemv_quant_i8_kernel(const GemvParams p) {
-    PlainPolicy pol{p, nullptr, 0.f, 0.f, 0};
+    using Policy = PlainPolicy<FULL>;
+    Policy pol{p, nullptr, 0.f, 0.f, 0};
     const uint32_t ngroups = (p.nrows + R - 1) / R;
     if constexpr (!F::F32X) {
         if (p.ncols <= 64 * F::TILE) {
-            gemv_i8_body<F, R, D, true, PlainPolicy, XPART>(p, pol, blockIdx.x, gridDim.x,
-                                                            p.active_waves, ngroups);
+            gemv_i8_body<F, R, D, true, Policy, XPART, FULL>(p, pol, blockIdx.x, gridDim.x,
+                                                             p.active_waves, ngroups);
             return;
         }
     }
-    gemv_i8_body<F, R, D, false, PlainPolicy, XPART>(p, pol, blockIdx.x, gridDim.x, p.active_waves,
-                                                     ngroups);
+    gemv_i8_body<F, R, D, false, Policy, XPART, FULL>(p, pol, blockIdx.x, gridDim.x, p.active_waves,
+                                                      ngroups);
 }
 
 // ------------------------------------------------------------------------
-// Fused multi-matrix launch.  Up to three matrices that consume the same input
-// vector share one launch (Q, K and V; gate and up): each workgroup works on one
-// of them (so mixed quantization formats are fine: the format decides the
-// workgroup's staging layout and inner loop), and the row pairs of a wave get an
-// epilogue:
+// Fused multi-matrix launches.  Up to three matrices that consume the same input vector share one launch
+// (Q, K and V): each workgroup works on one of them (so mixed quantization formats are fine: the format
+// decides the workgroup's staging layout and inner loop), and the row pairs of a wave get an epilogue:
 //   PLAIN  out[row] = dot (+ bias) (+ out)
 //   ROPE   the pair (2g, 2g+1) is rotated by the RoPE angle of pair g before it
 //          is stored (ops/rope.wgsl:35-58, adjacent-pair variant)
+// Outputs may be displaced by pos * out_pos_stride (KV-cache column of the current position).
+// A gate and an up matrix share one launch of another kernel (GatedPolicy):
 //   SILU   the wave holds row g of the gate matrix and row g of the up matrix and
 //          stores up * gate / (1 + exp(-gate))   (ops/silu.wgsl:13-27)
-// Outputs may be displaced by pos * out_pos_stride (KV-cache column of the
-// current position).
+// One kernel for all three modes took longer: the arguments lie in memory that no cache holds when a launch starts (two
+// unused job records of 112 bytes 0.24 us), and both matrices' planes were fetched and picked from (0.35 us).  us per launch in a
+// recorded graph, Q8_0: gate and up 768x288 4.01 -> 3.12, plain rows 3.81 -> 3.38 (the single-matrix kernel 2.8); gate and
+// up 11008x4096 in Q4_K 12.6 -> 11.8.
 enum { JOB_PLAIN = 0, JOB_ROPE = 1, JOB_SILU = 2 };
 
 struct GemvJob {
     const uint8_t *a0, *a1, *a2, *a3;  // matrix planes
-    const uint8_t *b0, *b1, *b2, *b3;  // second matrix (SILU: a = gate, b = up)
     float *out;
     const float *bias;
     uint32_t nrows;
-    int type, mode, accumulate;
+    uint32_t kind;  // format, mode and whether out is added to: GEMV_KIND
     uint32_t out_pos_stride;
     uint32_t wg_begin, wg_count;  // workgroups assigned to this matrix
     uint32_t active_waves;        // waves of a workgroup that walk its row pairs
+    __host__ __device__ int type() const { return (int)(kind & 0xffu); }
+    __host__ __device__ int mode() const { return (int)((kind >> 8) & 0xffu); }
+    __device__ bool accumulate() const { return kind >> 16; }
 };
+constexpr uint32_t gemv_kind(int type, int mode, int accumulate) {
+    return (uint32_t)type | (uint32_t)mode << 8 | (accumulate ? 1u << 16 : 0u);
+}
 
 struct FusedParams {
     GemvJob jobs[3];
+    const float *ln_g, *ln_b;
     const float *x;
     uint32_t ncols;
-    const float *norm_w;
     float norm_eps;
-    const float *ln_g, *ln_b;
+    const float *norm_w;
     DynPos pos;
     uint32_t head_size;
     float rope_base;
@@ -1389,14 +1439,12 @@ struct FusedParams {
     int njobs;
 };
 
-// A group is a pair of rows whose tiles a wave loads together and multiplies with one
-// read of its tile of x:
-//   PLAIN / ROPE  rows 2g and 2g+1 of the matrix
-//   SILU          row g of the gate matrix and row g of the up matrix
+// A group is the pair of rows 2g and 2g+1, whose tiles a wave loads together and multiplies with one
+// read of its tile of x.
 struct JobPolicy {
     static constexpr int S = 1;
     const GemvJob &j;
-    const GemvParams &pa, &pb;  // plane views of the two matrices
+    const GemvParams &p;
     DynPos dpos;
     uint32_t head_size;
     float rope_base;
@@ -1406,17 +1454,8 @@ struct JobPolicy {
                          bool ok) const {
         static_assert(R == 2, "fused launches work on row pairs");
         if (!ok) g = 0;
-        const bool silu = j.mode == JOB_SILU;
-        // plane pointers are picked one by one (wave-uniform selects): choosing between
-        // the two parameter blocks by reference would force them into memory
-        GemvParams q{};
-        q.p0 = silu ? pb.p0 : pa.p0;
-        q.p1 = silu ? pb.p1 : pa.p1;
-        q.p2 = silu ? pb.p2 : pa.p2;
-        q.p3 = silu ? pb.p3 : pa.p3;
-        q.ncols = pa.ncols;
-        WF::load(w[0], WF::row_base(pa, silu ? g : 2 * g), tile);
-        WF::load(w[1], WF::row_base(q, silu ? g : min(2 * g + 1, j.nrows - 1)), tile);
+        WF::load(w[0], WF::row_base(p, 2 * g), tile);
+        WF::load(w[1], WF::row_base(p, min(2 * g + 1, j.nrows - 1)), tile);
     }
     // Lanes 2i and 2i+1 hold the two results of group g0 + i * GW.  prefetch()
     // fetches what the epilogue of the first segment needs at kernel start.
@@ -1439,7 +1478,6 @@ struct JobPolicy {
             pre_bias = pre_out = 0.f;
             pre_cs = make_float2(1.f, 0.f);
         }
-        if (j.mode == JOB_SILU) return;
         const uint32_t row = 2 * (g0 + (lane >> 1) * GW) + (lane & 1);
         if (!(lane < 2 * my_groups && row < j.nrows)) return;
         // what depends on the position waits for the late call: the output column of a
@@ -1448,14 +1486,14 @@ struct JobPolicy {
         const bool cs_needs_pos = dpos.ptr && !rope_cs;
         if (!late) {
             if (j.bias) pre_bias = j.bias[row];
-            if (j.accumulate && !out_needs_pos) pre_out = (j.out + (size_t)dpos.val * j.out_pos_stride)[row];
-            if (j.mode == JOB_ROPE && !cs_needs_pos) {
+            if (j.accumulate() && !out_needs_pos) pre_out = (j.out + (size_t)dpos.val * j.out_pos_stride)[row];
+            if (j.mode() == JOB_ROPE && !cs_needs_pos) {
                 pos = dpos.val;
                 pre_cs = rope_entry(row);
             }
         } else {
-            if (j.accumulate && out_needs_pos) pre_out = (j.out + (size_t)pos * j.out_pos_stride)[row];
-            if (j.mode == JOB_ROPE && cs_needs_pos) pre_cs = rope_entry(row);
+            if (j.accumulate() && out_needs_pos) pre_out = (j.out + (size_t)pos * j.out_pos_stride)[row];
+            if (j.mode() == JOB_ROPE && cs_needs_pos) pre_cs = rope_entry(row);
         }
     }
     template <int R>
@@ -1463,45 +1501,64 @@ struct JobPolicy {
         const uint32_t g = g0 + (lane >> 1) * GW, sub = lane & 1;
         const bool valid = lane < n;
         float *out = j.out + (size_t)pos * j.out_pos_stride;
-        if (j.mode == JOB_SILU) {
-            const float up = dpp_f32<0xB1>(mine);  // the neighbouring lane's value
-            if (valid && sub == 0) out[g] = up * (mine / (1.0f + expf(-mine)));
-            return;
-        }
         const uint32_t row = 2 * g + sub;
         float t = mine + pre_bias;
-        if (j.mode == JOB_ROPE) {  // ROPE matrices have an even number of rows
+        if (j.mode() == JOB_ROPE) {  // ROPE matrices have an even number of rows
             const float other = dpp_f32<0xB1>(t);
             // (x, y) = (even row, odd row):  x' = cs x - sn y,  y' = sn x + cs y
             t = sub ? pre_cs.y * other + pre_cs.x * t : pre_cs.x * t - pre_cs.y * other;
         }
-        if (valid && row < j.nrows) out[row] = j.accumulate ? pre_out + t : t;
+        if (valid && row < j.nrows) out[row] = j.accumulate() ? pre_out + t : t;
     }
 };
 
-template <class F, int D>
+// Row g of the gate matrix and row g of the up matrix.
+struct GatedPolicy {
+    static constexpr int S = 1;
+    const GemvParams &gate, &up;
+    template <class WF, int R>
+    __device__ void load(typename WF::Row (&w)[R], uint32_t g, uint32_t, uint32_t tile, bool ok) const {
+        static_assert(R == 2, "fused launches work on row pairs");
+        if (!ok) g = 0;
+        WF::load(w[0], WF::row_base(gate, g), tile);
+        WF::load(w[1], WF::row_base(up, g), tile);
+    }
+    __device__ const uint32_t *pos_ptr() const { return nullptr; }
+    __device__ void set_pos(uint32_t) {}
+    template <int R>
+    __device__ void prefetch(bool, uint32_t, uint32_t, uint32_t, uint32_t) {}
+    template <int R>
+    __device__ void finish(float mine, uint32_t n, uint32_t g0, uint32_t GW, uint32_t lane) {
+        const float u = dpp_f32<0xB1>(mine);  // the neighbouring lane's value
+        if (lane < n && (lane & 1) == 0) gate.out[g0 + (lane >> 1) * GW] = u * (mine / (1.0f + expf(-mine)));
+    }
+};
+
+template <class F, int D, bool FULL>
 __device__ __forceinline__ void fused_job_body(const FusedParams &P, const GemvJob &j) {
-    GemvParams xp{};
-    xp.x = P.x;
-    xp.ncols = P.ncols;
-    xp.norm_w = P.norm_w;
-    xp.norm_eps = P.norm_eps;
-    xp.ln_g = P.ln_g;
-    xp.ln_b = P.ln_b;
-    xp.nrows = j.nrows;
-    GemvParams pa = xp, pb = xp;
-    pa.p0 = j.a0; pa.p1 = j.a1; pa.p2 = j.a2; pa.p3 = j.a3;
-    pb.p0 = j.b0; pb.p1 = j.b1; pb.p2 = j.b2; pb.p3 = j.b3;
-    JobPolicy pol{j, pa, pb, P.pos, P.head_size, P.rope_base, P.rope_cs, 0.f, 0.f, make_float2(1.f, 0.f), 0};
-    const uint32_t ngroups = j.mode == JOB_SILU ? j.nrows : (j.nrows + 1) / 2;
+    GemvParams p{};
+    p.x = P.x;
+    p.ncols = P.ncols;
+    p.norm_w = P.norm_w;
+    p.norm_eps = P.norm_eps;
+    if constexpr (FULL) {
+        p.ln_g = P.ln_g;
+        p.ln_b = P.ln_b;
+    }
+    p.nrows = j.nrows;
+    p.p0 = j.a0;
+    p.p1 = j.a1;
+    p.p2 = j.a2;
+    p.p3 = j.a3;
+    JobPolicy pol{j, p, P.pos, P.head_size, P.rope_base, P.rope_cs, 0.f, 0.f, make_float2(1.f, 0.f), 0};
+    const uint32_t ngroups = (j.nrows + 1) / 2, wg = blockIdx.x - j.wg_begin;
     if constexpr (!F::F32X) {
         if (P.ncols <= 64 * F::TILE) {
-            gemv_i8_body<F, 2, D, true>(xp, pol, blockIdx.x - j.wg_begin, j.wg_count, j.active_waves,
-                                        ngroups);
+            gemv_i8_body<F, 2, D, true, JobPolicy, false, FULL>(p, pol, wg, j.wg_count, j.active_waves, ngroups);
             return;
         }
     }
-    gemv_i8_body<F, 2, D, false>(xp, pol, blockIdx.x - j.wg_begin, j.wg_count, j.active_waves, ngroups);
+    gemv_i8_body<F, 2, D, false, JobPolicy, false, FULL>(p, pol, wg, j.wg_count, j.active_waves, ngroups);
 }
 
 // The format struct of a GGUF type: integer-dot (F32 false) or fp32-activation.
@@ -1533,7 +1590,7 @@ template <> struct FusedFmt<kLegacyWide + WGML_Q5_1, false> { using T = IFmtLega
 // a launch may differ in format (Q4_K / Q6_K / Q8_0, decided per workgroup), else the one
 // format all of them have (smaller code, registers of that format only).  F32: fp32
 // activations (the three main formats only).
-template <int D, int MAXT, int MINW, int FMT, bool F32 = false>
+template <int D, int MAXT, int MINW, int FMT, bool F32 = false, bool FULL = false>
 __global__ __launch_bounds__(MAXT, MINW) void gemv_fused_kernel(const FusedParams P) {
     // All three job records are fetched at once and the workgroup's own is picked field by
     // field afterwards: indexing the kernel arguments with the job number would put a second
@@ -1544,20 +1601,71 @@ __global__ __launch_bounds__(MAXT, MINW) void gemv_fused_kernel(const FusedParam
     const GemvJob &j0 = P.jobs[0], &j1 = P.jobs[1], &j2 = P.jobs[2];
 #define WGML_PICK(f) (is2 ? j2.f : (is1 ? j1.f : j0.f))
     const GemvJob j{WGML_PICK(a0), WGML_PICK(a1), WGML_PICK(a2), WGML_PICK(a3),
-                    WGML_PICK(b0), WGML_PICK(b1), WGML_PICK(b2), WGML_PICK(b3),
-                    WGML_PICK(out), WGML_PICK(bias), WGML_PICK(nrows), WGML_PICK(type),
-                    WGML_PICK(mode), WGML_PICK(accumulate), WGML_PICK(out_pos_stride),
-                    WGML_PICK(wg_begin), WGML_PICK(wg_count), WGML_PICK(active_waves)};
-#undef WGML_PICK
+                    WGML_PICK(out), WGML_PICK(bias), WGML_PICK(nrows), WGML_PICK(kind),
+                    WGML_PICK(out_pos_stride), WGML_PICK(wg_begin), WGML_PICK(wg_count),
+                    WGML_PICK(active_waves)};
     if constexpr (FMT != 0) {
-        fused_job_body<typename FusedFmt<FMT, F32>::T, D>(P, j);
+        fused_job_body<typename FusedFmt<FMT, F32>::T, D, FULL>(P, j);
     } else {
-        switch (j.type) {
-        case WGML_Q4_K: fused_job_body<typename FusedFmt<WGML_Q4_K, F32>::T, D>(P, j); break;
-        case WGML_Q6_K: fused_job_body<typename FusedFmt<WGML_Q6_K, F32>::T, D>(P, j); break;
-        default: fused_job_body<typename FusedFmt<WGML_Q8_0, F32>::T, D>(P, j); break;
+        switch (j.type()) {
+        case WGML_Q4_K: fused_job_body<typename FusedFmt<WGML_Q4_K, F32>::T, D, FULL>(P, j); break;
+        case WGML_Q6_K: fused_job_body<typename FusedFmt<WGML_Q6_K, F32>::T, D, FULL>(P, j); break;
+        default: fused_job_body<typename FusedFmt<WGML_Q8_0, F32>::T, D, FULL>(P, j); break;
         }
     }
+}
+
+// The launch of a gate and an up matrix (of one format).
+struct GatedParams {
+    const uint8_t *a0, *a1, *a2, *a3;  // gate
+    const uint8_t *b0, *b1, *b2, *b3;  // up
+    const float *x, *norm_w;
+    float *out;
+    float norm_eps;
+    uint32_t nrows, ncols, active_waves;
+};
+template <int MAXT, int FMT, bool F32 = false>
+__global__ __launch_bounds__(MAXT, 1) void gemv_gated_kernel(const GatedParams P) {
+    using F = typename FusedFmt<FMT, F32>::T;
+    GemvParams a{};
+    a.x = P.x;
+    a.out = P.out;
+    a.nrows = P.nrows;
+    a.ncols = P.ncols;
+    a.norm_w = P.norm_w;
+    a.norm_eps = P.norm_eps;
+    GemvParams b = a;
+    a.p0 = P.a0;
+    a.p1 = P.a1;
+    a.p2 = P.a2;
+    a.p3 = P.a3;
+    b.p0 = P.b0;
+    b.p1 = P.b1;
+    b.p2 = P.b2;
+    b.p3 = P.b3;
+    GatedPolicy pol{a, b};
+    if constexpr (!F::F32X) {
+        if (P.ncols <= 64 * F::TILE) {
+            gemv_i8_body<F, 2, 1, true>(a, pol, blockIdx.x, gridDim.x, P.active_waves, P.nrows);
+            return;
+        }
+    }
+    gemv_i8_body<F, 2, 1, false>(a, pol, blockIdx.x, gridDim.x, P.active_waves, P.nrows);
+}
+
+// A format's kernels (the fp32-activation ones with F32).
+template <int TYPE, bool F32, bool FULL>
+GemvKernels gemv_kernels_of() {
+    using F = typename FusedFmt<TYPE, F32>::T;
+    GemvKernels k{};
+    k.plain = (const void *)gemv_quant_i8_kernel<F, 1, 1, 1024, 4, false, FULL>;
+    k.fused1024 = (const void *)gemv_fused_kernel<1, 1024, 1, TYPE, F32, FULL>;
+    k.fused768 = (const void *)gemv_fused_kernel<1, 768, 1, TYPE, F32, FULL>;
+    if constexpr (!FULL) {
+        k.gated1024 = (const void *)gemv_gated_kernel<1024, TYPE, F32>;
+        k.gated768 = (const void *)gemv_gated_kernel<768, TYPE, F32>;
+    }
+    return k;
 }
 
 // Pairs of the jobs in ROPE mode in the Neox variant: half a head, and 2^32 over it rounded up (g / half is

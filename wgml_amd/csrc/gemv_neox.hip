@@ -53,20 +53,20 @@ struct NeoxPolicy {
         const bool cs_needs_pos = dpos.ptr && !rope_cs;
         if (!late && j.bias) pre_bias = j.bias[row];
         if (!late) pos = dpos.val;
-        if (j.accumulate && late == out_needs_pos) pre_out = (j.out + (size_t)pos * j.out_pos_stride)[row];
-        if (j.mode == JOB_ROPE && late == cs_needs_pos) pre_cs = entry(g);
+        if (j.accumulate() && late == out_needs_pos) pre_out = (j.out + (size_t)pos * j.out_pos_stride)[row];
+        if (j.mode() == JOB_ROPE && late == cs_needs_pos) pre_cs = entry(g);
     }
     template <int R>
     __device__ void finish(float mine, uint32_t n, uint32_t g0, uint32_t GW, uint32_t lane) {
         const uint32_t sub = lane & 1, row = row_of(g0 + (lane >> 1) * GW) + sub * step();
         float *out = j.out + (size_t)pos * j.out_pos_stride;
         float t = mine + pre_bias;
-        if (j.mode == JOB_ROPE) {
+        if (j.mode() == JOB_ROPE) {
             const float other = dpp_f32<0xB1>(t);
             // (x, y) = (first row, second row):  x' = cs x - sn y,  y' = sn x + cs y
             t = sub ? pre_cs.y * other + pre_cs.x * t : pre_cs.x * t - pre_cs.y * other;
         }
-        if (lane < n && row < j.nrows) out[row] = j.accumulate ? pre_out + t : t;
+        if (lane < n && row < j.nrows) out[row] = j.accumulate() ? pre_out + t : t;
     }
 };
 
@@ -77,14 +77,12 @@ __device__ __forceinline__ void neox_job_body(const FusedParams &P, const GemvJo
     p.ncols = P.ncols;
     p.norm_w = P.norm_w;
     p.norm_eps = P.norm_eps;
-    p.ln_g = P.ln_g;
-    p.ln_b = P.ln_b;
     p.nrows = j.nrows;
     p.p0 = j.a0;
     p.p1 = j.a1;
     p.p2 = j.a2;
     p.p3 = j.a3;
-    if (j.mode != JOB_ROPE) pairs = {};
+    if (j.mode() != JOB_ROPE) pairs = {};
     NeoxPolicy pol{j, p, P.pos, P.rope_cs, P.head_size, P.rope_base, pairs, 0.f, 0.f, make_float2(1.f, 0.f), 0};
     const uint32_t ngroups = (j.nrows + 1) / 2, wg = blockIdx.x - j.wg_begin;
     if (P.ncols <= 64 * F::TILE)
@@ -99,17 +97,14 @@ __global__ __launch_bounds__(MAXT, MINW) void gemv_fused_neox_kernel(const Fused
     const bool is1 = P.njobs > 1 && blockIdx.x >= P.jobs[1].wg_begin;
     const bool is2 = P.njobs > 2 && blockIdx.x >= P.jobs[2].wg_begin;
     const GemvJob &j0 = P.jobs[0], &j1 = P.jobs[1], &j2 = P.jobs[2];
-#define WGML_PICK(f) (is2 ? j2.f : (is1 ? j1.f : j0.f))
     const GemvJob j{WGML_PICK(a0), WGML_PICK(a1), WGML_PICK(a2), WGML_PICK(a3),
-                    nullptr, nullptr, nullptr, nullptr,
-                    WGML_PICK(out), WGML_PICK(bias), WGML_PICK(nrows), WGML_PICK(type),
-                    WGML_PICK(mode), WGML_PICK(accumulate), WGML_PICK(out_pos_stride),
-                    WGML_PICK(wg_begin), WGML_PICK(wg_count), WGML_PICK(active_waves)};
-#undef WGML_PICK
+                    WGML_PICK(out), WGML_PICK(bias), WGML_PICK(nrows), WGML_PICK(kind),
+                    WGML_PICK(out_pos_stride), WGML_PICK(wg_begin), WGML_PICK(wg_count),
+                    WGML_PICK(active_waves)};
     if constexpr (FMT != 0) {
         neox_job_body<typename FusedFmt<FMT, false>::T>(P, j, pairs);
     } else {
-        switch (j.type) {
+        switch (j.type()) {
         case WGML_Q4_K: neox_job_body<IFmtQ4K>(P, j, pairs); break;
         case WGML_Q6_K: neox_job_body<IFmtQ6K>(P, j, pairs); break;
         default: neox_job_body<IFmtQ8_0>(P, j, pairs); break;
