@@ -1,0 +1,39 @@
+"""GPU: short contexts in one workgroup per head, or per head and slice of the value dimensions (heads of more than 64): head sizes whose
+slices are uneven, every place of a position in a quad and a round of 64, grouped heads, and an output that lies on the query.
+
+Bound: scores and sums are fp32 over at most 256 positions and 128 dimensions; 2e-5 of the largest result is about four times what is
+observed."""
+import numpy as np
+import pytest
+
+import wgml_amd as W
+
+pytestmark = pytest.mark.gpu
+
+
+def reference(q, k, v, n_heads, kv_mul, hs, pos):
+    out = np.empty(n_heads * hs)
+    for h in range(n_heads):
+        kv = h // kv_mul * hs
+        s = k[:pos + 1, kv:kv + hs].astype(np.float64) @ q[h * hs:(h + 1) * hs].astype(np.float64) / np.sqrt(hs)
+        p = np.exp(s - s.max())
+        out[h * hs:(h + 1) * hs] = (p / p.sum()) @ v[:pos + 1, kv:kv + hs].astype(np.float64)
+    return out
+
+
+@pytest.mark.parametrize("n_heads,kv_mul,hs", [(3, 1, 4), (5, 1, 64), (3, 1, 68), (6, 3, 72), (4, 2, 96), (7, 1, 100), (8, 8, 124),
+                                               (32, 4, 128), (2, 1, 128), (300, 1, 80)])
+@pytest.mark.parametrize("pos", [0, 2, 3, 4, 62, 63, 64, 127, 200, 255])
+@pytest.mark.parametrize("same", [False, True])
+def test_short_contexts(gpu, n_heads, kv_mul, hs, pos, same):
+    kv_dim = n_heads // kv_mul * hs
+    rng = np.random.default_rng(hs + pos)
+    q = rng.standard_normal(n_heads * hs).astype(np.float32)
+    k, v = (rng.standard_normal((256, kv_dim)).astype(np.float32) for _ in range(2))
+    k[pos + 1:], v[pos + 1:] = np.nan, np.nan  # rows beyond the position may be read, not used
+    qv = W.GpuVector.init(gpu, q)
+    out = qv if same else W.GpuVector.uninit(gpu, n_heads * hs)
+    p = W.BatchedMultiqueryAttentionParams(256, kv_dim, kv_mul, n_heads, hs, pos)
+    W.BatchedMultiqueryAttention.from_device(gpu).dispatch_multi(p, qv, W.GpuMatrix.init(gpu, k), W.GpuMatrix.init(gpu, v), out)
+    ref = reference(q, k, v, n_heads, kv_mul, hs, pos)
+    assert np.abs(out.read() - ref).max() <= 2e-5 * np.abs(ref).max()

@@ -31,6 +31,7 @@
 // heads of 128 beyond position 256, -1.2 % on 12 heads of 64, -16 % at 8192 positions of
 // 8 KV heads, where one workgroup merges the four heads of its group in turn.)
 #include <algorithm>
+#include <type_traits>
 
 #include "common.h"
 #include "device_utils.h"
@@ -51,7 +52,7 @@ struct AttnArgs {
     DynPos pos;
     uint32_t chunk;  // positions per wave
     uint32_t spec_rows;  // rows of the caches that exist (may be read before pos is known)
-    uint32_t spec_sets;  // register sets whose quads are requested before pos is known (>= 1)
+    uint32_t slice_f4;   // SLICED: float4 of V's rows that a workgroup weighs (1 .. 16)
     uint32_t n_wg_y;
     int direct;  // 1: grid.y == 1 and the workgroup writes xb itself
 };
@@ -304,19 +305,43 @@ __device__ __forceinline__ float4 axpby4(const float4 a, float sa, const float4 
     return make_float4(fmaf(a.x, sa, b.x * sb), fmaf(a.y, sa, b.y * sb), fmaf(a.z, sa, b.z * sb),
                        fmaf(a.w, sa, b.w * sb));
 }
-__device__ __forceinline__ float shfl_xor_f32(float v, int mask) { return __shfl_xor(v, mask, 64); }
 
-// NS register sets of QS quads each take turns (NS * QS quads of a wave in flight).  Less is
-// more here: one set of one quad -- a wave requests the K and V rows of four positions, waits,
-// consumes them and requests the next four; the other waves of the CU cover the wait -- is the
-// fastest at every length measured (per layer, attention + merge, us; sets x quads 1x1 / 2x1 /
-// 1x2 / 2x2 / 1x4: 32 heads of 128 at position 150: 4.38 / 4.62 / 4.54 / 4.84 / 5.94, at 1000:
-// 9.41 / 9.61 / 9.57 / 10.26 / 10.41; 8 KV heads x 4 at 8192: 20.2 / 20.6 / 21.3 / 21.8 / 21.5;
-// four sets of two were slower still), as with the GEMV's weight tiles: requests beyond what
-// keeps the memory system busy only queue.
-template <int NV4, int KM, int NW, int NS = 1, int QS = 1>
+// A wave has one quad in flight: it requests the K and V rows of four positions, waits, consumes them and requests the next
+// four; the other waves of the CU cover the wait.  More is slower (per layer, attention + merge, us; register sets x quads
+// per set 1x1 / 2x1 / 1x2 / 2x2 / 1x4: 32 heads of 128 at position 150: 4.38 / 4.62 / 4.54 / 4.84 / 5.94, at 1000:
+// 9.41 / 9.61 / 9.57 / 10.26 / 10.41; 8 KV heads x 4 at 8192: 20.2 / 20.6 / 21.3 / 21.8 / 21.5), as with the GEMV's weight
+// tiles: requests beyond what keeps the memory system busy only queue.
+//
+// SLICED (one workgroup per head and slice, blockIdx.y the slice, no partial results): a workgroup reads all of K, but weighs only
+// its slice of V's dimensions (a.slice_f4 float4 of a row, one per lane).  One compute unit takes about 30 GB/s whatever is
+// in flight, so a head's rows are what a short context waits for, and these are three quarters of them.  Query heads that share
+// a KV head read its rows again, each on compute units of its own.  Quarters of a wave meet by lane swaps (with two rounds of
+// ds_bpermute per value the 16 waves' merges were a sixth of the launch), and the waves' weights are made one per lane.
+// us per layer, one workgroup per head group, bpermutes -> now: 32 heads of 128 at position 150 5.14 -> 4.45, at 250 7.69 -> 6.1, at
+// 20 4.21 -> 3.30; 8 KV heads x 4 at 150 6.51 -> 4.06; 4 x 4 at 25 4.94 -> 3.12; 12 heads of 64 at 150 3.97 -> 3.71.  With partial
+// results and the merge launch (beyond 256 planned positions): 32 heads at 400 7.41 -> 7.29, 8 x 4 at 8192 19.2 -> 18.9.
+__device__ __forceinline__ void swap_halves(float v, float &lower, float &upper) {  // lanes i and i + 32
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    lower = __uint_as_float(r[0]);
+    upper = __uint_as_float(r[1]);
+}
+__device__ __forceinline__ void swap_rows(float v, float &even, float &odd) {  // rows of 16 lanes 2 i and 2 i + 1
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    even = __uint_as_float(r[0]);
+    odd = __uint_as_float(r[1]);
+}
+template <bool HALVES>
+__device__ __forceinline__ void swap_pair(float v, float &a, float &b) {
+    if constexpr (HALVES)
+        swap_halves(v, a, b);
+    else
+        swap_rows(v, a, b);
+}
+
+template <int NV4, int KM, int NW, bool SLICED = false>
 __global__ __launch_bounds__(NW * 64) void attn_fast_kernel(const AttnArgs a) {
-    constexpr int HSP = NV4 * 64;  // dimension capacity: 16 lanes x 4 x NV4
+    constexpr int NVV = SLICED ? 1 : NV4;  // float4 of V per lane
+    constexpr int HSP = NVV * 64;          // dimension capacity: 16 lanes x 4 x NVV
     __shared__ float sm_m[NW][KM], sm_l[NW][KM];
     __shared__ float sm_acc[NW][KM][HSP];
 
@@ -327,7 +352,7 @@ __global__ __launch_bounds__(NW * 64) void attn_fast_kernel(const AttnArgs a) {
     const uint32_t hs = a.head_size;
     const uint32_t h0 = blockIdx.x * KM;
     const uint32_t kvh = h0 / a.kv_mul;
-    const uint32_t gid = blockIdx.y * NW + wave, total = a.n_wg_y * NW;
+    const uint32_t gid = SLICED ? wave : blockIdx.y * NW + wave, total = SLICED ? NW : a.n_wg_y * NW;
     const float inv_sqrt_hs = 1.0f / sqrtf((float)hs);
     const float4 zero4 = make_float4(0.f, 0.f, 0.f, 0.f);
     const float *kb = a.kc + (size_t)kvh * hs;
@@ -342,56 +367,32 @@ __global__ __launch_bounds__(NW * 64) void attn_fast_kernel(const AttnArgs a) {
         dv[v] = (sub + 16 * v) * 4 < hs;
         cv[v] = min(sub + 16 * v, hs / 4 - 1);
     }
+    // (lanes beyond a slice read its last float4 again)
+    const uint32_t slice0 = SLICED ? blockIdx.y * a.slice_f4 : 0;
+    const uint32_t cs = min(slice0 + min(sub, a.slice_f4 - 1), hs / 4 - 1);
 
-    // This wave's quads are gid, gid + total, ...  NS register sets of QS quads
-    // each take turns: while one is consumed the others' loads (if NS > 1) are in flight.
-    // The quads of the first set are requested before the position is known (`spec_rows` rows
-    // of the caches may be read; rows beyond the position are masked out below),
-    // the others once it is, and only those that hold a position <= pos.
-    float4 kS[NS][QS][NV4], vS[NS][QS][NV4];
+    // This wave's quads are gid, gid + total, ...  The first is requested before the position is known where it lies inside
+    // the caches whatever the position is (`spec_rows` rows may be read; those beyond the position are masked out below: a
+    // recorded step is planned for a range of positions whose lower end lies beyond what the first quads of all waves cover, so
+    // nothing is read in vain).
+    float4 k4[NV4], v4[NVV];
 #pragma unroll
-    for (int s = 0; s < NS; ++s) {
+    for (int v = 0; v < NV4; ++v) k4[v] = zero4;
 #pragma unroll
-        for (int u = 0; u < QS; ++u) {
+    for (int v = 0; v < NVV; ++v) v4[v] = zero4;
+    auto request = [&](uint32_t quad, uint32_t last) {
+        const uint32_t tt = min(quad * 4 + quarter, last);
+        const float4 *kp = reinterpret_cast<const float4 *>(kb + (size_t)tt * a.kv_dim);
+        const float4 *vp = reinterpret_cast<const float4 *>(vb + (size_t)tt * a.kv_dim);
 #pragma unroll
-            for (int v = 0; v < NV4; ++v) kS[s][u][v] = vS[s][u][v] = zero4;
-        }
-    }
-    // requests quads number i0 + u (u_begin <= u < QS) of this wave into a set
-    auto request = [&](float4(&kk)[QS][NV4], float4(&vv)[QS][NV4], uint32_t i0, uint32_t last,
-                       int u_begin, uint32_t nq_limit) {
+        for (int v = 0; v < NV4; ++v) k4[v] = kp[cv[v]];
 #pragma unroll
-        for (int u = 0; u < QS; ++u) {
-            const uint32_t quad = (i0 + u) * total + gid;
-            if (u >= u_begin && quad < nq_limit) {  // uniform over the wave
-                const uint32_t tt = min(quad * 4 + quarter, last);
-                const float4 *kp = reinterpret_cast<const float4 *>(kb + (size_t)tt * a.kv_dim);
-                const float4 *vp = reinterpret_cast<const float4 *>(vb + (size_t)tt * a.kv_dim);
-#pragma unroll
-                for (int v = 0; v < NV4; ++v) kk[u][v] = kp[cv[v]];
-#pragma unroll
-                for (int v = 0; v < NV4; ++v) vv[u][v] = vp[cv[v]];
-            }
-        }
+        for (int v = 0; v < NVV; ++v) v4[v] = vp[SLICED ? cs : cv[v]];
     };
-    // Quads that lie inside the caches whatever the position are requested right away: those
-    // of the first `spec_sets` register sets (one: a recorded step is planned for a range of
-    // positions whose lower end lies beyond what the first sets of all waves cover, so nothing
-    // is read in vain).
-    const uint32_t spec_quads = a.spec_rows / 4;  // whole quads below spec_rows
-    int n_spec[NS];
-#pragma unroll
-    for (int s = 0; s < NS; ++s) {
-        // the set's leading quads that lie below spec_rows (a wave's quads ascend)
-        n_spec[s] = 0;
-        if ((uint32_t)s < a.spec_sets) {
-#pragma unroll
-            for (int u = 0; u < QS; ++u) n_spec[s] += ((uint32_t)(QS * s + u) * total + gid < spec_quads) ? 1 : 0;
-        }
-        if (n_spec[s]) request(kS[s], vS[s], QS * s, a.spec_rows - 1, 0, spec_quads);
-    }
+    const bool early = gid < a.spec_rows / 4;
+    if (early) request(gid, a.spec_rows - 1);
 
-    float4 q[KM][NV4], acc[KM][NV4];
+    float4 q[KM][NV4], acc[KM][NVV];
     float mx[KM], l[KM];
 #pragma unroll
     for (int m = 0; m < KM; ++m) {
@@ -402,79 +403,73 @@ __global__ __launch_bounds__(NW * 64) void attn_fast_kernel(const AttnArgs a) {
             const float4 qv = reinterpret_cast<const float4 *>(a.q + (size_t)(h0 + m) * hs)[cv[v]];
             q[m][v] = make_float4(dv[v] ? qv.x : 0.f, dv[v] ? qv.y : 0.f, dv[v] ? qv.z : 0.f,
                                   dv[v] ? qv.w : 0.f);
-            acc[m][v] = zero4;
         }
+#pragma unroll
+        for (int v = 0; v < NVV; ++v) acc[m][v] = zero4;
     }
 
     const uint32_t pos = dyn_pos(a.pos);
-    const uint32_t n_used = fast_n_used(pos, a.n_wg_y, NW);  // workgroups with work
-    if (blockIdx.y >= n_used) {
-        // no position for this workgroup: a neutral partial (max -inf, sum 0), so that the
-        // merge need not know the position to tell which partials count
-        if (threadIdx.x < KM) {
-            float *p = a.ws_ml + ((size_t)(h0 + threadIdx.x) * a.n_wg_y + blockIdx.y) * 2;
-            p[0] = -INFINITY;
-            p[1] = 0.f;
+    if constexpr (!SLICED) {
+        if (blockIdx.y >= fast_n_used(pos, a.n_wg_y, NW)) {
+            // no position for this workgroup: a neutral partial (max -inf, sum 0), so that the
+            // merge need not know the position to tell which partials count
+            if (threadIdx.x < KM) {
+                float *p = a.ws_ml + ((size_t)(h0 + threadIdx.x) * a.n_wg_y + blockIdx.y) * 2;
+                p[0] = -INFINITY;
+                p[1] = 0.f;
+            }
+            return;
         }
-        return;
     }
     const uint32_t nq = pos / 4 + 1;
-    // online-softmax update with the quads of a set
-    auto consume = [&](const float4(&kk)[QS][NV4], const float4(&vv)[QS][NV4], uint32_t i0) {
+    if (!early && gid < nq) request(gid, pos);
+    for (uint32_t quad = gid; quad < nq; quad += total) {
+        // uniform within each 16-lane row, so the row reductions below see whole rows
+        if (quad * 4 + quarter <= pos) {
 #pragma unroll
-        for (int u = 0; u < QS; ++u) {
-            // uniform within each 16-lane row, so the row reductions below see whole rows
-            if (((i0 + u) * total + gid) * 4 + quarter <= pos) {
+            for (int m = 0; m < KM; ++m) {
+                float part = 0.f;
 #pragma unroll
-                for (int m = 0; m < KM; ++m) {
-                    float part = 0.f;
+                for (int v = 0; v < NV4; ++v) part = dot4(q[m][v], k4[v], part);
+                const float s = row16_sum(part) * inv_sqrt_hs;
+                const float mn = fmaxf(mx[m], s);
+                const float sc = __expf(mx[m] - mn);
+                const float p = __expf(s - mn);
+                l[m] = fmaf(l[m], sc, p);
 #pragma unroll
-                    for (int v = 0; v < NV4; ++v) part = dot4(q[m][v], kk[u][v], part);
-                    const float s = row16_sum(part) * inv_sqrt_hs;
-                    const float mn = fmaxf(mx[m], s);
-                    const float sc = __expf(mx[m] - mn);
-                    const float p = __expf(s - mn);
-                    l[m] = fmaf(l[m], sc, p);
-#pragma unroll
-                    for (int v = 0; v < NV4; ++v) acc[m][v] = axpby4(acc[m][v], sc, vv[u][v], p);
-                    mx[m] = mn;
-                }
+                for (int v = 0; v < NVV; ++v) acc[m][v] = axpby4(acc[m][v], sc, v4[v], p);
+                mx[m] = mn;
             }
         }
-    };
-#pragma unroll
-    for (int s = 0; s < NS; ++s) request(kS[s], vS[s], QS * s, pos, n_spec[s], nq);
-    for (uint32_t i0 = 0; i0 * total + gid < nq; i0 += QS * NS) {
-#pragma unroll
-        for (int s = 0; s < NS; ++s) {
-            consume(kS[s], vS[s], i0 + QS * s);
-            request(kS[s], vS[s], i0 + QS * s + QS * NS, pos, 0, nq);
-        }
+        if (quad + total < nq) request(quad + total, pos);
     }
 
     // merge the four quarters of the wave (every lane ends up with the merged state)
-#pragma unroll
-    for (int step = 16; step <= 32; step <<= 1) {
+    auto merge_quarters = [&](auto halves_c) {
+        constexpr bool H = decltype(halves_c)::value;
 #pragma unroll
         for (int m = 0; m < KM; ++m) {
-            const float om = shfl_xor_f32(mx[m], step), ol = shfl_xor_f32(l[m], step);
-            const float M = fmaxf(mx[m], om);
-            const float sa = mx[m] == -INFINITY ? 0.f : __expf(mx[m] - M);
-            const float sb = om == -INFINITY ? 0.f : __expf(om - M);
-            l[m] = fmaf(l[m], sa, ol * sb);
+            float m0, m1, l0, l1, a0, a1;
+            swap_pair<H>(mx[m], m0, m1);
+            swap_pair<H>(l[m], l0, l1);
+            const float M = fmaxf(m0, m1);
+            const float s0 = m0 == -INFINITY ? 0.f : __expf(m0 - M), s1 = m1 == -INFINITY ? 0.f : __expf(m1 - M);
+            l[m] = fmaf(l0, s0, l1 * s1);
 #pragma unroll
-            for (int v = 0; v < NV4; ++v) {
-                float4 o;
-                o.x = shfl_xor_f32(acc[m][v].x, step);
-                o.y = shfl_xor_f32(acc[m][v].y, step);
-                o.z = shfl_xor_f32(acc[m][v].z, step);
-                o.w = shfl_xor_f32(acc[m][v].w, step);
-                acc[m][v] = axpby4(acc[m][v], sa, o, sb);
+            for (int v = 0; v < NVV; ++v) {
+                float *x = &acc[m][v].x;
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    swap_pair<H>(x[c], a0, a1);
+                    x[c] = fmaf(a0, s0, a1 * s1);
+                }
             }
             mx[m] = M;
         }
-    }
-    // merge the waves of this workgroup
+    };
+    merge_quarters(std::false_type{});
+    merge_quarters(std::true_type{});
+    // merge the waves of this workgroup: lane w of a row of 16 weighs wave w (or w % 4)
 #pragma unroll
     for (int m = 0; m < KM; ++m) {
         if (lane == 0) {
@@ -483,25 +478,35 @@ __global__ __launch_bounds__(NW * 64) void attn_fast_kernel(const AttnArgs a) {
         }
         if (quarter == 0) {
 #pragma unroll
-            for (int v = 0; v < NV4; ++v)
+            for (int v = 0; v < NVV; ++v)
                 reinterpret_cast<float4 *>(&sm_acc[wave][m][0])[sub + 16 * v] = acc[m][v];
         }
     }
     __syncthreads();
-    for (uint32_t i = threadIdx.x; i < KM * HSP; i += blockDim.x) {
-        const uint32_t m = i / HSP, d = i % HSP;
-        float M = sm_m[0][m];
-#pragma unroll
-        for (int w = 1; w < NW; ++w) M = fmaxf(M, sm_m[w][m]);
-        float L = 0.f, o = 0.f;
-#pragma unroll
-        for (int w = 0; w < NW; ++w) {
-            const float mw = sm_m[w][m];
-            const float wgt = mw == -INFINITY ? 0.f : __expf(mw - M);
-            L = fmaf(sm_l[w][m], wgt, L);
-            o = fmaf(sm_acc[w][m][d], wgt, o);
+    for (uint32_t i = threadIdx.x; i < KM * HSP; i += NW * 64) {
+        const uint32_t m = i / HSP, d = i % HSP;  // (m is the same in all lanes of a wave: HSP is a multiple of 64)
+        const float mw = sm_m[lane % NW][m];
+        float M = fmaxf(mw, dpp_f32<0xB1>(mw));
+        M = fmaxf(M, dpp_f32<0x4E>(M));
+        if (NW == 16) {
+            M = fmaxf(M, dpp_f32<0x141>(M));
+            M = fmaxf(M, dpp_f32<0x140>(M));
         }
-        if (a.n_wg_y == 1) {
+        const float wgt = mw == -INFINITY ? 0.f : __expf(mw - M);
+        float L = sm_l[lane % NW][m] * wgt;
+        L += dpp_f32<0xB1>(L);
+        L += dpp_f32<0x4E>(L);
+        if (NW == 16) {
+            L += dpp_f32<0x141>(L);
+            L += dpp_f32<0x140>(L);
+        }
+        float o = 0.f;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) o = fmaf(sm_acc[w][m][d], readlane_f32(wgt, w), o);
+        if constexpr (SLICED) {
+            const uint32_t at = slice0 * 4 + d;
+            if (d < a.slice_f4 * 4 && at < hs) a.xb[(size_t)h0 * hs + at] = o / L;
+        } else if (a.n_wg_y == 1) {
             if (d < hs) a.xb[(size_t)(h0 + m) * hs + d] = o / L;
         } else {
             const size_t slot = (size_t)(h0 + m) * a.n_wg_y + blockIdx.y;
@@ -574,8 +579,8 @@ int launch_nv(wgml_ctx *ctx, const AttnArgs &a, int km, dim3 grid) {
 template <int NV4, int NW>
 int launch_fast_nv(wgml_ctx *ctx, const AttnArgs &a, int km, dim3 grid) {
     const dim3 block(NW * 64);
-    // the planner keeps km * NV4 within the register budget of the variant
-    constexpr int kMaxKmNv = NW == 16 ? 4 : 8;
+    // the planner keeps km * NV4 within the register budget of the variant (16 waves: one head)
+    constexpr int kMaxKmNv = NW == 16 ? NV4 : 8;
     if (km * NV4 > kMaxKmNv)
         return set_error(WGML_E_INVALID, "attention: no kernel for km %d, %d float4 per lane", km,
                          NV4);
@@ -641,10 +646,9 @@ static int make_fast_plan(wgml_ctx *ctx, const wgml_attn_params &p, uint32_t pla
     pl.km = 1;
     if (p.kv_mul == 2 || p.kv_mul == 4) pl.km = (int)p.kv_mul;
     if (p.kv_mul == 8) pl.km = 4;
-    // register budget (q and acc are km * nv float4 each): 128 VGPRs for the
-    // 16-wave variant, 256 for the 4-wave one
-    const int max_kmnv = pl.wide ? 4 : 8;
-    while (pl.km > 1 && pl.km * pl.nv > max_kmnv) pl.km >>= 1;
+    if (pl.wide) pl.km = 1;  // (query heads that share a KV head read its rows again, on other compute units)
+    // register budget (q and acc are km * nv float4 each): 256 VGPRs
+    while (pl.km > 1 && pl.km * pl.nv > 8) pl.km >>= 1;
     pl.groups = p.n_heads / pl.km;
     pl.chunk = 0;  // derived from the position on the device
     pl.hsp = (uint32_t)pl.nv * 64;
@@ -771,11 +775,19 @@ int launch_attention_planned(wgml_ctx *ctx, const wgml_attn_params &p, DynPos po
         a.pos = pos;
         a.n_wg_y = pl.n_wg_y;
         a.spec_rows = cache_rows;
-        // (all sets at short planned lengths was measured: the launch reads up to twice the
-        // rows it needs and gets slower, 5.1 against 4.7 us with four workgroups per head)
-        a.spec_sets = 1u;
         const dim3 grid(pl.groups, pl.n_wg_y);
-        if (pl.wide) return launch_fast<16>(ctx, a, pl.nv, pl.km, grid);
+        if (pl.wide) {
+            // Heads of more than 64 dimensions in two slices (four and eight are no faster).  One slice of a head is written
+            // while the other may still read its q: not where these overlap.
+            const size_t dim = (size_t)p.n_heads * p.head_size;
+            const bool apart = (uintptr_t)(q + dim) <= (uintptr_t)xb || (uintptr_t)(xb + dim) <= (uintptr_t)q;
+            if (pl.nv != 2 || !apart) return launch_fast<16>(ctx, a, pl.nv, pl.km, grid);
+            a.slice_f4 = (p.head_size / 4 + 1) / 2;
+            attn_fast_kernel<2, 1, 16, true><<<dim3(p.n_heads, 2), dim3(1024), 0, ctx->stream>>>(a);
+            WGML_CHECK_LAUNCH();
+            ctx->launches++;
+            return WGML_OK;
+        }
         WGML_TRY(workspace((size_t)p.n_heads * pl.n_wg_y * (2 + pl.hsp) * 4, &a.ws));
         a.ws_ml = a.ws + (size_t)p.n_heads * pl.n_wg_y * pl.hsp;
         WGML_TRY(launch_fast<WAVES>(ctx, a, pl.nv, pl.km, grid));
