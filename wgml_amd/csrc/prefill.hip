@@ -173,13 +173,22 @@ __device__ __forceinline__ void load8(float (&o)[8], const float *p) {  // 16-by
     o[7] = b.w;
 }
 
+// Token of workgroup w.  Eight neighbouring tokens share every 128-byte line of the packed activations (16 bytes each), and
+// workgroup w runs on XCD w % 8: in runs of more than 64 tokens 8 i .. 8 i + 7 go to one XCD, whose L2 then writes whole
+// lines; in the order of the tokens eight L2s write a sixteen-byte piece of each.  us per launch, in order / so: 1000 rows
+// of 4096 to 14336 columns 36 -> 23, 128 rows 8.3 -> 7.7; 45 rows 5.8 / 5.9 (three XCDs have all the work).
+constexpr uint32_t kPrepInOrder = 64;
+__device__ __forceinline__ uint32_t prep_token(uint32_t w, uint32_t T) {
+    return T <= kPrepInOrder ? w : w / 64 * 64 + (w & 7) * 8 + (w / 8 & 7);
+}
+
 constexpr int PREP_THREADS = 1024;
 constexpr int PREP_GROUPS = 2;  // groups of 8 columns a thread keeps in registers
 // A form of its own for LayerNorm and for GELU: tested per element at run time they cost the other
 // rows 3 % of a short prompt (8 layers of the 7B shape, 45 tokens in plain f16: 1620 us against 1574).
 enum PrepMode { PREP_RMS, PREP_LN, PREP_GELU };
 // Bound by its chain of one memory trip (row, partial sums and norm weights together), a reduction and
-// a store: 8.4 us for 128 rows of 4096 that add four partial sums, 5.8 us for 21 rows of 3072 (9.5 and 6.4 with
+// a store: 7.7 us for 128 rows of 4096 that add four partial sums, 5.8 us for 21 rows of 3072 (9.5 and 6.4 with
 // the weights requested after the first of two reductions).
 // One workgroup per token: X[t] (fp32, optionally RMS-normalised with weights w as
 // the reference does: (x * rsqrt(mean(x^2) + eps)) * w, ops/rms_norm.rs:55-63) -> f16
@@ -198,7 +207,8 @@ __global__ __launch_bounds__(PREP_THREADS) void prep_x_kernel(float *__restrict_
                                                      float *__restrict__ xscale, uint32_t K,
                                                      uint32_t kpad, uint32_t T, uint32_t nt) {
     __shared__ float red[32];
-    const uint32_t t = blockIdx.x, tid = threadIdx.x;
+    const uint32_t t = prep_token(blockIdx.x, T), tid = threadIdx.x;
+    if (t >= T) return;
     // 16-byte word of (token t, columns 8 k8 .. 8 k8 + 7)
     auto word_index = [&](uint32_t k8) {
         const uint32_t c = k8 >> 3, s2 = (k8 >> 2) & 1, g = k8 & 3;
@@ -889,7 +899,8 @@ int launch_prefill_prep(wgml_ctx *ctx, float *x, uint32_t x_stride, const float 
         return set_error(WGML_E_INVALID, "prefill_prep: pending gate/up partial sums need a gated row of at "
                                          "most %d columns", 8 * PREP_GROUPS * PREP_THREADS);
     const auto kernel = ln_beta ? prep_x_kernel<PREP_LN> : gelu ? prep_x_kernel<PREP_GELU> : prep_x_kernel<PREP_RMS>;
-    kernel<<<dim3(T), dim3(PREP_THREADS), 0, ctx->stream>>>(
+    // (whole rounds of the eight XCDs, see prep_token; workgroups beyond T end at once)
+    kernel<<<dim3(T <= kPrepInOrder ? T : (T + 63) / 64 * 64), dim3(PREP_THREADS), 0, ctx->stream>>>(
         x, x_stride, pending ? ctx->gemm_part : nullptr, pending, pair, ln_beta ? ln_beta : up, norm_w, eps,
         reinterpret_cast<uint4 *>(xh), ctx->gemm_precise ? reinterpret_cast<uint4 *>(ctx->prefill_xl) : nullptr,
         reinterpret_cast<_Float16 *>(ctx->prefill_xsum), xscale, K, prefill_kpad(K), T, prefill_tpad(T) / 16);
