@@ -173,6 +173,13 @@ struct AttnPartials {
     uint32_t n = 0, hsp = 0, head_size = 0;
 };
 
+// The largest of some results of a product, and the first row that has it.
+struct RowMaximum {
+    float value;
+    uint32_t row;
+};
+constexpr uint32_t kMaxRowMaxima = 16384;  // 32 waves on each of 256 compute units, twice
+
 struct GemvEpilogue {
     // out[r] = acc (+ bias[r]) (+ out[r] if accumulate)
     const float *bias = nullptr;
@@ -190,6 +197,10 @@ struct GemvEpilogue {
     // activation applied to acc + bias before it is stored: 0 none, 1 GELU (tanh form,
     // ops/unary.rs:106-110)
     int act = 0;
+    // room for kMaxRowMaxima: every wave of the product leaves the largest of its results and its row, where the kernel that
+    // takes the product can (*n_maxima: how many there are, 0 where none; n_maxima and maxima come together)
+    RowMaximum *maxima = nullptr;
+    uint32_t *n_maxima = nullptr;
     // partials.n > 0: the input vector is the merged attention output of these partial results
     // (the `v` argument is ignored); integer-dot kernels of Q8_0 / Q4_K / Q6_K only, up to 16
     // partial results per head
@@ -245,6 +256,8 @@ GemvKernels gemv_legacy_kernels(int fmt);  // gemv_legacy.hip: a 32-element form
 // gemv_full.hip: with LayerNorm and activation (a format, kLegacyWide + one or kFusedDenseF32; no gated ones);
 // `rows` of a group of the plain kernel: 1, or 2 in Q8_0
 GemvKernels gemv_full_kernels(int fmt, bool f32, int rows);
+// gemv_maxima.hip: the plain kernel that leaves RowMaximums (same arguments)
+const void *gemv_maxima_kernel(int fmt, bool f32, int rows);
 
 int launch_gemv_quant(wgml_ctx *ctx, float *out, const wgml_qmat *m, const float *v,
                       const GemvEpilogue &ep);
@@ -313,9 +326,11 @@ struct NextEmbed {
     const float *pos_table;  // optional (GPT-2's learned positions)
     uint32_t n_pos;          // rows of pos_table: no row is read for a position beyond them
 };
+// With n_maxima the arg-max is that of these maxima, which the product that wrote v has left; v is not read.
 int launch_argmax_next(wgml_ctx *ctx, const float *v, uint32_t n, DynState *dyn,
                        const uint32_t *prompt, uint32_t *tokens_out,
-                       const NextEmbed *embed = nullptr);
+                       const NextEmbed *embed = nullptr, const RowMaximum *maxima = nullptr,
+                       uint32_t n_maxima = 0);
 int launch_dequantize(wgml_ctx *ctx, float *out, const wgml_qmat *m);
 
 // ---- batched products for prompt processing (prefill.hip) ---------------------

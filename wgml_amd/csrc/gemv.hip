@@ -16,6 +16,11 @@ template __global__ void gemv_gated_kernel<1024, WGML_Q6_K>(const GatedParams);
 template __global__ void gemv_fused_kernel<1, 1024, 1, WGML_Q8_0, false>(const FusedParams);
 template __global__ void gemv_quant_i8_kernel<IFmtQ8_0, 1, 1, 1024, 8, false>(const GemvParams);
 template __global__ void gemv_gated_kernel<1024, WGML_Q8_0>(const GatedParams);
+// (the output matrix of a token loop)
+template __global__ void gemv_quant_i8_kernel<IFmtQ6K, 1, 1, 1024, 4, false, EXTRA_MAXIMA>(const GemvParams);
+template __global__ void gemv_quant_i8_kernel<IFmtQ8_0, 2, 1, 1024, 4, false, EXTRA_MAXIMA>(const GemvParams);
+template __global__ void gemv_quant_i8_kernel<IFmtQ8_0, 1, 1, 1024, 8, false, EXTRA_MAXIMA>(const GemvParams);
+template __global__ void gemv_quant_i8_kernel<IFmtQ4K, 1, 1, 1024, 8, false, EXTRA_MAXIMA>(const GemvParams);
 
 // ------------------------------------------------------------- dense f32 ----
 // out = A v, A row-major f32 (p.p0).  One wave per row, float4 loads, x from LDS.  For what the
@@ -136,7 +141,9 @@ size_t lds_bytes_of(uint32_t ncols) {
     return ntiles_pad * 2 * (F::TILE / 16) * 16 + ntiles_pad * (F::NXB + F::NSUM) * 4;
 }
 // `fn`: a gemv_quant_i8_kernel with R rows per group and workgroups of `maxt` threads.
-int launch_plain(wgml_ctx *ctx, const void *fn, uint32_t R, uint32_t maxt, GemvParams p, size_t lds) {
+// `n_maxima`: fn leaves maxima (EXTRA_MAXIMA); receives how many, 0 (and none are left) if they are more than kMaxRowMaxima.
+int launch_plain(wgml_ctx *ctx, const void *fn, uint32_t R, uint32_t maxt, GemvParams p, size_t lds,
+                 uint32_t *n_maxima = nullptr) {
     int per_cu = 1;
     WGML_TRY(blocks_per_cu(ctx, fn, (int)maxt, lds, &per_cu));
     const uint32_t cu = ctx->n_cu > 0 ? (uint32_t)ctx->n_cu : 256u;
@@ -147,6 +154,12 @@ int launch_plain(wgml_ctx *ctx, const void *fn, uint32_t R, uint32_t maxt, GemvP
     if (min_c > maxt / 64) min_c = maxt / 64;
     const WgPlan plan = plan_groups(ngroups, cu * (uint32_t)per_cu, maxt / 64, 64 / R, min_c);
     p.active_waves = plan.active_waves;
+    if (n_maxima) {
+        // a wave's number is that of its first row-group
+        const uint32_t waves = plan.wgs * plan.active_waves, n = waves < ngroups ? waves : ngroups;
+        *n_maxima = n <= kMaxRowMaxima ? n : 0;
+        if (!*n_maxima) p.maxima = nullptr;
+    }
     void *args[] = {&p};
     WGML_CHECK_HIP(hipLaunchKernel(fn, dim3(plan.wgs), dim3(maxt), args, lds, ctx->stream));
     WGML_CHECK_LAUNCH();
@@ -354,7 +367,7 @@ static size_t lds_bytes_fused(int type, uint32_t ncols, bool f32) {
 static bool main_format(int type) { return type == WGML_Q4_K || type == WGML_Q6_K || type == WGML_Q8_0; }
 
 // With LayerNorm or activation (gemv_full.hip): one variant per format, Q8_0 in one or two rows per wave.
-static int launch_full(wgml_ctx *ctx, const wgml_qmat *m, const GemvParams &p) {
+static int launch_full(wgml_ctx *ctx, const wgml_qmat *m, const GemvParams &p, uint32_t *n_maxima) {
     if (m->type == WGML_F32 && !dense_f32_in_shared_body(m))
         return set_error(WGML_E_UNSUPPORTED, "gemv_quant: LayerNorm / activation folding needs rows of a "
                                              "multiple of 16 elements");
@@ -372,7 +385,39 @@ static int launch_full(wgml_ctx *ctx, const wgml_qmat *m, const GemvParams &p) {
                     : legacy_format(m->type) ? legacy_kernel_format(m->type, p.ncols)
                                              : m->type;
     const int rows = m->type == WGML_Q8_0 && !f32 ? rows_per_wave_q8(p) : 1;
-    return launch_plain(ctx, gemv_full_kernels(fmt, f32, rows).plain, (uint32_t)rows, 1024, p, lds);
+    return launch_plain(ctx, gemv_full_kernels(fmt, f32, rows).plain, (uint32_t)rows, 1024, p, lds, n_maxima);
+}
+
+// The kernel that leaves maxima for a plain product (gemv_maxima.hip: one row per wave, one tile in flight, workgroups of 16
+// waves), or null where the product runs in another shape: launch-shape overrides, Q8_0 rows that have four tiles in
+// flight, dense rows that the general kernel takes, rows beyond the LDS limit (the caller's own path refuses them).
+static const void *maxima_kernel_for(const wgml_ctx *ctx, const wgml_qmat *m, const GemvParams &p, uint32_t *rows,
+                                     size_t *lds) {
+    for (int key : {WGML_TUNE_GEMV_ROWS_PER_WAVE, WGML_TUNE_GEMV_WAVES_PER_WG, WGML_TUNE_GEMV_DEPTH})
+        if (ctx->tuning[key]) return nullptr;
+    const bool dense = m->type == WGML_F32;
+    if (p.part_n || (dense && (!dense_f32_in_shared_body(m) ||
+                               dense_f32_general_faster(ctx, p.nrows, p.ncols, p.norm_w != nullptr))))
+        return nullptr;
+    const bool f32 = dense || (main_format(m->type) && ctx->tuning[WGML_TUNE_GEMV_F32_ACTIVATIONS]);
+    if (m->type == WGML_Q8_0 && !f32 && p.ncols > 8192) return nullptr;
+    *lds = lds_bytes_fused(m->type, p.ncols, f32);
+    if (*lds > kMaxLds) return nullptr;
+    *rows = m->type == WGML_Q8_0 && !f32 ? (uint32_t)rows_per_wave_q8(p) : 1u;
+    if (!f32) {
+        switch (m->type) {
+        case WGML_Q6_K: return (const void *)gemv_quant_i8_kernel<IFmtQ6K, 1, 1, 1024, 4, false, EXTRA_MAXIMA>;
+        case WGML_Q4_K: return (const void *)gemv_quant_i8_kernel<IFmtQ4K, 1, 1, 1024, 8, false, EXTRA_MAXIMA>;
+        case WGML_Q8_0:
+            if (*rows == 2) return (const void *)gemv_quant_i8_kernel<IFmtQ8_0, 2, 1, 1024, 4, false, EXTRA_MAXIMA>;
+            return (const void *)gemv_quant_i8_kernel<IFmtQ8_0, 1, 1, 1024, 8, false, EXTRA_MAXIMA>;
+        default: break;
+        }
+    }
+    return gemv_maxima_kernel(dense                     ? kFusedDenseF32
+                              : legacy_format(m->type) ? legacy_kernel_format(m->type, p.ncols)
+                                                       : m->type,
+                              f32, (int)*rows);
 }
 
 int launch_gemv_quant(wgml_ctx *ctx, float *out, const wgml_qmat *m, const float *v,
@@ -412,7 +457,15 @@ int launch_gemv_quant(wgml_ctx *ctx, float *out, const wgml_qmat *m, const float
     } else if ((uintptr_t)v % 16 != 0) {
         return set_error(WGML_E_INVALID, "gemv_quant: the input vector must be 16-byte aligned");
     }
-    if (p.ln_g || p.act) return launch_full(ctx, m, p);
+    p.maxima = ep.maxima;
+    if (ep.n_maxima) *ep.n_maxima = 0;
+    if (p.ln_g || p.act) return launch_full(ctx, m, p, ep.n_maxima);
+    if (ep.n_maxima) {
+        uint32_t rows = 1;
+        size_t lds = 0;
+        if (const void *fn = maxima_kernel_for(ctx, m, p, &rows, &lds))
+            return launch_plain(ctx, fn, rows, 1024, p, lds, ep.n_maxima);
+    }
     if (dense_f32_in_shared_body(m) && !dense_f32_general_faster(ctx, p.nrows, p.ncols, p.norm_w != nullptr))
         return launch_dense_f32(ctx, p);
     if (m->type == WGML_F32) {

@@ -13,7 +13,7 @@ GemvKernels wgml::gemv_full_kernels(int fmt, bool f32, int rows) {
     switch (fmt) {
     case WGML_Q8_0: {
         GemvKernels k = gemv_kernels_of<WGML_Q8_0, false, true>();
-        if (rows == 2) k.plain = (const void *)gemv_quant_i8_kernel<IFmtQ8_0, 2, 1, 1024, 4, false, true>;
+        if (rows == 2) k.plain = (const void *)gemv_quant_i8_kernel<IFmtQ8_0, 2, 1, 1024, 4, false, EXTRA_FULL | EXTRA_MAXIMA>;
         return k;
     }
     case WGML_Q4_K: return gemv_kernels_of<WGML_Q4_K, false, true>();

@@ -55,7 +55,14 @@ struct GemvParams {
     // results per head (AttnPartials in common.h); x itself is then not read
     const float *part_o, *part_ml;
     uint32_t part_n, part_hsp, part_hs, part_hs_inv;  // part_hs_inv = ceil(2^32 / part_hs)
+    // kernels with EXTRA_MAXIMA: (largest result, its row) of the wave whose first row-group is g goes to maxima[g]
+    RowMaximum *maxima;
 };
+
+// What a single-matrix kernel can do beside the product (bits).  Kernels of their own (gemv_full.hip, gemv_maxima.hip): the
+// code that the others jump over costs every launch 0.05 to 0.1 us.
+enum { EXTRA_FULL = 1,     // x may go through a LayerNorm, results through an activation
+       EXTRA_MAXIMA = 2 };  // every wave leaves the largest of its results
 
 // Merging attention partial results (see AttnPartials) for float4 number g4 of the merged
 // output: the partial results of its head are taken in eight at a time, the way an online
@@ -887,8 +894,9 @@ struct FFmt {
 };
 
 // Row source / sink of a plain single-matrix GEMV: group g = rows g*R .. g*R+R-1.
-template <bool FULL>
+template <int EXTRA>
 struct PlainPolicy {
+    static constexpr bool FULL = EXTRA & EXTRA_FULL;
     static constexpr int S = 1;  // passes per group
     const GemvParams &p;
     // `ok` false: the load still happens, from row-group 0 (a wave's loads are never
@@ -932,6 +940,17 @@ struct PlainPolicy {
                 if (p.act == 1) v = gelu_tanh(v);
             }
             out[row] = v + pre_out;
+            if constexpr ((EXTRA & EXTRA_MAXIMA) != 0) mine = v + pre_out;
+        }
+        if constexpr ((EXTRA & EXTRA_MAXIMA) != 0) {
+            // The first of the largest results: rows ascend with the lane.  A sequential scan for v > best from row 0 on
+            // passes over NaN, except in row 0, which then stays the best.
+            if (!p.maxima) return;
+            float v = lane < n && row < p.nrows && mine == mine ? mine : -INFINITY;
+            if (row == 0 && mine != mine) v = INFINITY;
+            const float best = wave_max(v);
+            const uint64_t at = __ballot(lane < n && v == best);
+            if (lane == (uint32_t)__builtin_ctzll(at)) p.maxima[g0] = RowMaximum{best, row};
         }
     }
 };
@@ -948,8 +967,7 @@ struct PlainPolicy {
 // XREG: rows fit one step (ncols <= 64 tiles), so a lane's tile of x is the same
 // for every row and is read from LDS once instead of once per row.
 // XPART: x is not read from p.x but merged from attention partial results (merged_partials).
-// FULL: x may go through a LayerNorm (p.ln_g) on its way, and results through an activation.  Kernels of
-// their own (gemv_full.hip): the code that the others jump over costs every launch 0.05 to 0.1 us.
+// FULL: x may go through a LayerNorm (p.ln_g) on its way, and results through an activation.
 template <class F, int R, int D, bool XREG, class Policy, bool XPART = false, bool FULL = false>
 __device__ __forceinline__ void gemv_i8_body(const GemvParams &p, Policy &pol, uint32_t wg,
                                              uint32_t nwg, uint32_t nw, uint32_t ngroups) {
@@ -1372,9 +1390,10 @@ __device__ __forceinline__ void gemv_i8_body(const GemvParams &p, Policy &pol, u
 // MINW: waves per SIMD the register allocation must leave room for (MAXT / 256 = one
 // workgroup per CU; twice that caps the kernel at 64 vector registers, so that two
 // 1024-thread workgroups share a CU).
-template <class F, int R, int D, int MAXT, int MINW = MAXT / 256, bool XPART = false, bool FULL = false>
+template <class F, int R, int D, int MAXT, int MINW = MAXT / 256, bool XPART = false, int EXTRA = 0>
 __global__ __launch_bounds__(MAXT, MINW) void gemv_quant_i8_kernel(const GemvParams p) {
-    using Policy = PlainPolicy<FULL>;
+    using Policy = PlainPolicy<EXTRA>;
+    constexpr bool FULL = Policy::FULL;
     Policy pol{p, nullptr, 0.f, 0.f, 0};
     const uint32_t ngroups = (p.nrows + R - 1) / R;
     if constexpr (!F::F32X) {
@@ -1658,7 +1677,7 @@ template <int TYPE, bool F32, bool FULL>
 GemvKernels gemv_kernels_of() {
     using F = typename FusedFmt<TYPE, F32>::T;
     GemvKernels k{};
-    k.plain = (const void *)gemv_quant_i8_kernel<F, 1, 1, 1024, 4, false, FULL>;
+    k.plain = (const void *)gemv_quant_i8_kernel<F, 1, 1, 1024, 4, false, FULL ? EXTRA_FULL | EXTRA_MAXIMA : 0>;
     k.fused1024 = (const void *)gemv_fused_kernel<1, 1024, 1, TYPE, F32, FULL>;
     k.fused768 = (const void *)gemv_fused_kernel<1, 768, 1, TYPE, F32, FULL>;
     if constexpr (!FULL) {

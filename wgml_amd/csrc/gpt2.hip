@@ -32,6 +32,7 @@ struct wgml_gpt2 {
     // recorded token loop: position / token / output cursor on the device
     DynState *dyn = nullptr;
     uint32_t *d_prompt = nullptr, *d_tokens = nullptr;
+    RowMaximum *maxima = nullptr;  // kMaxRowMaxima: what the output product leaves for the arg-max
     // the recorded step, one capture per bucket of positions (plan_bucket)
     hipGraph_t graph[kMaxPlanBuckets] = {};
     hipGraphExec_t graph_exec[kMaxPlanBuckets] = {};
@@ -118,6 +119,8 @@ int wgml_gpt2_create(wgml_ctx *ctx, const wgml_gpt2_params *p, wgml_gpt2 **out) 
         m->d_prompt = reinterpret_cast<uint32_t *>(tmp);
         A(&tmp, p->n_seq, true);
         m->d_tokens = reinterpret_cast<uint32_t *>(tmp);
+        A(&tmp, kMaxRowMaxima * (sizeof(RowMaximum) / sizeof(float)), true);
+        m->maxima = reinterpret_cast<RowMaximum *>(tmp);
     }
     for (auto &l : m->layers) {
         A(&l.key_cache, (uint64_t)p->n_embd * p->n_seq, true);
@@ -246,10 +249,11 @@ bool can_fold(const wgml_gpt2 *m) {
     return true;
 }
 
+// n_maxima non-null: the output product may leave the largest logit of each of its waves in m->maxima (their number, or 0).
 // embed == false: m->layer_input already holds wte[:, token] + wpe[:, pos] (the sampling launch
 // of the step before wrote it).
 int enqueue_step(wgml_gpt2 *m, bool dynamic, uint32_t token, uint32_t pos,
-                 uint32_t plan_positions = 0, bool embed = true) {
+                 uint32_t plan_positions = 0, bool embed = true, uint32_t *n_maxima = nullptr) {
     const wgml_gpt2_params &p = m->p;
     wgml_ctx *ctx = m->ctx;
     const uint32_t n = p.n_embd;
@@ -335,6 +339,10 @@ int enqueue_step(wgml_gpt2 *m, bool dynamic, uint32_t token, uint32_t pos,
         GemvEpilogue e;
         e.ln_gamma = m->ln_f_g;
         e.ln_beta = m->ln_f_b;
+        if (n_maxima) {
+            e.maxima = m->maxima;
+            e.n_maxima = n_maxima;
+        }
         WGML_TRY(launch_gemv_quant(ctx, m->curr_vocab, m->lm_head, m->layer_input, e));
     } else {
         WGML_TRY(launch_layernorm(ctx, m->curr_768, m->layer_input, m->ln_f_g, m->ln_f_b, n));
@@ -379,9 +387,11 @@ constexpr uint32_t kStepsPerGraph = 8;
 // follows.  The loop's first step finds it written by loop_first_embed.
 int enqueue_loop_step(wgml_gpt2 *m, uint32_t plan) {
     const wgml_gpt2_params &p = m->p;
-    WGML_TRY(enqueue_step(m, true, 0, 0, plan, false));
+    uint32_t n_maxima = 0;
+    WGML_TRY(enqueue_step(m, true, 0, 0, plan, false, &n_maxima));
     const NextEmbed ne{m->layer_input, m->wte, p.n_embd, nullptr, 2, 0.f, m->wpe, p.n_seq};
-    return launch_argmax_next(m->ctx, m->curr_vocab, p.n_vocab, m->dyn, m->d_prompt, m->d_tokens, &ne);
+    return launch_argmax_next(m->ctx, m->curr_vocab, p.n_vocab, m->dyn, m->d_prompt, m->d_tokens, &ne,
+                              m->maxima, n_maxima);
 }
 int loop_first_embed(wgml_gpt2 *m) {
     return launch_embed(m->ctx, m->layer_input, m->wte, m->p.n_embd, DynPos{&m->dyn->token, 0}, nullptr, 2,

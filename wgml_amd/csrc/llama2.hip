@@ -42,6 +42,7 @@ struct wgml_llama2 {
     // token-loop state on the device
     DynState *dyn = nullptr;
     uint32_t *d_prompt = nullptr, *d_tokens = nullptr;  // seq_len entries each
+    RowMaximum *maxima = nullptr;  // kMaxRowMaxima: what the output product leaves for the arg-max
     // the recorded step, one capture per bucket of positions (plan_bucket)
     hipGraph_t graph[kMaxPlanBuckets] = {};
     hipGraphExec_t graph_exec[kMaxPlanBuckets] = {};
@@ -123,10 +124,11 @@ void drop_graph(wgml_llama2 *m) {
 // fusion 0: one launch per reference op.  1: bias and residual adds folded into
 // the GEMV epilogues.  2: additionally every RMSNorm folded into the staging of
 // the GEMVs that consume it.
+//   n_maxima non-null: the output product may leave the largest logit of each of its waves in m->maxima (their number, or 0).
 //   embed == false : m->x and the RoPE table already hold the token's embedding and the
 //                     position's angles (the sampling launch of the step before wrote them).
 int enqueue_step(wgml_llama2 *m, bool dynamic, uint32_t token, uint32_t pos,
-                 uint32_t plan_positions = 0, bool embed = true) {
+                 uint32_t plan_positions = 0, bool embed = true, uint32_t *n_maxima = nullptr) {
     const wgml_llama2_config &c = m->cfg;
     wgml_ctx *ctx = m->ctx;
     const uint32_t dim = c.dim, kv_dim = m->kv_dim;
@@ -284,6 +286,10 @@ int enqueue_step(wgml_llama2 *m, bool dynamic, uint32_t token, uint32_t pos,
     } else {
         WGML_TRY(launch_rms_norm(ctx, c.rms_norm_eps, m->xb, m->x, m->output_norm, dim));
     }
+    if (n_maxima) {
+        eo.maxima = m->maxima;
+        eo.n_maxima = n_maxima;
+    }
     WGML_TRY(launch_gemv_quant(ctx, m->logits, m->output, out_in, eo));
     return WGML_OK;
 }
@@ -310,9 +316,11 @@ constexpr uint32_t kStepsPerGraph = 8;
 // The loop's first step finds them written by loop_first_embed.
 int enqueue_loop_step(wgml_llama2 *m, uint32_t plan) {
     const wgml_llama2_config &c = m->cfg;
-    WGML_TRY(enqueue_step(m, true, 0, 0, plan, false));
+    uint32_t n_maxima = 0;
+    WGML_TRY(enqueue_step(m, true, 0, 0, plan, false, &n_maxima));
     const NextEmbed ne{m->x, m->token_embd, c.dim, m->rope_cs, m->head_size, c.rope_base_freq, nullptr, 0};
-    return launch_argmax_next(m->ctx, m->logits, c.vocab_size, m->dyn, m->d_prompt, m->d_tokens, &ne);
+    return launch_argmax_next(m->ctx, m->logits, c.vocab_size, m->dyn, m->d_prompt, m->d_tokens, &ne,
+                              m->maxima, n_maxima);
 }
 int loop_first_embed(wgml_llama2 *m) {
     const wgml_llama2_config &c = m->cfg;
@@ -771,6 +779,7 @@ int wgml_llama2_create(wgml_ctx *ctx, const wgml_llama2_config *cfg, int model_t
     if (rc == WGML_OK) rc = dev_alloc_bytes(m, (void **)&m->dyn, 256, true);
     if (rc == WGML_OK) rc = dev_alloc_bytes(m, (void **)&m->d_prompt, (uint64_t)cfg->seq_len * 4, true);
     if (rc == WGML_OK) rc = dev_alloc_bytes(m, (void **)&m->d_tokens, (uint64_t)cfg->seq_len * 4, true);
+    if (rc == WGML_OK) rc = dev_alloc_bytes(m, (void **)&m->maxima, kMaxRowMaxima * sizeof(RowMaximum), true);
     if (rc == WGML_OK && hipStreamSynchronize(ctx->stream) != hipSuccess)
         rc = set_error(WGML_E_HIP, "wgml_llama2_create: synchronize failed");
     if (rc != WGML_OK) {
