@@ -136,12 +136,12 @@ WGML_API int wgml_buf_zero(wgml_buf *buf);
  *      GgufTensorData::to_gpu_matrix (gguf.rs:131-184) ---------------------- *
  * `gguf_bytes` is the tensor exactly as stored in a GGUF file: row-major,
  * nrows rows of ncols/elems_per_block blocks.  Every block format the reference keeps
- * quantized on the GPU (gguf.rs:172-182) stays quantized here: WGML_Q8_0 and WGML_Q6_K are
- * re-laid out into aligned planes on the device (same bytes in total, see the layout
- * notes in csrc/common.h), WGML_Q4_K, WGML_Q4_0, WGML_Q4_1, WGML_Q5_0, WGML_Q5_1,
+ * quantized on the GPU (gguf.rs:172-182) stays quantized here: WGML_Q8_0, WGML_Q6_K, WGML_Q4_0,
+ * WGML_Q4_1, WGML_Q5_0 and WGML_Q5_1 are re-laid out into aligned planes on the device (same bytes
+ * in total, see the layout notes in csrc/common.h), WGML_Q4_K,
  * WGML_Q5_K and WGML_Q8_K keep the GGUF bytes unchanged; the values are those of
- * Block*::dequantize in every case.  WGML_F16 is expanded to f32 on the device at
- * creation, as to_gpu_matrix does (the matrix then reports WGML_F32).  Other tags give
+ * Block*::dequantize in every case.  A WGML_F16 matrix reports WGML_F32, as to_gpu_matrix expands it:
+ * on the device it keeps its 16 bits where the products can read them, with the same results.  Other tags give
  * WGML_E_UNSUPPORTED.  Unlike the reference there is no pairing rule (ncols % 64 /
  * % 512): any ncols that is a multiple of the block length stays quantized. */
 WGML_API int wgml_quant_matrix_create(wgml_ctx *ctx, int type, uint32_t nrows, uint32_t ncols,

@@ -348,6 +348,13 @@ static bool dense_f32_general_faster(const wgml_ctx *ctx, uint32_t nrows, uint32
     return ncols <= 256 && (nrows <= 32768 || nrows > cu * 16 * 64);
 }
 
+// F16 tensors stay 16 bits wide where the shared body always takes their products (dense_f32_general_faster: never beyond
+// 512 columns); narrower or ragged rows are expanded to f32 when the matrix is created.
+bool gemv_keeps_f16(uint32_t ncols) {
+    return ncols > 512 && ncols % FmtF16::TILE == 0 && (size_t)ncols * 4 <= kMaxLds;
+}
+static int dense_format(const wgml_qmat *m) { return m->half ? kFusedDenseF16 : kFusedDenseF32; }
+
 bool gemv_partials_supported(const wgml_ctx *, const wgml_qmat *m) {
     return m && (m->type == WGML_Q4_K || m->type == WGML_Q6_K || m->type == WGML_Q8_0);
 }
@@ -381,7 +388,7 @@ static int launch_full(wgml_ctx *ctx, const wgml_qmat *m, const GemvParams &p, u
     if (lds > kMaxLds)
         return set_error(WGML_E_UNSUPPORTED, "gemv_quant: %u columns need %zu bytes of LDS (limit %zu)", p.ncols, lds,
                          kMaxLds);
-    const int fmt = m->type == WGML_F32 ? kFusedDenseF32
+    const int fmt = m->type == WGML_F32 ? dense_format(m)
                     : legacy_format(m->type) ? legacy_kernel_format(m->type, p.ncols)
                                              : m->type;
     const int rows = m->type == WGML_Q8_0 && !f32 ? rows_per_wave_q8(p) : 1;
@@ -414,10 +421,10 @@ static const void *maxima_kernel_for(const wgml_ctx *ctx, const wgml_qmat *m, co
         default: break;
         }
     }
-    return gemv_maxima_kernel(dense                     ? kFusedDenseF32
+    return gemv_maxima_kernel(dense                     ? dense_format(m)
                               : legacy_format(m->type) ? legacy_kernel_format(m->type, p.ncols)
                                                        : m->type,
-                              f32, (int)*rows);
+                              f32);
 }
 
 int launch_gemv_quant(wgml_ctx *ctx, float *out, const wgml_qmat *m, const float *v,
@@ -466,6 +473,7 @@ int launch_gemv_quant(wgml_ctx *ctx, float *out, const wgml_qmat *m, const float
         if (const void *fn = maxima_kernel_for(ctx, m, p, &rows, &lds))
             return launch_plain(ctx, fn, rows, 1024, p, lds, ep.n_maxima);
     }
+    if (m->half) return launch_plain(ctx, gemv_f16_kernels().plain, 1, 1024, p, lds_bytes_of<FFmt<FmtF16>>(p.ncols));
     if (dense_f32_in_shared_body(m) && !dense_f32_general_faster(ctx, p.nrows, p.ncols, p.norm_w != nullptr))
         return launch_dense_f32(ctx, p);
     if (m->type == WGML_F32) {
@@ -518,7 +526,7 @@ bool gemv_fused_set_supported(const wgml_ctx *ctx, const wgml_qmat *const *mats,
     bool same = true, all_main = true;
     for (int i = 0; i < n; ++i) {
         if (!gemv_fused_supported(mats[i])) return false;
-        same = same && mats[i]->type == mats[0]->type;
+        same = same && mats[i]->type == mats[0]->type && mats[i]->half == mats[0]->half;
         all_main = all_main && main_format(mats[i]->type);
     }
     if (ctx->tuning[WGML_TUNE_GEMV_F32_ACTIVATIONS]) return all_main || (same && mats[0]->type == WGML_F32);
@@ -530,10 +538,11 @@ static int fused_format(const FusedGemv &f, uint32_t ncols) {
     const int type = f.jobs[0].a->type;
     for (int i = 1; i < f.njobs; ++i)
         if (f.jobs[i].a->type != type) return 0;
-    return type == WGML_F32 ? kFusedDenseF32 : legacy_format(type) ? legacy_kernel_format(type, ncols) : type;
+    return type == WGML_F32 ? dense_format(f.jobs[0].a) : legacy_format(type) ? legacy_kernel_format(type, ncols) : type;
 }
 static GemvKernels fused_kernels(int fmt, bool f32) {
     if (fmt == kFusedDenseF32) return dense_f32_kernels();
+    if (fmt == kFusedDenseF16) return gemv_f16_kernels();
     if (f32) {
         switch (fmt) {
         case WGML_Q4_K: return gemv_kernels_of<WGML_Q4_K, true, false>();
@@ -572,7 +581,7 @@ static uint32_t fused_workgroups(const wgml_ctx *ctx, int per_cu, uint64_t bytes
 static int launch_gated(wgml_ctx *ctx, const FusedGemv &f, const FusedGemvJob &s, uint32_t threads) {
     const uint32_t ncols = s.a->ncols;
     const bool f32 = ctx->tuning[WGML_TUNE_GEMV_F32_ACTIVATIONS] != 0;
-    if (!s.b || s.b->type != s.a->type || s.b->nrows != s.a->nrows || s.b->ncols != ncols || s.row0 || s.nrows)
+    if (!s.b || s.b->type != s.a->type || s.b->half != s.a->half || s.b->nrows != s.a->nrows || s.b->ncols != ncols || s.row0 || s.nrows)
         return set_error(WGML_E_INVALID, "gemv_fused: gate/up matrices differ");
     if (f.ln_gamma) return set_error(WGML_E_UNSUPPORTED, "gemv_fused: a gated job behind a LayerNorm");
     FusedGemv one = f;
@@ -629,7 +638,7 @@ static int launch_jobs(wgml_ctx *ctx, const FusedGemv &f, uint32_t threads) {
                 return set_error(WGML_E_INVALID, "gemv_fused: job %d: bad row slice", i);
             const uint64_t r = s.row0, nb = r * (ncols / 256), nb32 = r * (ncols / 32);
             switch (s.a->type) {
-            case WGML_F32: j.a0 += r * ncols * 4; break;
+            case WGML_F32: j.a0 += r * ncols * (s.a->half ? 2 : 4); break;
             case WGML_Q4_K: j.a0 += nb * 144; break;
             case WGML_Q5_K: j.a0 += nb * 176; break;
             case WGML_Q8_K: j.a0 += nb * 292; break;
@@ -660,11 +669,12 @@ static int launch_jobs(wgml_ctx *ctx, const FusedGemv &f, uint32_t threads) {
     const int fmt = fused_format(f, ncols);
     // (heads of two elements: both RoPE variants rotate the same pairs)
     const bool neox = f.rope_neox && P.head_size > 2;
-    if (neox && (f32 || fmt == kFusedDenseF32))
+    const bool dense = fmt == kFusedDenseF32 || fmt == kFusedDenseF16;
+    if (neox && (f32 || dense))
         return set_error(WGML_E_UNSUPPORTED, "gemv_fused: Neox RoPE takes the integer-dot formats only");
     if (P.ln_g && (neox || fmt == 0))
         return set_error(WGML_E_UNSUPPORTED, "gemv_fused: LayerNorm before Neox RoPE or mixed formats");
-    const GemvKernels k = P.ln_g ? gemv_full_kernels(fmt, f32 || fmt == kFusedDenseF32, 1) : fused_kernels(fmt, f32);
+    const GemvKernels k = P.ln_g ? gemv_full_kernels(fmt, f32 || dense, 1) : fused_kernels(fmt, f32);
     const void *const kern = neox ? gemv_neox_kernel(fmt, (int)threads) : threads == 768 ? k.fused768 : k.fused1024;
     int per_cu = 1;
     WGML_TRY(blocks_per_cu(ctx, kern, (int)threads, lds, &per_cu));
@@ -725,7 +735,7 @@ int launch_gemv_fused(wgml_ctx *ctx, const FusedGemv &f) {
             return set_error(WGML_E_UNSUPPORTED, "gemv_fused: fp32 activations exist for Q4_K, Q6_K "
                                                  "and Q8_0 only");
         gated = gated || s.mode == FUSED_SILU;
-        mixed = mixed || s.a->type != f.jobs[0].a->type;
+        mixed = mixed || s.a->type != f.jobs[0].a->type || s.a->half != f.jobs[0].a->half;
         all_main = all_main && main_format(s.a->type);
         const uint32_t rows = s.nrows ? s.nrows : s.a->nrows - s.row0;
         pairs += s.mode == FUSED_SILU ? rows : (rows + 1) / 2;

@@ -7,6 +7,7 @@ GemvKernels wgml::gemv_full_kernels(int fmt, bool f32, int rows) {
         case WGML_Q4_K: return gemv_kernels_of<WGML_Q4_K, true, true>();
         case WGML_Q6_K: return gemv_kernels_of<WGML_Q6_K, true, true>();
         case WGML_Q8_0: return gemv_kernels_of<WGML_Q8_0, true, true>();
+        case kFusedDenseF16: return gemv_kernels_of<kFusedDenseF16, true, true>();
         default: return gemv_kernels_of<kFusedDenseF32, true, true>();
         }
     }

