@@ -614,16 +614,27 @@ __global__ __launch_bounds__(256) void attn_rows_kernel(const AttnRowsArgs a) {
 //   online softmax per token: maximum and sum over the lane's 4 rows and the 4 lane groups;
 //   O^T[dim][token] += V^T · P^T : A = V^T (lane n = dimension 16 b + n, k-slot g = row 4 g + i
 //                     in step i), B = the lane's own P values -- no transposition anywhere.
+// Both operands are loaded as they lie in memory.  A row of K belongs to lanes n, n + 16, ..., and loads in that order are 64
+// pieces of 16 bytes: a wave brings its block in whole rows and turns it in LDS, in a place of its own (no barriers; KS keeps
+// the sixteen rows of a read on different banks).  The products of PV take their dimensions so that a lane's are neighbours: one
+// load of V for four products.  V is requested before the scores, the next block of K behind them.  us per launch, both in
+// operand order -> so: 1000 tokens, 32 heads of 128 140 -> 106; 200 behind 1900 130 -> 92; 401 behind 1500 (32 heads of 64)
+// 93 -> 80; 700 behind 100 (20 of 96) 50 -> 41; 128 9.5 -> 8.7; in eight waves 45 behind 300 17.9 -> 13.5, 21 behind 600 (24
+// heads) 25 -> 18.5.  Bound by the fp32 MFMAs, 57 of those 106 us, and by a wave's vector instructions beside them.
+// Three waves per SIMD, or four where the registers of a smaller head let them: 106 us, with two 117.
 // WAVES 4: several workgroups fit a compute unit and cover each other's waits.  WAVES 8, where there are fewer
-// workgroups than compute units (a short run behind a long context): twice the waves share the cache rows,
-// and a wave requests its next block of them before it multiplies one (21 tokens behind 600, 24 heads of 128:
-// 39 -> 25 us; 45 behind 300, 32 heads: 24.5 -> 18; with 256 workgroups 9.8 us with four waves, 11.3 with eight).
+// workgroups than compute units (a short run behind a long context): twice the waves share the cache rows.
 template <int HS16, int WAVES>
-__global__ __launch_bounds__(WAVES * 64) void attn_block_kernel(const AttnRowsArgs a, uint32_t T) {
-    constexpr int HS = HS16 * 16;
-    __shared__ float sm_m[4][16], sm_l[4][16];
-    __shared__ float sm_o[4][HS][17];
-    const uint32_t h = blockIdx.x, t0 = blockIdx.y * 16;
+__global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(HS16 > 5 ? 3 : 4))) void attn_block_kernel(const AttnRowsArgs a, uint32_t T) {
+    constexpr int HS = HS16 * 16, KS = HS + 4;                      // KS: floats of a staged row of K
+    constexpr int VW = HS16 % 4 == 0 ? 4 : HS16 % 2 == 0 ? 2 : 1;  // floats of V per load
+    constexpr int STAGE = 16 * KS, MERGE = HS * 17, PER_WAVE = STAGE > MERGE ? STAGE : MERGE;
+    typedef float vrow_t __attribute__((ext_vector_type(VW)));
+    __shared__ float sm_m[WAVES][16], sm_l[WAVES][16];
+    __shared__ __attribute__((aligned(16))) float sm[WAVES][PER_WAVE];  // a wave's block of K, then its results
+    // the heads in eight groups, one on each XCD, and the longest workgroups first
+    const uint32_t h = gridDim.x % 8 ? blockIdx.x : (blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8;
+    const uint32_t t0 = (gridDim.y - 1 - blockIdx.y) * 16;
     const uint32_t lane = threadIdx.x & 63;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const uint32_t n = lane & 15, g = lane >> 4;
@@ -633,6 +644,31 @@ __global__ __launch_bounds__(WAVES * 64) void attn_block_kernel(const AttnRowsAr
     const uint32_t tq = min(t0 + n, T - 1), pos_q = a.pos0 + tq;
     const uint32_t last_pos = a.pos0 + min(t0 + 15, T - 1);  // rows 0 .. last_pos exist
     const uint32_t nblk = last_pos / 16 + 1;
+    const uint32_t kv_bytes = a.kv_dim * 4;
+    // a block of K as it lies in memory: 16-byte word 64 c + lane of its 16 rows
+    floatx4 k[HS16];
+    auto load_k = [&](uint32_t blk) {  // rows past the end repeat the last one and do not count
+        const char *base = reinterpret_cast<const char *>(a.kc + (size_t)blk * 16 * a.kv_dim + head_off);
+        const uint32_t last = last_pos - blk * 16;
+#pragma unroll
+        for (int c = 0; c < HS16; ++c) {
+            const uint32_t w = 64 * c + lane, row = w / (HS / 4), col = w % (HS / 4) * 16;
+            k[c] = *reinterpret_cast<const floatx4 *>(base + (min(row, last) * kv_bytes + col));
+        }
+    };
+    // V^T: lane n has VW neighbouring dimensions of row 4 g + i, one for each of VW products
+    vrow_t v[HS16 / VW][4];
+    auto load_v = [&](uint32_t blk) {
+        const char *base = reinterpret_cast<const char *>(a.vc + (size_t)blk * 16 * a.kv_dim + head_off);
+        const uint32_t last = last_pos - blk * 16;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t at = min(4 * g + i, last) * kv_bytes + 4 * VW * n;
+#pragma unroll
+            for (int j = 0; j < HS16 / VW; ++j) v[j][i] = *reinterpret_cast<const vrow_t *>(base + at + 64 * VW * j);
+        }
+    };
+    load_k(min(wave, nblk - 1));
     float4 q[HS16];
 #pragma unroll
     for (int c = 0; c < HS16; ++c)
@@ -641,35 +677,30 @@ __global__ __launch_bounds__(WAVES * 64) void attn_block_kernel(const AttnRowsAr
 #pragma unroll
     for (int b = 0; b < HS16; ++b) acc[b] = floatx4{0.f, 0.f, 0.f, 0.f};
     float m = -INFINITY, l = 0.f;
-    struct Rows {
-        float4 k[HS16];
-        float v[HS16][4];
-    };
-    auto load = [&](Rows &r, uint32_t blk) {  // rows past the end repeat the last one and do not count
+    for (uint32_t blk = wave; blk < nblk; blk += WAVES) {  // uniform over the wave
         const uint32_t pbase = blk * 16;
-        const float *krow = a.kc + (size_t)min(pbase + n, last_pos) * a.kv_dim + head_off + 4 * g;
 #pragma unroll
-        for (int c = 0; c < HS16; ++c) r.k[c] = *reinterpret_cast<const float4 *>(krow + 16 * c);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const float *vrow = a.vc + (size_t)min(pbase + 4 * g + i, last_pos) * a.kv_dim + head_off + n;
-#pragma unroll
-            for (int b = 0; b < HS16; ++b) r.v[b][i] = vrow[16 * b];
+        for (int c = 0; c < HS16; ++c) {
+            const uint32_t w = 64 * c + lane, row = w / (HS / 4), col = w % (HS / 4) * 4;
+            *reinterpret_cast<floatx4 *>(&sm[wave][row * KS + col]) = k[c];
         }
-    };
-    constexpr bool AHEAD = WAVES == 8;
-    auto step = [&](const Rows &r, uint32_t blk) {
-        const uint32_t pbase = blk * 16;
-        const float4(&k)[HS16] = r.k;
-        const float(&v)[HS16][4] = r.v;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");  // (the wave's own rows: no barrier)
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        load_v(blk);
+        __builtin_amdgcn_sched_barrier(0);  // requested before the products, not between them
         floatx4 s = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int c = 0; c < HS16; ++c) {
-            s = __builtin_amdgcn_mfma_f32_16x16x4f32(k[c].x, q[c].x, s, 0, 0, 0);
-            s = __builtin_amdgcn_mfma_f32_16x16x4f32(k[c].y, q[c].y, s, 0, 0, 0);
-            s = __builtin_amdgcn_mfma_f32_16x16x4f32(k[c].z, q[c].z, s, 0, 0, 0);
-            s = __builtin_amdgcn_mfma_f32_16x16x4f32(k[c].w, q[c].w, s, 0, 0, 0);
+            const float4 kf = *reinterpret_cast<const float4 *>(&sm[wave][n * KS + 16 * c + 4 * g]);
+            s = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.x, q[c].x, s, 0, 0, 0);
+            s = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.y, q[c].y, s, 0, 0, 0);
+            s = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.z, q[c].z, s, 0, 0, 0);
+            s = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.w, q[c].w, s, 0, 0, 0);
         }
+        __builtin_amdgcn_sched_barrier(0);
+        load_k(min(blk + WAVES, nblk - 1));
+        __builtin_amdgcn_sched_barrier(0);
         // s[i] = score of row pbase + 4 g + i for token n; rows after the token's position do not count
         float sc[4], mloc = -INFINITY;
 #pragma unroll
@@ -695,58 +726,43 @@ __global__ __launch_bounds__(WAVES * 64) void attn_block_kernel(const AttnRowsAr
         for (int b = 0; b < HS16; ++b) {
             acc[b] = floatx4{acc[b][0] * scale, acc[b][1] * scale, acc[b][2] * scale, acc[b][3] * scale};
 #pragma unroll
-            for (int i = 0; i < 4; ++i) acc[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[b][i], p[i], acc[b], 0, 0, 0);
+            for (int i = 0; i < 4; ++i)
+                acc[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[b / VW][i][b % VW], p[i], acc[b], 0, 0, 0);
         }
-    };
-    if (AHEAD) {
-        Rows r0, r1;
-        if (wave < nblk) load(r0, wave);
-        for (uint32_t blk = wave; blk < nblk; blk += 2 * WAVES) {  // uniform over the wave
-            load(r1, blk + WAVES);
-            __builtin_amdgcn_sched_barrier(0);  // requested before the products, not between them
-            step(r0, blk);
-            if (blk + WAVES >= nblk) break;
-            load(r0, blk + 2 * WAVES);
-            __builtin_amdgcn_sched_barrier(0);
-            step(r1, blk + WAVES);
-        }
-    } else {
-        for (uint32_t blk = wave; blk < nblk; blk += WAVES) {
-            Rows r;
-            load(r, blk);
-            step(r, blk);
-        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
     }
-    // acc[b][i] = O^T[dimension 16 b + 4 g + i][token n] of this wave's rows; merge the waves, eight of
+    // acc[b][i] = O^T[dimension dim(b, i)][token n] of this wave's rows; merge the waves, eight of
     // them in two steps (wave w takes up wave w + 4 first)
-    auto leave = [&](uint32_t w) {
+    auto dim = [&](int b, int i) { return 16 * VW * (b / VW) + VW * (4 * g + i) + b % VW; };
+    auto leave = [&]() {
         if (g == 0) {
-            sm_m[w][n] = m;
-            sm_l[w][n] = l;
+            sm_m[wave][n] = m;
+            sm_l[wave][n] = l;
         }
 #pragma unroll
         for (int b = 0; b < HS16; ++b) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) sm_o[w][16 * b + 4 * g + i][n] = acc[b][i];
+            for (int i = 0; i < 4; ++i) sm[wave][dim(b, i) * 17 + n] = acc[b][i];
         }
     };
     if (WAVES == 8) {
-        if (wave >= 4) leave(wave - 4);
+        if (wave >= 4) leave();
         __syncthreads();
         if (wave < 4) {
-            const float m2 = sm_m[wave][n], l2 = sm_l[wave][n], mn = fmaxf(m, m2);
+            const float m2 = sm_m[wave + 4][n], l2 = sm_l[wave + 4][n], mn = fmaxf(m, m2);
             const float s1 = m == -INFINITY ? 0.f : __expf(m - mn), s2 = m2 == -INFINITY ? 0.f : __expf(m2 - mn);
 #pragma unroll
             for (int b = 0; b < HS16; ++b) {
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
-                    acc[b][i] = fmaf(acc[b][i], s1, sm_o[wave][16 * b + 4 * g + i][n] * s2);
+                    acc[b][i] = fmaf(acc[b][i], s1, sm[wave + 4][dim(b, i) * 17 + n] * s2);
             }
             l = fmaf(l, s1, l2 * s2);
             m = mn;
         }
     }
-    if (wave < 4) leave(wave);
+    if (wave < 4) leave();
     __syncthreads();
     for (uint32_t idx = threadIdx.x; idx < 16 * HS; idx += WAVES * 64) {
         const uint32_t tok = idx / HS, d = idx % HS;
@@ -757,7 +773,7 @@ __global__ __launch_bounds__(WAVES * 64) void attn_block_kernel(const AttnRowsAr
         for (int w = 0; w < 4; ++w) {
             const float wgt = sm_m[w][tok] == -INFINITY ? 0.f : __expf(sm_m[w][tok] - M);
             L = fmaf(sm_l[w][tok], wgt, L);
-            o = fmaf(sm_o[w][d][tok], wgt, o);
+            o = fmaf(sm[w][d * 17 + tok], wgt, o);
         }
         a.xb[(size_t)(t0 + tok) * a.xb_stride + (size_t)h * HS + d] = o / L;
     }
