@@ -16,7 +16,7 @@ multiply the quantized weights with activations rounded to 16-bit block fixed
 point on the integer dot-product units and accumulate in i32 / f32) with the
 same decode on fp32 activations beside it; the logit error of the GPU step
 against the CPU oracle on the positions the CPU baseline runs; the HBM roofline
-of the dominant kernel (gemv_fused_kernel as launched for the gate/up
+of the dominant kernel (gemv_gated_kernel as launched for the gate/up
 projections) measured with HIP events on the library's own stream, launch by
 launch as rocprofv3 sees it, and inside a recorded graph as the decode loop
 runs it; a GEMV sweep over the model's four matrix shapes for the three
@@ -544,7 +544,7 @@ def main():
         for _ in range(3):
             W.OpAssign(gpu, W.OpAssignVariant.Copy).dispatch(dst, src)
         gpu.synchronize()
-        print(json.dumps({"kernel": "gemv_fused_kernel gate+up", "us_per_launch": round(us, 3),
+        print(json.dumps({"kernel": "gemv_gated_kernel gate+up", "us_per_launch": round(us, 3),
                           "bytes_per_launch": b, "GB/s": round(b / us * 1e-3, 1),
                           "calibration": "op_assign Copy of 67108864 f32: 268435456 B read, "
                                          "268435456 B written per launch"}), flush=True)
@@ -708,7 +708,7 @@ def main():
                     "frac": round(gbs / HBM_PEAK_GBS, 4), "traffic": traffic,
                     "achievable": chain,
                     "traffic_source": traffic_src,
-                    "kernel": "gemv_fused_kernel, gate+up launch: 2 x Q4_K 11008x4096, RMSNorm "
+                    "kernel": "gemv_gated_kernel, gate+up launch: 2 x Q4_K 11008x4096, RMSNorm "
                               "folded into staging, SiLU epilogue",
                     "bytes_per_launch": b, "us_per_launch": round(us_eager, 3),
                     "timing": "HIP events around back-to-back launches on the library's stream, "
@@ -719,7 +719,7 @@ def main():
                     "plain_gemv_q4_k_11008x4096_in_graph": {"us_per_launch": round(us1, 3),
                                                             "bytes_per_launch": b1,
                                                             "GB/s": round(b1 / us1 * 1e-3, 1)}}
-        log(f"dominant kernel gemv_fused_kernel gate+up: {us_eager:.2f} us launch by launch "
+        log(f"dominant kernel gemv_gated_kernel gate+up: {us_eager:.2f} us launch by launch "
             f"({gbs:.0f} GB/s), {us_graph:.2f} us in a graph; plain Q4_K gemv 11008x4096: "
             f"{us1:.2f} us, {b1 / us1 * 1e-3:.0f} GB/s")
 
