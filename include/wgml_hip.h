@@ -100,8 +100,9 @@ enum {
     WGML_TUNE_GEMM_K_SPLIT,                  /* 1..8 workgroups share the K range of a batched product */
     WGML_TUNE_PREFILL_ATTENTION_PER_TOKEN,   /* 1: one workgroup per (head, token) in the prompt pass */
     WGML_TUNE_ATTN_WIDE_POSITIONS,           /* decode attention planned for up to this many positions
-                                                (at most 2^20) runs as one workgroup per head group,
-                                                without partial results */
+                                                (at most 2^20) runs without partial results, as one
+                                                workgroup per head, two per head or one per two heads that
+                                                share a KV head */
     WGML_TUNE_ATTN_SPLITS,                   /* workgroups that share the positions of a head group, 2..64 */
     WGML_TUNE_ATTN_MERGE,                    /* attention followed by a quantized GEMV on its output
                                                 (wgml_attention_gemv_quant, the decoders' layers): 1 = the

@@ -11,6 +11,7 @@ enum { MAX_FUNCTIONS = 4096, MAX_LAUNCHES = 1 << 16, MAX_BLOCKS = 1 << 14 };
 static struct { const void *fn; const char *name; } functions[MAX_FUNCTIONS];
 static int n_functions;
 static const char *launches[MAX_LAUNCHES];
+static dim3 grids[MAX_LAUNCHES];
 static int n_launches;
 static struct { void *p; size_t bytes; } blocks[MAX_BLOCKS];
 static int n_blocks, n_pinned;
@@ -25,6 +26,7 @@ void host_hip_fail_kernel(const char *part) { strncpy(failing, part, sizeof(fail
 void host_hip_clear(void) { n_launches = 0; }
 int host_hip_launches(void) { return n_launches; }
 const char *host_hip_launch(int i) { return launches[i]; }
+unsigned host_hip_workgroups(int i) { return grids[i].x * grids[i].y * grids[i].z; }
 size_t host_hip_allocated(void) { return allocated; }
 int host_hip_pinned(void) { return n_pinned; } /* requests for pinned memory so far */
 
@@ -62,7 +64,10 @@ hipError_t hipLaunchKernel(const void *fn, dim3 grid, dim3 block, void **args, s
     if (failing[0] && strstr(name, failing)) return done(hipErrorLaunchFailure);
     if (!grid.x || !grid.y || !grid.z || !block.x || block.x * block.y * block.z > 1024 || lds > 160 * 1024)
         return done(hipErrorInvalidConfiguration);
-    if (n_launches < MAX_LAUNCHES) launches[n_launches++] = name;
+    if (n_launches < MAX_LAUNCHES) {
+        launches[n_launches] = name;
+        grids[n_launches++] = grid;
+    }
     return hipSuccess;
 }
 hipError_t hipFuncSetAttribute(const void *f, hipFuncAttribute a, int v) { (void)f; (void)a; (void)v; return hipSuccess; }

@@ -28,6 +28,10 @@ def launched(call):
     call()
     return [fake.host_hip_launch(i).decode() for i in range(fake.host_hip_launches())]
 
+def workgroups(call):
+    "of each kernel that `call` launches"
+    return [fake.host_hip_workgroups(i) for i in range(len(launched(call)))]
+
 def count(names, part):
     return sum(part in n for n in names)
 

@@ -1,5 +1,5 @@
-"""GPU: short contexts in one workgroup per head, or per head and slice of the value dimensions (heads of more than 64): head sizes whose
-slices are uneven, every place of a position in a quad and a round of 64, grouped heads, and an output that lies on the query.
+"""GPU: short contexts in one workgroup per head, per head and slice of the value dimensions (heads of more than 64) or, with many heads,
+per two heads: head sizes whose slices are uneven, every place of a position in a quad and a round of 64, grouped heads, and an output that lies on the query.
 
 Bound: scores and sums are fp32 over at most 256 positions and 128 dimensions; 2e-5 of the largest result is about four times what is
 observed."""
@@ -31,9 +31,23 @@ def test_short_contexts(gpu, n_heads, kv_mul, hs, pos, same):
     q = rng.standard_normal(n_heads * hs).astype(np.float32)
     k, v = (rng.standard_normal((256, kv_dim)).astype(np.float32) for _ in range(2))
     k[pos + 1:], v[pos + 1:] = np.nan, np.nan  # rows beyond the position may be read, not used
+    run(gpu, n_heads, kv_mul, hs, pos, same, q, k, v)
+
+
+@pytest.mark.parametrize("n_heads,kv_mul,hs", [(129, 3, 128), (160, 1, 68), (130, 2, 128), (162, 6, 72), (256, 8, 100), (256, 4, 64),
+                                               (256, 256, 4), (270, 5, 64)])
+@pytest.mark.parametrize("pos", [0, 3, 64, 130, 255])
+def test_more_heads_than_compute_units_take_in_slices(gpu, n_heads, kv_mul, hs, pos):
+    rng = np.random.default_rng(n_heads + pos)
+    k, v = (rng.standard_normal((256, n_heads // kv_mul * hs)).astype(np.float32) for _ in range(2))
+    k[pos + 1:], v[pos + 1:] = np.nan, np.nan
+    run(gpu, n_heads, kv_mul, hs, pos, pos % 2 == 1, rng.standard_normal(n_heads * hs).astype(np.float32), k, v)
+
+
+def run(gpu, n_heads, kv_mul, hs, pos, same, q, k, v):
     qv = W.GpuVector.init(gpu, q)
     out = qv if same else W.GpuVector.uninit(gpu, n_heads * hs)
-    p = W.BatchedMultiqueryAttentionParams(256, kv_dim, kv_mul, n_heads, hs, pos)
+    p = W.BatchedMultiqueryAttentionParams(256, k.shape[1], kv_mul, n_heads, hs, pos)
     W.BatchedMultiqueryAttention.from_device(gpu).dispatch_multi(p, qv, W.GpuMatrix.init(gpu, k), W.GpuMatrix.init(gpu, v), out)
     ref = reference(q, k, v, n_heads, kv_mul, hs, pos)
     assert np.abs(out.read() - ref).max() <= 2e-5 * np.abs(ref).max()

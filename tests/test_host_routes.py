@@ -188,3 +188,22 @@ def test_longer_prompts_pin_no_new_memory(runtime):
         assert m.generate_sampled(np.zeros(n, np.uint32), n + 9, 0.7, 0.9, 1).size == n + 9
     assert fake.host_hip_pinned() == before + 1
     """)
+
+
+def test_short_contexts_share_the_compute_units_out(runtime):
+    # two slices per head while all have a compute unit (256), then one workgroup per head, or per two that share rows
+    host_hip.run(runtime, """
+    def attention(n_heads, kv_mul, hs):
+        kv_dim = n_heads // kv_mul * hs
+        q, out = W.GpuVector.uninit(gpu, n_heads * hs), W.GpuVector.uninit(gpu, n_heads * hs)
+        k, v = (W.GpuMatrix.init(gpu, np.zeros((256, kv_dim), np.float32)) for _ in range(2))
+        p = W.BatchedMultiqueryAttentionParams(256, kv_dim, kv_mul, n_heads, hs, 40)
+        run = lambda: W.BatchedMultiqueryAttention.from_device(gpu).dispatch_multi(p, q, k, v, out)
+        assert count(launched(run), "attn_fast_kernel") == 1
+        return workgroups(run)[0]
+
+    for n_heads, kv_mul, hs, want in ((32, 1, 128, 64), (128, 8, 128, 256), (129, 3, 128, 129), (130, 1, 68, 130), (132, 4, 68, 66),
+                                      (160, 8, 128, 80), (129, 3, 68, 129), (192, 6, 96, 96), (192, 3, 128, 192), (256, 8, 128, 128), (12, 1, 64, 12),
+                                      (252, 4, 64, 252), (256, 4, 64, 128), (255, 5, 64, 255), (300, 1, 64, 300)):
+        assert attention(n_heads, kv_mul, hs) == want, (n_heads, kv_mul, hs)
+    """)

@@ -314,8 +314,7 @@ __device__ __forceinline__ float4 axpby4(const float4 a, float sa, const float4 
 //
 // SLICED (one workgroup per head and slice, blockIdx.y the slice, no partial results): a workgroup reads all of K, but weighs only
 // its slice of V's dimensions (a.slice_f4 float4 of a row, one per lane).  One compute unit takes about 30 GB/s whatever is
-// in flight, so a head's rows are what a short context waits for, and these are three quarters of them.  Query heads that share
-// a KV head read its rows again, each on compute units of its own.  Quarters of a wave meet by lane swaps (with two rounds of
+// in flight, so a head's rows are what a short context waits for, and these are three quarters of them.  Quarters of a wave meet by lane swaps (with two rounds of
 // ds_bpermute per value the 16 waves' merges were a sixth of the launch), and the waves' weights are made one per lane.
 // us per layer, one workgroup per head group, bpermutes -> now: 32 heads of 128 at position 150 5.14 -> 4.45, at 250 7.69 -> 6.1, at
 // 20 4.21 -> 3.30; 8 KV heads x 4 at 150 6.51 -> 4.06; 4 x 4 at 25 4.94 -> 3.12; 12 heads of 64 at 150 3.97 -> 3.71.  With partial
@@ -579,8 +578,8 @@ int launch_nv(wgml_ctx *ctx, const AttnArgs &a, int km, dim3 grid) {
 template <int NV4, int NW>
 int launch_fast_nv(wgml_ctx *ctx, const AttnArgs &a, int km, dim3 grid) {
     const dim3 block(NW * 64);
-    // the planner keeps km * NV4 within the register budget of the variant (16 waves: one head)
-    constexpr int kMaxKmNv = NW == 16 ? NV4 : 8;
+    // the planner keeps km * NV4 within the register budget of the variant (16 waves: two heads at most)
+    constexpr int kMaxKmNv = NW == 16 ? 2 * NV4 : 8;
     if (km * NV4 > kMaxKmNv)
         return set_error(WGML_E_INVALID, "attention: no kernel for km %d, %d float4 per lane", km,
                          NV4);
@@ -619,7 +618,8 @@ namespace wgml {
 struct AttnPlan {
     int nv, km;
     uint32_t groups, chunk, n_wg_y, hsp;
-    int wide;  // fast plan: one 16-wave workgroup per head group, no partials
+    int wide;  // fast plan: 16-wave workgroups, no partials
+    int slices;  // wide: workgroups that share the value dimensions of a head
 };
 
 // The fast kernel needs float4-addressable heads; `aligned` says that q and the
@@ -629,7 +629,7 @@ static bool fast_ok(const wgml_attn_params &p, bool aligned, bool wants_scores) 
            p.head_size <= 256;
 }
 
-constexpr uint32_t kWidePositions = 256;  // up to here one workgroup per head group
+constexpr uint32_t kWidePositions = 256;  // up to here no partial results
 // the most partial results per head that a consumer merges while it stages its input
 // (launch_gemv_quant with GemvEpilogue::partials)
 constexpr uint32_t kMaxFoldedPartials = 16;
@@ -646,7 +646,20 @@ static int make_fast_plan(wgml_ctx *ctx, const wgml_attn_params &p, uint32_t pla
     pl.km = 1;
     if (p.kv_mul == 2 || p.kv_mul == 4) pl.km = (int)p.kv_mul;
     if (p.kv_mul == 8) pl.km = 4;
-    if (pl.wide) pl.km = 1;  // (query heads that share a KV head read its rows again, on other compute units)
+    pl.slices = 1;
+    const uint32_t cu = ctx->n_cu > 0 ? (uint32_t)ctx->n_cu : 256u;
+    if (pl.wide) {
+        // A compute unit's share of the rows is what such a launch waits for.  Two slices of a head while all workgroups get a
+        // compute unit of their own (128 heads of 128 at position 250: 7.0 us, one workgroup per head 7.2; 130 heads 11.0 and
+        // 7.4); four and eight are no faster.  Query heads that share a KV head read its rows again, on other compute units, as
+        // long as there are enough of these, and two of them share a workgroup beyond.  us at positions 20 / 120 / 250, one by one and in
+        // twos: 160 heads of 128 in groups of 8 4.3 / 6.0 / 8.7 and 4.7 / 6.3 / 7.9, 256 heads 4.9 / 7.3 / 11.6 and 5.0 / 6.4 / 8.5
+        // (in slices 5.0 / 7.2 / 13.6); heads of 64: 256 of them 3.7 / 5.0 / 7.1 and 3.8 / 5.0 / 6.2, 224 3.6 / 4.8 / 6.6 one by one.
+        // Fours are slower than twos up to 512 heads.
+        const bool many = pl.nv == 2 ? p.n_heads > cu / 2 : p.n_heads >= cu;
+        pl.km = many && p.kv_mul % 2 == 0 ? 2 : 1;
+        if (pl.nv == 2 && !many) pl.slices = 2;
+    }
     // register budget (q and acc are km * nv float4 each): 256 VGPRs
     while (pl.km > 1 && pl.km * pl.nv > 8) pl.km >>= 1;
     pl.groups = p.n_heads / pl.km;
@@ -656,7 +669,6 @@ static int make_fast_plan(wgml_ctx *ctx, const wgml_attn_params &p, uint32_t pla
         pl.n_wg_y = 1;
         return WGML_OK;
     }
-    const uint32_t cu = ctx->n_cu > 0 ? (uint32_t)ctx->n_cu : 256u;
     // about two workgroups per CU, each with at least 64 positions at full length (four
     // quads per wave; measured on 32 x 128 and 12 x 64 heads, shorter shares only add
     // partial results for the merge to read) -- or 32 positions while that keeps the partial
@@ -777,11 +789,10 @@ int launch_attention_planned(wgml_ctx *ctx, const wgml_attn_params &p, DynPos po
         a.spec_rows = cache_rows;
         const dim3 grid(pl.groups, pl.n_wg_y);
         if (pl.wide) {
-            // Heads of more than 64 dimensions in two slices (four and eight are no faster).  One slice of a head is written
-            // while the other may still read its q: not where these overlap.
+            // One slice of a head is written while the other may still read its q: not where these overlap.
             const size_t dim = (size_t)p.n_heads * p.head_size;
             const bool apart = (uintptr_t)(q + dim) <= (uintptr_t)xb || (uintptr_t)(xb + dim) <= (uintptr_t)q;
-            if (pl.nv != 2 || !apart) return launch_fast<16>(ctx, a, pl.nv, pl.km, grid);
+            if (pl.slices == 1 || !apart) return launch_fast<16>(ctx, a, pl.nv, pl.km, grid);
             a.slice_f4 = (p.head_size / 4 + 1) / 2;
             attn_fast_kernel<2, 1, 16, true><<<dim3(p.n_heads, 2), dim3(1024), 0, ctx->stream>>>(a);
             WGML_CHECK_LAUNCH();
