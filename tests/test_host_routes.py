@@ -207,3 +207,19 @@ def test_short_contexts_share_the_compute_units_out(runtime):
                                       (252, 4, 64, 252), (256, 4, 64, 128), (255, 5, 64, 255), (300, 1, 64, 300)):
         assert attention(n_heads, kv_mul, hs) == want, (n_heads, kv_mul, hs)
     """)
+
+
+def test_short_runs_pack_their_tokens_in_order(runtime):
+    # (nothing of the longer runs' order in their kernel)
+    host_hip.run(runtime, """
+    def packing(qtype, n):
+        m = W.GpuQuantMatrix(gpu, qtype, 64, 256, np.zeros(W.quant_bytes(qtype, 64 * 256), np.uint8))
+        out, x = W.GpuVector.uninit(gpu, n * 64), W.GpuVector.uninit(gpu, n * 256)
+        run = lambda: W.GemmQuant.from_device(gpu).dispatch(out, m, x, n)
+        return "prep_x_kernelILi0ELb1E" in launched(run)[0], workgroups(run)[0]
+
+    for n in (1, 17, 63, 64):
+        assert packing(W.Q8_0, n) == packing(W.Q4_K, n) == (True, n)
+    for n in (65, 100, 128):
+        assert packing(W.Q8_0, n) == packing(W.Q4_K, n) == (False, 128)
+    """)

@@ -176,10 +176,12 @@ __device__ __forceinline__ void load8(float (&o)[8], const float *p) {  // 16-by
 // Token of workgroup w.  Eight neighbouring tokens share every 128-byte line of the packed activations (16 bytes each), and
 // workgroup w runs on XCD w % 8: in runs of more than 64 tokens 8 i .. 8 i + 7 go to one XCD, whose L2 then writes whole
 // lines; in the order of the tokens eight L2s write a sixteen-byte piece of each.  us per launch, in order / so: 1000 rows
-// of 4096 to 14336 columns 36 -> 23, 128 rows 8.3 -> 7.7; 45 rows 5.8 / 5.9 (three XCDs have all the work).
+// of 4096 to 14336 columns 36 -> 23, 128 rows 8.3 -> 7.7; 45 rows 5.8 / 5.9 (three XCDs have all the work).  A kernel of its
+// own for each: the order chosen and workgroups beyond T ended at run time cost short runs 0.1 to 0.3 us of 4 to 5.
 constexpr uint32_t kPrepInOrder = 64;
-__device__ __forceinline__ uint32_t prep_token(uint32_t w, uint32_t T) {
-    return T <= kPrepInOrder ? w : w / 64 * 64 + (w & 7) * 8 + (w / 8 & 7);
+template <bool IN_ORDER>
+__device__ __forceinline__ uint32_t prep_token(uint32_t w) {
+    return IN_ORDER ? w : w / 64 * 64 + (w & 7) * 8 + (w / 8 & 7);
 }
 
 constexpr int PREP_THREADS = 1024;
@@ -196,7 +198,7 @@ enum PrepMode { PREP_RMS, PREP_LN, PREP_GELU };
 // largest |x| into (512, 1024]; the factor to undo it goes to xscale[t].  Columns from K on are zero (tokens
 // from T on hold anything: a token's results are its own).  With `up` non-null the input is the gated activation
 // up[k] * silu(x[k]) (ops/silu.wgsl:13-27) instead of x itself (no normalisation then).
-template <int MODE>
+template <int MODE, bool IN_ORDER>
 __global__ __launch_bounds__(PREP_THREADS) void prep_x_kernel(float *__restrict__ x, uint32_t x_stride,
                                                      const float *__restrict__ part, uint32_t part_ks,
                                                      uint32_t part_pair,
@@ -207,8 +209,8 @@ __global__ __launch_bounds__(PREP_THREADS) void prep_x_kernel(float *__restrict_
                                                      float *__restrict__ xscale, uint32_t K,
                                                      uint32_t kpad, uint32_t T, uint32_t nt) {
     __shared__ float red[32];
-    const uint32_t t = prep_token(blockIdx.x, T), tid = threadIdx.x;
-    if (t >= T) return;
+    const uint32_t t = prep_token<IN_ORDER>(blockIdx.x), tid = threadIdx.x;
+    if (!IN_ORDER && t >= T) return;
     // 16-byte word of (token t, columns 8 k8 .. 8 k8 + 7)
     auto word_index = [&](uint32_t k8) {
         const uint32_t c = k8 >> 3, s2 = (k8 >> 2) & 1, g = k8 & 3;
@@ -914,9 +916,12 @@ int launch_prefill_prep(wgml_ctx *ctx, float *x, uint32_t x_stride, const float 
           ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(up)) & 15u) == 0))
         return set_error(WGML_E_INVALID, "prefill_prep: pending gate/up partial sums need a gated row of at "
                                          "most %d columns", 8 * PREP_GROUPS * PREP_THREADS);
-    const auto kernel = ln_beta ? prep_x_kernel<PREP_LN> : gelu ? prep_x_kernel<PREP_GELU> : prep_x_kernel<PREP_RMS>;
+    const bool in_order = T <= kPrepInOrder;
+    const auto kernel = ln_beta ? (in_order ? prep_x_kernel<PREP_LN, true> : prep_x_kernel<PREP_LN, false>)
+                        : gelu  ? (in_order ? prep_x_kernel<PREP_GELU, true> : prep_x_kernel<PREP_GELU, false>)
+                                : (in_order ? prep_x_kernel<PREP_RMS, true> : prep_x_kernel<PREP_RMS, false>);
     // (whole rounds of the eight XCDs, see prep_token; workgroups beyond T end at once)
-    kernel<<<dim3(T <= kPrepInOrder ? T : (T + 63) / 64 * 64), dim3(PREP_THREADS), 0, ctx->stream>>>(
+    kernel<<<dim3(in_order ? T : (T + 63) / 64 * 64), dim3(PREP_THREADS), 0, ctx->stream>>>(
         x, x_stride, pending ? ctx->gemm_part : nullptr, pending, pair, ln_beta ? ln_beta : up, norm_w, eps,
         reinterpret_cast<uint4 *>(xh), ctx->gemm_precise ? reinterpret_cast<uint4 *>(ctx->prefill_xl) : nullptr,
         reinterpret_cast<_Float16 *>(ctx->prefill_xsum), xscale, K, prefill_kpad(K), T, prefill_tpad(T) / 16);
