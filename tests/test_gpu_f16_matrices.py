@@ -80,7 +80,7 @@ def test_gpt2(gpu, dim):
 
 @pytest.mark.parametrize("mixed", [False, True])
 def test_llama(gpu, mixed):
-    """Mixed: F16 beside F32 matrices of the same layer, which no launch takes together (sums in another order then)."""
+    """Mixed: F16 beside F32 matrices of the same layer."""
     cfg = Llama2Config(dim=768, hidden_dim=1280, n_layers=2, n_q_heads=12, n_kv_heads=6, vocab_size=1009, seq_len=64,
                        rope_base_freq=10000.0, rms_norm_eps=1e-5)
     other = lambda k, i: W.F32 if k in ("attn_k", "ffn_up") else W.F16  # noqa: E731
@@ -93,3 +93,16 @@ def test_llama(gpu, mixed):
         assert np.abs(got[0][1] - got[1][1]).max() <= 2e-5 * np.abs(got[1][1]).max()
     else:
         assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1])
+
+
+@pytest.mark.parametrize("f32", [("attn_k", "ffn_up"), ("attn_q", "ffn_gate"), ("attn_k", "attn_v"), ("attn_v",), ("ffn_gate",)])
+@pytest.mark.parametrize("dim,hidden,heads,kv", [(544, 1040, 17, 17), (768, 1280, 12, 6), (1040, 2064, 13, 13)])
+def test_f16_beside_f32_in_one_launch(gpu, f32, dim, hidden, heads, kv):
+    """The values and the order of the sums are those of a layer all in F32."""
+    cfg = Llama2Config(dim=dim, hidden_dim=hidden, n_layers=2, n_q_heads=heads, n_kv_heads=kv, vocab_size=331, seq_len=64,
+                       rope_base_freq=10000.0, rms_norm_eps=1e-5)
+    got = []
+    for of in (lambda k, i: W.F32 if k in f32 else W.F16, lambda k, i: W.F32):
+        m = Llama2(gpu, cfg).load(converted(synth_llama(cfg, 9, "f32"), ["output"], of))
+        got.append((m.decode_greedy(3, 0, 20), m.logits()))
+    assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1])

@@ -223,3 +223,21 @@ def test_short_runs_pack_their_tokens_in_order(runtime):
     for n in (65, 100, 128):
         assert packing(W.Q8_0, n) == packing(W.Q4_K, n) == (False, 128)
     """)
+
+
+def test_f16_beside_f32_takes_no_more_launches(runtime):
+    # a layer that mixes them in Q/K/V or gate/up, at widths where F16 stays 16 bits wide
+    host_hip.run(runtime, """
+    cfg = Llama2Config(768, 2048, 2, 12, 12, 331, 64)
+    def launches(f16):
+        m = llama(gpu, cfg, W.F32)
+        for l in range(cfg.n_layers):
+            for name, (r, k) in {"attn_q": (768, 768), "attn_k": (768, 768), "ffn_gate": (2048, 768), "ffn_up": (2048, 768)}.items():
+                if name in f16:
+                    m.set_matrix(name, l, HostMatrix(W.F16, r, k, np.zeros(2 * r * k, np.uint8)))
+        return launched(lambda: m.forward(0, 0))
+
+    plain = launches(())
+    for f16 in (("attn_q",), ("ffn_up",), ("attn_k", "ffn_gate"), ("attn_q", "attn_k", "ffn_gate", "ffn_up")):
+        assert len(launches(f16)) == len(plain), f16
+    """)

@@ -119,7 +119,7 @@ struct wgml_qmat {
     uint8_t *base = nullptr;  // device allocation
     uint64_t alloc_bytes = 0;
     uint8_t *p0 = nullptr, *p1 = nullptr, *p2 = nullptr, *p3 = nullptr;  // planes
-    bool half = false;  // type F32 whose values lie in p0 as f16 (an F16 tensor that only FmtF16's kernels read)
+    bool half = false;  // type F32 whose values lie in p0 as f16 (an F16 tensor that only FmtF16's and FmtDenseMix' kernels read)
     // upper bound on |w| over the dequantized matrix (Q8_0 / Q4_K / Q6_K; inf for NaN / inf
     // scales): the batched products need it below kGemmMaxWeight
     float max_abs = 0.f;
@@ -243,7 +243,7 @@ constexpr uint32_t kFusedNeoxRows = 1u << 24;  // rows / 2 * head_size / 2 stays
 bool gemv_fused_supported(const wgml_qmat *m);
 bool gemv_keeps_f16(uint32_t ncols);  // F16 tensors of that width stay 16 bits wide (wgml_qmat::half)
 // the matrices can share one launch_gemv_fused (with the context's settings): one format, or a
-// mix of Q4_K / Q6_K / Q8_0
+// mix of Q4_K / Q6_K / Q8_0 or of F16 / F32
 bool gemv_fused_set_supported(const wgml_ctx *ctx, const wgml_qmat *const *mats, int n);
 // launch_gemv_quant takes GemvEpilogue::partials for this matrix (with the context's settings)
 bool gemv_partials_supported(const wgml_ctx *ctx, const wgml_qmat *m);
@@ -256,6 +256,7 @@ struct GemvKernels {
 };
 GemvKernels gemv_legacy_kernels(int fmt);  // gemv_legacy.hip: a 32-element format, or kLegacyWide + one
 GemvKernels gemv_f16_kernels();            // gemv_f16.hip: F16 tensors (wgml_qmat::half)
+GemvKernels gemv_dense_mix_kernels();      // gemv_f16.hip: F16 and F32 tensors together (fused launches only)
 // gemv_full.hip: with LayerNorm and activation (a format, kLegacyWide + one or kFusedDenseF32; no gated ones);
 // `rows` of a group of the plain kernel: 1, or 2 in Q8_0
 GemvKernels gemv_full_kernels(int fmt, bool f32, int rows);

@@ -526,23 +526,30 @@ bool gemv_fused_set_supported(const wgml_ctx *ctx, const wgml_qmat *const *mats,
     bool same = true, all_main = true;
     for (int i = 0; i < n; ++i) {
         if (!gemv_fused_supported(mats[i])) return false;
-        same = same && mats[i]->type == mats[0]->type && mats[i]->half == mats[0]->half;
+        same = same && mats[i]->type == mats[0]->type;
         all_main = all_main && main_format(mats[i]->type);
     }
     if (ctx->tuning[WGML_TUNE_GEMV_F32_ACTIVATIONS]) return all_main || (same && mats[0]->type == WGML_F32);
     return same || all_main;
 }
 
-// The format number of a fused launch's kernel: that of its matrices, or 0 for a mix of the main ones.
+// The format number of a fused launch's kernel: that of its matrices, kFusedDenseMix for F16 beside F32, or 0 for a mix of the
+// main ones.  (us per token of six layers with K and up in F32 and the rest in F16: a launch per operation, as any other mix takes, 187
+// for 640 columns and 225 for 1024; in one launch 119 and 150.)
 static int fused_format(const FusedGemv &f, uint32_t ncols) {
     const int type = f.jobs[0].a->type;
-    for (int i = 1; i < f.njobs; ++i)
+    bool mix = false;
+    for (int i = 0; i < f.njobs; ++i) {
         if (f.jobs[i].a->type != type) return 0;
+        mix = mix || f.jobs[i].a->half != f.jobs[0].a->half || (f.jobs[i].mode == FUSED_SILU && f.jobs[i].b->half != f.jobs[0].a->half);
+    }
+    if (mix) return kFusedDenseMix;
     return type == WGML_F32 ? dense_format(f.jobs[0].a) : legacy_format(type) ? legacy_kernel_format(type, ncols) : type;
 }
 static GemvKernels fused_kernels(int fmt, bool f32) {
     if (fmt == kFusedDenseF32) return dense_f32_kernels();
     if (fmt == kFusedDenseF16) return gemv_f16_kernels();
+    if (fmt == kFusedDenseMix) return gemv_dense_mix_kernels();
     if (f32) {
         switch (fmt) {
         case WGML_Q4_K: return gemv_kernels_of<WGML_Q4_K, true, false>();
@@ -578,10 +585,13 @@ static uint32_t fused_workgroups(const wgml_ctx *ctx, int per_cu, uint64_t bytes
     return bytes <= (uint64_t(64) << 20) ? cu : cu * (uint32_t)per_cu;
 }
 
+// Plane p1 as a kernel gets it: FmtDenseMix tells F32 tensors by their having none.
+static const uint8_t *plane1(const wgml_qmat *m) { return m->type == WGML_F32 && !m->half ? nullptr : m->p1; }
+
 static int launch_gated(wgml_ctx *ctx, const FusedGemv &f, const FusedGemvJob &s, uint32_t threads) {
     const uint32_t ncols = s.a->ncols;
     const bool f32 = ctx->tuning[WGML_TUNE_GEMV_F32_ACTIVATIONS] != 0;
-    if (!s.b || s.b->type != s.a->type || s.b->half != s.a->half || s.b->nrows != s.a->nrows || s.b->ncols != ncols || s.row0 || s.nrows)
+    if (!s.b || s.b->type != s.a->type || s.b->nrows != s.a->nrows || s.b->ncols != ncols || s.row0 || s.nrows)
         return set_error(WGML_E_INVALID, "gemv_fused: gate/up matrices differ");
     if (f.ln_gamma) return set_error(WGML_E_UNSUPPORTED, "gemv_fused: a gated job behind a LayerNorm");
     FusedGemv one = f;
@@ -592,12 +602,12 @@ static int launch_gated(wgml_ctx *ctx, const FusedGemv &f, const FusedGemvJob &s
     const size_t lds = lds_bytes_fused(s.a->type, ncols, f32);
     if (lds > kMaxLds)
         return set_error(WGML_E_UNSUPPORTED, "gemv_fused: %u columns need %zu bytes of LDS", ncols, lds);
-    GatedParams P{s.a->p0, s.a->p1, s.a->p2, s.a->p3, s.b->p0, s.b->p1, s.b->p2, s.b->p3, f.x, f.norm_w, s.out,
+    GatedParams P{s.a->p0, plane1(s.a), s.a->p2, s.a->p3, s.b->p0, plane1(s.b), s.b->p2, s.b->p3, f.x, f.norm_w, s.out,
                   f.norm_eps, s.a->nrows, ncols, 0};
     int per_cu = 1;
     WGML_TRY(blocks_per_cu(ctx, kern, (int)threads, lds, &per_cu));
     const uint32_t nwaves = threads / 64;
-    const WgPlan plan = plan_groups(P.nrows, fused_workgroups(ctx, per_cu, s.a->gguf_bytes * 2), nwaves, 32);
+    const WgPlan plan = plan_groups(P.nrows, fused_workgroups(ctx, per_cu, s.a->gguf_bytes + s.b->gguf_bytes), nwaves, 32);
     P.active_waves = plan.active_waves;
     void *args[] = {&P};
     WGML_CHECK_HIP(hipLaunchKernel(kern, dim3(plan.wgs), dim3(threads), args, lds, ctx->stream));
@@ -628,7 +638,7 @@ static int launch_jobs(wgml_ctx *ctx, const FusedGemv &f, uint32_t threads) {
     for (int i = 0; i < f.njobs; ++i) {
         const FusedGemvJob &s = f.jobs[i];
         GemvJob &j = P.jobs[i];
-        j.a0 = s.a->p0; j.a1 = s.a->p1; j.a2 = s.a->p2; j.a3 = s.a->p3;
+        j.a0 = s.a->p0; j.a1 = plane1(s.a); j.a2 = s.a->p2; j.a3 = s.a->p3;
         j.out = s.out;
         j.bias = s.bias;
         j.nrows = s.a->nrows;
@@ -669,10 +679,10 @@ static int launch_jobs(wgml_ctx *ctx, const FusedGemv &f, uint32_t threads) {
     const int fmt = fused_format(f, ncols);
     // (heads of two elements: both RoPE variants rotate the same pairs)
     const bool neox = f.rope_neox && P.head_size > 2;
-    const bool dense = fmt == kFusedDenseF32 || fmt == kFusedDenseF16;
+    const bool dense = fmt == kFusedDenseF32 || fmt == kFusedDenseF16 || fmt == kFusedDenseMix;
     if (neox && (f32 || dense))
         return set_error(WGML_E_UNSUPPORTED, "gemv_fused: Neox RoPE takes the integer-dot formats only");
-    if (P.ln_g && (neox || fmt == 0))
+    if (P.ln_g && (neox || fmt == 0 || fmt == kFusedDenseMix))
         return set_error(WGML_E_UNSUPPORTED, "gemv_fused: LayerNorm before Neox RoPE or mixed formats");
     const GemvKernels k = P.ln_g ? gemv_full_kernels(fmt, f32 || dense, 1) : fused_kernels(fmt, f32);
     const void *const kern = neox ? gemv_neox_kernel(fmt, (int)threads) : threads == 768 ? k.fused768 : k.fused1024;
@@ -735,7 +745,7 @@ int launch_gemv_fused(wgml_ctx *ctx, const FusedGemv &f) {
             return set_error(WGML_E_UNSUPPORTED, "gemv_fused: fp32 activations exist for Q4_K, Q6_K "
                                                  "and Q8_0 only");
         gated = gated || s.mode == FUSED_SILU;
-        mixed = mixed || s.a->type != f.jobs[0].a->type || s.a->half != f.jobs[0].a->half;
+        mixed = mixed || s.a->type != f.jobs[0].a->type;
         all_main = all_main && main_format(s.a->type);
         const uint32_t rows = s.nrows ? s.nrows : s.a->nrows - s.row0;
         pairs += s.mode == FUSED_SILU ? rows : (rows + 1) / 2;

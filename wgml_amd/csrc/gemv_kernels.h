@@ -530,6 +530,53 @@ struct FmtF16 {
     }
 };
 
+// F16 and F32 tensors in one launch (a file may mix them in a layer): plane pointer p1 is null for F32.  The values and order of the
+// other two, a matrix' rows as words of 16 bytes (F16: the second word again in place of the third and fourth).
+struct FmtDenseMix {
+    static constexpr int TILE = 16;
+    static constexpr int CHUNKS = 4;
+    static constexpr int NSUM = 0;
+    struct Row {
+        uint4 a[4];
+        bool half;
+    };
+    struct RowBase {
+        const uint4 *row;
+        bool half;
+    };
+    __device__ static RowBase row_base(const GemvParams &p, uint32_t row) {
+        const bool half = p.p1 != nullptr;
+        return {reinterpret_cast<const uint4 *>(p.p0) + (size_t)row * (p.ncols / (half ? 8 : 4)), half};
+    }
+    __device__ static void map(uint32_t g, uint32_t &tile, uint32_t &chunk) { FmtF32::map(g, tile, chunk); }
+    __device__ static void load(Row &w, const RowBase &rb, uint32_t tile) {
+        const uint32_t n = rb.half ? 2 : 4;
+        w.half = rb.half;
+#pragma unroll
+        for (uint32_t c = 0; c < 4; ++c) w.a[c] = rb.row[(size_t)tile * n + min(c, n - 1)];
+    }
+    template <int R>
+    __device__ static void accumulate(const Row (&w)[R], const float4 *xl, const float *, uint32_t,
+                                      float (&acc)[R]) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const float4 xv = xl[c * 64];
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const uint32_t bits[2] = {c & 1 ? w[r].a[c / 2].z : w[r].a[c / 2].x, c & 1 ? w[r].a[c / 2].w : w[r].a[c / 2].y};
+                _Float16 h[4];
+                __builtin_memcpy(h, bits, 8);
+                float v[4];
+                __builtin_memcpy(v, &w[r].a[c], 16);
+                acc[r] = fmaf(w[r].half ? (float)h[0] : v[0], xv.x, acc[r]);
+                acc[r] = fmaf(w[r].half ? (float)h[1] : v[1], xv.y, acc[r]);
+                acc[r] = fmaf(w[r].half ? (float)h[2] : v[2], xv.z, acc[r]);
+                acc[r] = fmaf(w[r].half ? (float)h[3] : v[3], xv.w, acc[r]);
+            }
+        }
+    }
+};
+
 // LDS layout: x as float4 xs[step][chunk][lane]; then sums[sum][tile_padded].
 template <class F>
 __device__ __forceinline__ uint32_t lds_slot(uint32_t tile, uint32_t chunk) {
@@ -1630,9 +1677,10 @@ template <> struct FusedFmt<WGML_Q4_K, true> { using T = FFmt<FmtQ4K>; };
 template <> struct FusedFmt<WGML_Q6_K, true> { using T = FFmt<FmtQ6K>; };
 template <> struct FusedFmt<WGML_Q8_0, true> { using T = FFmt<FmtQ8_0>; };
 // (WGML_F32 is 0, which as FMT stands for mixed formats)
-constexpr int kFusedDenseF32 = 1000, kFusedDenseF16 = 1001;
+constexpr int kFusedDenseF32 = 1000, kFusedDenseF16 = 1001, kFusedDenseMix = 1002;
 template <> struct FusedFmt<kFusedDenseF32, true> { using T = FFmt<FmtF32>; };
 template <> struct FusedFmt<kFusedDenseF16, true> { using T = FFmt<FmtF16>; };
+template <> struct FusedFmt<kFusedDenseMix, true> { using T = FFmt<FmtDenseMix>; };
 // A format number for kernels whose tiles are two blocks of a 32-element format.
 constexpr int kLegacyWide = 2000;
 template <> struct FusedFmt<WGML_Q5_K, false> { using T = IFmtQ5K; };
