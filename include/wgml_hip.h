@@ -150,7 +150,8 @@ WGML_API int wgml_quant_matrix_create(wgml_ctx *ctx, int type, uint32_t nrows, u
 WGML_API int wgml_quant_matrix_destroy(wgml_qmat *m);
 WGML_API int wgml_quant_matrix_shape(const wgml_qmat *m, int *type, uint32_t *nrows,
                                      uint32_t *ncols); /* GpuQuantMatrix::shape */
-/* Size of the tensor in GGUF bytes (the algorithmic weight traffic of one GEMV). */
+/* Size of the tensor in GGUF bytes (the algorithmic weight traffic of one GEMV); of a WGML_F16 matrix that was expanded,
+ * that of its f32 values. */
 WGML_API uint64_t wgml_quant_matrix_gguf_bytes(const wgml_qmat *m);
 /* An upper bound on the magnitude of the matrix's dequantized weights, computed on the device
  * when the matrix is created (Q8_0 / Q4_K / Q6_K; 0 for other formats; infinity when a block

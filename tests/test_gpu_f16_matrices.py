@@ -24,7 +24,8 @@ def halves(rng, n):
 
 def product(gpu, qtype, data, rows, cols, x):
     m = W.GpuQuantMatrix(gpu, qtype, rows, cols, data.view(np.uint8).reshape(-1))
-    assert m.shape() == (W.F32, rows, cols) and m.gguf_bytes() == 4 * rows * cols
+    kept = qtype == W.F16 and 512 < cols <= 32768 and cols % 16 == 0
+    assert m.shape() == (W.F32, rows, cols) and m.gguf_bytes() == (2 if kept else 4) * rows * cols
     out = W.GpuVector.uninit(gpu, rows)
     W.GemvQuant.from_device(gpu).dispatch(out, m, W.GpuVector.init(gpu, x))
     return out.read(), m

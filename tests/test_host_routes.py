@@ -241,3 +241,12 @@ def test_f16_beside_f32_takes_no_more_launches(runtime):
     for f16 in (("attn_q",), ("ffn_up",), ("attn_k", "ffn_gate"), ("attn_q", "attn_k", "ffn_gate", "ffn_up")):
         assert len(launches(f16)) == len(plain), f16
     """)
+
+
+def test_bytes_of_f16_matrices(runtime):
+    # what a product streams; the rule that shares fused launches out goes by it (64 MB: one workgroup per compute unit)
+    host_hip.run(runtime, """
+    for qtype, cols, per in ((W.F16, 768, 2), (W.F16, 32768, 2), (W.F16, 512, 4), (W.F16, 772, 4), (W.F16, 32784, 4), (W.F32, 768, 4)):
+        m = W.GpuQuantMatrix(gpu, qtype, 5, cols, np.zeros((2 if qtype == W.F16 else 4) * 5 * cols, np.uint8))
+        assert m.gguf_bytes() == per * 5 * cols and m.shape() == (W.F32, 5, cols), (qtype, cols)
+    """)

@@ -579,7 +579,7 @@ static GemvKernels fused_kernels(int fmt, bool f32) {
 // more than 64 MB.  A second workgroup on a compute unit stages x again, and the waves' row pairs are fewer and less even.  us
 // per launch, as many as fit (two of 64 registers) / one per compute unit: gate and up 8192x3072 in Q4_0 9.2 / 7.8, Q4_1 9.7 / 8.2,
 // Q8_0 (53 MB) 11.8 / 11.6, 9216x3072 rows in pairs in Q8_0 9.2 / 8.8, 2304x768 3.8 / 3.4; gate and up 11008x4096 in Q8_0 (96 MB)
-// 19.0 / 19.5.
+// 19.0 / 19.5; F16 2304x4096 9.4 / 8.8, 5120x3072 (63 MB) 12.8 / 12.4, rows in pairs 9216x3072 12.2 / 11.6, 5120x4096 9.95 / 10.1.
 static uint32_t fused_workgroups(const wgml_ctx *ctx, int per_cu, uint64_t bytes) {
     const uint32_t cu = ctx->n_cu > 0 ? (uint32_t)ctx->n_cu : 256u;
     return bytes <= (uint64_t(64) << 20) ? cu : cu * (uint32_t)per_cu;

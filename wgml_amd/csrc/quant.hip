@@ -369,8 +369,7 @@ int wgml_quant_matrix_create(wgml_ctx *ctx, int type, uint32_t nrows, uint32_t n
     if (!be)
         return set_error(WGML_E_UNSUPPORTED,
                          "wgml_quant_matrix_create: quantization type %d is not supported "
-                         "(F32, Q8_0, Q4_0, Q4_1, Q5_0, Q5_1, Q4_K, Q5_K, Q6_K, Q8_K; F16 is "
-                         "expanded to f32)",
+                         "(F32, F16, Q8_0, Q4_0, Q4_1, Q5_0, Q5_1, Q4_K, Q5_K, Q6_K, Q8_K)",
                          type);
     WGML_REQUIRE(nrows > 0 && ncols > 0, "wgml_quant_matrix_create: empty matrix %ux%u", nrows,
                  ncols);
@@ -393,7 +392,7 @@ int wgml_quant_matrix_create(wgml_ctx *ctx, int type, uint32_t nrows, uint32_t n
     m->half = half;
     m->nrows = nrows;
     m->ncols = ncols;
-    m->gguf_bytes = f32 ? nelem * 4 : gguf;
+    m->gguf_bytes = expand ? nelem * 4 : gguf;
 
     const bool has_m = type == WGML_Q4_1 || type == WGML_Q5_1, has_qh = type == WGML_Q5_0 || type == WGML_Q5_1;
     const bool legacy = has_m || has_qh || type == WGML_Q4_0;
@@ -449,7 +448,6 @@ int wgml_quant_matrix_create(wgml_ctx *ctx, int type, uint32_t nrows, uint32_t n
     const uint64_t end = type == WGML_Q8_0 ? o1 + nblocks * 2
                          : type == WGML_Q6_K ? o3 + nblocks * 2
                          : legacy            ? o1 + nblocks * (has_m ? 4 : 2)
-                         : half              ? gguf
                                              : m->gguf_bytes;
     e = hipMemsetAsync(m->base + end, 0, total - end, ctx->stream);
     if (e != hipSuccess) return fail(e, "spare bytes");
