@@ -14,7 +14,7 @@ static const char *launches[MAX_LAUNCHES];
 static dim3 grids[MAX_LAUNCHES];
 static int n_launches;
 static struct { void *p; size_t bytes; } blocks[MAX_BLOCKS];
-static int n_blocks, n_pinned;
+static int n_blocks, n_pinned, blocks_per_cu = 1;
 static size_t allocated, malloc_limit = (size_t)-1;
 static char failing[64];
 static hipError_t last_error;
@@ -27,6 +27,7 @@ void host_hip_clear(void) { n_launches = 0; }
 int host_hip_launches(void) { return n_launches; }
 const char *host_hip_launch(int i) { return launches[i]; }
 unsigned host_hip_workgroups(int i) { return grids[i].x * grids[i].y * grids[i].z; }
+void host_hip_blocks_per_cu(int n) { blocks_per_cu = n; } /* of every kernel; asked for once per kernel and size of LDS */
 size_t host_hip_allocated(void) { return allocated; }
 int host_hip_pinned(void) { return n_pinned; } /* requests for pinned memory so far */
 
@@ -73,7 +74,7 @@ hipError_t hipLaunchKernel(const void *fn, dim3 grid, dim3 block, void **args, s
 hipError_t hipFuncSetAttribute(const void *f, hipFuncAttribute a, int v) { (void)f; (void)a; (void)v; return hipSuccess; }
 hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int *n, const void *f, int threads, size_t lds) {
     (void)f; (void)threads; (void)lds;
-    *n = 1;
+    *n = blocks_per_cu;
     return hipSuccess;
 }
 hipError_t hipGetLastError(void) { hipError_t e = last_error; last_error = hipSuccess; return e; }

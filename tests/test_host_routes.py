@@ -250,3 +250,23 @@ def test_bytes_of_f16_matrices(runtime):
         m = W.GpuQuantMatrix(gpu, qtype, 5, cols, np.zeros((2 if qtype == W.F16 else 4) * 5 * cols, np.uint8))
         assert m.gguf_bytes() == per * 5 * cols and m.shape() == (W.F32, 5, cols), (qtype, cols)
     """)
+
+
+def test_workgroups_of_products_with_fp32_activations(runtime):
+    host_hip.run(runtime, """
+    fake.host_hip_blocks_per_cu(2)
+    def grid(qtype, nrows, ncols):
+        m = W.GpuQuantMatrix(gpu, qtype, nrows, ncols, np.zeros(4 * nrows * ncols if qtype == W.F32 else W.quant_bytes(qtype, nrows * ncols), np.uint8))
+        out, x = W.GpuVector.uninit(gpu, nrows), W.GpuVector.uninit(gpu, ncols)
+        return workgroups(lambda: W.GemvQuant(gpu).dispatch(out, m, x))
+
+    for shape in ((6000, 1024), (10239, 1024), (20000, 528), (20000, 1040), (6000, 2048)):
+        assert grid(W.F32, *shape)[0] <= 256, shape
+    for shape in ((10240, 1024), (20000, 896), (12000, 1808), (12000, 2048)):
+        assert grid(W.F32, *shape)[0] > 256, shape
+    gpu.set_tuning(gpu.TUNE_GEMV_F32_ACTIVATIONS, 1)
+    for shape in ((6144, 1024), (5000, 4096), (10239, 256), (20000, 4096)):
+        assert grid(W.Q6_K, *shape)[0] <= 256, shape
+    for shape in ((10240, 256), (20000, 2048)):
+        assert grid(W.Q6_K, *shape)[0] > 256, shape
+    """)

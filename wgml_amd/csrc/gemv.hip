@@ -142,10 +142,12 @@ size_t lds_bytes_of(uint32_t ncols) {
 }
 // `fn`: a gemv_quant_i8_kernel with R rows per group and workgroups of `maxt` threads.
 // `n_maxima`: fn leaves maxima (EXTRA_MAXIMA); receives how many, 0 (and none are left) if they are more than kMaxRowMaxima.
+// `cap`: workgroups per compute unit at most.
 int launch_plain(wgml_ctx *ctx, const void *fn, uint32_t R, uint32_t maxt, GemvParams p, size_t lds,
-                 uint32_t *n_maxima = nullptr) {
+                 uint32_t *n_maxima = nullptr, int cap = 8) {
     int per_cu = 1;
     WGML_TRY(blocks_per_cu(ctx, fn, (int)maxt, lds, &per_cu));
+    if (per_cu > cap) per_cu = cap;
     const uint32_t cu = ctx->n_cu > 0 ? (uint32_t)ctx->n_cu : 256u;
     // One workgroup per CU with all its waves at work rather than two half-empty ones
     // (each would stage x), as long as that still gives every CU a workgroup (min_c).
@@ -168,8 +170,21 @@ int launch_plain(wgml_ctx *ctx, const void *fn, uint32_t R, uint32_t maxt, GemvP
 }
 
 template <class F, int R, int D, int MAXT, int MINW = MAXT / 256, bool XPART = false>
-int launch_variant_i8(wgml_ctx *ctx, const GemvParams &p, size_t lds) {
-    return launch_plain(ctx, (const void *)gemv_quant_i8_kernel<F, R, D, MAXT, MINW, XPART>, R, MAXT, p, lds);
+int launch_variant_i8(wgml_ctx *ctx, const GemvParams &p, size_t lds, int cap = 8) {
+    return launch_plain(ctx, (const void *)gemv_quant_i8_kernel<F, R, D, MAXT, MINW, XPART>, R, MAXT, p, lds, nullptr, cap);
+}
+
+// Workgroups per compute unit, at most, of a plain product with fp32 activations.  Two share the loads of a tall matrix better as long
+// as its rows fill the lanes of their steps (f32: 1024 columns a step); below 40 rows per compute unit the second ones are too few to
+// come out even.  us, two / one: f32 50257x272 14.4 / 13.3, x512 19.0 / 17.6, x768 26.5 / 25.6, x896 30.5 / 30.7, x1008 35.2 / 36.4,
+// x1280 44.3 / 42.2, x2048 70.1 / 71.5; 16384x1024 12.7 / 13.0, 8200x1024 7.9 / 7.7, 6000x2048 11.8 / 10.2; Q6_K 50257x768 22.5 / 23.8,
+// 32000x2048 14.9 / 16.5, x4096 21.1 / 20.6, 11008x4096 9.4 / 9.2, 8192x3072 6.8 / 6.7, 6144x1024 5.9 / 5.3, 5000x4096 6.9 / 6.1.
+template <class WF>
+int f32_wgs_per_cu(const wgml_ctx *ctx, const GemvParams &p) {
+    const uint32_t cu = ctx->n_cu > 0 ? (uint32_t)ctx->n_cu : 256u, steps = (p.ncols + 1023) / 1024;
+    if (std::is_same_v<WF, FmtF32>) return p.nrows >= 40 * cu && p.ncols >= steps * 896 ? 2 : 1;
+    if (std::is_same_v<WF, FmtQ6K>) return p.nrows >= 40 * cu && p.ncols <= 2048 ? 2 : 1;
+    return 8;
 }
 
 bool legacy_format(int type) {
@@ -262,8 +277,7 @@ int launch_fmt_i8(wgml_ctx *ctx, const GemvParams &p) {
     }
 }
 
-// fp32-activation path: the same body with x staged as floats.  16-wave workgroups, one per
-// compute unit (the expansion needs the registers), or 8-wave workgroups with two tiles in flight
+// fp32-activation path: the same body with x staged as floats.  16-wave workgroups, or 8-wave workgroups with two tiles in flight
 // per wave when WGML_TUNE_GEMV_WAVES_PER_WG is 8.
 template <class WF>
 int launch_fmt_f32(wgml_ctx *ctx, const GemvParams &p) {
@@ -283,7 +297,7 @@ int launch_fmt_f32(wgml_ctx *ctx, const GemvParams &p) {
     if constexpr (!std::is_same_v<WF, FmtF32>) {
         if (waves == 8) return launch_variant_i8<F, 1, 2, 512, 2>(ctx, p, lds);
     }
-    return launch_variant_i8<F, 1, 1, 1024, 4>(ctx, p, lds);
+    return launch_variant_i8<F, 1, 1, 1024, 4>(ctx, p, lds, f32_wgs_per_cu<WF>(ctx, p));
 }
 
 }  // namespace
@@ -470,8 +484,12 @@ int launch_gemv_quant(wgml_ctx *ctx, float *out, const wgml_qmat *m, const float
     if (ep.n_maxima) {
         uint32_t rows = 1;
         size_t lds = 0;
-        if (const void *fn = maxima_kernel_for(ctx, m, p, &rows, &lds))
-            return launch_plain(ctx, fn, rows, 1024, p, lds, ep.n_maxima);
+        if (const void *fn = maxima_kernel_for(ctx, m, p, &rows, &lds)) {
+            const int cap = m->type == WGML_F32 && !m->half                                          ? f32_wgs_per_cu<FmtF32>(ctx, p)
+                            : m->type == WGML_Q6_K && ctx->tuning[WGML_TUNE_GEMV_F32_ACTIVATIONS] ? f32_wgs_per_cu<FmtQ6K>(ctx, p)
+                                                                                                  : 8;
+            return launch_plain(ctx, fn, rows, 1024, p, lds, ep.n_maxima, cap);
+        }
     }
     if (m->half) return launch_plain(ctx, gemv_f16_kernels().plain, 1, 1024, p, lds_bytes_of<FFmt<FmtF16>>(p.ncols));
     if (dense_f32_in_shared_body(m) && !dense_f32_general_faster(ctx, p.nrows, p.ncols, p.norm_w != nullptr))
