@@ -270,3 +270,17 @@ def test_workgroups_of_products_with_fp32_activations(runtime):
     for shape in ((10240, 256), (20000, 2048)):
         assert grid(W.Q6_K, *shape)[0] > 256, shape
     """)
+
+
+def test_workgroups_of_large_q5_1_matrices(runtime):
+    host_hip.run(runtime, """
+    fake.host_hip_blocks_per_cu(2)
+    def grid(qtype, nrows, ncols):
+        m = W.GpuQuantMatrix(gpu, qtype, nrows, ncols, np.zeros(W.quant_bytes(qtype, nrows * ncols), np.uint8))
+        out, x = W.GpuVector.uninit(gpu, nrows), W.GpuVector.uninit(gpu, ncols)
+        return workgroups(lambda: W.GemvQuant(gpu).dispatch(out, m, x))[0]
+
+    for ncols, limit in ((8192, 43690), (2048, 174762), (3072, 116508)):  # rows of 256 MB
+        assert grid(W.Q5_1, limit, ncols) > 256 and grid(W.Q5_1, limit + 1, ncols) == 256, ncols
+    assert grid(W.Q5_1, 200000, 2112) > 256 and grid(W.Q5_0, 45000, 8192) > 256  # lanes without a tile; another format
+    """, timeout=300)

@@ -199,6 +199,16 @@ int legacy_kernel_format(int type, uint32_t ncols) {
     return ncols > 2048 && ncols % 64 == 0 ? kLegacyWide + type : type;
 }
 
+// Workgroups per compute unit, at most.  Q5_1 matrices of more than 256 MB whose rows fill the lanes are faster with one (the file's
+// blocks, of 24 bytes, streamed better than three planes do).  us, blocks as in the file / planes, two workgroups / one: 128256x4096 68.2 /
+// 69.3 / 67.2, 64000x8192 68.1 / 71.6 / 70.0, 256000x2048 64.4 / 67.9 / 66.4, 151936x3584 75.6 / 72.8 / 70.6; 64000x4096 36.3 / 34.6 / 35.2,
+// 128256x5120 92.9 / 92.3 / 94.1.
+int legacy_wgs_per_cu(int type, const GemvParams &p) {
+    if (type != WGML_Q5_1 || (uint64_t)p.nrows * (p.ncols / 32) * 24 <= (uint64_t(256) << 20)) return 8;
+    const uint32_t tiles = p.ncols / (legacy_kernel_format(type, p.ncols) == type ? 32 : 64), steps = (tiles + 63) / 64;
+    return tiles >= steps * 48 ? 1 : 8;
+}
+
 size_t lds_bytes_legacy(int type, uint32_t ncols) {
     return legacy_kernel_format(type, ncols) == type ? lds_bytes_of<IFmtLegacy<false, false, 1>>(ncols)
                                                      : lds_bytes_of<IFmtLegacy<false, false, 2>>(ncols);
@@ -210,7 +220,8 @@ int launch_legacy(wgml_ctx *ctx, int type, const GemvParams &p) {
     if (lds > kMaxLds)
         return set_error(WGML_E_UNSUPPORTED, "gemv_quant: %u columns need %zu bytes of LDS (limit %zu)", p.ncols, lds,
                          kMaxLds);
-    return launch_plain(ctx, gemv_legacy_kernels(legacy_kernel_format(type, p.ncols)).plain, 1, 1024, p, lds);
+    return launch_plain(ctx, gemv_legacy_kernels(legacy_kernel_format(type, p.ncols)).plain, 1, 1024, p, lds, nullptr,
+                        legacy_wgs_per_cu(type, p));
 }
 
 template <class F, int R, int D>
@@ -487,7 +498,7 @@ int launch_gemv_quant(wgml_ctx *ctx, float *out, const wgml_qmat *m, const float
         if (const void *fn = maxima_kernel_for(ctx, m, p, &rows, &lds)) {
             const int cap = m->type == WGML_F32 && !m->half                                          ? f32_wgs_per_cu<FmtF32>(ctx, p)
                             : m->type == WGML_Q6_K && ctx->tuning[WGML_TUNE_GEMV_F32_ACTIVATIONS] ? f32_wgs_per_cu<FmtQ6K>(ctx, p)
-                                                                                                  : 8;
+                                                                                                  : legacy_wgs_per_cu(m->type, p);
             return launch_plain(ctx, fn, rows, 1024, p, lds, ep.n_maxima, cap);
         }
     }
