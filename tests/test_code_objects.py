@@ -50,3 +50,12 @@ def test_batched_products_keep_everything_in_registers(all_kernels):
     assert len(gemm) == 9 * 2 * 7  # formats, precisions, 16 .. 128 tokens and long runs
     for name, k in gemm.items():
         assert k[".vgpr_spill_count"] == 0 and k[".private_segment_fixed_size"] == 0, name
+
+
+def test_default_matrix_vector_products_keep_everything_in_registers(all_kernels):
+    # (the launch-shape overrides reach the others: two rows per wave or a second tile in flight in Q4_K and Q6_K)
+    gemv = {n: k for n, k in all_kernels.items() if "gemv_" in n}
+    assert len(gemv) > 150
+    spilled = [n for n, k in gemv.items() if k[".vgpr_spill_count"] or k[".private_segment_fixed_size"]]
+    for name in spilled:
+        assert re.search(r"gemv_quant_i8_kernelINS_7IFmtQ[46]KELi(1ELi[234]|2ELi2)ELi1024E", name), name

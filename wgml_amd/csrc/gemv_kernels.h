@@ -1131,20 +1131,25 @@ __device__ __forceinline__ void gemv_i8_body(const GemvParams &p, Policy &pol, u
     float4 xv[XP], nv[XP], bv[XP];
     const float4 *gsrc = ln_g ? reinterpret_cast<const float4 *>(ln_g) : nw4;
     const float4 *bsrc = FULL ? reinterpret_cast<const float4 *>(p.ln_b) : nullptr;
-    float4 xrow[FULL ? LN_REGS : 1];
-    if constexpr (FULL) {
 #pragma unroll
-        for (int i = 0; i < LN_REGS; ++i) {
-            xrow[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (ln_row && stager && lane + 64 * i < n4) xrow[i] = x4[lane + 64 * i];
+    for (int i = 0; i < XP; ++i) {
+        xv[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+        nv[i] = make_float4(1.f, 1.f, 1.f, 1.f);
+        bv[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+    // such a row takes the places of the second and third float4, which nobody has then (sixteen registers of its own: 128 and a
+    // spill in the Q/K/V kernel of Q5_1)
+    auto row_part = [&](int i) -> float4 & { return i < 2 ? xv[1 + i] : nv[i - 1]; };
+    if constexpr (FULL) {
+        if (ln_row && stager) {
+#pragma unroll
+            for (int i = 0; i < LN_REGS; ++i)
+                row_part(i) = lane + 64 * i < n4 ? x4[lane + 64 * i] : make_float4(0.f, 0.f, 0.f, 0.f);
         }
     }
 #pragma unroll
     for (int i = 0; i < XP; ++i) {
         const uint32_t g4 = stager ? tid + i * sthreads : n4;
-        xv[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-        nv[i] = make_float4(1.f, 1.f, 1.f, 1.f);
-        bv[i] = make_float4(0.f, 0.f, 0.f, 0.f);
         if (g4 < n4) {
             if constexpr (!XPART) xv[i] = x4[g4];
             if (gsrc) nv[i] = gsrc[g4];
@@ -1181,14 +1186,18 @@ __device__ __forceinline__ void gemv_i8_body(const GemvParams &p, Policy &pol, u
         if constexpr (FULL) if (ln_row) {
             float s1 = 0.f;
 #pragma unroll
-            for (int i = 0; i < LN_REGS; ++i) s1 += (xrow[i].x + xrow[i].y) + (xrow[i].z + xrow[i].w);
+            for (int i = 0; i < LN_REGS; ++i) {
+                const float4 v = row_part(i);
+                s1 += (v.x + v.y) + (v.z + v.w);
+            }
             const float mean = wave_sum(s1) / (float)p.ncols;
             float s2 = 0.f;
 #pragma unroll
             for (int i = 0; i < LN_REGS; ++i) {
                 const bool there = lane + 64 * i < n4;
-                const float a = there ? xrow[i].x - mean : 0.f, b = there ? xrow[i].y - mean : 0.f,
-                            c = there ? xrow[i].z - mean : 0.f, d = there ? xrow[i].w - mean : 0.f;
+                const float4 v = row_part(i);
+                const float a = there ? v.x - mean : 0.f, b = there ? v.y - mean : 0.f, c = there ? v.z - mean : 0.f,
+                            d = there ? v.w - mean : 0.f;
                 s2 = fmaf(a, a, s2);
                 s2 = fmaf(b, b, s2);
                 s2 = fmaf(c, c, s2);
