@@ -86,8 +86,8 @@ WGML_API int wgml_ctx_stream(wgml_ctx *ctx, void **stream);
  * kernel variant; value 0 restores the heuristic.  The reference has compile-time constants in
  * this role (USE_OPTIMIZED, ops/gemv_quant.rs:15; USE_MATMUL_ATTN, models/llama2/transformer.rs:444).
  * Results stay within the documented tolerances for every setting.  Values outside a key's range
- * are refused.  A model re-records its decode step the next time it runs after a change (launch
- * sequences recorded under other settings are dropped). */
+ * are refused.  Rows, waves and depth do not reach products with a folded LayerNorm or activation (GPT-2's).  A model
+ * re-records its decode step the next time it runs after a change (launch sequences recorded under other settings are dropped). */
 enum {
     WGML_TUNE_GEMV_ROWS_PER_WAVE = 0,        /* 1 or 2 rows of a quantized GEMV per wave and step */
     WGML_TUNE_GEMV_WAVES_PER_WG,             /* 4, 8 or 16; 12 for the multi-matrix launches only

@@ -284,3 +284,24 @@ def test_workgroups_of_large_q5_1_matrices(runtime):
         assert grid(W.Q5_1, limit, ncols) > 256 and grid(W.Q5_1, limit + 1, ncols) == 256, ncols
     assert grid(W.Q5_1, 200000, 2112) > 256 and grid(W.Q5_0, 45000, 8192) > 256  # lanes without a tile; another format
     """, timeout=300)
+
+
+def test_launch_shapes_do_not_bound_the_folded_layernorm(runtime):
+    # its kernels have workgroups of 1024 threads whatever the overrides say (they refused rows of more than 12 columns per thread
+    # of a smaller workgroup that never ran)
+    host_hip.run(runtime, """
+    n = 6400
+    p = Gpt2Params(n_vocab=64, n_seq=8, n_embd=n, n_head=50, n_layer=1, ff_len=64, attn_b=3 * n)
+    w = Gpt2HostWeights(params=p)
+    w.layers.append({"attn_w": zeros(W.Q8_0, 3 * n, n), "attn_proj_w": zeros(W.Q8_0, n, n), "mlp_fc_w": zeros(W.Q8_0, 64, n),
+                     "mlp_proj_w": zeros(W.Q8_0, n, 64)} | {k: np.zeros(c, np.float32) for k, c in
+                    dict(attn_b=3 * n, attn_proj_b=n, mlp_fc_b=64, mlp_proj_b=n, ln_1_g=n, ln_1_b=n, ln_2_g=n, ln_2_b=n).items()})
+    w.wte, w.wpe, w.lm_head = np.zeros((64, n), np.float32), np.zeros((8, n), np.float32), zeros(W.Q8_0, 64, n)
+    w.ln_f_g = w.ln_f_b = np.zeros(n, np.float32)
+    m = Gpt2(gpu, p).load(w)
+    plain = launched(lambda: m.forward(0, 0))
+    for waves in (4, 8, 16, 12):
+        gpu.set_tuning(gpu.TUNE_GEMV_WAVES_PER_WG, waves)
+        names = launched(lambda: m.forward(0, 0))
+        assert len(names) == len(plain) and names[-1] == plain[-1], waves
+    """)

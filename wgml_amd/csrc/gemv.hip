@@ -398,16 +398,16 @@ static size_t lds_bytes_fused(int type, uint32_t ncols, bool f32) {
 
 static bool main_format(int type) { return type == WGML_Q4_K || type == WGML_Q6_K || type == WGML_Q8_0; }
 
-// With LayerNorm or activation (gemv_full.hip): one variant per format, Q8_0 in one or two rows per wave.
+// With LayerNorm or activation (gemv_full.hip): one variant per format, Q8_0 in one or two rows per wave; the overrides of rows, waves and
+// depth do not reach these.  (Q8_0 rows of more than 8192 columns with four tiles in flight, as without LayerNorm: a GPT-2 of 8448 columns
+// with 50257 logits 264 us per token, with one tile 259.)
 static int launch_full(wgml_ctx *ctx, const wgml_qmat *m, const GemvParams &p, uint32_t *n_maxima) {
     if (m->type == WGML_F32 && !dense_f32_in_shared_body(m))
         return set_error(WGML_E_UNSUPPORTED, "gemv_quant: LayerNorm / activation folding needs rows of a "
                                              "multiple of 16 elements");
     if (p.part_n) return set_error(WGML_E_UNSUPPORTED, "gemv_quant: no merging kernel with an activation");
     const bool f32 = m->type == WGML_F32 || (main_format(m->type) && ctx->tuning[WGML_TUNE_GEMV_F32_ACTIVATIONS]);
-    const int waves = main_format(m->type) ? ctx->tuning[WGML_TUNE_GEMV_WAVES_PER_WG] : 0;
-    const uint32_t threads = waves == 8 ? 512u : waves && waves < 8 && !f32 ? 256u : 1024u;
-    if (p.ln_g && (p.ncols >> 2) > 3u * threads)  // XP float4 per thread
+    if (p.ln_g && (p.ncols >> 2) > 3u * 1024u)  // XP float4 per thread
         return set_error(WGML_E_UNSUPPORTED, "gemv_quant: %u columns are too many for the folded LayerNorm", p.ncols);
     const size_t lds = lds_bytes_fused(m->type, p.ncols, f32);
     if (lds > kMaxLds)
