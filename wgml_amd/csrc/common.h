@@ -332,9 +332,8 @@ struct NextEmbed {
 };
 // With n_maxima the arg-max is that of these maxima, which the product that wrote v has left; v is not read.
 int launch_argmax_next(wgml_ctx *ctx, const float *v, uint32_t n, DynState *dyn,
-                       const uint32_t *prompt, uint32_t *tokens_out,
-                       const NextEmbed *embed = nullptr, const RowMaximum *maxima = nullptr,
-                       uint32_t n_maxima = 0);
+                       const uint32_t *prompt, uint32_t *tokens_out, const NextEmbed &embed,
+                       const RowMaximum *maxima = nullptr, uint32_t n_maxima = 0);
 int launch_dequantize(wgml_ctx *ctx, float *out, const wgml_qmat *m);
 
 // ---- batched products for prompt processing (prefill.hip) ---------------------

@@ -390,7 +390,7 @@ int enqueue_loop_step(wgml_gpt2 *m, uint32_t plan) {
     uint32_t n_maxima = 0;
     WGML_TRY(enqueue_step(m, true, 0, 0, plan, false, &n_maxima));
     const NextEmbed ne{m->layer_input, m->wte, p.n_embd, nullptr, 2, 0.f, m->wpe, p.n_seq};
-    return launch_argmax_next(m->ctx, m->curr_vocab, p.n_vocab, m->dyn, m->d_prompt, m->d_tokens, &ne,
+    return launch_argmax_next(m->ctx, m->curr_vocab, p.n_vocab, m->dyn, m->d_prompt, m->d_tokens, ne,
                               m->maxima, n_maxima);
 }
 int loop_first_embed(wgml_gpt2 *m) {
@@ -620,7 +620,7 @@ int enqueue_prompt(wgml_gpt2 *m, uint32_t np, const DynState &at) {
     }
     WGML_CHECK_HIP(hipMemcpyAsync(m->dyn, &at, sizeof(at), hipMemcpyHostToDevice, ctx->stream));
     const NextEmbed ne{m->layer_input, m->wte, p.n_embd, nullptr, 2, 0.f, m->wpe, p.n_seq};
-    return launch_argmax_next(ctx, m->curr_vocab, p.n_vocab, m->dyn, m->d_prompt, m->d_tokens, &ne);
+    return launch_argmax_next(ctx, m->curr_vocab, p.n_vocab, m->dyn, m->d_prompt, m->d_tokens, ne);
 }
 
 }  // namespace

@@ -319,7 +319,7 @@ int enqueue_loop_step(wgml_llama2 *m, uint32_t plan) {
     uint32_t n_maxima = 0;
     WGML_TRY(enqueue_step(m, true, 0, 0, plan, false, &n_maxima));
     const NextEmbed ne{m->x, m->token_embd, c.dim, m->rope_cs, m->head_size, c.rope_base_freq, nullptr, 0};
-    return launch_argmax_next(m->ctx, m->logits, c.vocab_size, m->dyn, m->d_prompt, m->d_tokens, &ne,
+    return launch_argmax_next(m->ctx, m->logits, c.vocab_size, m->dyn, m->d_prompt, m->d_tokens, ne,
                               m->maxima, n_maxima);
 }
 int loop_first_embed(wgml_llama2 *m) {

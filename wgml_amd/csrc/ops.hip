@@ -278,26 +278,6 @@ __global__ __launch_bounds__(1024) void argmax_kernel(const float *__restrict__ 
     if (threadIdx.x == 0) out[blockIdx.x] = idx;
 }
 
-// Greedy sampling + the token loop's bookkeeping on the device
-// (ChatLlama2::forward / sample_next_token with temperature 0,
-// wgml-chat/src/chat_llama2.rs:51-153, wgml-chat/src/sampler.rs:91-111): records
-// the arg-max, picks the next input token (a forced prompt token wins over the
-// sample) and advances the position, so that the next step can be enqueued
-// without a host round trip.
-__global__ __launch_bounds__(1024) void argmax_next_kernel(const float *__restrict__ v, uint32_t n,
-                                                           DynState *dyn,
-                                                           const uint32_t *__restrict__ prompt,
-                                                           uint32_t *__restrict__ tokens_out) {
-    const uint32_t idx = block_argmax(v, n);
-    if (threadIdx.x == 0) {
-        const uint32_t pos = dyn->pos, cnt = dyn->count;
-        tokens_out[cnt] = idx;
-        dyn->token = (pos + 1 < dyn->n_prompt) ? prompt[pos + 1] : idx;
-        dyn->pos = pos + 1;
-        dyn->count = cnt + 1;
-    }
-}
-
 // What embed_kernel does for a token and position that this launch has chosen (the same expressions, so the same bits).
 __device__ __forceinline__ void next_rope(const NextEmbed &e, uint32_t pos, uint32_t i) {
     const float head_dim = (float)(2 * i);
@@ -314,7 +294,13 @@ __device__ __forceinline__ void next_row(const NextEmbed &e, uint32_t tok, uint3
     }
 }
 
-// argmax_next_kernel followed, in the same launch, by the embedding of the token just chosen: the next step of the loop
+// Greedy sampling + the token loop's bookkeeping on the device
+// (ChatLlama2::forward / sample_next_token with temperature 0,
+// wgml-chat/src/chat_llama2.rs:51-153, wgml-chat/src/sampler.rs:91-111): records
+// the arg-max, picks the next input token (a forced prompt token wins over the
+// sample) and advances the position, so that the next step can be enqueued
+// without a host round trip.
+// It is followed, in the same launch, by the embedding of the token just chosen: the next step of the loop
 // needs no launch of its own for it.
 __global__ __launch_bounds__(1024) void argmax_next_embed_kernel(const float *__restrict__ v, uint32_t n,
                                                                  DynState *dyn,
@@ -516,20 +502,15 @@ int launch_embed(wgml_ctx *ctx, float *x, const float *table, uint32_t dim, DynP
 }
 
 int launch_argmax_next(wgml_ctx *ctx, const float *v, uint32_t n, DynState *dyn,
-                       const uint32_t *prompt, uint32_t *tokens_out, const NextEmbed *embed,
+                       const uint32_t *prompt, uint32_t *tokens_out, const NextEmbed &embed,
                        const RowMaximum *maxima, uint32_t n_maxima) {
-    if (embed) {
-        if (embed->rope_cs && embed->head_size / 2 > 1024)
-            return set_error(WGML_E_UNSUPPORTED, "argmax_next: head_size %u too large", embed->head_size);
-        if (n_maxima)
-            maxima_next_embed_kernel<<<dim3(1), dim3(1024), 0, ctx->stream>>>(maxima, n_maxima, dyn, prompt,
-                                                                             tokens_out, *embed);
-        else
-            argmax_next_embed_kernel<<<dim3(1), dim3(1024), 0, ctx->stream>>>(v, n, dyn, prompt, tokens_out,
-                                                                             *embed);
-    } else {
-        argmax_next_kernel<<<dim3(1), dim3(1024), 0, ctx->stream>>>(v, n, dyn, prompt, tokens_out);
-    }
+    if (embed.rope_cs && embed.head_size / 2 > 1024)
+        return set_error(WGML_E_UNSUPPORTED, "argmax_next: head_size %u too large", embed.head_size);
+    if (n_maxima)
+        maxima_next_embed_kernel<<<dim3(1), dim3(1024), 0, ctx->stream>>>(maxima, n_maxima, dyn, prompt,
+                                                                         tokens_out, embed);
+    else
+        argmax_next_embed_kernel<<<dim3(1), dim3(1024), 0, ctx->stream>>>(v, n, dyn, prompt, tokens_out, embed);
     WGML_CHECK_LAUNCH();
     ctx->launches++;
     return WGML_OK;
