@@ -1,6 +1,6 @@
 """GPU: the arg-max of a token loop taken from the maxima that the output product's waves leave, against the arg-max kernel over the
 logits (decode_greedy_sync: a launch of its own, a read-back per token): every format and both activations, fewer rows than waves,
-one row and several per wave, rows in pairs (Q8_0, 16384 rows and up to 1024 columns), more rows than kMaxRowMaxima row groups hold;
+one row and several per wave, rows in pairs (Q8_0, 16384 rows and up to 1024 columns), as many waves as there is room for maxima and more;
 then ties, infinities and NaN, where the first largest logit counts and only a NaN in row 0 does.  Tokens are equal."""
 import numpy as np
 import pytest
@@ -63,8 +63,17 @@ def test_fp32_activations(gpu, qtype):
 
 
 def test_tall(gpu):
-    """More results than the waves of one round of workgroups park: 300001 rows."""
+    """Many results per wave: 300001 rows, at most 8192 waves."""
     same_tokens(model(gpu, W.Q8_0, 300001, 256), 7)
+
+
+@pytest.mark.parametrize("vocab", [1048576, 1048578])
+def test_more_waves_than_room_for_maxima(gpu, vocab):
+    """A wave parks 64 results: from 1048577 rows on there are more waves than kMaxRowMaxima, and the arg-max is that of the logits
+    (test_host_routes.py sees the kernels)."""
+    weights = np.resize(np.random.default_rng(1).standard_normal((50021, 64)).astype(np.float32), (vocab, 64))  # ties between waves
+    weights[vocab - 3] = 1.5 * weights[17]
+    same_tokens(model(gpu, W.Q8_0, vocab, 64, weights), 7, steps=4)
 
 
 @pytest.mark.parametrize("qtype", [W.F32, W.F16])

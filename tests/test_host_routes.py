@@ -305,3 +305,15 @@ def test_launch_shapes_do_not_bound_the_folded_layernorm(runtime):
         names = launched(lambda: m.forward(0, 0))
         assert len(names) == len(plain) and names[-1] == plain[-1], waves
     """)
+
+
+def test_maxima_of_more_waves_than_there_is_room_for(runtime):
+    # a wave parks 64 results: 1048576 rows are 16384 waves
+    host_hip.run(runtime, """
+    def arg_max(vocab):
+        names = launched(lambda: llama(gpu, Llama2Config(64, 64, 1, 1, 1, vocab, 16)).decode_greedy(1, 0, 1))
+        return [n for n in names if "next_embed" in n][0]
+
+    assert "maxima_next_embed" in arg_max(331) and "maxima_next_embed" in arg_max(1048576)
+    assert "argmax_next_embed" in arg_max(1048578)
+    """)
