@@ -1,4 +1,4 @@
-"""Dense f32 matrices (F32 tensors, F16 ones expanded at creation): rows of a multiple of 16 columns
+"""Dense f32 matrices (F32 tensors, and F16 ones, expanded at creation up to 512 columns and of the same bits beyond): rows of a multiple of 16 columns
 in the shared GEMV body, other widths and most narrow matrices on the general kernel
 (test_host_routes.py has the line).  Against float64."""
 import numpy as np

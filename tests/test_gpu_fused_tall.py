@@ -2,8 +2,9 @@
 gate/up pairs and row pairs (rotated at position 0, which changes nothing, and plain), more rows than one round of workgroups parks,
 and a gated job beside a plain one.
 
-Bound: activations are 16-bit block fixed point (2^-16 of a block's largest value) in the quantized formats and fp32 in the dense ones;
-2e-4 of the largest result is what the other tests of these kernels allow."""
+Bound: the quantized formats take activations as 16-bit block fixed point, in steps of 2^-15 of a block's largest value, which is 2 to 3
+standard deviations: an error of 2e-5 of a result's, at random.  Gating multiplies two such results.  2e-4 of the largest result is
+ten times that (the dense formats' fp32 sums are far below)."""
 import numpy as np
 import pytest
 

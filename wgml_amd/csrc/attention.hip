@@ -371,9 +371,9 @@ __global__ __launch_bounds__(NW * 64) void attn_fast_kernel(const AttnArgs a) {
     const uint32_t cs = min(slice0 + min(sub, a.slice_f4 - 1), hs / 4 - 1);
 
     // This wave's quads are gid, gid + total, ...  The first is requested before the position is known where it lies inside
-    // the caches whatever the position is (`spec_rows` rows may be read; those beyond the position are masked out below: a
-    // recorded step is planned for a range of positions whose lower end lies beyond what the first quads of all waves cover, so
-    // nothing is read in vain).
+    // the caches whatever the position is (`spec_rows` rows may be read; those beyond the position are masked out below, so a step at
+    // one of the first 63 positions reads up to 64 rows; the later ranges that a recorded step is planned for begin beyond what the
+    // first quads of all waves cover).
     float4 k4[NV4], v4[NVV];
 #pragma unroll
     for (int v = 0; v < NV4; ++v) k4[v] = zero4;
@@ -684,8 +684,7 @@ static int make_fast_plan(wgml_ctx *ctx, const wgml_attn_params &p, uint32_t pla
     // short contexts of a folded plan: up to one workgroup per CU
     if (folded && plan_positions <= kWidePositions) {
         max_y = (cu + pl.groups - 1) / pl.groups;
-        // four quads per wave: both register sets, all of them requested before the position
-        // is known; and few partial results, which every workgroup of the consumer merges
+        // four quads per wave, and few partial results, which every workgroup of the consumer merges
         const uint32_t enough = (plan_positions + 16 * WAVES - 1) / (16 * WAVES);
         if (max_y > enough) max_y = enough;
         if (max_y > kMaxFoldedPartials) max_y = kMaxFoldedPartials;

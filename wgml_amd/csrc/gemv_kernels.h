@@ -445,12 +445,12 @@ struct FmtQ5K {
 };
 
 // ------------------------------------------------------------- dense f32 ----
-// Rows of a multiple of 16 floats (F32 tensors, and F16 ones, which are expanded when the matrix
-// is created).  A tile is 16 elements, 64 bytes: a wave's step covers 1024 columns and asks for
+// Rows of a multiple of 16 floats (F32 tensors, and F16 ones that are expanded when the matrix
+// is created, see gemv_keeps_f16).  A tile is 16 elements, 64 bytes: a wave's step covers 1024 columns and asks for
 // 4 KB, as the quantized formats do.  No sums of x are needed.  HBM-bound where tall (GPT-2's
 // 50257x768 output projection), launch-bound elsewhere: what it brings is the folded norms,
-// epilogues and Q/K/V launch, and with them the recorded step -- GPT-2 124M from an F16 file
-// 331 us per token, 625 with a launch per operation and gemv_f32_kernel.
+// epilogues and Q/K/V launch, and with them the recorded step -- GPT-2 124M with its matrices in f32
+// 283 us per token, 625 with a launch per operation and gemv_f32_kernel.
 struct FmtF32 {
     static constexpr int TILE = 16;
     static constexpr int CHUNKS = 4;
